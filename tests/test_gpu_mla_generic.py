@@ -100,6 +100,27 @@ def test_weight_forms_at_the_usual_widths(bits, group, scale_dtype, heads, lens)
     print(what, assert_attention_close(got.reshape(want.shape), want, what))
 
 
+@pytest.mark.parametrize("bits,group,scale_dtype,nope,value,heads,lens,rows", [
+    (8, 128, O.SCALE_BF16, 128, 128, 128, [300], 5),     # 640 (row, head) pairs: absorb on the matrix cores, part of a block of sixteen rows
+    (8, 64, O.SCALE_F16, 128, 128, 64, [90, 700], 17),   # one row past a block; scales that need three query terms
+    (4, 32, O.SCALE_BF16, 128, 128, 48, [200], 130),     # workgroups of sixteen waves, the smallest scale group
+    (8, 512, O.SCALE_F32, 192, 256, 32, [150], 129),     # two column halves a head, one scale a row, sixteen value waves
+    (4, 128, O.SCALE_BF16, 192, 256, 64, [400, 100], 3), # few rows, wide values
+    (8, 128, O.SCALE_BF16, 96, 40, 20, [33], 2),         # widths without a matrix-core form, a partial block of value columns
+    (8, 256, O.SCALE_F16, 256, 130, 8, [5000], 1),       # the widest query and a wide split merge
+    (8, 16, O.SCALE_BF16, 128, 128, 16, [70], 4)])       # groups narrower than a matrix step: the vector kernels
+def test_weight_codes_at_the_edges_of_their_kernels(bits, group, scale_dtype, nope, value, heads, lens, rows):
+    """kv_b as codes over 512 + 64 columns: every kernel of the absorb and the projection at the sizes where it starts,
+    ends or fills a tile in part.  The codes are exact in the matrix cores and the query and merged rows carry 24 bits, so
+    the bound is that of the attention itself."""
+    case = make_mla_chunk_case(bits + group + heads, lens, rows, heads, nope=nope, value=value, block_tokens=16)
+    set_weight_form(case, bits, group=group, scale_dtype=scale_dtype)
+    want_f, _ = oracle_mla_chunk(case)
+    got = run_mla_chunk(case).cpu().numpy()
+    what = f"kv_b {bits}-bit group={group} nope={nope} value={value} heads={heads} rows={rows}"
+    print(what, assert_attention_close(got, want_f, what))
+
+
 def test_weight_forms_at_other_widths_and_chunks():
     case = make_mla_chunk_case(91, [200, 64], 5, 6, nope=64, rope=32, value=64, latent=256, block_tokens=16)
     set_weight_form(case, 8, group=64, scale_dtype=O.SCALE_BF16)

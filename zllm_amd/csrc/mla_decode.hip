@@ -52,6 +52,57 @@ union Frag {
     f16x8 h;
 };
 
+// kv_b as codes (W8A16 / W4A16): 32-bit words, codes low bits first, value (code - 128) or (code - 8) times the scale of
+// (row, column / group).  The codes are small integers, exact in bf16.
+template <int BITS> struct Bf16Codes {
+    unsigned int word[16 / BITS]; // one 32-bit word of codes as packed bf16 pairs: 2 registers of 8-bit codes, 4 of 4-bit ones
+};
+template <int BITS> __device__ __forceinline__ float code_value(unsigned int word, int i)
+{
+    if constexpr (BITS == 8) {
+        return (float)(signed char)((word ^ 0x80808080u) >> (8 * i));
+    } else {
+        return (float)((int)((word >> (4 * i)) & 15u) - 8);
+    }
+}
+template <int BITS> __device__ __forceinline__ Bf16Codes<BITS> codes_to_bf16(unsigned int word)
+{
+    Bf16Codes<BITS> out;
+#pragma unroll
+    for (int i = 0; i < 16 / BITS; ++i) {
+        out.word[i] = pack_bf16_trunc(code_value<BITS>(word, 2 * i), code_value<BITS>(word, 2 * i + 1));
+    }
+    return out;
+}
+// Scales to LDS as f32: entry i is the scale at index at(i) of the scale plane.  All of a thread's are requested before the
+// first is stored (N = the most a thread has), and the type is decided once, outside the loads.
+template <int N, class At> __device__ __forceinline__ void stage_scales(const MlaDecodeParams& p, float* to, unsigned int count, const At& at)
+{
+    const unsigned int threads = blockDim.x;
+    unsigned int bits[N];
+    if (p.kv_b_scale_dtype == 2) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const unsigned int i = threadIdx.x + threads * n;
+            bits[n] = i < count ? ((const unsigned int*)p.kv_b_scales)[at(i)] : 0u;
+        }
+    } else {
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const unsigned int i = threadIdx.x + threads * n;
+            bits[n] = i < count ? ((const unsigned short*)p.kv_b_scales)[at(i)] : 0u;
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        const unsigned int i = threadIdx.x + threads * n;
+        if (i < count) {
+            to[i] = p.kv_b_scale_dtype == 2 ? __uint_as_float(bits[n])
+                                            : (p.kv_b_scale_dtype == 1 ? f16_bits_to_f32((unsigned short)bits[n]) : __uint_as_float(bits[n] << 16));
+        }
+    }
+}
+
 // Chunk swizzle for the 64-bank LDS (256 B per cycle).  A tile row is 72 chunks of 16 B, i.e. 8 chunks past a
 // multiple of 256 B, so the row's parity already selects the upper or lower 128 B of a bank line; XOR-ing
 // row bits 1 and 2 into chunk bits 1 and 2 spreads eight rows over all sixteen 16-byte slots.  Measured with
@@ -232,12 +283,16 @@ template <int R> __global__ __launch_bounds__(256) void mla_absorb_rows(MlaDecod
 // waves take blocks of sixteen rows in turn, a wave (or the 2 to 16 waves that share a block) all 512 latent columns.
 // NOPE query columns and COLS latent columns a workgroup: 128 x 512, or 192 x 256 with the two column halves in
 // workgroups of their own (blockIdx.z), which is what fits the LDS.
-template <int WAVES, int NOPE, int COLS> __global__ __launch_bounds__(64 * WAVES) void mla_absorb_mfma(MlaDecodeParams p)
+//
+// BITS 8 / 4: kv_b as codes.  The codes are staged as bf16 integers in the same place, and the scale of (k, column group)
+// multiplies the query instead: q scale is carried as TERMS bf16 terms (two hold the product of two bf16 numbers exactly,
+// three hold all 24 bits of an f32 for f16 and f32 scales), so the products stay exact.
+template <int WAVES, int NOPE, int COLS, int BITS = 16, int TERMS = 1> __global__ __launch_bounds__(64 * WAVES) void mla_absorb_mfma(MlaDecodeParams p)
 {
     constexpr int kRowBytes = COLS * 2 + 16; // LDS bytes of one weight row: sixteen rows start in different banks
-    constexpr int kRowChunks = COLS / 8;     // its 16-byte chunks
     const unsigned int col0 = blockIdx.z * COLS;
     __shared__ __align__(16) unsigned char w_lds[NOPE * kRowBytes];
+    __shared__ __align__(16) float s_lds[BITS == 16 ? 1 : NOPE * (COLS / 32)]; // [column group][k]
     const unsigned int head = blockIdx.x;
     const unsigned int tid = threadIdx.x;
     const unsigned int lane = tid & 63u;
@@ -246,21 +301,39 @@ template <int WAVES, int NOPE, int COLS> __global__ __launch_bounds__(64 * WAVES
     const unsigned int m = lane & 15u;
     const unsigned int j = lane >> 4;
     {
-        const unsigned char* w = (const unsigned char*)(p.kv_b + (size_t)head * p.kv_head_dim * kLatent + col0);
-        // NOPE * COLS / 8 16-byte chunks (chunk c % kRowChunks of weight row c / kRowChunks), all of a thread's requested
-        // before any is stored
-        constexpr int kPerThread = NOPE * kRowChunks / (64 * WAVES);
-        static_assert(NOPE * kRowChunks % (64 * WAVES) == 0, "whole chunks per thread");
+        // 16-byte pieces (piece c % kRowPieces of weight row c / kRowPieces), all of a thread's requested before any is stored
+        constexpr int kRowPieces = COLS * BITS / 128;
+        constexpr int kPieces = NOPE * kRowPieces;
+        constexpr int kPerThread = (kPieces + 64 * WAVES - 1) / (64 * WAVES);
+        const unsigned char* w = (const unsigned char*)p.kv_b + ((size_t)head * p.kv_head_dim * kLatent + col0) * BITS / 8;
         u32x4 staged[kPerThread];
 #pragma unroll
         for (int i = 0; i < kPerThread; ++i) {
             const unsigned int c = tid + 64u * WAVES * i;
-            staged[i] = *(const u32x4*)(w + (size_t)(c / kRowChunks) * (kLatent * 2) + (c % kRowChunks) * 16u);
+            if (kPieces % (64 * WAVES) == 0 || c < kPieces) {
+                staged[i] = *(const u32x4*)(w + (size_t)(c / kRowPieces) * (kLatent * BITS / 8) + (c % kRowPieces) * 16u);
+            }
+        }
+        if constexpr (BITS != 16) {
+            const unsigned int group = min(p.kv_b_group, (unsigned int)COLS);
+            stage_scales<NOPE * (COLS / 32) / (64 * WAVES)>(p, s_lds, NOPE * (COLS / group), [&](unsigned int i) {
+                return ((size_t)head * p.kv_head_dim + i % NOPE) * (kLatent / p.kv_b_group) + (col0 + i / NOPE * group) / p.kv_b_group;
+            });
         }
 #pragma unroll
         for (int i = 0; i < kPerThread; ++i) {
             const unsigned int c = tid + 64u * WAVES * i;
-            *(u32x4*)(w_lds + (c / kRowChunks) * kRowBytes + (c % kRowChunks) * 16u) = staged[i];
+            if (kPieces % (64 * WAVES) == 0 || c < kPieces) {
+                unsigned char* at = w_lds + (c / kRowPieces) * kRowBytes + (c % kRowPieces) * (256u / BITS);
+                if constexpr (BITS == 16) {
+                    *(u32x4*)at = staged[i];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        *(Bf16Codes<BITS>*)(at + e * (64 / BITS)) = codes_to_bf16<BITS>(staged[i][e]);
+                    }
+                }
+            }
         }
     }
     __syncthreads();
@@ -314,7 +387,32 @@ template <int WAVES, int NOPE, int COLS> __global__ __launch_bounds__(64 * WAVES
             }
         }
         unsigned short* qa = p.absorbed + ((size_t)(row0 + m) * p.heads + head) * (kLatent + kRope) + col0 + 4u * j;
+        [[maybe_unused]] Frag qs[TERMS][NOPE / 32];
+        [[maybe_unused]] unsigned int scaled_for = ~0u; // column group qs was made for
         for (unsigned int nt = tile0; nt < tile0 + tiles; ++nt) {
+            if constexpr (BITS != 16) {
+                const unsigned int g = nt * 16u / min(p.kv_b_group, (unsigned int)COLS);
+                if (g != scaled_for) {
+                    scaled_for = g;
+#pragma unroll
+                    for (int ks = 0; ks < NOPE / 32; ++ks) {
+                        const f32x4 s0 = *(const f32x4*)(s_lds + g * NOPE + ks * 32u + 4u * j), s1 = *(const f32x4*)(s_lds + g * NOPE + ks * 32u + 16u + 4u * j);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const f32x4& sc = e < 2 ? s0 : s1;
+                            float x0 = __uint_as_float(qf[ks].u[e] << 16) * sc[2 * (e & 1)];
+                            float x1 = __uint_as_float(qf[ks].u[e] & 0xffff0000u) * sc[2 * (e & 1) + 1];
+#pragma unroll
+                            for (int t = 0; t < TERMS; ++t) {
+                                const unsigned int term = pack_bf16_hw(x0, x1);
+                                qs[t][ks].u[e] = term;
+                                x0 -= __uint_as_float(term << 16);
+                                x1 -= __uint_as_float(term & 0xffff0000u);
+                            }
+                        }
+                    }
+                }
+            }
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ks = 0; ks < NOPE / 32; ++ks) {
@@ -325,7 +423,14 @@ template <int WAVES, int NOPE, int COLS> __global__ __launch_bounds__(64 * WAVES
                 const unsigned char* at = frag_at + ks * 32 * kRowBytes + nt * 32u;
                 wf.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(at));
                 wf.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(at + 16 * kRowBytes));
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf.b, qf[ks].b, acc, 0, 0, 0);
+                if constexpr (BITS == 16) {
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf.b, qf[ks].b, acc, 0, 0, 0);
+                } else {
+#pragma unroll
+                    for (int t = TERMS - 1; t >= 0; --t) {
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf.b, qs[t][ks].b, acc, 0, 0, 0);
+                    }
+                }
             }
             if (row0 + m < p.batch) { // lane (m, j) holds latent columns 16 nt + 4 j .. + 4 of row m
                 *(u32x2*)(qa + nt * 16u) = u32x2{pack_bf16_rne(acc[0], acc[1]), pack_bf16_rne(acc[2], acc[3])};
@@ -1263,13 +1368,171 @@ __global__ __launch_bounds__(256) void mla_project(MlaDecodeParams p)
     project_head(p, head, b, x, blockIdx.z * 32u, min(p.value_dim, blockIdx.z * 32u + 32u));
 }
 
+// The two weight stages of a decode call with kv_b as codes, few rows (a single sequence has as many (row, head) pairs as
+// heads).  Memory latency is all there is: 32 heads of 8-bit weights are 2 MB a stage.  A thread of the absorb owns one
+// 32-bit word of codes (4 or 8 latent columns) and a quarter of the query columns, one per wave, up to TRIP of whose words
+// it requests at once; the four waves' sums meet in LDS.  grid = (heads, batch, BITS / 4), 256 threads.  Products are formed
+// as code x (query x scale): exact in f32 for bf16 scales.
+// One row of 32 heads, 8-bit codes in groups of 128: absorb 103 -> 5.8 us against mla_absorb_any, which reads the codes an
+// element at a time; a whole decode pass (append included) over 32 K tokens 255 -> 39.5 us.  A chunk of 512 rows of 128 heads
+// runs the matrix-core kernels: absorb 38.7 us and merge + projection 55.7 (bf16 weights: 34.3 and 46.4).
+template <int BITS, int TRIP> __global__ __launch_bounds__(256) void mla_absorb_codes(MlaDecodeParams p)
+{
+    constexpr unsigned int kPerWord = 32 / BITS, kWords = kLatent / kPerWord; // columns of a word, words of a weight row
+    __shared__ float q_sh[1024];
+    __shared__ float s_sh[256 * 16]; // [query column][column group] of up to 256 query columns, 16 groups at most
+    __shared__ __align__(16) float sum_sh[4][64 * kPerWord];
+    const unsigned int head = blockIdx.x;
+    const unsigned int b = blockIdx.y;
+    const unsigned int lane = threadIdx.x & 63u;
+    const unsigned int wave = threadIdx.x >> 6;
+    const unsigned int word = blockIdx.z * 64u + lane;
+    const unsigned int quarter = (p.nope_dim + 3u) / 4u;
+    const unsigned int k_begin = min(wave * quarter, p.nope_dim), k_end = min(k_begin + quarter, p.nope_dim);
+    const unsigned int* w = (const unsigned int*)p.kv_b + (size_t)head * p.kv_head_dim * kWords + word;
+    const unsigned int groups = kLatent / p.kv_b_group;
+    const unsigned int g = word * kPerWord / p.kv_b_group;
+    unsigned int raw[TRIP];
+    auto fetch = [&](unsigned int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < TRIP; ++u) {
+            const unsigned int k = min(k0 + u, p.nope_dim - 1u);
+            raw[u] = w[(size_t)k * kWords];
+        }
+    };
+    fetch(k_begin);
+    stage_scales<16>(p, s_sh, p.nope_dim * groups, [&](unsigned int i) { return (size_t)head * p.kv_head_dim * groups + i; });
+    const size_t q_base = ((size_t)b * p.heads + head) * p.q_head_dim;
+    for (unsigned int i = threadIdx.x; i < p.q_head_dim; i += 256u) {
+        // the oracle takes a bf16 query (src/kernel/cpu/mla.rs:958-961)
+        q_sh[i] = bf16_bits_to_f32(f32_to_bf16_bits(load_as_f32(p.q, q_base + i, p.q_dtype)));
+    }
+    __syncthreads();
+    float acc[kPerWord];
+#pragma unroll
+    for (unsigned int e = 0; e < kPerWord; ++e) {
+        acc[e] = 0.0f;
+    }
+    for (unsigned int k0 = k_begin; k0 < k_end; k0 += TRIP) {
+#pragma unroll
+        for (int u = 0; u < TRIP; ++u) {
+            const unsigned int k = min(k0 + u, p.nope_dim - 1u);
+            const float x = k0 + u < k_end ? q_sh[k] * s_sh[k * groups + g] : 0.0f;
+#pragma unroll
+            for (unsigned int e = 0; e < kPerWord; ++e) {
+                acc[e] = fmaf(x, code_value<BITS>(raw[u], e), acc[e]);
+            }
+        }
+        if (k0 + TRIP < k_end) {
+            fetch(k0 + TRIP);
+        }
+    }
+#pragma unroll
+    for (unsigned int e = 0; e < kPerWord; ++e) {
+        sum_sh[wave][lane * kPerWord + e] = acc[e];
+    }
+    __syncthreads();
+    unsigned short* qa = p.absorbed + ((size_t)b * p.heads + head) * (kLatent + kRope);
+    for (unsigned int c = threadIdx.x; c < 32u * kPerWord; c += 256u) {
+        const float2 s0 = *(const float2*)&sum_sh[0][2 * c], s1 = *(const float2*)&sum_sh[1][2 * c], s2 = *(const float2*)&sum_sh[2][2 * c],
+                     s3 = *(const float2*)&sum_sh[3][2 * c];
+        *(unsigned int*)(qa + blockIdx.z * 64u * kPerWord + 2u * c) = pack_bf16_rne((s0.x + s1.x) + (s2.x + s3.x), (s0.y + s1.y) + (s2.y + s3.y));
+    }
+    if (blockIdx.z == 0u && threadIdx.x < kRope) {
+        qa[kLatent + threadIdx.x] = f32_to_bf16_bits(q_sh[p.nope_dim + threadIdx.x]);
+    }
+}
+
+// A value column's weights as a lane holds them, kv_b as codes: lane = (column, slice lane % 8); a slice owns the codes of
+// 16 bytes out of every 128 of a weight row (16 or 32 latent columns), so the eight slices fetch whole lines.
+template <int BITS> struct CodeColumn {
+    static constexpr int kPer16 = 128 / BITS, kPieces = 64 / kPer16; // columns of a 16-byte piece, pieces of a lane
+    u32x4 raw[kPieces];
+    unsigned int scale[kPieces];
+
+    __device__ __forceinline__ void fetch(const MlaDecodeParams& p, unsigned int head, unsigned int v, unsigned int slice)
+    {
+        const size_t row = (size_t)head * p.kv_head_dim + p.nope_dim + min(v, p.value_dim - 1u);
+        const unsigned char* w = (const unsigned char*)p.kv_b + row * (kLatent * BITS / 8) + slice * 16u;
+        const size_t scales = row * (kLatent / p.kv_b_group);
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            raw[i] = *(const u32x4*)(w + 128 * i);
+        }
+        if (p.kv_b_scale_dtype == 2) {
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) {
+                scale[i] = ((const unsigned int*)p.kv_b_scales)[scales + (i * 8u + slice) * kPer16 / p.kv_b_group];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) {
+                scale[i] = ((const unsigned short*)p.kv_b_scales)[scales + (i * 8u + slice) * kPer16 / p.kv_b_group];
+            }
+        }
+    }
+    // x[i * kPer16 + e] = merged value of latent column (8 i + slice) kPer16 + e; the sum over all slices ends up in slice 7
+    __device__ __forceinline__ float dot(const MlaDecodeParams& p, const f32x4 (&x)[16]) const
+    {
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            float part = 0.0f;
+#pragma unroll
+            for (int e = 0; e < kPer16; ++e) {
+                part = fmaf(x[i * (kPer16 / 4) + e / 4][e & 3], code_value<BITS>(raw[i][e * BITS / 32], e & (32 / BITS - 1)), part);
+            }
+            const float s = p.kv_b_scale_dtype == 2 ? __uint_as_float(scale[i])
+                                                    : (p.kv_b_scale_dtype == 1 ? f16_bits_to_f32((unsigned short)scale[i]) : __uint_as_float(scale[i] << 16));
+            sum = fmaf(part, s, sum);
+        }
+        sum += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(sum), 0x114, 0xf, 0xf, true)); // row_shr:4
+        sum += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(sum), 0x112, 0xf, 0xf, true)); // row_shr:2
+        sum += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(sum), 0x111, 0xf, 0xf, true)); // row_shr:1
+        return sum;
+    }
+    static __device__ __forceinline__ void merged_row(const float* row, unsigned int slice, f32x4 (&x)[16])
+    {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            x[i] = *(const f32x4*)(row + (i / (kPer16 / 4) * 8u + slice) * kPer16 + i % (kPer16 / 4) * 4u);
+        }
+    }
+};
+
+__device__ __forceinline__ void store_value(const MlaDecodeParams& p, unsigned int head, unsigned int b, unsigned int v, float sum)
+{
+    const size_t at = ((size_t)b * p.heads + head) * (p.out_compact ? p.value_dim : p.q_head_dim) + v;
+    if (p.out_dtype == 0) {
+        ((float*)p.out)[at] = sum;
+    } else {
+        ((unsigned short*)p.out)[at] = f32_to_bf16_bits(sum);
+    }
+}
+
+// Projection of the merged rows in the workspace.  grid = (heads, batch, value_dim / 32 rounded up), 256 threads.
+template <int BITS> __global__ __launch_bounds__(256) void mla_project_codes(MlaDecodeParams p)
+{
+    const unsigned int slice = threadIdx.x & 7u;
+    const unsigned int v = blockIdx.z * 32u + (threadIdx.x >> 3);
+    CodeColumn<BITS> w;
+    w.fetch(p, blockIdx.x, v, slice);
+    f32x4 x[16];
+    CodeColumn<BITS>::merged_row(p.weighted + ((size_t)blockIdx.y * p.heads + blockIdx.x) * kLatent, slice, x);
+    const float sum = w.dot(p, x);
+    if (slice == 7u && v < p.value_dim) {
+        store_value(p, blockIdx.x, blockIdx.y, v, sum);
+    }
+}
+
 // grid = (heads, batch): split merge and projection in one kernel when both stages run.  The merge is the
 // log-sum-exp combine of the split records (same algebra as the stand-alone merge, base 2): threads =
 // (128 column quads) x (2 split lanes), all loads of a lane issued before any is used; the merged row goes
 // through LDS to the projection's register layout instead of through the workspace.  With the usual value width
 // (128 columns) a thread's weight vectors for all four passes of the projection are requested first of all, so that
 // the kernel is two memory round trips long (sequence length, then records and weights together) instead of seven.
-__global__ __launch_bounds__(256) void mla_merge_project(MlaDecodeParams p)
+// BITS 8 / 4: kv_b as codes; the weights of up to 128 value columns are requested first of all in the same way.
+template <int BITS> __global__ __launch_bounds__(256) void mla_merge_project(MlaDecodeParams p)
 {
     const unsigned int head = blockIdx.x;
     const unsigned int b = blockIdx.y;
@@ -1279,7 +1542,14 @@ __global__ __launch_bounds__(256) void mla_merge_project(MlaDecodeParams p)
     const unsigned int wave = threadIdx.x >> 6;
     const unsigned int slice = lane & 7u;
     const unsigned int sub = lane >> 3;
-    const bool wide = p.value_dim == 128u;
+    const bool wide = BITS == 16 && p.value_dim == 128u;
+    [[maybe_unused]] CodeColumn<BITS == 16 ? 8 : BITS> code_w[4];
+    if constexpr (BITS != 16) {
+#pragma unroll
+        for (int pass = 0; pass < 4; ++pass) {
+            code_w[pass].fetch(p, head, 32u * pass + (threadIdx.x >> 3), slice);
+        }
+    }
     u32x4 raw[4][8];
     const unsigned short* w_head = p.kv_b + ((size_t)head * p.kv_head_dim + p.nope_dim) * kLatent + slice * 8u;
     if (wide) {
@@ -1360,6 +1630,24 @@ __global__ __launch_bounds__(256) void mla_merge_project(MlaDecodeParams p)
         *(f32x4*)(merged + quad * 4u) = result;
     }
     __syncthreads();
+    if constexpr (BITS != 16) {
+        f32x4 x[16];
+        CodeColumn<BITS>::merged_row(merged, slice, x);
+        for (unsigned int v0 = threadIdx.x >> 3; v0 < p.value_dim; v0 += 128u) {
+#pragma unroll
+            for (int pass = 0; pass < 4; ++pass) {
+                const unsigned int v = v0 + 32u * pass;
+                const float sum = code_w[pass].dot(p, x);
+                if (slice == 7u && v < p.value_dim) {
+                    store_value(p, head, b, v, sum);
+                }
+                if (v + 128u < p.value_dim) {
+                    code_w[pass].fetch(p, head, v + 128u, slice);
+                }
+            }
+        }
+        return;
+    }
     if (wide) { // the other two passes' weights travel while the merged row is read back
 #pragma unroll
         for (int pass = 2; pass < 4; ++pass) {
@@ -1620,13 +1908,18 @@ template <int R> __global__ __launch_bounds__(256) void mla_merge_project_rows(M
 // its sum divided out.  Modes 1 and 2 leave the registers for two workgroups per compute unit.
 constexpr int kMergedStride = kLatent + 8; // bf16 elements: sixteen rows' 16-byte fragments start in different banks
 // WAVES: 8 (value widths up to 128) or 16 (up to 256; modes 1 and 2, whose registers allow 1,024 threads).
-template <int MODE, int WAVES = 8> __global__ __launch_bounds__(64 * WAVES) void mla_merge_project_mfma(MlaDecodeParams p)
+//
+// BITS 8 / 4: kv_b as codes, fed to the matrix cores as bf16 integers; a column group's sum is multiplied by the scale of
+// (value column, group) in f32.  The merged rows are carried as three bf16 terms there, all 24 bits of the f32.
+template <int MODE, int WAVES = 8, int BITS = 16> __global__ __launch_bounds__(64 * WAVES) void mla_merge_project_mfma(MlaDecodeParams p)
 {
     static_assert(WAVES == 8 || MODE != 0, "the record-folding form needs the registers of 512 threads");
+    constexpr int TERMS = BITS == 16 ? 2 : 3;
     constexpr unsigned int RG = WAVES / 2;  // groups of 128 threads: thread group rb takes rows rb, rb + RG, ...
     constexpr int RPT = 16 / RG;            // rows of a block per thread
-    // the merged rows as two bf16 terms (value = hi + lo keeps 16 bits of the f32), split once by the thread that merged them
-    __shared__ __align__(16) unsigned short merged_hi[16][kMergedStride], merged_lo[16][kMergedStride];
+    // the merged rows as bf16 terms (value = hi + lo keeps 16 bits of the f32), split once by the thread that merged them
+    __shared__ __align__(16) unsigned short merged[TERMS][16][kMergedStride];
+    __shared__ __align__(16) float s_lds[BITS == 16 ? 1 : (kLatent / 32) * WAVES * 16]; // [column group][value column]
     const unsigned int head = blockIdx.x;
     const unsigned int tid = threadIdx.x;
     const unsigned int quad = tid & 127u;
@@ -1639,9 +1932,37 @@ template <int MODE, int WAVES = 8> __global__ __launch_bounds__(64 * WAVES) void
     Frag wf[16];
     {
         const unsigned int v = min(wave * 16u + m, p.value_dim - 1u);
+        if constexpr (BITS == 16) {
 #pragma unroll
-        for (int ks = 0; ks < 16; ++ks) {
-            wf[ks].u = *(const u32x4*)(w_head + (size_t)v * kLatent + ks * 32 + 8u * j);
+            for (int ks = 0; ks < 16; ++ks) {
+                wf[ks].u = *(const u32x4*)(w_head + (size_t)v * kLatent + ks * 32 + 8u * j);
+            }
+        } else {
+            const size_t first = (size_t)head * p.kv_head_dim + p.nope_dim; // kv_b row of value column 0
+            const unsigned int* words = (const unsigned int*)p.kv_b + (first + v) * (kLatent * BITS / 32) + j * (BITS / 4);
+            unsigned int raw[16][BITS / 4];
+#pragma unroll
+            for (int ks = 0; ks < 16; ++ks) {
+#pragma unroll
+                for (int e = 0; e < BITS / 4; ++e) {
+                    raw[ks][e] = words[ks * BITS + e];
+                }
+            }
+            const unsigned int groups = kLatent / p.kv_b_group;
+            stage_scales<kLatent / 32 / 4>(p, s_lds, WAVES * 16u * groups, [&](unsigned int i) {
+                return (first + min(i % (WAVES * 16u), p.value_dim - 1u)) * groups + i / (WAVES * 16u);
+            });
+#pragma unroll
+            for (int ks = 0; ks < 16; ++ks) {
+#pragma unroll
+                for (int e = 0; e < BITS / 4; ++e) {
+                    const Bf16Codes<BITS> c = codes_to_bf16<BITS>(raw[ks][e]);
+#pragma unroll
+                    for (int u = 0; u < 16 / BITS; ++u) {
+                        wf[ks].u[e * (16 / BITS) + u] = c.word[u];
+                    }
+                }
+            }
         }
     }
     // the merged values of this thread's four rows (rb, rb + 4, rb + 8, rb + 12 of the block at row0) and four columns
@@ -1752,12 +2073,14 @@ template <int MODE, int WAVES = 8> __global__ __launch_bounds__(64 * WAVES) void
         const unsigned int rb = tid >> 7;
 #pragma unroll
         for (int u = 0; u < RPT; ++u) {
-            const f32x4 x = next_rows[u];
-            const u32x2 hi = {pack_bf16_rne(x[0], x[1]), pack_bf16_rne(x[2], x[3])};
-            const u32x2 lo = {pack_bf16_rne(x[0] - __uint_as_float(hi[0] << 16), x[1] - __uint_as_float(hi[0] & 0xffff0000u)),
-                              pack_bf16_rne(x[2] - __uint_as_float(hi[1] << 16), x[3] - __uint_as_float(hi[1] & 0xffff0000u))};
-            *(u32x2*)(&merged_hi[rb + RG * u][quad * 4u]) = hi;
-            *(u32x2*)(&merged_lo[rb + RG * u][quad * 4u]) = lo;
+            f32x4 x = next_rows[u];
+#pragma unroll
+            for (int t = 0; t < TERMS; ++t) {
+                const u32x2 term = {pack_bf16_rne(x[0], x[1]), pack_bf16_rne(x[2], x[3])};
+                *(u32x2*)(&merged[t][rb + RG * u][quad * 4u]) = term;
+                x -= f32x4{__uint_as_float(term[0] << 16), __uint_as_float(term[0] & 0xffff0000u), __uint_as_float(term[1] << 16),
+                           __uint_as_float(term[1] & 0xffff0000u)};
+            }
         }
     }
     __syncthreads();
@@ -1767,13 +2090,32 @@ template <int MODE, int WAVES = 8> __global__ __launch_bounds__(64 * WAVES) void
     // ---- projection
     const unsigned int out_stride = p.out_compact ? p.value_dim : p.q_head_dim;
     f32x4 out_acc = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (BITS == 16) {
 #pragma unroll
-    for (int ks = 0; ks < 16; ++ks) {
-        Frag hi, lo;
-        hi.u = *(const u32x4*)(&merged_hi[m][ks * 32 + 8u * j]);
-        lo.u = *(const u32x4*)(&merged_lo[m][ks * 32 + 8u * j]);
-        out_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks].b, hi.b, out_acc, 0, 0, 0);
-        out_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks].b, lo.b, out_acc, 0, 0, 0);
+        for (int ks = 0; ks < 16; ++ks) {
+#pragma unroll
+            for (int t = 0; t < TERMS; ++t) {
+                Frag x;
+                x.u = *(const u32x4*)(&merged[t][m][ks * 32 + 8u * j]);
+                out_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks].b, x.b, out_acc, 0, 0, 0);
+            }
+        }
+    } else {
+        const unsigned int steps = p.kv_b_group / 32u; // 32-column steps of a scale group: 1, 2, 4, 8 or 16
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 16; ++ks) {
+#pragma unroll
+            for (int t = TERMS - 1; t >= 0; --t) {
+                Frag x;
+                x.u = *(const u32x4*)(&merged[t][m][ks * 32 + 8u * j]);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks].b, x.b, acc, 0, 0, 0);
+            }
+            if (((ks + 1u) & (steps - 1u)) == 0u) {
+                out_acc += acc * *(const f32x4*)(s_lds + (ks / steps) * (WAVES * 16u) + wave * 16u + 4u * j);
+                acc = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
     }
     if (row0 + m < p.batch) { // lane (m, j) holds value columns 16 wave + 4 j .. + 4 of row m
         const size_t base = ((size_t)(row0 + m) * p.heads + head) * out_stride;
@@ -1803,6 +2145,27 @@ static unsigned int row_block_groups(const MlaDecodeParams& p)
     const unsigned int blocks = (p.batch + 15u) / 16u;
     const unsigned int per_head = (256u + p.heads - 1u) / p.heads;
     return blocks < per_head ? blocks : per_head;
+}
+
+// Where the matrix-core stages take over from a workgroup per (row, head), by the number of such pairs: a few hundred
+// workgroups run side by side, beyond that they queue, while the matrix-core kernels read a head's weights once for sixteen
+// rows and cost the same for one row as for sixteen.  Measured, us per pair / on the matrix cores:
+//   absorb, 128 query columns: bf16 512 pairs 5.8 / 6.4, 640 pairs 8.5 / 7.1, 1920 pairs 16.9 / 7.1; 8-bit codes 352 pairs
+//   7.3 / 8.4, 480 pairs 11.2 / 8.7; 192 query columns: bf16 128 pairs 6.3 / 5.5, 8-bit codes 128 pairs 7.3 / 7.1
+//   merge and projection: bf16 512 pairs 7.4 / 11.7 (sixteen rows), 832 pairs 13.3 / 12.3 (26 rows), 1024 pairs 15.1 / 16.2
+//   (eight rows: half of a tile empty), 1408 pairs 19.8 / 16.6; 8-bit codes within 2 us of these
+static bool matrix_absorb(const MlaDecodeParams& p)
+{
+    const unsigned int pairs = p.batch * p.heads;
+    if ((p.q_head_dim & 3u) != 0) {
+        return false;
+    }
+    return p.nope_dim == 192u ? pairs >= 128u : p.nope_dim == 128u && pairs >= (p.kv_b_bits == 16u ? 576u : 448u);
+}
+
+static bool matrix_project(const MlaDecodeParams& p)
+{
+    return p.batch * p.heads >= (p.batch >= 16u ? 800u : 1200u);
 }
 
 // One workgroup per (row, head) folds 32 split records a round trip; the wide merge and the separate projection cost a
@@ -1837,6 +2200,94 @@ static hipError_t merge_into_workspace(const MlaDecodeParams& p, hipStream_t str
     return launch_split_merge(mp, stream);
 }
 
+// Waves of a matrix-core absorb workgroup that share a block of sixteen rows: as many as keeps every wave busy
+static unsigned int waves_per_block(const MlaDecodeParams& p, unsigned int waves)
+{
+    const unsigned int groups = row_block_groups(p);
+    const unsigned int blocks_here = ((p.batch + 15u) / 16u + groups - 1u) / groups;
+    unsigned int share = 1u;
+    while (share < waves && blocks_here * share < waves) {
+        share *= 2u;
+    }
+    return share;
+}
+
+// kv_b as 8- or 4-bit codes on the kernels of this file: scale groups of 32, 64, ... 512 columns (a 32-column matrix step
+// and a 16-byte piece of 4-bit codes lie in one group)
+static bool takes_codes(const MlaDecodeParams& p)
+{
+    return (p.kv_b_bits == 8u || p.kv_b_bits == 4u) && p.kv_b_group % 32u == 0 && p.nope_dim != 0u && p.nope_dim <= 256u;
+}
+
+template <int BITS> static hipError_t launch_absorb_codes(const MlaDecodeParams& p, hipStream_t stream)
+{
+    if (matrix_absorb(p)) {
+        MlaDecodeParams q = p;
+        const dim3 grid(p.heads, row_block_groups(p), p.nope_dim == 128u ? 1u : 2u);
+        // q x scale in two bf16 terms is exact for bf16 scales; f16 and f32 scales take three.  Sixteen waves a workgroup
+        // for a chunk as with bf16 weights, eight where the terms of a query do not fit a sixteenth of the registers
+        auto launch = [&](auto terms) {
+            constexpr int T = decltype(terms)::value;
+            constexpr int kMost = T == 2 ? 16 : 8;
+            const unsigned int waves = p.batch < 128u ? 4u : p.nope_dim == 128u ? kMost : 8u;
+            q.column_split = waves_per_block(p, waves);
+            if (p.nope_dim == 128u) {
+                waves != 4u ? mla_absorb_mfma<kMost, 128, 512, BITS, T><<<grid, dim3(64 * kMost), 0, stream>>>(q)
+                            : mla_absorb_mfma<4, 128, 512, BITS, T><<<grid, dim3(256), 0, stream>>>(q);
+            } else {
+                waves != 4u ? mla_absorb_mfma<8, 192, 256, BITS, T><<<grid, dim3(512), 0, stream>>>(q)
+                            : mla_absorb_mfma<4, 192, 256, BITS, T><<<grid, dim3(256), 0, stream>>>(q);
+            }
+        };
+        p.kv_b_scale_dtype == 0 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 3>{});
+    } else {
+        const dim3 grid(p.heads, p.batch, BITS / 4);
+        p.nope_dim <= 128u ? mla_absorb_codes<BITS, 32><<<grid, dim3(256), 0, stream>>>(p) : mla_absorb_codes<BITS, 48><<<grid, dim3(256), 0, stream>>>(p);
+    }
+    return hipGetLastError();
+}
+
+template <int BITS> static hipError_t launch_merge_project_codes(const MlaDecodeParams& p, unsigned int stages, hipStream_t stream)
+{
+    const bool both = (stages & 12u) == 12u;
+    const bool matrix = both && matrix_project(p) && p.value_dim <= 256u;
+    const bool wide_values = p.value_dim > 128u;
+    const bool unsplit = p.max_chunks == 1u;
+    const unsigned int groups = row_block_groups(p);
+    if (matrix && unsplit) {
+        const unsigned int blocks = (p.batch + 15u) / 16u;
+        const unsigned int twice = 2u * groups < blocks ? 2u * groups : blocks;
+        wide_values ? mla_merge_project_mfma<2, 16, BITS><<<dim3(p.heads, groups), dim3(1024), 0, stream>>>(p)
+                    : mla_merge_project_mfma<2, 8, BITS><<<dim3(p.heads, twice), dim3(512), 0, stream>>>(p);
+        return hipGetLastError();
+    }
+    if (matrix && !wide_values && p.batch > 64u) {
+        mla_merge_project_mfma<0, 8, BITS><<<dim3(p.heads, groups), dim3(512), 0, stream>>>(p);
+        return hipGetLastError();
+    }
+    if (both && !matrix && !wide_merge_pays(p)) {
+        mla_merge_project<BITS><<<dim3(p.heads, p.batch), dim3(256), 0, stream>>>(p);
+        return hipGetLastError();
+    }
+    if (stages & 4u) {
+        if (both && !matrix) {
+            mla_merge_wide<<<dim3(p.heads, p.batch, kWideParts), dim3(256), 0, stream>>>(p);
+        } else {
+            const hipError_t err = merge_into_workspace(p, stream);
+            if (err != hipSuccess) {
+                return err;
+            }
+        }
+    }
+    if (matrix) {
+        wide_values ? mla_merge_project_mfma<1, 16, BITS><<<dim3(p.heads, groups), dim3(1024), 0, stream>>>(p)
+                    : mla_merge_project_mfma<1, 8, BITS><<<dim3(p.heads, groups), dim3(512), 0, stream>>>(p);
+    } else if (stages & 8u) {
+        mla_project_codes<BITS><<<dim3(p.heads, p.batch, (p.value_dim + 31u) / 32u), dim3(256), 0, stream>>>(p);
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, hipStream_t stream)
 {
     const unsigned int stages = (stage_mask & 15u) == 0 ? 15u : (stage_mask & 15u);
@@ -1845,25 +2296,27 @@ hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, 
     // stages for other widths, absorb and projection (the stages that read kv_b) for other weight forms
     const bool usual_widths = p.latent_dim == (unsigned int)kLatent && p.rope_dim == 64u;
     const bool bf16_weights = p.kv_b_bits == 16u;
-    if ((stages & 1u) && !(usual_widths && bf16_weights)) {
+    const bool code_weights = usual_widths && takes_codes(p);
+    if ((stages & 1u) && code_weights) {
+        err = p.kv_b_bits == 8u ? launch_absorb_codes<8>(p, stream) : launch_absorb_codes<4>(p, stream);
+        if (err != hipSuccess) {
+            return err;
+        }
+    } else if ((stages & 1u) && !(usual_widths && bf16_weights)) {
         err = launch_mla_absorb_any(p, stream);
         if (err != hipSuccess) {
             return err;
         }
     } else if (stages & 1u) {
-        // Eight rows per workgroup share every weight load, and the workgroup then runs eight rows' sums: measured 28 us from
-        // 16 rows up to a few hundred, against 13 us (15 rows) to 27 us (32 rows) for one workgroup per row
-        if (p.batch >= 16u && (p.nope_dim == 128u || p.nope_dim == 192u) && (p.q_head_dim & 3u) == 0) { // sixteen rows a workgroup, on the matrix cores
+        // Other query widths: eight rows per workgroup share every weight load, and the workgroup then runs eight rows' sums:
+        // measured 28 us from 16 rows up to a few hundred, against 13 us (15 rows) to 27 us (32 rows) for one workgroup per row
+        if (matrix_absorb(p)) { // sixteen rows a workgroup, on the matrix cores
             // four waves for a decode batch, sixteen for a chunk (33 against 61 us on 512 rows of 128 heads; on 16 to 64 rows
             // the larger workgroup costs 4 us); as many waves share a block of sixteen rows as keeps every wave busy
             MlaDecodeParams q = p;
             const unsigned int groups = row_block_groups(p);
-            const unsigned int blocks_here = ((p.batch + 15u) / 16u + groups - 1u) / groups;
             const unsigned int waves = p.batch >= 128u ? 16u : 4u;
-            q.column_split = 1u;
-            while (q.column_split < waves && blocks_here * q.column_split < waves) {
-                q.column_split *= 2u;
-            }
+            q.column_split = waves_per_block(p, waves);
             if (p.nope_dim == 128u) {
                 waves == 16u ? mla_absorb_mfma<16, 128, 512><<<dim3(p.heads, groups), dim3(1024), 0, stream>>>(q)
                              : mla_absorb_mfma<4, 128, 512><<<dim3(p.heads, groups), dim3(256), 0, stream>>>(q);
@@ -1913,6 +2366,9 @@ hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, 
             return err;
         }
     }
+    if (code_weights) {
+        return p.kv_b_bits == 8u ? launch_merge_project_codes<8>(p, stages, stream) : launch_merge_project_codes<4>(p, stages, stream);
+    }
     if (!(usual_widths && bf16_weights)) {
         if (stages & 4u) {
             err = merge_into_workspace(p, stream);
@@ -1926,7 +2382,7 @@ hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, 
         // value widths up to 128 run eight waves, up to 256 sixteen (not the record-folding form, whose registers stop at 512 threads)
         const bool wide_values = p.value_dim > 128u;
         const bool two_step = p.max_chunks > 1u && p.batch <= 64u;
-        if (p.batch >= 16u && (p.value_dim <= 128u || (p.value_dim <= 256u && (two_step || p.max_chunks == 1u)))) {
+        if (matrix_project(p) && (p.value_dim <= 128u || (p.value_dim <= 256u && (two_step || p.max_chunks == 1u)))) {
             // sixteen rows a workgroup, the projection on the matrix cores.
             // Up to 64 rows the fused kernel is at most 256 workgroups, each a chain of round trips (lengths, records four
             // splits at a time, projection); the split-merge kernel reads the same records with a thread per (row, head,
@@ -1950,7 +2406,7 @@ hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, 
             } else {
                 mla_merge_project_mfma<0, 8><<<grid, dim3(512), 0, stream>>>(p);
             }
-        } else if (p.batch >= 16u) { // eight rows share every weight load of the projection
+        } else if (p.batch >= 16u && matrix_project(p)) { // eight rows share every weight load of the projection
             mla_merge_project_rows<8><<<dim3(p.heads, (p.batch + 7u) / 8u), dim3(256), 0, stream>>>(p);
         } else if (wide_merge_pays(p)) {
             // few rows, each cut into many splits: the merge by eight workgroups per (row, head), then the projection
@@ -1961,7 +2417,7 @@ hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, 
             }
             mla_project<<<dim3(p.heads, p.batch, (p.value_dim + 31u) / 32u), dim3(256), 0, stream>>>(p);
         } else {
-            mla_merge_project<<<dim3(p.heads, p.batch), dim3(256), 0, stream>>>(p);
+            mla_merge_project<16><<<dim3(p.heads, p.batch), dim3(256), 0, stream>>>(p);
         }
         return hipGetLastError();
     }

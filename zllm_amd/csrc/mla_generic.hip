@@ -1,7 +1,8 @@
 // Absorbed MLA decode for the geometries and weight formats the matrix-core kernels do not take: any latent width that
 // Q8g64 groups divide (64 .. 1024 columns), any even rope width up to 256, and kv_b as f32, bf16, or 8- / 4-bit codes
 // with a scale per row and column group (the formats of paged_weight,
-// src/kernel/rocm/hip/attention/paged_mla/source.hip:2-26).  Vector ALU only: the work is a few dot products per
+// src/kernel/rocm/hip/attention/paged_mla/source.hip:2-26; at 512 + 64 columns codes in groups of at least 32 columns have
+// kernels of their own in mla_decode.hip).  Vector ALU only: the work is a few dot products per
 // token, and these shapes are the small ones (the reference's own rank-64 case, src/kernel/cpu/mla.rs:1166-1195).
 //
 //   absorb   q_abs[h, c] = sum_k q_nope[h, k] * W[h, k, c], k ascending, product and sum rounded separately, result
