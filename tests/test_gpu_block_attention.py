@@ -101,6 +101,19 @@ def test_varlen_segments(kv, d, hq, hkv, q_kind, block_tokens):
     assert_attention_close(out, want, f"varlen {kv} d={d}")
 
 
+@pytest.mark.parametrize("kv,d", [("f16", 128), ("f16", 256), ("q8", 64), ("q8", 128)])
+@pytest.mark.parametrize("rows,heads", [(127, 8), (129, 8), (577, 64)])
+def test_segments_that_end_beside_tile_and_wave_edges(kv, d, rows, heads):
+    """One query head per KV head, so that tiles are 128 or 256 rows and waves 16 or 32 of them: segments that end one row
+    before, on and after those edges and one-key rows among them; 64 heads x 577 rows fill the device and
+    run without KV splits, the shorter calls with what the plan gives them."""
+    offsets = [o for o in (0, 1, 15, 17, 32, 63, 96, 127, 128, 129, 255, 257, 512, 545) if o < rows] + [rows]
+    visible = varlen_ranges(offsets, offsets)
+    visible[100] = (0, 1)
+    out, want = run_block(200 + rows, rows, rows, heads, heads, d, visible, kv=kv)
+    assert_attention_close(out, want, f"tile edges {kv} d={d} rows={rows}")
+
+
 @pytest.mark.parametrize("workspace", [True, False])
 def test_random_ranges_and_fewer_keys_than_rows(workspace):
     """Arbitrary [start, end) per row (not monotone, not causal), one-key rows, and a call with more query rows than cache

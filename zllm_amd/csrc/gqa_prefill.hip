@@ -115,6 +115,58 @@ __device__ __forceinline__ SplitRange split_range(const GqaPrefillParams& p, uns
     return r;
 }
 
+// The visible range of a row tile whose rows bring their own ends, or ranges (src/attention/block.rs:10-16): the union over
+// the rows.  A lane takes every 64th row and the wave folds what they found: one loop over the rows, the same for every
+// lane, is a chain of scalar loads.  Packed segments (16 heads of 128, 4,100 f16 rows in nine segments) went from 218 us
+// and a 32 us split merge to 68 us without one, by this, tiles of 128 rows, wide query loads and the skipped steps below
+// together; 2,580 rows of 32 / 8 heads of 256 in thirteen segments 230 -> 92 us a pass.
+__device__ __forceinline__ void given_range(const GqaPrefillParams& p, unsigned int row0, unsigned int last_row, unsigned int lane, unsigned int& t_begin,
+                                            unsigned int& t_end)
+{
+    const bool ranges = p.visible_starts != nullptr;
+    unsigned int end = ranges ? 0u : t_end, begin = ranges ? 0xffffffffu : t_begin;
+    for (unsigned int r = row0 + lane; r <= last_row; r += 64u) {
+        const unsigned int given_end = min(p.visible_ends[r], p.position + p.rows);
+        end = max(end, given_end);
+        if (ranges) {
+            begin = min(begin, min(p.visible_starts[r], given_end));
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        end = max(end, (unsigned int)__shfl_xor((int)end, off));
+        begin = min(begin, (unsigned int)__shfl_xor((int)begin, off));
+    }
+    t_end = __builtin_amdgcn_readfirstlane(end);
+    t_begin = __builtin_amdgcn_readfirstlane(begin);
+}
+
+// Eight consecutive query elements (16-byte aligned: the query is, and head_dim is a multiple of 64).  One element at a
+// time, a lane sends 32 to 128 two-byte loads before the first step: 1,000 rows of 32 / 8 heads 54.6 -> 49.1 us, a sliding
+// layer of 2,048 rows (16 / 8 heads of 256, window 1,024) 108.9 -> 86.3 us.
+__device__ __forceinline__ void widen8(const u32x4& raw, int dtype, float (&x)[8])
+{
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        x[2 * e] = dtype == 1 ? __uint_as_float(raw[e] << 16) : f16_bits_to_f32((unsigned short)(raw[e] & 0xffffu));
+        x[2 * e + 1] = dtype == 1 ? __uint_as_float(raw[e] & 0xffff0000u) : f16_bits_to_f32((unsigned short)(raw[e] >> 16));
+    }
+}
+
+__device__ __forceinline__ void load_query8(const void* q, size_t at, int dtype, float (&x)[8])
+{
+    if (dtype == 0) {
+        const f32x4 a = *(const f32x4*)((const float*)q + at), b = *(const f32x4*)((const float*)q + at + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[e] = a[e];
+            x[4 + e] = b[e];
+        }
+        return;
+    }
+    widen8(*(const u32x4*)((const unsigned short*)q + at), dtype, x);
+}
+
 __device__ __forceinline__ void store_empty_record(const GqaPrefillParams& p, unsigned int row, unsigned int head)
 {
     const size_t rec = ((size_t)row * p.max_chunks + blockIdx.z) * p.num_heads + head;
@@ -191,18 +243,8 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
     const unsigned int last_row = min(row0 + rows_per_wg, p.rows) - 1u;
     unsigned int t_end = p.position + last_row + 1u;
     unsigned int t_begin = 0;
-    if (p.visible_starts != nullptr) { // explicit ranges (src/attention/block.rs:10-16): the union of the rows' own
-        t_end = 0u;
-        t_begin = 0xffffffffu;
-        for (unsigned int r = row0; r <= last_row; ++r) { // uniform over the workgroup: scalar loads
-            const unsigned int given_end = min(p.visible_ends[r], p.position + p.rows);
-            t_end = max(t_end, given_end);
-            t_begin = min(t_begin, min(p.visible_starts[r], given_end));
-        }
-    } else if (p.visible_ends != nullptr) {
-        for (unsigned int r = row0; r <= last_row; ++r) { // uniform over the workgroup: scalar loads
-            t_end = max(t_end, min(p.visible_ends[r], p.position + p.rows));
-        }
+    if (p.visible_ends != nullptr) {
+        given_range(p, row0, last_row, lane, t_begin, t_end);
     }
     if (p.window != 0 && p.visible_starts == nullptr) {
         const unsigned int first_pos = p.position + row0 + 1u;
@@ -247,9 +289,14 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
             for (int ks = 0; ks < 4; ++ks) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float x = col_valid[ct] ? load_as_f32(p.q, ((size_t)r * p.num_heads + col_head[ct]) * kD + ks * 32 + j * 8 + e, p.q_dtype) : 0.0f;
-                    qx[ct][ks][e] = x;
-                    q_amax = fmaxf(q_amax, fabsf(x));
+                    qx[ct][ks][e] = 0.0f;
+                }
+                if (col_valid[ct]) {
+                    load_query8(p.q, ((size_t)r * p.num_heads + col_head[ct]) * kD + ks * 32 + j * 8, p.q_dtype, qx[ct][ks]);
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    q_amax = fmaxf(q_amax, fabsf(qx[ct][ks][e]));
                 }
             }
         }
@@ -718,8 +765,7 @@ template <int D> struct TileShape {
     static constexpr int kRow = D * 2;            // bytes of one token of one KV head as f16
     static constexpr int kTile = kStep * kRow;    // one 32-token tile
     static constexpr int kChunks = D / 8;         // 16-byte chunks per row
-    static constexpr int kCT = D == 256 ? 1 : 2;  // 16-column MFMA tiles per wave
-    static constexpr int kCols = 8 * 16 * kCT;    // (row, head-in-group) pairs per workgroup
+    static constexpr int kCT = D == 256 ? 1 : 2;  // 16-column MFMA tiles per wave (128 (row, head-in-group) pairs per workgroup each)
     static constexpr int kKS = D / 32;            // k-steps of the score product
     static constexpr int kDT = D / 16;            // 16-dim tiles of the output
     static constexpr int kLoads = kChunks / 8;    // staging loads per thread and step (16 bytes of f16, or 8 codes)
@@ -728,11 +774,11 @@ template <int D> struct TileShape {
 };
 
 // KV: 0 = Q8g64 (SDT names the scale type: bf16, f16 or f32), 1 = f16 rows
-template <int D, int KV, int SDT, bool SOFTCAP, bool POW2>
+// CT: 16-column MFMA tiles per wave, TileShape<D>::kCT or, for f16 rows at head_dim 128, one (gqa_prefill_half_tiles)
+template <int D, int KV, int SDT, bool SOFTCAP, bool POW2, int CT = TileShape<D>::kCT>
 __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
 {
     using C = TileShape<D>;
-    constexpr int CT = C::kCT;
     constexpr int G = C::kG;
     constexpr bool Q8 = KV == 0;
     static_assert(C::kLoads >= 1, "a staging thread owns at least one chunk");
@@ -763,7 +809,7 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
     // the short tiles of the first ones had finished: a first chunk of 4,096 rows took 495 us instead of 300), and the
     // KV head is the fast index, so that with eight KV heads every XCD reads the cache of one.
     const unsigned int kvh = blockIdx.x % p.num_kv_heads;
-    const unsigned int rows_per_wg = max(1u, (unsigned int)C::kCols / p.group);
+    const unsigned int rows_per_wg = max(1u, 128u * CT / p.group);
     const unsigned int row0 = (gridDim.x / p.num_kv_heads - 1u - blockIdx.x / p.num_kv_heads) * rows_per_wg;
     const unsigned int cols_used = rows_per_wg * p.group;
 
@@ -771,18 +817,8 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
     const unsigned int last_row = min(row0 + rows_per_wg, p.rows) - 1u;
     unsigned int t_end = p.position + last_row + 1u;
     unsigned int t_begin = 0;
-    if (p.visible_starts != nullptr) { // explicit ranges (src/attention/block.rs:10-16): the union of the rows' own
-        t_end = 0u;
-        t_begin = 0xffffffffu;
-        for (unsigned int r = row0; r <= last_row; ++r) {
-            const unsigned int given_end = min(p.visible_ends[r], p.position + p.rows);
-            t_end = max(t_end, given_end);
-            t_begin = min(t_begin, min(p.visible_starts[r], given_end));
-        }
-    } else if (p.visible_ends != nullptr) {
-        for (unsigned int r = row0; r <= last_row; ++r) {
-            t_end = max(t_end, min(p.visible_ends[r], p.position + p.rows));
-        }
+    if (p.visible_ends != nullptr) {
+        given_range(p, row0, last_row, lane, t_begin, t_end);
     }
     if (p.window != 0 && p.visible_starts == nullptr) {
         const unsigned int first_pos = p.position + row0 + 1u;
@@ -817,15 +853,26 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
             col_head[ct] = kvh * p.group + col % p.group;
             col_valid[ct] = col < cols_used && r < p.rows;
         }
-        // two passes over the query (maximum, then conversion): keeping all of it in f32 would not fit the registers
+        // the 16-bit query as it is first, for its maximum, then converted in place: all of it in f32 would not fit the registers
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
 #pragma unroll
             for (int ks = 0; ks < C::kKS; ++ks) {
+                qf[ct][ks].u = u32x4{0u, 0u, 0u, 0u};
+                if (col_valid[ct]) {
+                    qf[ct][ks].u = *(const u32x4*)((const unsigned short*)p.q + ((size_t)col_row[ct] * p.num_heads + col_head[ct]) * D + ks * 32 + j * 8);
+                }
+            }
+        }
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+#pragma unroll
+            for (int ks = 0; ks < C::kKS; ++ks) {
+                float x[8];
+                widen8(qf[ct][ks].u, p.q_dtype, x);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float x = col_valid[ct] ? load_as_f32(p.q, ((size_t)col_row[ct] * p.num_heads + col_head[ct]) * D + ks * 32 + j * 8 + e, p.q_dtype) : 0.0f;
-                    q_amax = fmaxf(q_amax, fabsf(x));
+                    q_amax = fmaxf(q_amax, fabsf(x[e]));
                 }
             }
         }
@@ -839,12 +886,11 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
         for (int ct = 0; ct < CT; ++ct) {
 #pragma unroll
             for (int ks = 0; ks < C::kKS; ++ks) {
+                float x[8];
+                widen8(qf[ct][ks].u, p.q_dtype, x);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const size_t at = ((size_t)col_row[ct] * p.num_heads + col_head[ct]) * D + ks * 32 + j * 8 + 2 * e;
-                    const float x0 = col_valid[ct] ? load_as_f32(p.q, at, p.q_dtype) : 0.0f;
-                    const float x1 = col_valid[ct] ? load_as_f32(p.q, at + 1, p.q_dtype) : 0.0f;
-                    qf[ct][ks].u[e] = pack_f16_hw(x0 * q_mul, x1 * q_mul);
+                    qf[ct][ks].u[e] = pack_f16_hw(x[2 * e] * q_mul, x[2 * e + 1] * q_mul);
                 }
             }
         }
@@ -970,6 +1016,7 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
     float run_max[CT], run_sum[CT], ref_shift[CT];
     unsigned int vis_lo[CT], vis_hi[CT];
     unsigned int wave_min_hi = 0xffffffffu, wave_max_lo = 0u;
+    unsigned int wave_max_hi = 0u, wave_min_lo = 0xffffffffu; // tokens outside [min_lo, max_hi) are nobody's in the wave
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
         run_max[ct] = kNegInf;
@@ -988,14 +1035,20 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
         vis_lo[ct] = lo;
         wave_min_hi = min(wave_min_hi, vis_hi[ct]);
         wave_max_lo = max(wave_max_lo, vis_lo[ct]);
+        wave_max_hi = max(wave_max_hi, vis_hi[ct]);
+        wave_min_lo = min(wave_min_lo, col_valid[ct] ? vis_lo[ct] : 0xffffffffu);
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         wave_min_hi = min(wave_min_hi, (unsigned int)__shfl_xor((int)wave_min_hi, off));
         wave_max_lo = max(wave_max_lo, (unsigned int)__shfl_xor((int)wave_max_lo, off));
+        wave_max_hi = max(wave_max_hi, (unsigned int)__shfl_xor((int)wave_max_hi, off));
+        wave_min_lo = min(wave_min_lo, (unsigned int)__shfl_xor((int)wave_min_lo, off));
     }
     wave_min_hi = __builtin_amdgcn_readfirstlane(wave_min_hi);
     wave_max_lo = __builtin_amdgcn_readfirstlane(wave_max_lo);
+    wave_max_hi = __builtin_amdgcn_readfirstlane(wave_max_hi);
+    wave_min_lo = __builtin_amdgcn_readfirstlane(wave_min_lo);
 
     // LDS byte offsets of the lane's fragments as finished sums.  K: chunk 4 ks + j of row m; the swizzle permutes
     // ks inside a group of four, so four registers serve every k-step (ks / 4 selects 256 bytes further, an immediate).
@@ -1207,7 +1260,11 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
                 v_shift = kPBias + (float)(127 - (int)wv);
             }
         }
-        compute_step(buf, t0, v_shift, acc_fix, window_moved);
+        // A tile of packed segments walks the union of its rows' ranges, a wave only what some row of its own sees (a step
+        // whose every score is masked leaves maximum, sum and accumulators as they are unless the V window moved).
+        if (window_moved || (t0 < wave_max_hi && t0 + kStep > wave_min_lo)) {
+            compute_step(buf, t0, v_shift, acc_fix, window_moved);
+        }
     };
     auto two_steps = [&](unsigned int step, int set) __attribute__((always_inline)) {
         const unsigned int t0 = part.begin + step * kStep;
@@ -1284,19 +1341,22 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
     }
 }
 
-template <int D, int KV, int SDT> static hipError_t launch_prefill_tiles(const GqaPrefillParams& p, hipStream_t stream)
+template <int D, int KV, int SDT, int CT = TileShape<D>::kCT> static hipError_t launch_prefill_tiles(const GqaPrefillParams& p, hipStream_t stream)
 {
-    const unsigned int cols = TileShape<D>::kCols;
+    if (p.q_dtype == 0) {
+        return hipErrorInvalidValue; // the tiles hold a 16-bit query; f32 ones run as decode items
+    }
+    const unsigned int cols = 128u * CT;
     const unsigned int rows_per_wg = p.group >= cols ? 1u : cols / p.group;
     const dim3 grid((p.rows + rows_per_wg - 1) / rows_per_wg * p.num_kv_heads, 1, p.max_chunks > 1u ? p.max_chunks : 1u);
     const bool cap = p.softcap > 0.0f;
     const bool pow2 = (p.block_tokens & (p.block_tokens - 1u)) == 0 && p.table != nullptr;
     if (cap) {
-        pow2 ? gqa_prefill_tiles<D, KV, SDT, true, true><<<grid, dim3(512), 0, stream>>>(p)
-             : gqa_prefill_tiles<D, KV, SDT, true, false><<<grid, dim3(512), 0, stream>>>(p);
+        pow2 ? gqa_prefill_tiles<D, KV, SDT, true, true, CT><<<grid, dim3(512), 0, stream>>>(p)
+             : gqa_prefill_tiles<D, KV, SDT, true, false, CT><<<grid, dim3(512), 0, stream>>>(p);
     } else {
-        pow2 ? gqa_prefill_tiles<D, KV, SDT, false, true><<<grid, dim3(512), 0, stream>>>(p)
-             : gqa_prefill_tiles<D, KV, SDT, false, false><<<grid, dim3(512), 0, stream>>>(p);
+        pow2 ? gqa_prefill_tiles<D, KV, SDT, false, true, CT><<<grid, dim3(512), 0, stream>>>(p)
+             : gqa_prefill_tiles<D, KV, SDT, false, false, CT><<<grid, dim3(512), 0, stream>>>(p);
     }
     return hipGetLastError();
 }
@@ -1304,14 +1364,17 @@ template <int D, int KV, int SDT> static hipError_t launch_prefill_tiles(const G
 } // namespace
 
 bool gqa_prefill_half_tiles(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
-                            unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype)
+                            unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges)
 {
-    if (kv_format != 0 || head_dim != (unsigned int)kD || scale_dtype == 2 || num_kv_heads == 0) {
-        return false; // not gqa_prefill_q8's geometry
+    if (head_dim != (unsigned int)kD || (kv_format == 0 && scale_dtype == 2) || num_kv_heads == 0) {
+        return false; // neither gqa_prefill_q8's geometry nor f16 rows of head_dim 128
     }
     const unsigned int group = num_heads / num_kv_heads;
     if (group == 0 || group > 128u) {
         return false;
+    }
+    if (kv_format == 1 && ranges) {
+        return true; // packed segments: a smaller tile meets fewer of them, and there are twice as many tiles
     }
     if (q_dtype == 0) {
         return true; // f32 queries travel as two f16 fragments: a wave has the registers for one column tile of them
@@ -1332,6 +1395,10 @@ bool gqa_prefill_half_tiles(unsigned int rows, unsigned int position, unsigned i
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scale_dtype, hipStream_t stream)
 {
     if (kv_format == 1) { // f16 rows
+        if (p.head_dim == 128u && gqa_prefill_half_tiles(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scale_dtype, p.q_dtype,
+                                                         p.visible_starts != nullptr)) {
+            return launch_prefill_tiles<128, 1, 0, 1>(p, stream);
+        }
         if (p.head_dim == 128u) {
             return launch_prefill_tiles<128, 1, 0>(p, stream);
         }
@@ -1358,7 +1425,8 @@ hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scal
         return launch_prefill_tiles<128, 0, 2>(p, stream);
     }
     const unsigned int full_rows = p.group >= 256u ? 1u : 256u / p.group;
-    const bool halves = gqa_prefill_half_tiles(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scale_dtype, p.q_dtype);
+    const bool halves = gqa_prefill_half_tiles(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scale_dtype, p.q_dtype,
+                                               p.visible_starts != nullptr);
     const unsigned int rows_per_wg = halves ? (p.group >= 128u ? 1u : 128u / p.group) : full_rows;
     const dim3 grid((p.rows + rows_per_wg - 1) / rows_per_wg * p.num_kv_heads, 1, p.max_chunks > 1u ? p.max_chunks : 1u);
     const bool cap = p.softcap > 0.0f;
