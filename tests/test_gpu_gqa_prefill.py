@@ -250,6 +250,19 @@ def test_prefill_value_magnitudes(rule, exponent):
     print("spike", _close_at_scale(*run_case(44, 600, 90, 8, 2, rule=rule, v_gain=spike), "one large row"))
 
 
+@pytest.mark.parametrize("prefix,chunk,hq,hkv,extra", [(0, 1, 8, 2, {}), (0, 16, 8, 2, {}), (0, 33, 8, 2, {}), (0, 64, 2, 2, {}), (0, 65, 2, 2, {}),
+                                                       (0, 97, 64, 1, {}), (40, 161, 12, 4, {}), (31, 16, 8, 2, {"softcap": 30.0}), (3000, 9, 14, 2, {}),
+                                                       (3000, 9, 14, 2, {"workspace": False}), (200, 16, 8, 2, {"window": 70}), (0, 200, 8, 2, {"gate_cols": 1})])
+def test_prefill_waves_share_a_range(prefix, chunk, hq, hkv, extra):
+    """Chunks whose row tiles have 64 pairs, where half of a workgroup's waves take the odd 32-token tiles of the range: ranges of
+    one tile, of an even and an odd number of tiles, KV splits of them, and V rows whose magnitude changes by 2^9 from tile to
+    tile, so that the two halves meet with different maxima and V windows."""
+    tile = np.arange(prefix + chunk) // 32
+    for gain in (1.0, np.where(tile % 2 == 0, 2.0**9, 1.0), np.where(tile % 2 == 1, 2.0**9, 1.0)):
+        out, want = run_case(500 + prefix + chunk, prefix, chunk, hq, hkv, v_gain=gain, outliers=True, **extra)
+        _close_at_scale(out, want, f"prefix={prefix} chunk={chunk} {hq}/{hkv}")
+
+
 @pytest.mark.parametrize("q_exp,k_exp", [(12, -12), (-14, 14), (20, 0), (0, -20), (-9, -9)])
 def test_prefill_query_and_key_magnitudes(q_exp, k_exp):
     """Queries and keys far from unit magnitude with the score scale compensating: the kernel multiplies its query

@@ -201,9 +201,14 @@ __device__ __forceinline__ void store_split_record(const GqaPrefillParams& p, un
 // fragment read from LDS feeds two MFMAs; one makes it 128 pairs, for chunks whose full-size row tiles would be one round
 // of very unequal workgroups (a first chunk: the last tile walks the whole chunk, the first 64 keys) -- twice as many
 // workgroups, handed out longest first, even that out.
-template <int SDT, bool SOFTCAP, bool POW2, int CT = 2, bool QLO = false>
+// KS (with CT == 1): waves 0..3 and 4..7 own the same 64 pairs, the first four attend the even tiles of the range and the
+// others the odd ones, each with its own maximum, sum and V window; the halves meet in LDS at the end.  A launch of at most
+// a workgroup per compute unit lasts as long as its longest range, step after step, with two waves a SIMD to hide each
+// other's latencies: half the steps for half the pairs lets the short ranges fill the other half of that time.
+template <int SDT, bool SOFTCAP, bool POW2, int CT = 2, bool QLO = false, bool KS = false>
 __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
 {
+    static_assert(!KS || CT == 1, "a range is shared by waves of one column tile");
     constexpr int kColTiles = CT; // inside the kernel the name means this instantiation's count
     // Four tile buffers: a pass of the main loop attends two 32-token tiles (buffers 2 s and 2 s + 1) while the next two
     // are loaded, converted and stored into the other pair, with one barrier per 64 tokens.
@@ -227,6 +232,8 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
     const unsigned int tid = threadIdx.x;
     const unsigned int lane = tid & 63u;
     const unsigned int wave = tid >> 6;
+    const unsigned int col_wave = KS ? wave & 3u : wave; // whose columns
+    const unsigned int odd = KS ? wave >> 2 : 0u;        // which tile of a pair of tiles
     const unsigned int m = lane & 15u;
     const unsigned int j = lane >> 4;
     // Workgroups are handed out in the order of their linear index: the row tile is the slow index and the one with the
@@ -234,7 +241,7 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
     // the short tiles of the first ones had finished: a first chunk of 4,096 rows took 495 us instead of 300), and the
     // KV head is the fast index, so that with eight KV heads every XCD reads the cache of one.
     const unsigned int kvh = blockIdx.x % p.num_kv_heads;
-    const unsigned int rows_per_wg = max(1u, (128u * CT) / p.group);
+    const unsigned int rows_per_wg = max(1u, (KS ? 64u : 128u * CT) / p.group);
     const unsigned int row0 = (gridDim.x / p.num_kv_heads - 1u - blockIdx.x / p.num_kv_heads) * rows_per_wg;
     const unsigned int cols_used = rows_per_wg * p.group;
 
@@ -255,8 +262,8 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
     if (!part.live) {
 #pragma unroll
         for (int ct = 0; ct < kColTiles; ++ct) {
-            const unsigned int col = wave * (16u * kColTiles) + ct * 16u + m;
-            if (col < cols_used && row0 + col / p.group < p.rows && j == 0) {
+            const unsigned int col = col_wave * (16u * kColTiles) + ct * 16u + m;
+            if (col < cols_used && row0 + col / p.group < p.rows && j == 0 && odd == 0u) {
                 store_empty_record(p, row0 + col / p.group, kvh * p.group + col % p.group);
             }
         }
@@ -280,7 +287,7 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
         float q_amax = 0.0f;
 #pragma unroll
         for (int ct = 0; ct < kColTiles; ++ct) {
-            const unsigned int col = wave * (16u * kColTiles) + ct * 16u + m;
+            const unsigned int col = col_wave * (16u * kColTiles) + ct * 16u + m;
             const unsigned int r = row0 + col / p.group;
             col_row[ct] = r;
             col_head[ct] = kvh * p.group + col % p.group;
@@ -397,7 +404,7 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
     };
     // (biased) exponent of the largest V scale of the tile in `buf`, folded into the running one
     auto window_of = [&](int buf, unsigned int wv) __attribute__((always_inline)) -> unsigned int {
-        const f32x4 tops = *(const f32x4*)&lds_top[buf][4];
+        const f32x4 tops = *(const f32x4*)&lds_top[buf + odd][4];
         const float top = fmaxf(fmaxf(tops[0], tops[1]), fmaxf(tops[2], tops[3]));
         return max(wv, (unsigned int)__builtin_amdgcn_readfirstlane(window_exponent(top)));
     };
@@ -452,6 +459,7 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
     // parts from the optimizer, which would otherwise split the sums again to save the registers.
     unsigned int qk_at[2][2], pv_at[2][4];
     const unsigned int tr_row = 4u * j + (m >> 2);
+    const unsigned int odd_scales = 4u * j + odd * (2u * kStep); // KS: a tile further in the scales too
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
         const unsigned int qk_group = g == 0 ? (m & 1u) * 128u : 128u - (m & 1u) * 128u;
@@ -459,11 +467,17 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             qk_at[g][h] = m * kRowBytes + ((((unsigned int)h << 2 | j) ^ (m & 6u)) << 4) + qk_group;
+            if constexpr (KS) {
+                qk_at[g][h] += odd * kTileBytes;
+            }
             asm volatile("" : "+v"(qk_at[g][h]));
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             pv_at[g][q] = tr_row * kRowBytes + ((((unsigned int)q << 1 | ((m & 3u) >> 1)) ^ (tr_row & 6u)) << 4) + (m & 1u) * 8u + pv_group;
+            if constexpr (KS) {
+                pv_at[g][q] += odd * kTileBytes;
+            }
             asm volatile("" : "+v"(pv_at[g][q]));
         }
     }
@@ -485,7 +499,7 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
                 Frag k0, k1;
                 k0.u = *(const u32x4*)(kt + qk_at[g][0] + i * 16 * kRowBytes);
                 k1.u = *(const u32x4*)(kt + qk_at[g][1] + i * 16 * kRowBytes);
-                const f32x4 gs = *(const f32x4*)(&lds_ks[buf][g][i * 16 + 4 * j]);
+                const f32x4 gs = *(const f32x4*)(&lds_ks[buf][g][i * 16 + (KS ? odd_scales : 4 * j)]);
 #pragma unroll
                 for (int ct = 0; ct < kColTiles; ++ct) {
                     f32x4 d = {0.f, 0.f, 0.f, 0.f};
@@ -522,8 +536,8 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
         load_vfrags(vf[0], 0);
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-            gsv[g][0] = *(const f32x4*)(&lds_vs[buf][g][4 * j]);
-            gsv[g][1] = *(const f32x4*)(&lds_vs[buf][g][16 + 4 * j]);
+            gsv[g][0] = *(const f32x4*)(&lds_vs[buf][g][KS ? odd_scales : 4 * j]);
+            gsv[g][1] = *(const f32x4*)(&lds_vs[buf][g][16 + (KS ? odd_scales : 4 * j)]);
         }
         PREFILL_PHASE_FENCE();
         // ---- online softmax per column --------------------------------------------------------------
@@ -665,44 +679,105 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
         }
         compute_step(buf, t0, v_shift, acc_fix, window_moved);
     };
-    // Tiles `step` and `step + 1` are in the buffers of `set`; the two after them travel, one at a time through the same
-    // registers, into the other pair, which nobody reads before the barrier.
-    auto two_steps = [&](unsigned int step, int set) __attribute__((always_inline)) {
-        const unsigned int t0 = part.begin + step * kStep;
-        // rows past the end of the visible range repeat its last one: the loads stay inside the sequence's pages
-        load_step(regs, t0 + 2u * kStep, entry_next);
-        entry_next = entry_of(t0 + 3u * kStep + st_token);
-        attend_tile(t0, 2 * set);
-        store_step(regs, 2 * (set ^ 1));
-        PREFILL_PHASE_FENCE(); // the two tiles are attended one after the other: interleaved, their operands do not fit the registers
-        load_step(regs, t0 + 3u * kStep, entry_next);
-        entry_next = entry_of(t0 + 4u * kStep + st_token);
-        attend_tile(t0 + kStep, 2 * set + 1);
-        store_step(regs, 2 * (set ^ 1) + 1);
-        __syncthreads();
-    };
-    unsigned int step = 0;
-    for (; step + 4 <= steps; step += 4) {
-        two_steps(step, 0);
-        two_steps(step + 2u, 1);
-    }
-    if (step + 2 <= steps) {
-        two_steps(step, 0);
-        step += 2;
-        if (step < steps) { // the odd tile at the end sits in the first buffer of the other pair
-            attend_tile(part.begin + step * kStep, 2);
+    if constexpr (KS) {
+        // one pass: tiles `step` and `step + 1` of the buffers of `set`, one to each half of the waves; the two after them
+        // travel meanwhile.  A range of an odd number of tiles leaves the odd waves out of its last pass.
+        StepRegs regs_odd;
+        unsigned int entry_odd = entry_of(part.begin + 3u * kStep + st_token);
+        auto pass = [&](unsigned int step, int set) __attribute__((always_inline)) {
+            const unsigned int t0 = part.begin + step * kStep;
+            const bool more = step + 2u < steps;
+            if (more) {
+                load_step(regs, t0 + 2u * kStep, entry_next);
+                load_step(regs_odd, t0 + 3u * kStep, entry_odd);
+                entry_next = entry_of(t0 + 4u * kStep + st_token);
+                entry_odd = entry_of(t0 + 5u * kStep + st_token);
+            }
+            if (step + odd < steps) {
+                attend_tile(t0 + odd * kStep, 2 * set);
+            }
+            if (more) {
+                store_step(regs, 2 * (set ^ 1));
+                store_step(regs_odd, 2 * (set ^ 1) + 1);
+            }
+            __syncthreads();
+        };
+        for (unsigned int step = 0; step < steps; step += 4) {
+            pass(step, 0);
+            if (step + 2u < steps) {
+                pass(step + 2u, 1);
+            }
         }
-    } else if (step < steps) {
-        attend_tile(part.begin + step * kStep, 0);
+    } else {
+        // Tiles `step` and `step + 1` are in the buffers of `set`; the two after them travel, one at a time through the same
+        // registers, into the other pair, which nobody reads before the barrier.
+        auto two_steps = [&](unsigned int step, int set) __attribute__((always_inline)) {
+            const unsigned int t0 = part.begin + step * kStep;
+            // rows past the end of the visible range repeat its last one: the loads stay inside the sequence's pages
+            load_step(regs, t0 + 2u * kStep, entry_next);
+            entry_next = entry_of(t0 + 3u * kStep + st_token);
+            attend_tile(t0, 2 * set);
+            store_step(regs, 2 * (set ^ 1));
+            PREFILL_PHASE_FENCE(); // the two tiles are attended one after the other: interleaved, their operands do not fit the registers
+            load_step(regs, t0 + 3u * kStep, entry_next);
+            entry_next = entry_of(t0 + 4u * kStep + st_token);
+            attend_tile(t0 + kStep, 2 * set + 1);
+            store_step(regs, 2 * (set ^ 1) + 1);
+            __syncthreads();
+        };
+        unsigned int step = 0;
+        for (; step + 4 <= steps; step += 4) {
+            two_steps(step, 0);
+            two_steps(step + 2u, 1);
+        }
+        if (step + 2 <= steps) {
+            two_steps(step, 0);
+            step += 2;
+            if (step < steps) { // the odd tile at the end sits in the first buffer of the other pair
+                attend_tile(part.begin + step * kStep, 2);
+            }
+        } else if (step < steps) {
+            attend_tile(part.begin + step * kStep, 0);
+        }
     }
 
     // ---- normalise and store ------------------------------------------------------------------------
 #pragma unroll
     for (int ct = 0; ct < kColTiles; ++ct) {
-        const float total = wave_sum_16x4(run_sum[ct]);
+        float total = wave_sum_16x4(run_sum[ct]);
+        if constexpr (KS) { // the last pass ended with a barrier: nobody reads the tiles any more
+            static_assert(sizeof(lds.k) >= 4 * 8 * 64 * sizeof(f32x4) && sizeof(lds.v) >= 4 * 3 * 64 * sizeof(float), "the odd waves' state fits the tiles");
+            f32x4* const far_acc = (f32x4*)&lds_k[0][0] + col_wave * (8u * 64u) + lane;
+            float* const far = (float*)&lds_v[0][0] + col_wave * (3u * 64u) + lane;
+            if (odd != 0u) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    far_acc[t * 64] = acc[ct][t];
+                }
+                far[0] = run_max[ct];
+                far[64] = total;
+                far[128] = v_shift;
+            }
+            __syncthreads();
+            if (odd != 0u) {
+                return;
+            }
+            // to the larger maximum and the smaller of the two powers of two: both factors are at most one
+            const float far_max = far[0], far_shift = far[128];
+            const float top = fmaxf(run_max[ct], far_max), shift = fminf(v_shift, far_shift);
+            const float near_by = run_max[ct] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(run_max[ct] - top + (shift - v_shift));
+            const float far_by = far_max == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(far_max - top + (shift - far_shift));
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                acc[ct][t] = acc[ct][t] * near_by + far_acc[t * 64] * far_by;
+            }
+            total = total * near_by + far[64] * far_by;
+            run_max[ct] = top;
+            v_shift = shift;
+        }
         {
             // recomputed rather than kept: these would sit in registers through the whole main loop
-            const unsigned int col = wave * (16u * kColTiles) + ct * 16u + m;
+            const unsigned int col = col_wave * (16u * kColTiles) + ct * 16u + m;
             col_row[ct] = row0 + col / p.group;
             col_head[ct] = kvh * p.group + col % p.group;
             col_valid[ct] = col < cols_used && col_row[ct] < p.rows;
@@ -774,7 +849,7 @@ template <int D> struct TileShape {
 };
 
 // KV: 0 = Q8g64 (SDT names the scale type: bf16, f16 or f32), 1 = f16 rows
-// CT: 16-column MFMA tiles per wave, TileShape<D>::kCT or, for f16 rows at head_dim 128, one (gqa_prefill_half_tiles)
+// CT: 16-column MFMA tiles per wave, TileShape<D>::kCT or, for f16 rows at head_dim 128, one (gqa_prefill_tile_pairs)
 template <int D, int KV, int SDT, bool SOFTCAP, bool POW2, int CT = TileShape<D>::kCT>
 __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
 {
@@ -1363,40 +1438,49 @@ template <int D, int KV, int SDT, int CT = TileShape<D>::kCT> static hipError_t 
 
 } // namespace
 
-bool gqa_prefill_half_tiles(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
-                            unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges)
+unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
+                                    unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges)
 {
     if (head_dim != (unsigned int)kD || (kv_format == 0 && scale_dtype == 2) || num_kv_heads == 0) {
-        return false; // neither gqa_prefill_q8's geometry nor f16 rows of head_dim 128
+        return head_dim == 256u ? 128u : 256u; // neither gqa_prefill_q8's geometry nor f16 rows of head_dim 128
     }
     const unsigned int group = num_heads / num_kv_heads;
     if (group == 0 || group > 128u) {
-        return false;
+        return 256u;
     }
     if (kv_format == 1 && ranges) {
-        return true; // packed segments: a smaller tile meets fewer of them, and there are twice as many tiles
+        return 128u; // packed segments: a smaller tile meets fewer of them, and there are twice as many tiles
     }
     if (q_dtype == 0) {
-        return true; // f32 queries travel as two f16 fragments: a wave has the registers for one column tile of them
+        return 128u; // f32 queries travel as two f16 fragments: a wave has the registers for one column tile of them
     }
-    if ((unsigned long long)rows * group <= 128u) {
-        return true; // the whole chunk fits a half tile: a full one would be half empty at least
+    const bool can_share = kv_format == 0 && group <= 64u; // gqa_prefill_q8 with KS
+    const unsigned long long pairs = (unsigned long long)rows * group;
+    if (pairs <= 128u) {
+        return can_share && pairs <= 64u ? 64u : 128u; // the whole chunk fits the tile: a larger one would be half empty at least
     }
-    if (window != 0u) {
-        return false;
+    if (window != 0u || (unsigned long long)position * 4u > rows) {
+        return 256u;
     }
-    const unsigned int full_rows = 256u / group;
-    const unsigned long long full_tiles = ((unsigned long long)rows + full_rows - 1) / full_rows * num_kv_heads;
     // measured on 32 query / 8 KV heads: 2,048 rows at position 0 140 -> 122 us, 256 rows 40 -> 26 us; at position 1,024
     // (ranges 1 : 3) the half tiles' dearer steps cost what the evening out gains, 190 -> 200 us
-    return full_tiles <= kComputeUnitsPrefill && (unsigned long long)position * 4u <= rows;
+    auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
+    // Tiles of 64 stage every key for half the pairs: 1,000 rows (250 tiles of 128) 70.6 -> 62.0 us, 2,048 rows of 16 / 4
+    // heads 102.6 -> 89.4, 256 rows 35.4 -> 25.2; beyond a workgroup per compute unit the staging shows, 1,040 rows (264 tiles
+    // of 128) 82 -> 94, 2,000 rows 115 -> 157.  Capped at 128 registers for two workgroups a compute unit they spill inside
+    // the loop and take twice as long.
+    if (can_share && tiles_of(128u) <= kComputeUnitsPrefill) {
+        return 64u;
+    }
+    return tiles_of(256u) <= kComputeUnitsPrefill ? 128u : 256u;
 }
 
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scale_dtype, hipStream_t stream)
 {
+    const unsigned int tile_pairs = gqa_prefill_tile_pairs(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scale_dtype,
+                                                           p.q_dtype, p.visible_starts != nullptr);
     if (kv_format == 1) { // f16 rows
-        if (p.head_dim == 128u && gqa_prefill_half_tiles(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scale_dtype, p.q_dtype,
-                                                         p.visible_starts != nullptr)) {
+        if (p.head_dim == 128u && tile_pairs == 128u) {
             return launch_prefill_tiles<128, 1, 0, 1>(p, stream);
         }
         if (p.head_dim == 128u) {
@@ -1424,10 +1508,7 @@ hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scal
     if (scale_dtype == 2) { // f32 scales at head_dim 128: the tile kernel (gqa_prefill_q8 reads 16-bit scales)
         return launch_prefill_tiles<128, 0, 2>(p, stream);
     }
-    const unsigned int full_rows = p.group >= 256u ? 1u : 256u / p.group;
-    const bool halves = gqa_prefill_half_tiles(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scale_dtype, p.q_dtype,
-                                               p.visible_starts != nullptr);
-    const unsigned int rows_per_wg = halves ? (p.group >= 128u ? 1u : 128u / p.group) : full_rows;
+    const unsigned int rows_per_wg = p.group >= tile_pairs ? 1u : tile_pairs / p.group;
     const dim3 grid((p.rows + rows_per_wg - 1) / rows_per_wg * p.num_kv_heads, 1, p.max_chunks > 1u ? p.max_chunks : 1u);
     const bool cap = p.softcap > 0.0f;
     const bool pow2 = (p.block_tokens & (p.block_tokens - 1u)) == 0 && p.table != nullptr;
@@ -1435,9 +1516,11 @@ hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scal
     auto launch = [&](auto sdt, auto softcap, auto table_pow2) {
         constexpr int S = decltype(sdt)::value;
         constexpr bool C = decltype(softcap)::value, P = decltype(table_pow2)::value;
-        if (halves && p.q_dtype == 0) {
+        if (tile_pairs == 64u) {
+            gqa_prefill_q8<S, C, P, 1, false, true><<<grid, block, 0, stream>>>(p);
+        } else if (tile_pairs == 128u && p.q_dtype == 0) {
             gqa_prefill_q8<S, C, P, 1, true><<<grid, block, 0, stream>>>(p);
-        } else if (halves) {
+        } else if (tile_pairs == 128u) {
             gqa_prefill_q8<S, C, P, 1><<<grid, block, 0, stream>>>(p);
         } else {
             gqa_prefill_q8<S, C, P, 2><<<grid, block, 0, stream>>>(p);

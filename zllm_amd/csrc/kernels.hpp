@@ -179,13 +179,15 @@ struct MlaDecodeParams {
     unsigned int query_rows;
 };
 
-// Chunked prefill at head_dim 128 over Q8g64 rows with 16-bit scales or f16 rows: whether the chunk runs row tiles of 128
-// (row, head) pairs instead of 256.  True for a chunk whose pairs all fit the smaller tile, for f16 rows with explicit
-// ranges (`ranges`), and for a chunk that is much longer than what lies before it (its row tiles' ranges grow from almost
-// nothing to the whole chunk) when the full-size tiles would be at most one workgroup per compute unit: twice as many
-// workgroups, handed out longest first, even the launch out.  The split planner and the launcher both ask.
-bool gqa_prefill_half_tiles(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
-                            unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges);
+// (row, query head) pairs of a row tile of the chunked-prefill kernels: 256, 128 at head_dim 256, and at head_dim 128 over
+// Q8g64 rows with 16-bit scales or f16 rows 128 for f32 queries, for a chunk whose pairs all fit, for f16 rows with
+// explicit ranges (`ranges`), and for a chunk that is much longer than what lies before it (its row tiles' ranges grow
+// from almost nothing to the whole chunk) when the full-size tiles would be at most one workgroup per compute unit: twice
+// as many workgroups, handed out longest first, even the launch out.  64 where the same holds for the tiles of 128 over
+// Q8g64 rows, or all pairs fit: half of a workgroup's waves then take every other 32 tokens of the range.  The split
+// planner and the launcher both ask.
+unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
+                                    unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges);
 
 // KV heads (= waves) per GQA decode workgroup for a head dimension.
 unsigned int gqa_decode_max_waves(unsigned int head_dim);
