@@ -1448,8 +1448,12 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
     if (group == 0 || group > 128u) {
         return 256u;
     }
+    auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
     if (kv_format == 1 && ranges) {
-        return 128u; // packed segments: a smaller tile meets fewer of them, and there are twice as many tiles
+        // Packed segments: a smaller tile meets fewer of them and there are twice as many, until the full ones are most of two
+        // rounds of the device: 16 / 4 heads, 4,100 rows in one segment (260 full tiles) 323 -> 300 us, in eight 90 -> 79; 16 / 8
+        // heads, 6,000 rows (376) 485 -> 461; but 32 / 8 heads, 4,326 rows (544) 541 -> 565, 16 / 4, 8,000 rows (500) 630 -> 784.
+        return tiles_of(256u) * 2u <= kComputeUnitsPrefill * 3u ? 128u : 256u;
     }
     if (q_dtype == 0) {
         return 128u; // f32 queries travel as two f16 fragments: a wave has the registers for one column tile of them
@@ -1464,7 +1468,6 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
     }
     // measured on 32 query / 8 KV heads: 2,048 rows at position 0 140 -> 122 us, 256 rows 40 -> 26 us; at position 1,024
     // (ranges 1 : 3) the half tiles' dearer steps cost what the evening out gains, 190 -> 200 us
-    auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
     // Tiles of 64 stage every key for half the pairs: 1,000 rows (250 tiles of 128) 70.6 -> 62.0 us, 2,048 rows of 16 / 4
     // heads 102.6 -> 89.4, 256 rows 35.4 -> 25.2; beyond a workgroup per compute unit the staging shows, 1,040 rows (264 tiles
     // of 128) 82 -> 94, 2,000 rows 115 -> 157.  Capped at 128 registers for two workgroups a compute unit they spill inside
