@@ -161,3 +161,37 @@ def test_an_empty_range_gives_a_zero_row_and_bad_arguments_are_refused():
     with pytest.raises(capi.ZllmAttnError, match="visible_starts"):
         ops.gqa_prefill_chunk(q, *dev, None, 61, 8, 2, 128, 16, 0.09, window=8, visible_starts=upload(visible[:, 0].copy()),
                               visible_ends=upload(visible[:, 1].copy()))
+
+
+@pytest.mark.parametrize("kv,d,rows,q_kind", [("q8", 128, 16, "bf16"), ("q8", 128, 300, "bf16"), ("q8", 128, 300, "f32"), ("q8", 64, 16, "bf16"),
+                                              ("q8", 256, 300, "bf16"), ("f16", 128, 16, "bf16"), ("f16", 256, 300, "bf16")])
+@pytest.mark.parametrize("workspace", [True, False])
+def test_tiles_whose_every_range_ends_at_zero(kv, d, rows, q_kind, workspace):
+    """A row tile without a visible key stages nothing but rows of the call's own pages (the first one over and over: the
+    block table has no entry beyond the call's), and its output is zero; one range is given to the last row of the longer
+    calls, so that tiles with and without keys meet in one launch."""
+    from zllm_amd import capi, ops
+
+    page, hq, hkv = 16, 16, 4
+    cols, pages = hkv * d, (rows + 15) // 16
+    table = torch.arange(pages - 1, -1, -1, dtype=torch.int32, device="cuda")
+    torch.manual_seed(d + rows)
+    if kv == "q8":
+        planes = [torch.randint(-127, 128, (pages * page, cols), dtype=torch.int8, device="cuda"),
+                  torch.full((pages * page, cols // 64), 0.01, dtype=torch.float16, device="cuda")] * 2
+    else:
+        planes = [torch.randn(pages * page, cols, device="cuda").to(torch.float16), None] * 2
+    q = torch.randn((rows, hq * d), device="cuda").to(torch.float32 if q_kind == "f32" else torch.bfloat16)
+    starts = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    ends = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    if rows > 16:
+        starts[-1], ends[-1] = 3, 3 + 1
+    got = ops.gqa_prefill_chunk(q, *planes, table, 0, hq, hkv, d, page, d ** -0.5, kv_format=capi.KV_Q8G64 if kv == "q8" else capi.KV_F16,
+                                visible_starts=starts, visible_ends=ends, workspace=workspace).cpu()
+    assert not got[:-1].any()
+    if rows == 16:
+        assert not got[-1].any()
+    else:  # one key: its value row, whatever the scores
+        row = planes[2][table[0] * page + 3].float().cpu() * (0.01 if kv == "q8" else 1.0)
+        want = row.view(hkv, 1, d).expand(hkv, hq // hkv, d).reshape(-1)
+        assert (got[-1] - want).abs().max() <= 2e-3 * want.abs().max()

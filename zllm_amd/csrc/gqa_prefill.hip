@@ -105,7 +105,7 @@ __device__ __forceinline__ SplitRange split_range(const GqaPrefillParams& p, uns
 {
     SplitRange r = {t_begin, t_end, true};
     if (p.max_chunks > 1u) {
-        const unsigned int parts = min(p.max_chunks, (t_end - t_begin + p.chunk_tokens - 1u) / p.chunk_tokens);
+        const unsigned int parts = max(1u, min(p.max_chunks, (t_end - t_begin + p.chunk_tokens - 1u) / p.chunk_tokens)); // none is live in an empty range
         const unsigned int span = (((t_end - t_begin + parts - 1u) / parts) + 31u) & ~31u;
         const unsigned long long begin = (unsigned long long)t_begin + (unsigned long long)blockIdx.z * span;
         r.live = blockIdx.z < parts && begin < t_end;
@@ -341,7 +341,8 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
     const unsigned int k_row = p.num_kv_heads * kD;
     const unsigned int s_row = p.num_kv_heads * 4u; // two 16-bit scales per KV head
     const bool pow2 = POW2 || (p.block_tokens & (p.block_tokens - 1u)) == 0;
-    const unsigned int last_token = t_end - 1u;
+    // What the staging reads past the range is its last row again, and the first one where every range of the tile ends at 0
+    const unsigned int last_token = max(t_end, 1u) - 1u;
     // The block-table entry of a staging thread's token is fetched one step before the data that needs
     // it, so no step waits on a table -> data load chain.
     auto entry_of = [&](unsigned int token) __attribute__((always_inline)) -> unsigned int {
@@ -984,7 +985,7 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
     constexpr unsigned int kScaleBytes = SDT == 2 ? 4u : 2u;
     const unsigned int s_row = p.num_kv_heads * G * kScaleBytes;                                // bytes of one scale row
     const bool pow2 = POW2 || (p.block_tokens & (p.block_tokens - 1u)) == 0;
-    const unsigned int last_token = t_end - 1u;
+    const unsigned int last_token = max(t_end, 1u) - 1u; // ranges that all end at 0 stage the first row
     auto entry_of = [&](unsigned int token) __attribute__((always_inline)) -> unsigned int {
         token = min(token, last_token);
         const unsigned int page = pow2 ? token >> p.block_shift : token / p.block_tokens;
