@@ -561,6 +561,33 @@ def test_mla_matrix_core_stages_at_192_query_and_256_value_columns():
         print("mla 192/256 chunk", rows, assert_attention_close(got_c.reshape(want_c.shape), want_c, f"MLA 192/256 chunk of {rows}"))
 
 
+@pytest.mark.parametrize("nope,value", [(128, 128), (192, 256)])
+@pytest.mark.parametrize("rows,context", [(10, 700), (12, 40), (15, 1400)])
+def test_mla_projection_of_few_rows_keeps_all_bits_of_the_merged_rows(rows, context, nope, value):
+    """Ten to fifteen rows of 128 heads project on the matrix cores (at least 1,200 (row, head) pairs), split (700 and 1,400
+    tokens) or not (40).  The same records merged and projected stage by stage go through the f32 kernel; what is left between
+    the two is the order of 512 f32 additions, about 2^-25 sqrt(512 / 2) = 4.8e-7 in the 2-norm.  Merged rows of two bf16
+    terms would add 2^-18 / sqrt(3) = 2.2e-6."""
+    import ctypes as C
+
+    from zllm_amd import capi, ops
+
+    heads = 128
+    case = make_mla_case(600 + rows, [context] * rows, heads, nope=nope, value=value)
+    q, kv_b = to_torch_bf16(case["q_bits"], "cuda"), weight_args(case)[0]
+    keep = [upload(case[n]) for n in ("codes", "scales", "rope", "tables", "lens")]
+    args, out, workspace = ops.mla_decode_args(q, kv_b, *keep, heads, nope + 64, nope + value, 512, 64, case["block_tokens"], context)
+    outs = []
+    for masks in ((15,), (4, 8)):
+        for mask in masks:
+            args.stage_mask = mask
+            capi.check(capi.load().zllm_attn_mla_decode(C.byref(args), ops._stream()))
+        outs.append(out.double().cpu())
+    rel = float((outs[0] - outs[1]).norm() / outs[1].norm())
+    print("mla projection of few rows", rows, context, value, rel)
+    assert rel <= 1e-6
+
+
 def test_mla_chunk_query_types_on_the_matrix_core_absorb():
     case = make_mla_chunk_case(9, [300, 120], 20, 16)
     want_f, _ = oracle_mla_chunk(case)

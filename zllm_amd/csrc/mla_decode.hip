@@ -1910,11 +1910,14 @@ constexpr int kMergedStride = kLatent + 8; // bf16 elements: sixteen rows' 16-by
 // WAVES: 8 (value widths up to 128) or 16 (up to 256; modes 1 and 2, whose registers allow 1,024 threads).
 //
 // BITS 8 / 4: kv_b as codes, fed to the matrix cores as bf16 integers; a column group's sum is multiplied by the scale of
-// (value column, group) in f32.  The merged rows are carried as three bf16 terms there, all 24 bits of the f32.
-template <int MODE, int WAVES = 8, int BITS = 16> __global__ __launch_bounds__(64 * WAVES) void mla_merge_project_mfma(MlaDecodeParams p)
+// (value column, group) in f32.
+// TERMS: bf16 terms of a merged row.  Three hold all 24 bits of the f32 and are what codes take, and bf16 weights where the
+// call is fewer than sixteen rows: mla_merge_project, which those take below the line of matrix_project, reads the f32.
+// One more term costs 0.6 us there (12 rows of 128 heads in 2,048 tokens 17.2 -> 17.8), 6 us on 512 rows (47.3 -> 53.5).
+template <int MODE, int WAVES = 8, int BITS = 16, int TERMS = BITS == 16 ? 2 : 3>
+__global__ __launch_bounds__(64 * WAVES) void mla_merge_project_mfma(MlaDecodeParams p)
 {
     static_assert(WAVES == 8 || MODE != 0, "the record-folding form needs the registers of 512 threads");
-    constexpr int TERMS = BITS == 16 ? 2 : 3;
     constexpr unsigned int RG = WAVES / 2;  // groups of 128 threads: thread group rb takes rows rb, rb + RG, ...
     constexpr int RPT = 16 / RG;            // rows of a block per thread
     // the merged rows as bf16 terms (value = hi + lo keeps 16 bits of the f32), split once by the thread that merged them
@@ -2390,19 +2393,25 @@ hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, 
             // splits, 29.6 -> 25.7 us for 64 rows.  A long chunk keeps the fused kernel: its merged rows would cross the
             // workspace twice (134 MB each way for 512 rows).
             const dim3 grid(p.heads, row_block_groups(p));
+            const bool few = p.batch < 16u; // less than a block of rows: all of the merged rows' bits
             if (two_step) {
                 err = merge_into_workspace(p, stream);
                 if (err != hipSuccess) {
                     return err;
                 }
-                wide_values ? mla_merge_project_mfma<1, 16><<<grid, dim3(1024), 0, stream>>>(p) : mla_merge_project_mfma<1, 8><<<grid, dim3(512), 0, stream>>>(p);
+                if (wide_values) {
+                    (few ? mla_merge_project_mfma<1, 16, 16, 3> : mla_merge_project_mfma<1, 16>)<<<grid, dim3(1024), 0, stream>>>(p);
+                } else {
+                    (few ? mla_merge_project_mfma<1, 8, 16, 3> : mla_merge_project_mfma<1, 8>)<<<grid, dim3(512), 0, stream>>>(p);
+                }
             } else if (p.max_chunks == 1u && wide_values) {
-                mla_merge_project_mfma<2, 16><<<grid, dim3(1024), 0, stream>>>(p);
+                (few ? mla_merge_project_mfma<2, 16, 16, 3> : mla_merge_project_mfma<2, 16>)<<<grid, dim3(1024), 0, stream>>>(p);
             } else if (p.max_chunks == 1u) {
                 // one record a row: two workgroups of eight waves fit a compute unit, so twice the workgroups of the usual round
                 const unsigned int blocks = (p.batch + 15u) / 16u;
                 const unsigned int groups = 2u * row_block_groups(p);
-                mla_merge_project_mfma<2, 8><<<dim3(p.heads, groups < blocks ? groups : blocks), dim3(512), 0, stream>>>(p);
+                const dim3 twice(p.heads, groups < blocks ? groups : blocks);
+                (few ? mla_merge_project_mfma<2, 8, 16, 3> : mla_merge_project_mfma<2, 8>)<<<twice, dim3(512), 0, stream>>>(p);
             } else {
                 mla_merge_project_mfma<0, 8><<<grid, dim3(512), 0, stream>>>(p);
             }
