@@ -561,6 +561,48 @@ def test_mla_matrix_core_stages_at_192_query_and_256_value_columns():
         print("mla 192/256 chunk", rows, assert_attention_close(got_c.reshape(want_c.shape), want_c, f"MLA 192/256 chunk of {rows}"))
 
 
+@pytest.mark.parametrize("heads,rows", [(16, 31), (16, 32), (16, 33), (8, 64), (8, 65), (4, 128), (4, 129)])
+def test_mla_absorb_below_and_above_the_matrix_core_line(heads, rows):
+    """128 query columns: up to 512 (row, head) pairs a workgroup each, from 513 on the matrix cores.  Outputs against the
+    oracle, and the absorb alone takes about as long as that of 31 rows of 16 heads (6.5 us; 9.5 would be a second round of
+    workgroups): no size in between falls to the kernel of other query widths (29 us)."""
+    import ctypes as C
+
+    from zllm_amd import capi, ops
+
+    lens = [int(x) for x in np.random.default_rng(heads * rows).integers(1, 60, size=rows)]
+    case = make_mla_case(700 + heads + rows, lens, heads)
+    want, _ = oracle_mla(case)
+    got = run_mla(case).cpu().numpy()
+    print("mla absorb line", heads, rows, assert_attention_close(got.reshape(want.shape), want, f"MLA heads={heads} rows={rows}"))
+
+    def absorb_us(case):
+        keep = [to_torch_bf16(case["q_bits"], "cuda"), weight_args(case)[0]] + [upload(case[n]) for n in ("codes", "scales", "rope", "tables", "lens")]
+        args, _, _ = held = ops.mla_decode_args(*keep, case["heads"], 192, 256, 512, 64, case["block_tokens"], int(case["lens"].max()))
+        args.stage_mask = 1
+        call = lambda: capi.check(capi.load().zllm_attn_mla_decode(C.byref(args), ops._stream()))  # noqa: E731
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                call()
+        times = []
+        for _ in range(10):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            graph.replay()
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end) * 50.0)
+        del held
+        return min(times)
+
+    usual, here = absorb_us(make_mla_case(1, [8] * 31, 16)), absorb_us(case)
+    print("mla absorb us", heads, rows, usual, here)
+    assert here <= 2.0 * usual
+
+
 @pytest.mark.parametrize("nope,value", [(128, 128), (192, 256)])
 @pytest.mark.parametrize("rows,context", [(10, 700), (12, 40), (15, 1400)])
 def test_mla_projection_of_few_rows_keeps_all_bits_of_the_merged_rows(rows, context, nope, value):

@@ -2153,17 +2153,21 @@ static unsigned int row_block_groups(const MlaDecodeParams& p)
 // Where the matrix-core stages take over from a workgroup per (row, head), by the number of such pairs: a few hundred
 // workgroups run side by side, beyond that they queue, while the matrix-core kernels read a head's weights once for sixteen
 // rows and cost the same for one row as for sixteen.  Measured, us per pair / on the matrix cores:
-//   absorb, 128 query columns: bf16 512 pairs 5.8 / 6.4, 640 pairs 8.5 / 7.1, 1920 pairs 16.9 / 7.1; 8-bit codes 352 pairs
-//   7.3 / 8.4, 480 pairs 11.2 / 8.7; 192 query columns: bf16 128 pairs 6.3 / 5.5, 8-bit codes 128 pairs 7.3 / 7.1
+//   absorb, 128 query columns: bf16 512 pairs (16 heads) 6.7 / 7.8, 528 pairs 9.4 / 7.8, 1536 pairs 15.0 / 7.6; 8-bit codes
+//   352 pairs 7.3 / 8.4, 480 pairs 11.2 / 8.7; 192 query columns: bf16 128 pairs 7.0 / 6.8, 8-bit codes 128 pairs 8.0 / 8.4,
+//   256 pairs 9.1 / 8.4
 //   merge and projection: bf16 512 pairs 7.4 / 11.7 (sixteen rows), 832 pairs 13.3 / 12.3 (26 rows), 1024 pairs 15.1 / 16.2
 //   (eight rows: half of a tile empty), 1408 pairs 19.8 / 16.6; 8-bit codes within 2 us of these
+static bool matrix_absorb_widths(const MlaDecodeParams& p)
+{
+    return (p.q_head_dim & 3u) == 0 && (p.nope_dim == 128u || p.nope_dim == 192u);
+}
+
 static bool matrix_absorb(const MlaDecodeParams& p)
 {
     const unsigned int pairs = p.batch * p.heads;
-    if ((p.q_head_dim & 3u) != 0) {
-        return false;
-    }
-    return p.nope_dim == 192u ? pairs >= 128u : p.nope_dim == 128u && pairs >= (p.kv_b_bits == 16u ? 576u : 448u);
+    // bf16 weights: two workgroups a compute unit are the most that run side by side
+    return matrix_absorb_widths(p) && pairs >= (p.nope_dim == 192u ? 128u : p.kv_b_bits == 16u ? 513u : 448u);
 }
 
 static bool matrix_project(const MlaDecodeParams& p)
@@ -2311,8 +2315,6 @@ hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, 
             return err;
         }
     } else if (stages & 1u) {
-        // Other query widths: eight rows per workgroup share every weight load, and the workgroup then runs eight rows' sums:
-        // measured 28 us from 16 rows up to a few hundred, against 13 us (15 rows) to 27 us (32 rows) for one workgroup per row
         if (matrix_absorb(p)) { // sixteen rows a workgroup, on the matrix cores
             // four waves for a decode batch, sixteen for a chunk (33 against 61 us on 512 rows of 128 heads; on 16 to 64 rows
             // the larger workgroup costs 4 us); as many waves share a block of sixteen rows as keeps every wave busy
@@ -2327,7 +2329,11 @@ hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, 
                 waves == 16u ? mla_absorb_mfma<16, 192, 256><<<dim3(p.heads, groups, 2), dim3(1024), 0, stream>>>(q)
                              : mla_absorb_mfma<4, 192, 256><<<dim3(p.heads, groups, 2), dim3(256), 0, stream>>>(q);
             }
-        } else if (p.batch >= 32u && p.nope_dim <= 256u) {
+        } else if (p.batch >= 32u && p.nope_dim <= 256u && !matrix_absorb_widths(p)) {
+            // Other query widths: eight rows per workgroup share every weight load, and the workgroup then runs eight rows'
+            // sums: 28 us from 16 rows up to a few hundred, against 13 us (15 rows) to 27 us (32 rows) of 128 heads for one
+            // workgroup per row.  Where the matrix cores take over further up, one per row is the faster below that line:
+            // 16 heads x 32 rows 6.7 us against 28.9
             mla_absorb_rows<8><<<dim3(p.heads, (p.batch + 7u) / 8u), dim3(256), 0, stream>>>(p);
         } else {
             const unsigned int z = p.heads * p.batch <= 128u ? 4u : 1u;
