@@ -243,6 +243,27 @@ def test_prefill_workspace_covers_few_row_chunks_and_kv_splits(lib):
     assert sizes[1, 100] > 0                                            # still a decode item (its records are small)
 
 
+def _ranges_prefill_bytes(lib, rows, position, heads, kv_heads, kv_format, head_dim=128):
+    """Workspace of a chunk whose rows bring their own ranges (256 compute units where no device says otherwise)."""
+    starts = (C.c_uint32 * 1)()
+    pre = capi.GqaPrefillArgs(rows=rows, position=position, num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, block_tokens=16, score_scale=0.1,
+                              kv_format=kv_format, scale_dtype=capi.SCALE_F16, q_dtype=capi.DTYPE_BF16, out_dtype=capi.DTYPE_F32)
+    pre.visible_starts = pre.visible_ends = C.addressof(starts)  # the planner asks whether they are there
+    return lib.zllm_attn_gqa_prefill_workspace_bytes(C.byref(pre))
+
+
+def test_given_ranges_are_cut_into_kv_splits_behind_a_long_prefix_only(lib):
+    """Calls whose tiles fill the device: rows with nothing before them (packed segments) run unsplit, whatever their number;
+    behind a prefix the parts are kept where a round of the device saved is worth their records."""
+    for rows in (2600, 4100, 6000):
+        assert _ranges_prefill_bytes(lib, rows, 0, 16, 4, capi.KV_F16) == 0
+    for kv_format, head_dim, heads, kv_heads, rows, position in ((capi.KV_F16, 128, 16, 4, 2600, 12000), (capi.KV_F16, 128, 64, 8, 600, 12000),
+                                                                 (capi.KV_Q8G64, 128, 16, 4, 6000, 3000), (capi.KV_Q8G64, 64, 32, 8, 2600, 3000)):
+        assert _ranges_prefill_bytes(lib, rows, position, heads, kv_heads, kv_format, head_dim) > rows * heads * head_dim * 4
+    for heads, kv_heads, rows, position in ((32, 8, 2100, 1000), (16, 4, 4100, 1000)):  # 492 and 681 us cut, 365 and 547 whole
+        assert _ranges_prefill_bytes(lib, rows, position, heads, kv_heads, capi.KV_Q8G64) == 0
+
+
 def test_prefill_and_mla_argument_checks_without_a_gpu(lib):
     pre = capi.GqaPrefillArgs()
     pre.rows, pre.num_heads, pre.num_kv_heads, pre.head_dim, pre.block_tokens = 8, 8, 2, 128, 16

@@ -2,6 +2,8 @@
 `attention::block::attention_f32` (src/attention/block.rs:67-119): BlockAttentionSpec::visible, its varlen form (isolated
 segments, src/attention/block.rs:41-63) and asymmetric windows, over Q8g64 and f16 caches, through every route of the entry
 point (the chunk kernels, with and without KV splits, and rows run as decode items)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -161,6 +163,43 @@ def test_an_empty_range_gives_a_zero_row_and_bad_arguments_are_refused():
     with pytest.raises(capi.ZllmAttnError, match="visible_starts"):
         ops.gqa_prefill_chunk(q, *dev, None, 61, 8, 2, 128, 16, 0.09, window=8, visible_starts=upload(visible[:, 0].copy()),
                               visible_ends=upload(visible[:, 1].copy()))
+
+
+@pytest.mark.parametrize("kv,d,hq,hkv,prefix,rows", [("f16", 128, 64, 8, 12000, 600), ("q8", 64, 32, 8, 3000, 2600), ("q8", 128, 16, 4, 3000, 6000),
+                                                     ("f16", 256, 16, 8, 12000, 1100)])
+def test_ranges_behind_a_prefix_cut_and_whole(kv, d, hq, hkv, prefix, rows):
+    """Calls whose tiles fill the device and whose plan cuts them all the same (a prefix that most rows share): the split call
+    against the same call without a workspace, which walks every range whole.  A fifth of the rows sees a range of its own
+    inside the chunk, so that parts are empty in some tiles.  The two differ by the rounding of their probabilities to f16
+    against other references, 2^-11 each."""
+    from zllm_amd import capi, ops
+
+    page, total = 16, prefix + rows
+    cols, pages = hkv * d, (total + 15) // 16
+    torch.manual_seed(rows)
+    table = torch.randperm(pages, device="cuda").to(torch.int32)
+    if kv == "q8":
+        planes = []
+        for _ in range(2):
+            planes += [torch.zeros(pages * page, cols, dtype=torch.int8, device="cuda"), torch.zeros(pages * page, cols // 64, dtype=torch.int16, device="cuda")]
+            ops.q8g64_append(torch.randn(total, cols, device="cuda").to(torch.bfloat16), planes[-2], planes[-1], table, 0, page, capi.QUANT_METAL_GQA)
+    else:
+        planes = [torch.randn(pages * page, cols, device="cuda").to(torch.float16), None, torch.randn(pages * page, cols, device="cuda").to(torch.float16), None]
+    q = torch.randn((rows, hq * d), device="cuda").to(torch.bfloat16)
+    at = torch.arange(rows, device="cuda")
+    own = at >= rows * 4 // 5
+    starts = torch.where(own, prefix + at // 64 * 64, at % 7).to(torch.int32)
+    ends = torch.where(own, torch.clamp(prefix + at // 64 * 64 + 64, max=total), total - at % 5).to(torch.int32)
+    outs = []
+    for workspace in (True, False):
+        args, out, scratch = ops.gqa_prefill_chunk_args(q, *planes, table, prefix, hq, hkv, d, page, d ** -0.5, visible_starts=starts, visible_ends=ends,
+                                                        kv_format=capi.KV_Q8G64 if kv == "q8" else capi.KV_F16, workspace=workspace)
+        assert scratch is None or scratch.numel() > rows * hq * d * 4  # split records
+        capi.check(capi.load().zllm_attn_gqa_prefill_chunk(C.byref(args), ops._stream()))
+        outs.append(out.double())
+    rel = float((outs[0] - outs[1]).norm() / outs[1].norm())
+    print("ranges behind a prefix", kv, d, prefix, rows, rel)
+    assert rel <= 2.0 ** -11
 
 
 @pytest.mark.parametrize("kv,d,rows,q_kind", [("q8", 128, 16, "bf16"), ("q8", 128, 300, "bf16"), ("q8", 128, 300, "f32"), ("q8", 64, 16, "bf16"),

@@ -1109,14 +1109,6 @@ void plan_prefill_splits(const zllm_gqa_prefill_args* a, uint32_t* chunk_tokens,
                                                           a->scale_dtype, a->q_dtype, a->visible_starts != nullptr);
     const uint32_t tile_rows = columns / group > 0 ? columns / group : 1u;
     const uint64_t tiles = ((uint64_t)a->rows + tile_rows - 1) / tile_rows;
-    if (a->visible_starts != nullptr && tiles * a->num_kv_heads >= compute_units()) {
-        // Packed segments: a tile's range is a segment or two, not the whole of the rows, and the host does not know it.  Cut
-        // by the whole, most parts are empty and their records cost more than the attention (16 heads of 128 over 4,100 rows
-        // in nine segments: the split merge alone took 32 us).
-        *chunk_tokens = (uint32_t)align_up((uint64_t)a->position + a->rows, 32);
-        *max_chunks = 1;
-        return;
-    }
     uint64_t longest = (uint64_t)a->position + a->rows; // keys the last row tile may see
     if (a->window != 0 && (uint64_t)a->window + tile_rows + 32 < longest) {
         longest = (uint64_t)a->window + tile_rows + 32;
@@ -1129,6 +1121,23 @@ void plan_prefill_splits(const zllm_gqa_prefill_args* a, uint32_t* chunk_tokens,
         const uint64_t chunk = align_up((longest + keep - 1) / keep, 32);
         *chunk_tokens = (uint32_t)chunk;
         *max_chunks = (uint32_t)((longest + chunk - 1) / chunk);
+    }
+    const uint64_t cus = compute_units(), workgroups = tiles * a->num_kv_heads;
+    if (a->visible_starts != nullptr && workgroups >= cus && *max_chunks > 1) {
+        // Given ranges, and tiles enough for the device.  Packed segments: a tile's range is a segment or two, not the whole of
+        // the rows, and the host does not know it.  Cut by the whole, most parts are empty and their records cost more than
+        // the attention (16 heads of 128 over 4,100 rows in nine segments: the split merge alone took 32 us), so rows with
+        // nothing before them run unsplit.  Behind a prefix, which rows tend to share, the parts that even out a partly
+        // filled last round are kept where they save more than their records cost, about as long as 27 tokens of a
+        // workgroup's walk a megabyte (f16 rows, 16 / 4 heads of 128, unsplit -> split: 2,600 rows behind 12,000 664 -> 504 us,
+        // behind 1,000 189 -> 174, behind 300 159 -> 149; but 3,100 behind 6,000 430 -> 447; Q8g64 rows, 6,000 behind 3,000
+        // 918 -> 768, 4,100 behind 1,000 547 -> 681).
+        const uint64_t whole = (workgroups + cus - 1) / cus * (longest + 64);
+        const uint64_t cut = (workgroups * *max_chunks + cus - 1) / cus * ((uint64_t)*chunk_tokens + 64);
+        if (a->position == 0 || cut >= whole || (whole - cut) * 1000000 < 27 * record_bytes * *max_chunks) {
+            *chunk_tokens = (uint32_t)align_up(longest, 32);
+            *max_chunks = 1;
+        }
     }
 }
 
