@@ -260,6 +260,9 @@ def test_given_ranges_are_cut_into_kv_splits_behind_a_long_prefix_only(lib):
     for kv_format, head_dim, heads, kv_heads, rows, position in ((capi.KV_F16, 128, 16, 4, 2600, 12000), (capi.KV_F16, 128, 64, 8, 600, 12000),
                                                                  (capi.KV_Q8G64, 128, 16, 4, 6000, 3000), (capi.KV_Q8G64, 64, 32, 8, 2600, 3000)):
         assert _ranges_prefill_bytes(lib, rows, position, heads, kv_heads, kv_format, head_dim) > rows * heads * head_dim * 4
+    # f16 rows behind more keys than rows: tiles of 256 pairs, three parts of 80 (128 pairs: five of 152); few rows keep 128
+    assert 0 < _ranges_prefill_bytes(lib, 300, 12000, 64, 8, capi.KV_F16) < 4 * 300 * 64 * 128 * 4
+    assert 0 < _ranges_prefill_bytes(lib, 300, 12000, 16, 4, capi.KV_F16) < 7 * 300 * 16 * 128 * 4
     for heads, kv_heads, rows, position in ((32, 8, 2100, 1000), (16, 4, 4100, 1000)):  # 492 and 681 us cut, 365 and 547 whole
         assert _ranges_prefill_bytes(lib, rows, position, heads, kv_heads, capi.KV_Q8G64) == 0
 

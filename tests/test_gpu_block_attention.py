@@ -165,7 +165,8 @@ def test_an_empty_range_gives_a_zero_row_and_bad_arguments_are_refused():
                               visible_ends=upload(visible[:, 1].copy()))
 
 
-@pytest.mark.parametrize("kv,d,hq,hkv,prefix,rows", [("f16", 128, 64, 8, 12000, 600), ("q8", 64, 32, 8, 3000, 2600), ("q8", 128, 16, 4, 3000, 6000),
+@pytest.mark.parametrize("kv,d,hq,hkv,prefix,rows", [("f16", 128, 64, 8, 12000, 600), ("f16", 128, 16, 4, 12000, 2600),
+                                                     ("q8", 64, 32, 8, 3000, 2600), ("q8", 128, 16, 4, 3000, 6000),
                                                      ("f16", 256, 16, 8, 12000, 1100)])
 def test_ranges_behind_a_prefix_cut_and_whole(kv, d, hq, hkv, prefix, rows):
     """Calls whose tiles fill the device and whose plan cuts them all the same (a prefix that most rows share): the split call

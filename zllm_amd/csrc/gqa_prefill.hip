@@ -1450,10 +1450,13 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
         return 256u;
     }
     auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
-    if (kv_format == 1 && ranges) {
-        // Packed segments: a smaller tile meets fewer of them and there are twice as many, until the full ones are most of two
+    if (kv_format == 1 && ranges && (position <= rows || tiles_of(256u) * 5u <= kComputeUnitsPrefill)) {
+        // Packed segments: a smaller tile meets fewer of them and there are twice as many, until the full ones are one and a half
         // rounds of the device: 16 / 4 heads, 4,100 rows in one segment (260 full tiles) 323 -> 300 us, in eight 90 -> 79; 16 / 8
         // heads, 6,000 rows (376) 485 -> 461; but 32 / 8 heads, 4,326 rows (544) 541 -> 565, 16 / 4, 8,000 rows (500) 630 -> 784.
+        // Behind a prefix longer than the rows their ranges have most keys in common, and a full tile reads those for twice the
+        // rows: 16 / 4 heads, 2,600 rows behind 12,000 keys 508 -> 416, 600 rows of 64 / 8 446 -> 374.  The smaller ones stay for
+        // calls that leave the device idle: 300 rows of 16 / 4 (20 full tiles) behind 1,000 26 us against 37, behind 12,000 70 / 72.
         return tiles_of(256u) * 2u <= kComputeUnitsPrefill * 3u ? 128u : 256u;
     }
     if (q_dtype == 0) {
