@@ -106,14 +106,25 @@ def test_varlen_segments(kv, d, hq, hkv, q_kind, block_tokens):
 @pytest.mark.parametrize("kv,d", [("f16", 128), ("f16", 256), ("q8", 64), ("q8", 128)])
 @pytest.mark.parametrize("rows,heads", [(127, 8), (129, 8), (577, 64)])
 def test_segments_that_end_beside_tile_and_wave_edges(kv, d, rows, heads):
-    """One query head per KV head, so that tiles are 128 or 256 rows and waves 16 or 32 of them: segments that end one row
-    before, on and after those edges and one-key rows among them; 64 heads x 577 rows fill the device and
-    run without KV splits, the shorter calls with what the plan gives them."""
+    """One query head per KV head, so that tiles are 64, 128 or 256 rows and waves 16 or 32 of them: segments that end one
+    row before, on and after those edges and one-key rows among them; 64 heads x 577 rows fill the device and run without
+    KV splits (on tiles of 256 over Q8g64 rows of 128, of 128 over f16 rows), the shorter calls with what the plan gives them."""
     offsets = [o for o in (0, 1, 15, 17, 32, 63, 96, 127, 128, 129, 255, 257, 512, 545) if o < rows] + [rows]
     visible = varlen_ranges(offsets, offsets)
     visible[100] = (0, 1)
     out, want = run_block(200 + rows, rows, rows, heads, heads, d, visible, kv=kv)
     assert_attention_close(out, want, f"tile edges {kv} d={d} rows={rows}")
+
+
+@pytest.mark.parametrize("heads", [192, 193])
+def test_segments_on_both_sizes_of_f16_tiles(heads):
+    """Two full tiles a KV head: 384 of them, one and a half rounds of the device, still run as tiles of 128 rows, 386 as
+    tiles of 256, whose waves hold two 16-row column tiles.  Segments end beside 16, 32, 64 and 256 rows."""
+    offsets = [0, 15, 16, 31, 33, 64, 65, 127, 128, 200, 255, 257, 270]
+    visible = varlen_ranges(offsets, offsets)
+    visible[40] = (40, 41)
+    out, want = run_block(300 + heads, 270, 270, heads, heads, 128, visible, kv="f16")
+    assert_attention_close(out, want, f"f16 tiles, {heads} heads")
 
 
 @pytest.mark.parametrize("workspace", [True, False])

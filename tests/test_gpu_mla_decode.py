@@ -460,7 +460,7 @@ def run_mla_chunk(case, out_dtype=None, selection=None, compact=True, q_kind="bf
 
 
 @pytest.mark.parametrize("heads,lens,rows,block_tokens", [(16, [40], 8, 16), (128, [700, 300], 5, 16), (32, [1300, 64, 129], 64, 64),
-                                                          (20, [33, 97], 33, 16), (64, [2500], 3, 48)])
+                                                          (20, [33, 97], 33, 16), (64, [2500], 3, 48), (16, [260], 200, 16)])
 def test_mla_prefill_chunk_matches_oracle(heads, lens, rows, block_tokens):
     """Chunked MLA prefill: `rows` query rows per sequence, causal inside the chunk, f32 and bf16 output
     (the reference returns bf16 for more than one row, src/backend/rocm/attention.rs:17-19)."""
@@ -529,13 +529,31 @@ def test_mla_short_and_peaked_rows_in_the_narrow_layout(heads):
     print("mla narrow one key", heads, assert_attention_close(got_s.reshape(want_s.shape), want_s, f"MLA narrow one key heads={heads}", atol=1e-4))
 
 
+def mla_splits(case):
+    """KV splits that the plan gives the case (256 compute units)."""
+    import ctypes as C
+
+    from zllm_amd import capi
+
+    rows = case.get("rows", 1)
+    args = capi.MlaDecodeArgs(batch=len(case["lens"]), heads=case["heads"], q_head_dim=case["nope"] + case["rope_dim"],
+                              kv_head_dim=case["nope"] + case["value"], latent_dim=case["latent"], rope_dim=case["rope_dim"],
+                              table_stride=case["tables"].shape[1], max_ctx_len=int(case["lens"].max()), block_tokens=case["block_tokens"],
+                              q_dtype=capi.DTYPE_BF16, out_dtype=capi.DTYPE_F32, out_compact=1, query_rows=rows)
+    layout = capi.SplitRecordLayout()
+    capi.check(capi.load().zllm_attn_mla_decode_record_layout(C.byref(args), C.byref(layout)))
+    return layout.max_chunks
+
+
 def test_mla_batched_decode_on_the_matrix_core_stages():
-    """A decode batch of sixteen rows and more takes the matrix-core absorb and projection (one query row per sequence
-    here; chunks take them through test_mla_prefill_chunk_matches_oracle): 40 ragged sequences, strided and compact
-    output, and the query as bf16 and as f32 (one block of sixteen rows is partly empty: 40 = 2.5 blocks)."""
+    """A decode batch of 40 rows of 32 heads (1,280 (row, head) pairs) takes the matrix-core absorb and, split and of at
+    most 64 rows, the projection from merged rows (chunks take them through test_mla_prefill_chunk_matches_oracle): 40
+    ragged sequences, strided and compact output, and the query as bf16 and as f32 (one block of sixteen rows is partly
+    empty: 40 = 2.5 blocks)."""
     rng = np.random.default_rng(41)
     lens = [int(x) for x in rng.integers(1, 900, size=40)]
     case = make_mla_case(41, lens, 32)
+    assert mla_splits(case) > 1
     want_f, want_b = oracle_mla(case)
     got = run_mla(case).cpu().numpy()
     print("mla batch 40", assert_attention_close(got.reshape(want_f.shape), want_f, "MLA batch of 40"))
@@ -548,17 +566,33 @@ def test_mla_batched_decode_on_the_matrix_core_stages():
 def test_mla_matrix_core_stages_at_192_query_and_256_value_columns():
     """The reference's decode test has 192 query columns next to the rope and 256 value columns
     (src/kernel/rocm/hip/attention/paged_mla.rs:6226-6233).  The matrix-core absorb then stages half the latent columns
-    a workgroup, and the projection runs sixteen waves: a decode batch of 20 rows (split merge, then projection from
-    merged rows), a chunk of 40 rows (one record a row) and a chunk of 200 rows (sixteen-wave absorb)."""
-    case = make_mla_case(301, [int(x) for x in np.random.default_rng(301).integers(1, 700, size=20)], 16, nope=192, value=256)
+    a workgroup, and the projection runs sixteen waves: a decode batch of 20 rows of 64 heads (split merge, then projection
+    from merged rows), a chunk of 200 rows of 16 heads (one record a row, sixteen-wave absorb), and two sequences' chunks of
+    40 (more than 64 rows in splits: eight rows share the weights)."""
+    case = make_mla_case(301, [int(x) for x in np.random.default_rng(301).integers(1, 700, size=20)], 64, nope=192, value=256)
+    assert mla_splits(case) > 1
     want_f, _ = oracle_mla(case)
     got = run_mla(case).cpu().numpy()
     print("mla 192/256 batch", assert_attention_close(got.reshape(want_f.shape), want_f, "MLA 192/256 batch of 20"))
-    for rows, lens in ((40, [300, 120]), (200, [260])):
+    for rows, lens, split in ((40, [300, 120], True), (200, [260], False)):
         chunk = make_mla_chunk_case(302 + rows, lens, rows, 16, nope=192, value=256)
+        assert (mla_splits(chunk) > 1) == split
         want_c, _ = oracle_mla_chunk(chunk)
         got_c = run_mla_chunk(chunk).cpu().numpy()
         print("mla 192/256 chunk", rows, assert_attention_close(got_c.reshape(want_c.shape), want_c, f"MLA 192/256 chunk of {rows}"))
+
+
+@pytest.mark.parametrize("heads,rows,nope,value", [(16, 49, 128, 128), (16, 50, 128, 128), (16, 50, 128, 192), (128, 9, 128, 128), (128, 10, 128, 256),
+                                                   (4, 40, 96, 128), (8, 15, 192, 256), (8, 16, 192, 256), (8, 99, 192, 256), (8, 100, 192, 256)])
+def test_mla_weight_stages_below_and_above_their_lines(heads, rows, nope, value):
+    """The rules of the two weight stages, one size on either side: projection at 800 (row, head) pairs from sixteen rows
+    up, 1,200 below (784 / 800, 1,152 / 1,280, 792 / 800 with more than 64 rows); absorb of 192 query columns at 128 pairs (120 / 128), and a
+    query width without a matrix-core form (96), whose absorb takes eight rows a workgroup from 32 rows on."""
+    lens = [int(x) for x in np.random.default_rng(heads * rows).integers(1, 130, size=rows)]
+    case = make_mla_case(800 + heads + rows, lens, heads, nope=nope, value=value)
+    want, _ = oracle_mla(case)
+    got = run_mla(case).cpu().numpy()
+    print("mla stage lines", heads, rows, assert_attention_close(got.reshape(want.shape), want, f"MLA heads={heads} rows={rows} {nope}/{value}"))
 
 
 @pytest.mark.parametrize("heads,rows", [(16, 31), (16, 32), (16, 33), (8, 64), (8, 65), (4, 128), (4, 129)])
@@ -638,11 +672,11 @@ def test_mla_chunk_query_types_on_the_matrix_core_absorb():
         assert_attention_close(got, want_f, f"MLA chunk q as {q_kind}")
 
 
-@pytest.mark.parametrize("rows", [4, 11])
+@pytest.mark.parametrize("rows", [4, 11, 13])
 def test_mla_prefill_chunk_rows_equal_single_row_calls(rows):
     """Row r of a chunk is the decode step of a sequence that ends at that row.  With 8 query rows the call runs the
-    decode kernels: same bits.  With 22 it runs absorb and projection on the matrix cores, sixteen rows a workgroup: the
-    f32 sums run in another order, an absorbed query differs from the single-row one by a bf16 step in a few elements
+    decode kernels: same bits.  With 22 (704 (row, head) pairs) it runs the absorb on the matrix cores, sixteen rows a
+    workgroup, with 26 (832 pairs) the projection too: the f32 sums run in another order, an absorbed query differs from the single-row one by a bf16 step in a few elements
     out of a million, and the outputs agree to 5e-4."""
     case = make_mla_chunk_case(77, [600, 90], rows, 32)
     got = run_mla_chunk(case).cpu().numpy()

@@ -108,10 +108,25 @@ def test_weight_forms_at_the_usual_widths(bits, group, scale_dtype, heads, lens)
     (4, 128, O.SCALE_BF16, 192, 256, 64, [400, 100], 3), # few rows, wide values
     (8, 128, O.SCALE_BF16, 96, 40, 20, [33], 2),         # widths without a matrix-core form, a partial block of value columns
     (8, 256, O.SCALE_F16, 256, 130, 8, [5000], 1),       # the widest query and a wide split merge
+    (8, 128, O.SCALE_BF16, 128, 128, 16, [300], 70),     # more than 64 rows in splits: the projection folds the records itself
+    (4, 64, O.SCALE_F16, 128, 120, 16, [300], 70),
+    (8, 64, O.SCALE_BF16, 192, 256, 64, [700], 20),      # at most 64 rows in splits, wide values: sixteen waves over merged rows
+    (4, 128, O.SCALE_F32, 192, 200, 64, [700], 20),
+    (8, 128, O.SCALE_F16, 128, 128, 8, [200], 130),      # absorb of eight waves, three query terms
+    (4, 256, O.SCALE_F32, 128, 128, 8, [200], 130),
+    (8, 128, O.SCALE_BF16, 128, 128, 8, [200], 130),     # of sixteen, two terms; one record a row
+    (4, 128, O.SCALE_BF16, 128, 128, 64, [700], 20),     # of four, two terms; eight value waves over merged rows
+    (4, 64, O.SCALE_F16, 192, 256, 8, [260], 200),       # 192 query columns: eight waves, three terms; one record a row, wide values
+    (8, 64, O.SCALE_BF16, 192, 256, 8, [150], 129),      # two terms
+    (4, 128, O.SCALE_BF16, 192, 256, 8, [150], 129),
+    (8, 64, O.SCALE_F16, 192, 256, 64, [700], 3),        # four waves, three terms
+    (4, 128, O.SCALE_F32, 256, 130, 8, [5000], 1),       # a wide split merge, then the projection from the workspace
+    (8, 128, O.SCALE_F32, 128, 128, 8, [160], 56),       # 448 pairs: the first on the matrix-core absorb of 128 query columns
+    (4, 128, O.SCALE_F32, 128, 128, 8, [160], 55),       # 440: the last pair by pair
     (8, 16, O.SCALE_BF16, 128, 128, 16, [70], 4)])       # groups narrower than a matrix step: the vector kernels
 def test_weight_codes_at_the_edges_of_their_kernels(bits, group, scale_dtype, nope, value, heads, lens, rows):
-    """kv_b as codes over 512 + 64 columns: every kernel of the absorb and the projection at the sizes where it starts,
-    ends or fills a tile in part.  The codes are exact in the matrix cores and the query and merged rows carry 24 bits, so
+    """kv_b as codes over 512 + 64 columns: the kernels of the absorb and the projection at the sizes where they start,
+    end or fill a tile in part.  The codes are exact in the matrix cores and the query and merged rows carry 24 bits, so
     the bound is that of the attention itself."""
     case = make_mla_chunk_case(bits + group + heads, lens, rows, heads, nope=nope, value=value, block_tokens=16)
     set_weight_form(case, bits, group=group, scale_dtype=scale_dtype)

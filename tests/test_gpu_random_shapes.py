@@ -182,7 +182,7 @@ def test_random_mla_decode(it):
     rng = np.random.default_rng([404, it])
     heads = pick(rng, [1, 3, 16, 20, 40, 64, 65, 128])
     bt = pick(rng, [1, 16, 32, 48, 64, 128])
-    batch = pick(rng, [1, 2, 3, 4, 4, 17, 33])  # 16 rows and more take the matrix-core absorb and projection
+    batch = pick(rng, [1, 2, 3, 4, 4, 17, 33])  # 513 (row, head) pairs take the matrix-core absorb, 800 the projection (1,200 of fewer than sixteen rows)
     lens = [pick(rng, MLA_LENGTHS) for _ in range(batch)]
     if heads >= 64 or batch > 4:
         lens = [min(l, 700) for l in lens]
