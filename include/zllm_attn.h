@@ -510,9 +510,10 @@ typedef struct zllm_mla_decode_args {
      * src/backend/rocm/attention.rs:181-192).  kv_b_bits 0 or 16: bf16 at kv_b.  32: f32 at kv_b.  8 / 4: codes at kv_b,
      * packed low bits first into 32-bit words, ceil(latent_dim / (32 / bits)) words a row; element = (code - 128) or
      * (code - 8) times kv_b_scales[row * (latent_dim / kv_b_group) + column / kv_b_group], scales of kv_b_scale_dtype
-     * (ZLLM_SCALE_*).  Only the absorb and projection stages read kv_b: codes in groups of 32 columns and more feed the
-     * matrix cores (exact, the other operand in as many bf16 terms as its 24 bits take); f32 weights and narrower groups
-     * run on the vector ALUs, f32 throughout. */
+     * (ZLLM_SCALE_*).  Only the absorb and projection stages read kv_b.  At 512 + 64 columns codes in groups of 32 columns
+     * and more feed the matrix cores in calls of many (row, head) pairs (absorb: 128 or 192 query columns; exact, the other
+     * operand in as many bf16 terms as its 24 bits take).  Smaller calls, other widths, f32 weights and narrower groups run
+     * on the vector ALUs, f32 throughout. */
     const void* kv_b_scales;      /* [dev] or NULL */
     uint32_t kv_b_bits;
     uint32_t kv_b_group;          /* columns per scale; divides latent_dim */

@@ -1131,7 +1131,8 @@ void plan_prefill_splits(const zllm_gqa_prefill_args* a, uint32_t* chunk_tokens,
         // filled last round are kept where they save more than their records cost, about as long as 27 tokens of a
         // workgroup's walk a megabyte (f16 rows, 16 / 4 heads of 128, unsplit -> split: 2,600 rows behind 12,000 664 -> 504 us,
         // behind 1,000 189 -> 174, behind 300 159 -> 149; but 3,100 behind 6,000 430 -> 447; Q8g64 rows, 6,000 behind 3,000
-        // 918 -> 768, 4,100 behind 1,000 547 -> 681).
+        // 918 -> 768, 4,100 behind 1,000 547 -> 681).  With nothing before them one long segment, the case the parts would
+        // suit best, takes (16 / 4 heads of f16 rows, full tiles in parts / as it is) 328 / 285 us at 4,100 rows, 434 / 448 at 6,000.
         const uint64_t whole = (workgroups + cus - 1) / cus * (longest + 64);
         const uint64_t cut = (workgroups * *max_chunks + cus - 1) / cus * ((uint64_t)*chunk_tokens + 64);
         if (a->position == 0 || cut >= whole || (whole - cut) * 1000000 < 27 * record_bytes * *max_chunks) {
@@ -1221,10 +1222,13 @@ static uint64_t prefill_decode_route_bytes(const zllm_gqa_prefill_args* a)
 
 // A chunk of very few rows is a decode step in all but name (the reference decodes through this entry with one row,
 // src/backend/rocm/attention.rs:2202-2231): the chunk kernel would run row tiles that are all but empty.  With the
-// decode route's workspace such a chunk runs as decode items instead, each row re-reading the cache.  Measured on 32
-// query / 8 KV heads of 128 (us, decode items against the chunk kernel with KV splits): one row over 32 K tokens 24 / 71,
-// two 33 / 73, four 56 / 74, eight 104 / 78; eight rows over 2 K tokens 20 / 33 -- about 15 us + 0.34 ns per row and
-// token against 28 us + 1.5 ns per token (0.8 ns with half-size row tiles).
+// decode route's workspace such a chunk runs as decode items instead, each row re-reading the cache.  The rule stands on
+// measurements of the full-size tiles, 32 query / 8 KV heads of 128 (us, decode items against the chunk kernel with KV
+// splits): one row over 32 K tokens 24 / 71, two 33 / 73, four 56 / 74, eight 104 / 78; eight rows over 2 K tokens 20 / 33 --
+// about 15 us + 0.34 ns per row and token against 28 us + 1.5 ns per token (0.8 ns with smaller row tiles).
+// Tiles of 64 pairs (Q8g64 rows, 16-bit scales, head_dim 128) take 16 us + 0.8 ns per token: one row over 32 K tokens 25 / 42,
+// three 46 / 43, eight 108 / 44; eight over 2 K 21 / 18, sixteen 26 / 18; six over 8 K 31 / 21.  Time alone would draw the line
+// lower for those; the calls between keep the decode kernels' probabilities, which are wider than the f16 of a chunk.
 static bool few_rows_as_decode_items(const zllm_gqa_prefill_args* a)
 {
     if (a->rows > 16u) {
@@ -1234,8 +1238,8 @@ static bool few_rows_as_decode_items(const zllm_gqa_prefill_args* a)
     if (a->window != 0 && tokens > a->window) {
         tokens = a->window;
     }
-    // the chunk kernel's half-size row tiles (Q8g64 with 16-bit scales at head_dim 128, a chunk whose pairs fit one) walk
-    // a key in 0.8 ns: eight rows over 32 K tokens 54 us, where they would cost 104 as decode items
+    // the chunk kernel's smaller row tiles (Q8g64 with 16-bit scales at head_dim 128, a chunk whose pairs fit one) walk
+    // a key in 0.8 ns: eight rows over 32 K tokens 44 us, where they would cost 108 as decode items
     const bool half_tiles = a->kv_format == ZLLM_KV_Q8G64 &&
                             a->head_dim == 128 &&
                             zllm::gqa_prefill_tile_pairs(a->rows, a->position, a->window, a->num_heads, a->num_kv_heads, a->head_dim, a->kv_format, a->scale_dtype,

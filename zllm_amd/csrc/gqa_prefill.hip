@@ -1472,10 +1472,12 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
     }
     // measured on 32 query / 8 KV heads: 2,048 rows at position 0 140 -> 122 us, 256 rows 40 -> 26 us; at position 1,024
     // (ranges 1 : 3) the half tiles' dearer steps cost what the evening out gains, 190 -> 200 us
-    // Tiles of 64 stage every key for half the pairs: 1,000 rows (250 tiles of 128) 70.6 -> 62.0 us, 2,048 rows of 16 / 4
-    // heads 102.6 -> 89.4, 256 rows 35.4 -> 25.2; beyond a workgroup per compute unit the staging shows, 1,040 rows (264 tiles
-    // of 128) 82 -> 94, 2,000 rows 115 -> 157.  Capped at 128 registers for two workgroups a compute unit they spill inside
-    // the loop and take twice as long.
+    // Tiles of 64 stage every key for half the pairs (the attention alone, against tiles of 128): 1,000 rows of 32 / 8 heads (256
+    // tiles of 128) 50.2 -> 47.4 us, 504 rows 30.5 -> 22.4, 256 rows 18.9 -> 14.6, 2,048 rows of 16 / 4 heads 83.8 -> 78.0;
+    // beyond a workgroup per compute unit the staging shows, 1,040 rows (264 tiles of 128) 67 -> 79, 2,000 rows 98 -> 143.
+    // Capped at 128 registers for two workgroups a compute unit they spill inside the loop and take twice as long.
+    // Given ranges, as long for the first tile as for the last, take the same line: one segment of 1,100 rows (16 / 4 heads, 276
+    // tiles of 64) pays for its second round, 59 -> 77 us, but two of 600 rows of 32 / 8 take 32 us where 128 would be 41.
     if (can_share && tiles_of(128u) <= kComputeUnitsPrefill) {
         return 64u;
     }

@@ -181,7 +181,8 @@ struct MlaDecodeParams {
 
 // (row, query head) pairs of a row tile of the chunked-prefill kernels: 256, 128 at head_dim 256, and at head_dim 128 over
 // Q8g64 rows with 16-bit scales or f16 rows 128 for f32 queries, for a chunk whose pairs all fit, for f16 rows with
-// explicit ranges (`ranges`), and for a chunk that is much longer than what lies before it (its row tiles' ranges grow
+// explicit ranges (`ranges`) up to one and a half rounds of full-size tiles and not behind a longer prefix, unless they leave
+// most of the device idle, and for a chunk that is much longer than what lies before it (its row tiles' ranges grow
 // from almost nothing to the whole chunk) when the full-size tiles would be at most one workgroup per compute unit: twice
 // as many workgroups, handed out longest first, even the launch out.  64 where the same holds for the tiles of 128 over
 // Q8g64 rows, or all pairs fit: half of a workgroup's waves then take every other 32 tokens of the range.  The split

@@ -265,7 +265,7 @@ template <int R> __global__ __launch_bounds__(256) void mla_absorb_rows(MlaDecod
 }
 
 // ---------------------------------------------------------------------------------------------
-// absorb and projection on the matrix cores, for calls of sixteen rows and more
+// absorb and projection on the matrix cores, for calls of many (row, head) pairs (matrix_absorb, matrix_project)
 // ---------------------------------------------------------------------------------------------
 // The per-row kernels keep the oracle's summation order and cost a multiply and an add per weight and row on the vector
 // ALU: 28 us of absorb and 23 us of projection for 32 rows, more than the attention between them at short contexts.
@@ -2152,12 +2152,16 @@ static unsigned int row_block_groups(const MlaDecodeParams& p)
 
 // Where the matrix-core stages take over from a workgroup per (row, head), by the number of such pairs: a few hundred
 // workgroups run side by side, beyond that they queue, while the matrix-core kernels read a head's weights once for sixteen
-// rows and cost the same for one row as for sixteen.  Measured, us per pair / on the matrix cores:
+// rows and cost the same for one row as for sixteen.  Measured, us a workgroup per pair / on the matrix cores:
 //   absorb, 128 query columns: bf16 512 pairs (16 heads) 6.7 / 7.8, 528 pairs 9.4 / 7.8, 1536 pairs 15.0 / 7.6; 8-bit codes
-//   352 pairs 7.3 / 8.4, 480 pairs 11.2 / 8.7; 192 query columns: bf16 128 pairs 7.0 / 6.8, 8-bit codes 128 pairs 8.0 / 8.4,
-//   256 pairs 9.1 / 8.4
-//   merge and projection: bf16 512 pairs 7.4 / 11.7 (sixteen rows), 832 pairs 13.3 / 12.3 (26 rows), 1024 pairs 15.1 / 16.2
-//   (eight rows: half of a tile empty), 1408 pairs 19.8 / 16.6; 8-bit codes within 2 us of these
+//   384 pairs 8.0 / 9.5, 448 pairs 12.2 / 9.4; 4-bit codes 448 pairs 9.6 / 9.8, 512 pairs 9.7 / 9.6, 528 pairs 11.0 / 10.0
+//   192 query columns: bf16 128 pairs 7.0 / 6.8, 8-bit codes 128 pairs 8.0 / 8.4, 256 pairs 9.1 / 8.4; 4-bit 128 pairs 9.9 / 8.7
+//   merge and projection, 128 value columns: bf16 512 pairs (32 rows) 8.2 / 11.8, 640 pairs 11.7 / 11.6, 784 pairs 13.6 / 12.2,
+//   768 pairs in 96 rows 11.9 / 13.8; fewer than sixteen rows, part of a tile empty: 1024 pairs 16.0 / 16.8, 1280 pairs 18.8 /
+//   16.5; 4-bit codes 512 pairs 10.4 / 13.8, 784 pairs 18.0 / 14.4
+//   192 value columns: bf16 640 pairs 14.2 / 15.0, 784 pairs 15.8 / 15.6, 1024 pairs 16.3 / 16.8, eight rows 20.3 / 20.0
+//   256 value columns: bf16 512 pairs 10.8 / 16.9, 640 pairs 16.5 / 17.4, 784 pairs 18.0 / 17.0, 1024 pairs 18.5 / 18.5, eight
+//   rows 23.3 / 21.5, ten (1280) 30.1 / 21.3
 static bool matrix_absorb_widths(const MlaDecodeParams& p)
 {
     return (p.q_head_dim & 3u) == 0 && (p.nope_dim == 128u || p.nope_dim == 192u);
