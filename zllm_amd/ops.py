@@ -14,12 +14,14 @@ from . import capi
 _DTYPE = {torch.float32: capi.DTYPE_F32, torch.bfloat16: capi.DTYPE_BF16, torch.float16: capi.DTYPE_F16}
 
 
+# A decode step of a short context is a few launches of a few microseconds: what a call costs here counts as much as its
+# kernels.  Argument blocks are filled by one constructor call, in the order of their fields, with plain integers for pointers.
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())  # torch.cuda.current_stream() without the Stream object
 
 
 def _dev(t, name):
@@ -47,18 +49,12 @@ def gqa_prologue(q, k, v, q_norm, k_norm, cos, sin, k_codes, k_scales, v_codes, 
                  split_half=True, q_out_dtype=torch.float32, ring_capacity=0, positions=None):
     """Per-head RMSNorm + RoPE of Q and K, Q out as a tensor, K and V quantized into the pages (zllm_attn_gqa_prologue)."""
     rows = q.shape[0]
-    q_out = torch.empty((rows, num_heads * head_dim), dtype=q_out_dtype, device=q.device)
-    args = capi.GqaPrologueArgs()
-    args.q, args.k, args.v = _ptr(q), _ptr(k), _ptr(v)
-    args.q_norm, args.k_norm, args.cosine, args.sine = _ptr(q_norm), _ptr(k_norm), _ptr(cos), _ptr(sin)
-    args.q_out, args.k_codes, args.k_scales = _ptr(q_out), _ptr(k_codes), _ptr(k_scales)
-    args.v_codes, args.v_scales, args.table, args.positions = _ptr(v_codes), _ptr(v_scales), _ptr(table), _ptr(positions)
-    args.rows, args.num_heads, args.num_kv_heads, args.head_dim = rows, num_heads, num_kv_heads, head_dim
-    args.rotary_dim = rotary_dim
-    args.rope_table_rows = 0 if cos is None else cos.shape[0]
-    args.position, args.block_tokens, args.ring_capacity = position, block_tokens, ring_capacity
-    args.eps, args.weight_offset = eps, weight_offset
-    args.src_dtype, args.q_out_dtype, args.rule, args.split_half = _DTYPE[q.dtype], _DTYPE[q_out_dtype], rule, int(split_half)
+    q_out = q.new_empty((rows, num_heads * head_dim), dtype=q_out_dtype)
+    args = capi.GqaPrologueArgs(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(q_norm), _ptr(k_norm), _ptr(cos), _ptr(sin), q_out.data_ptr(), _ptr(k_codes),
+        _ptr(k_scales), _ptr(v_codes), _ptr(v_scales), _ptr(table), _ptr(positions), rows, num_heads, num_kv_heads, head_dim, rotary_dim,
+        0 if cos is None else cos.shape[0], position, block_tokens, ring_capacity, eps, weight_offset, _DTYPE[q.dtype],
+        _DTYPE[q_out_dtype], rule, int(split_half))
     capi.check(capi.load().zllm_attn_gqa_prologue(C.byref(args), _stream()))
     return q_out
 
@@ -98,37 +94,32 @@ def scatter_rows(plane, rows, table, first, block_tokens, ring_capacity=0):
 
 def gqa_decode_args(q, k_plane, k_scales, v_plane, v_scales, tables, kv_lens, num_heads, num_kv_heads, head_dim,
                     block_tokens, score_scale, max_kv_len, first_visible=None, softcap=0.0, ring_capacity=0,
-                    kv_format=capi.KV_Q8G64, scale_dtype=capi.SCALE_F16, out=None, workspace=None, total_kv_tokens=0, gate=None):
+                    kv_format=capi.KV_Q8G64, scale_dtype=capi.SCALE_F16, out=None, workspace=None, total_kv_tokens=0, gate=None,
+                    launched=False):
     batch = q.shape[0]
     if out is None:
-        out = torch.empty((batch, num_heads * head_dim), dtype=torch.float32, device=q.device)
-    args = capi.GqaDecodeArgs()
-    args.q, args.k_plane, args.k_scales = _ptr(q), _ptr(k_plane), _ptr(k_scales)
-    args.v_plane, args.v_scales = _ptr(v_plane), _ptr(v_scales)
-    args.tables, args.kv_lens, args.first_visible = _ptr(tables), _ptr(kv_lens), _ptr(first_visible)
-    args.out = _ptr(out)
-    args.batch, args.num_heads, args.num_kv_heads, args.head_dim = batch, num_heads, num_kv_heads, head_dim
-    args.table_stride = 0 if tables is None else tables.shape[1]
-    args.max_kv_len, args.block_tokens, args.ring_capacity = max_kv_len, block_tokens, ring_capacity
-    args.total_kv_tokens = total_kv_tokens
-    args.score_scale, args.softcap = score_scale, softcap
-    args.kv_format, args.scale_dtype, args.q_dtype = kv_format, scale_dtype, _DTYPE[q.dtype]
+        out = q.new_empty((batch, num_heads * head_dim), dtype=torch.float32)
+    args = capi.GqaDecodeArgs(
+        q.data_ptr(), _ptr(k_plane), _ptr(k_scales), _ptr(v_plane), _ptr(v_scales), _ptr(tables), _ptr(kv_lens), _ptr(first_visible),
+        out.data_ptr(), None, 0, batch, num_heads, num_kv_heads, head_dim, 0 if tables is None else tables.shape[1], max_kv_len,
+        total_kv_tokens, block_tokens, ring_capacity, score_scale, softcap, kv_format, scale_dtype, _DTYPE[q.dtype])
     if gate is not None:
-        args.gate, args.gate_cols, args.gate_dtype = _ptr(gate), gate.shape[1], _DTYPE[gate.dtype]
-    need = capi.load().zllm_attn_gqa_decode_workspace_bytes(C.byref(args))
-    if need == 0:
-        raise capi.ZllmAttnError(-1, capi.last_error())
+        args.gate, args.gate_cols, args.gate_dtype = gate.data_ptr(), gate.shape[1], _DTYPE[gate.dtype]
+    if not launched or workspace is None:  # a call that launches with the caller's workspace is checked by the launch itself
+        need = capi.load().zllm_attn_gqa_decode_workspace_bytes(C.byref(args))
+        if need == 0:
+            raise capi.ZllmAttnError(-1, capi.last_error())
     if workspace is False:  # the static-scratch entry point ignores both fields
         return args, out, None
     if workspace is None:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-    args.workspace, args.workspace_bytes = _ptr(workspace), workspace.numel()
+    args.workspace, args.workspace_bytes = workspace.data_ptr(), workspace.numel()
     return args, out, workspace
 
 
 def gqa_decode(*a, **kw):
     """Batched GQA decode over the paged cache (zllm_attn_gqa_decode).  Returns f32 [batch, Hq*d]."""
-    args, out, workspace = gqa_decode_args(*a, **kw)
+    args, out, workspace = gqa_decode_args(*a, launched=True, **kw)
     capi.check(capi.load().zllm_attn_gqa_decode(C.byref(args), _stream()))
     return out
 
@@ -147,17 +138,13 @@ def gqa_prefill_chunk_args(q, k_plane, k_scales, v_plane, v_scales, table, posit
     """The argument block of zllm_attn_gqa_prefill_chunk, the output tensor and the workspace tensor (None without one):
     for callers that launch the same call many times."""
     rows = q.shape[0]
-    out = torch.empty((rows, num_heads * head_dim), dtype=out_dtype, device=q.device)
-    args = capi.GqaPrefillArgs()
-    args.q, args.k_plane, args.k_scales = _ptr(q), _ptr(k_plane), _ptr(k_scales)
-    args.v_plane, args.v_scales, args.table, args.out = _ptr(v_plane), _ptr(v_scales), _ptr(table), _ptr(out)
-    args.rows, args.position, args.window = rows, position, window
-    args.num_heads, args.num_kv_heads, args.head_dim, args.block_tokens = num_heads, num_kv_heads, head_dim, block_tokens
-    args.score_scale, args.softcap = score_scale, softcap
-    args.kv_format, args.scale_dtype = kv_format, scale_dtype
-    args.q_dtype, args.out_dtype = _DTYPE[q.dtype], _DTYPE[out_dtype]
+    out = q.new_empty((rows, num_heads * head_dim), dtype=out_dtype)
+    args = capi.GqaPrefillArgs(
+        q.data_ptr(), _ptr(k_plane), _ptr(k_scales), _ptr(v_plane), _ptr(v_scales), _ptr(table), out.data_ptr(), None, 0, rows, position,
+        window, num_heads, num_kv_heads, head_dim, block_tokens, score_scale, softcap, kv_format, scale_dtype, _DTYPE[q.dtype],
+        _DTYPE[out_dtype])
     if gate is not None:
-        args.gate, args.gate_cols, args.gate_dtype = _ptr(gate), gate.shape[1], _DTYPE[gate.dtype]
+        args.gate, args.gate_cols, args.gate_dtype = gate.data_ptr(), gate.shape[1], _DTYPE[gate.dtype]
     args.visible_ends = _ptr(visible_ends)
     args.visible_starts = _ptr(visible_starts)
     args.table_stride = 0 if table is None else table.numel()
