@@ -1,0 +1,110 @@
+"""The chunk kernel over f16 rows of head_dim 128 that takes launches of more than 512 tiles of 128 (row, head) pairs
+(gqa_prefill_f16.hip): pages it addresses by scalars and others, groups that do and do not divide a tile, ranges that end inside
+a load's four rows, empty ranges, KV splits, output gate and types, against 64-bit attention on a few heads."""
+import numpy as np
+import pytest
+import torch
+
+from zllm_amd import capi, ops
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+
+
+def reference(q, k, v, lo, hi, scale, softcap):
+    """One head in 64 bits: q [rows, D], k / v [tokens, D], visible tokens [lo, hi) of each row."""
+    s = (q.double() @ k.double().T.contiguous()) * scale
+    if softcap:
+        s = torch.tanh(s / softcap) * softcap
+    t = torch.arange(k.shape[0], device=q.device)[None]
+    s = s.masked_fill(~((t >= lo[:, None]) & (t < hi[:, None])), float("-inf"))
+    top = s.amax(dim=1, keepdim=True)
+    p = torch.exp(s - torch.where(top == float("-inf"), torch.zeros_like(top), top))
+    total = p.sum(dim=1, keepdim=True)
+    return torch.where(total > 0, (p @ v.double()) / total, torch.zeros_like(q, dtype=torch.float64))
+
+
+def run(rows, position, heads, kv_heads, page, mode="causal", softcap=0.0, table=True, out_dtype=torch.float32, gate=False, workspace=True,
+        q_dtype=torch.bfloat16, spread=1.0):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + 7 * position + heads)
+    n = position + rows
+    pages = (n + page - 1) // page
+    cols = kv_heads * D
+    planes = [torch.full((pages * page, cols), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2)]  # behind the rows: garbage
+    order = torch.randperm(pages, generator=gen, device="cuda").to(torch.int32) if table else torch.arange(pages, dtype=torch.int32, device="cuda")
+    at = (order.long()[:, None] * page + torch.arange(page, device="cuda")).view(-1)[:n]
+    data = [torch.randn(n, cols, generator=gen, device="cuda").to(torch.float16) * f for f in (spread, 1.0)]
+    for plane, x in zip(planes, data):
+        plane[at] = x
+    q = torch.randn(rows, heads * D, generator=gen, device="cuda").to(q_dtype)
+    r = torch.arange(rows, device="cuda")
+    lo, hi, given = torch.zeros_like(r), position + r + 1, {}
+    if mode == "ends":  # rows read to the end of their block of 50
+        hi = torch.minimum((r // 50 + 1) * 50, torch.tensor(rows, device="cuda")) + position
+        given = dict(visible_ends=hi.to(torch.int32))
+    elif mode == "segments":  # unequal ones, the rows of every fifth see nothing
+        cuts = torch.tensor([0, 3, 130, 131, 400, 401, 700, 995], device="cuda")
+        which = torch.searchsorted(cuts, r, right=True) - 1
+        ends = torch.cat([cuts[1:], torch.tensor([rows], device="cuda")])
+        lo, hi = cuts[which], ends[which]
+        hi = torch.where(which % 5 == 4, lo, hi)
+        given = dict(visible_starts=lo.to(torch.int32), visible_ends=hi.to(torch.int32))
+    g = torch.randn(rows, heads * D, generator=gen, device="cuda") if gate else None
+    scale = D**-0.5
+    out = ops.gqa_prefill_chunk(q, planes[0], None, planes[1], None, order if table else None, position, heads, kv_heads, D, page, scale, softcap=softcap,
+                                kv_format=capi.KV_F16, out_dtype=out_dtype, gate=g, workspace=workspace, **given)
+    out = out.view(rows, heads, D)
+    for head in (0, heads // 2, heads - 1):
+        kvh = head // (heads // kv_heads)
+        k, v = (x.view(n, kv_heads, D)[:, kvh] for x in data)
+        want = reference(q.view(rows, heads, D)[:, head], k, v, lo, hi, scale, softcap)
+        if gate:
+            want = want * torch.sigmoid(g.view(rows, heads, D)[:, head].double())
+        # probabilities carried as f16 are off by at most 2^-12 of themselves and sum to one: 2^-12 of the largest value, all errors
+        # of one sign; f32 scores (|s| < 64 in base 2, the sum of 128 products) move a probability by less than 2^-14
+        bound = (2.0**-12 + 2.0**-14) * v.abs().max().item()
+        if out_dtype != torch.float32:
+            bound += want.abs().max().item() * (2.0**-8 if out_dtype == torch.bfloat16 else 2.0**-11)
+        err = (out[:, head].double() - want).abs().max().item()
+        assert np.isfinite(err) and err <= bound, f"head {head}: {err:.3e} > {bound:.3e}"
+
+
+# 64 KV heads: nine tiles of 128 rows each, 576 in all.  Pages of 8 and more are addressed by scalars
+@pytest.mark.parametrize("page", [8, 16, 64, 1024, 4, 1, 24])
+def test_pages(page):
+    run(1030, 0, 64, 64, page)
+
+
+@pytest.mark.parametrize("rows", [1025, 1027, 1055, 1056, 1057])  # the last tile of keys ends inside a load's four rows
+def test_row_remainders(rows):
+    run(rows, 0, 64, 64, 16)
+
+
+@pytest.mark.parametrize("heads,kv_heads,rows", [(24, 8, 2800), (72, 72, 900), (63, 9, 1100), (600, 600, 40)])
+def test_groups(heads, kv_heads, rows):
+    run(rows, 0, heads, kv_heads, 16)
+
+
+@pytest.mark.parametrize("mode", ["ends", "segments"])
+@pytest.mark.parametrize("page,table", [(16, True), (24, True), (16, False)])
+def test_given_ranges(mode, page, table):
+    run(1030, 0, 64, 64, page, mode=mode, table=table)
+
+
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("position", [37, 300, 2051])
+def test_behind_a_prefix(position, workspace):
+    run(1030, position, 64, 64, 16, workspace=workspace)
+
+
+@pytest.mark.parametrize("softcap", [5.0, 50.0, 300.0])
+def test_soft_caps(softcap):
+    run(1030, 0, 64, 64, 16, softcap=softcap)
+
+
+@pytest.mark.parametrize("out_dtype,gate,q_dtype,spread", [(torch.bfloat16, True, torch.float16, 1.0), (torch.float16, False, torch.bfloat16, 1.0),
+                                                           (torch.float32, True, torch.bfloat16, 4.0)])
+def test_outputs_and_queries(out_dtype, gate, q_dtype, spread):
+    run(1030, 0, 64, 64, 16, out_dtype=out_dtype, gate=gate, q_dtype=q_dtype, spread=spread)

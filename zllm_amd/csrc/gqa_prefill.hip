@@ -27,34 +27,20 @@
 // (running maximum, V window) is only touched when some lane's score passes it.
 #include <type_traits>
 
-#include "common.hpp"
-#include "kernels.hpp"
+#include "gqa_prefill.hpp"
 
 namespace zllm {
 
 namespace {
 
-// Fences for the instruction scheduler between the phases of a step (they keep the early LDS requests early).
-#define PREFILL_PHASE_FENCE() __builtin_amdgcn_sched_barrier(0)
-
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr int kStep = 32;                 // tokens per step
 constexpr int kD = 128;                   // head_dim handled by this kernel
 constexpr int kRowBytes = kD * 2;         // one token of one KV head as f16
 constexpr int kTileBytes = kStep * kRowBytes; // 8 KiB
-constexpr float kPBias = 8.0f;            // probabilities are carried as p * 2^8: f16 stays normal down to p = 2^-22
 constexpr float kLoThreshold = 8.0f;      // see the P.V stage
 constexpr int kColTiles = 2;              // 16-column MFMA tiles per wave
 constexpr int kWaves = 256 / (16 * kColTiles);
 constexpr int kThreads = 64 * kWaves;
 constexpr unsigned long long kComputeUnitsPrefill = 256; // compute units of the device the kernels are tuned for
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-union Frag {
-    u32x4 u;
-    f16x8 h;
-};
 
 // Chunk swizzle for the 64-bank LDS (256 B per cycle = one tile row).  Row bits 1 and 2 are XOR-ed into chunk
 // bits 1 and 2 and the row's parity into chunk bit 3 (the scale-group half of the row): the LDS serves a
@@ -71,15 +57,6 @@ __device__ __forceinline__ unsigned int tile_offset(unsigned int row, unsigned i
     return row * kRowBytes + ((chunk ^ swz(row)) << 4);
 }
 
-__device__ __forceinline__ float soft_tanh(float x)
-{
-    const float x2 = x * x;
-    const float poly = x * (1.0f + x2 * (-1.0f / 3.0f + x2 * (2.0f / 15.0f + x2 * (-17.0f / 315.0f))));
-    const float e = __builtin_amdgcn_exp2f(fminf(fabsf(x) * (2.0f * kLog2e), 80.0f));
-    const float big = copysignf(1.0f - __fdividef(2.0f, e + 1.0f), x);
-    return fabsf(x) < 0.1f ? poly : big;
-}
-
 struct StepRegs {
     u32x2 codes[2];        // codes 8 cc .. + 8 and 64 + 8 cc .. + 8 of the thread's plane (K: threads 0..255, V: 256..511)
     unsigned int scales;   // two 16-bit scales (groups 0, 1) of the token
@@ -89,30 +66,6 @@ struct StepRegs {
 __device__ __forceinline__ unsigned int window_exponent(float top)
 {
     return min(max((__float_as_uint(top) >> 23) & 0xffu, 2u), 252u);
-}
-
-// ---- KV splits of a chunk -------------------------------------------------------------------------------------
-// A chunk with few row tiles (a short chunk over a long prefix) leaves most CUs without a workgroup while each
-// workgroup walks the whole prefix.  With p.max_chunks > 1 workgroup z of a row tile attends part z of the tile's
-// visible range [t_begin, t_end) -- equal 32-aligned parts of at most p.chunk_tokens, as the decode kernels cut a
-// sequence -- and writes un-normalised records (sum of p v, running maximum, sum of p) that gqa_decode_merge combines;
-// parts beyond the tile's own count write empty records (maximum -inf, sum 0).
-struct SplitRange {
-    unsigned int begin, end;
-    bool live;
-};
-__device__ __forceinline__ SplitRange split_range(const GqaPrefillParams& p, unsigned int t_begin, unsigned int t_end)
-{
-    SplitRange r = {t_begin, t_end, true};
-    if (p.max_chunks > 1u) {
-        const unsigned int parts = max(1u, min(p.max_chunks, (t_end - t_begin + p.chunk_tokens - 1u) / p.chunk_tokens)); // none is live in an empty range
-        const unsigned int span = (((t_end - t_begin + parts - 1u) / parts) + 31u) & ~31u;
-        const unsigned long long begin = (unsigned long long)t_begin + (unsigned long long)blockIdx.z * span;
-        r.live = blockIdx.z < parts && begin < t_end;
-        r.begin = r.live ? (unsigned int)begin : t_begin;
-        r.end = r.live ? (unsigned int)min((unsigned long long)t_end, begin + span) : t_begin;
-    }
-    return r;
 }
 
 // The visible range of a row tile whose rows bring their own ends, or ranges (src/attention/block.rs:10-16): the union over
@@ -141,18 +94,6 @@ __device__ __forceinline__ void given_range(const GqaPrefillParams& p, unsigned 
     t_begin = __builtin_amdgcn_readfirstlane(begin);
 }
 
-// Eight consecutive query elements (16-byte aligned: the query is, and head_dim is a multiple of 64).  One element at a
-// time, a lane sends 32 to 128 two-byte loads before the first step: 1,000 rows of 32 / 8 heads 54.6 -> 49.1 us, a sliding
-// layer of 2,048 rows (16 / 8 heads of 256, window 1,024) 108.9 -> 86.3 us.
-__device__ __forceinline__ void widen8(const u32x4& raw, int dtype, float (&x)[8])
-{
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        x[2 * e] = dtype == 1 ? __uint_as_float(raw[e] << 16) : f16_bits_to_f32((unsigned short)(raw[e] & 0xffffu));
-        x[2 * e + 1] = dtype == 1 ? __uint_as_float(raw[e] & 0xffff0000u) : f16_bits_to_f32((unsigned short)(raw[e] >> 16));
-    }
-}
-
 __device__ __forceinline__ void load_query8(const void* q, size_t at, int dtype, float (&x)[8])
 {
     if (dtype == 0) {
@@ -165,13 +106,6 @@ __device__ __forceinline__ void load_query8(const void* q, size_t at, int dtype,
         return;
     }
     widen8(*(const u32x4*)((const unsigned short*)q + at), dtype, x);
-}
-
-__device__ __forceinline__ void store_empty_record(const GqaPrefillParams& p, unsigned int row, unsigned int head)
-{
-    const size_t rec = ((size_t)row * p.max_chunks + blockIdx.z) * p.num_heads + head;
-    p.stats[rec * 2] = kNegInf;
-    p.stats[rec * 2 + 1] = 0.0f;
 }
 
 // acc and total carry 2^v_shift (the bias that keeps f16 probabilities in range, less the V window): the records are
@@ -1439,6 +1373,28 @@ template <int D, int KV, int SDT, int CT = TileShape<D>::kCT> static hipError_t 
 
 } // namespace
 
+// More tiles of 128 pairs than two rounds of one workgroup a compute unit, f16 rows of head_dim 128: the kernel of which three
+// live on one (gqa_prefill_f16.hip).  Against the better of the tiles of this file (us, 32 / 8 heads where not given): first
+// chunks of 2,300 rows (576 tiles) 133 -> 116, 3,500 231 -> 199, 6,000 422 -> 399, 11,000 1,227 / 1,239; packed segments, 2,600
+// rows in 13 49 -> 39, 4,326 in five 155 -> 133, 16 / 16 heads, 4,100 in nine 66 -> 61, 8,000 in 24 93 -> 77, in one 612 -> 623.
+// Two rounds or less favour the waves of 16 pairs: 1,950 rows (488 tiles) 71 / 86, four segments of 4,096 (512) 98 / 103.
+// Behind a prefix every tile walks about as far, full-size ones read half the keys a pair, and what is gained is their unfilled
+// last round: 2,300 rows at 9,000 (288 full tiles) 670 -> 548, 2,600 at 2,600 (325) 321 -> 281, but 4,096 at 4,000 (512) 489 / 535.
+static bool gqa_prefill_takes_f16(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
+                                  unsigned int head_dim, int kv_format)
+{
+    const unsigned int group = num_heads / num_kv_heads;
+    if (kv_format != 1 || head_dim != 128u || window != 0u || group == 0u || group > 128u) {
+        return false;
+    }
+    auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
+    if (tiles_of(128u) <= kComputeUnitsPrefill * 2u) {
+        return false;
+    }
+    const unsigned long long full = tiles_of(256u), rounds = (full + kComputeUnitsPrefill - 1) / kComputeUnitsPrefill;
+    return (unsigned long long)position * 4u <= rows || full * 10u <= rounds * kComputeUnitsPrefill * 9u;
+}
+
 unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
                                     unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges)
 {
@@ -1450,14 +1406,16 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
         return 256u;
     }
     auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
+    if (gqa_prefill_takes_f16(rows, position, window, num_heads, num_kv_heads, head_dim, kv_format)) {
+        return 128u;
+    }
     if (kv_format == 1 && ranges && (position <= rows || tiles_of(256u) * 5u <= kComputeUnitsPrefill)) {
-        // Packed segments: a smaller tile meets fewer of them and there are twice as many, until the full ones are one and a half
-        // rounds of the device: 16 / 4 heads, 4,100 rows in one segment (260 full tiles) 323 -> 300 us, in eight 90 -> 79; 16 / 8
-        // heads, 6,000 rows (376) 485 -> 461; but 32 / 8 heads, 4,326 rows (544) 541 -> 565, 16 / 4, 8,000 rows (500) 630 -> 784.
-        // Behind a prefix longer than the rows their ranges have most keys in common, and a full tile reads those for twice the
-        // rows: 16 / 4 heads, 2,600 rows behind 12,000 keys 508 -> 416, 600 rows of 64 / 8 446 -> 374.  The smaller ones stay for
-        // calls that leave the device idle: 300 rows of 16 / 4 (20 full tiles) behind 1,000 26 us against 37, behind 12,000 70 / 72.
-        return tiles_of(256u) * 2u <= kComputeUnitsPrefill * 3u ? 128u : 256u;
+        // Packed segments: a smaller tile meets fewer of them, and up to two rounds of the device there are twice as many:
+        // 16 / 16 heads, 2,100 rows in four segments 63 -> 44 us, 3,900 in nine 60 -> 56.  Behind a prefix longer than the rows
+        // their ranges have most keys in common, and a full tile reads those for twice the rows: 16 / 4 heads, 2,600 rows behind
+        // 12,000 keys 508 -> 416, 600 rows of 64 / 8 446 -> 374.  The smaller ones stay for calls that leave the device idle: 300
+        // rows of 16 / 4 (20 full tiles) behind 1,000 26 us against 37, behind 12,000 70 / 72.
+        return tiles_of(128u) <= kComputeUnitsPrefill * 2u ? 128u : 256u;
     }
     if (q_dtype == 0) {
         return 128u; // f32 queries travel as two f16 fragments: a wave has the registers for one column tile of them
@@ -1489,6 +1447,9 @@ hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scal
     const unsigned int tile_pairs = gqa_prefill_tile_pairs(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scale_dtype,
                                                            p.q_dtype, p.visible_starts != nullptr);
     if (kv_format == 1) { // f16 rows
+        if (gqa_prefill_takes_f16(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format)) {
+            return launch_gqa_prefill_f16(p, stream);
+        }
         if (p.head_dim == 128u && tile_pairs == 128u) {
             return launch_prefill_tiles<128, 1, 0, 1>(p, stream);
         }

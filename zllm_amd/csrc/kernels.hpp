@@ -180,9 +180,9 @@ struct MlaDecodeParams {
 };
 
 // (row, query head) pairs of a row tile of the chunked-prefill kernels: 256, 128 at head_dim 256, and at head_dim 128 over
-// Q8g64 rows with 16-bit scales or f16 rows 128 for f32 queries, for a chunk whose pairs all fit, for f16 rows with
-// explicit ranges (`ranges`) up to one and a half rounds of full-size tiles and not behind a longer prefix, unless they leave
-// most of the device idle, and for a chunk that is much longer than what lies before it (its row tiles' ranges grow
+// Q8g64 rows with 16-bit scales or f16 rows 128 for f32 queries, for a chunk whose pairs all fit, for f16 rows where
+// gqa_prefill_f16.hip has the call, for f16 rows with explicit ranges (`ranges`) up to two rounds of such tiles and not behind a
+// longer prefix, unless they leave most of the device idle, and for a chunk that is much longer than what lies before it (its row tiles' ranges grow
 // from almost nothing to the whole chunk) when the full-size tiles would be at most one workgroup per compute unit: twice
 // as many workgroups, handed out longest first, even the launch out.  64 where the same holds for the tiles of 128 over
 // Q8g64 rows, or all pairs fit: half of a workgroup's waves then take every other 32 tokens of the range.  The split
@@ -204,6 +204,8 @@ hipError_t launch_gather_rows(const GatherParams& p, hipStream_t stream);
 // kv_format: 0 = Q8g64, 1 = f16; scale_dtype: 0 = bf16, 1 = f16 (Q8 only).
 hipError_t launch_gqa_decode(const GqaDecodeParams& p, int kv_format, int scale_dtype, unsigned int stages, hipStream_t stream);
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scale_dtype, hipStream_t stream);
+// f16 rows at head_dim 128, 16-bit queries, tiles of 128 pairs (gqa_prefill_f16.hip)
+hipError_t launch_gqa_prefill_f16(const GqaPrefillParams& p, hipStream_t stream);
 hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, hipStream_t stream);
 // The vector-ALU kernels for latent / rope widths other than 512 / 64 and for kv_b in other forms than bf16 (mla_generic.hip).
 hipError_t launch_mla_absorb_any(const MlaDecodeParams& p, hipStream_t stream);
