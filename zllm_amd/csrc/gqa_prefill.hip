@@ -24,7 +24,7 @@
 // The kernel is bound by the vector-ALU instructions it issues, not by the matrix cores, so whatever does not depend on
 // every (token, column) pair stays out of the common path of a step: the tile buffer is a literal (LDS addresses in
 // immediates), edge masks and the low-order P' pass sit behind wave-uniform branches, and a column's reference
-// (running maximum, V window) is only touched when some lane's score passes it.
+// (a running maximum, V window) is only touched when some lane's score passes it by more than 2^kSlack.
 #include <type_traits>
 
 #include "gqa_prefill.hpp"
@@ -36,7 +36,6 @@ namespace {
 constexpr int kD = 128;                   // head_dim handled by this kernel
 constexpr int kRowBytes = kD * 2;         // one token of one KV head as f16
 constexpr int kTileBytes = kStep * kRowBytes; // 8 KiB
-constexpr float kLoThreshold = 8.0f;      // see the P.V stage
 constexpr int kColTiles = 2;              // 16-column MFMA tiles per wave
 constexpr int kWaves = 256 / (16 * kColTiles);
 constexpr int kThreads = 64 * kWaves;
@@ -507,9 +506,9 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
             for (int e = 1; e < 8; ++e) {
                 lane_max = fmaxf(lane_max, sc[e]);
             }
-            // The reference point of the column (running maximum, V window) moves on few steps of a long prefix, so the
+            // The reference point of the column (a running maximum within 2^kSlack, V window) moves on few steps, so the
             // reduction across the wave's rows and the rescaling sit behind a test of the lane's own maximum.
-            if (__any(lane_max * mult > run_max[ct]) || window_moved) {
+            if (__any(lane_max * mult > run_max[ct] + kSlack) || window_moved) {
                 const float step_max = wave_max_16x4(lane_max) * mult;
                 const float new_max = fmaxf(run_max[ct], step_max);
                 const float safe_max = new_max == kNegInf ? 0.0f : new_max;
@@ -536,10 +535,7 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
             heavy = heavy || step_sum * kLoThreshold > run_sum[ct];
         }
         // ---- O^T += Vcodes^T . P'_g ----------------------------------------------------------------------
-        // P' is carried as f16 hi + lo (22 significant bits) while the probabilities a lane holds of this step weigh more
-        // than 1/8 of its running sum (a lane sums a quarter of the tokens, so each is < 1/32 of the row's sum);
-        // below that the hi term's rounding (2^-12 relative, random sign) moves the normalised output by
-        // < 2^-12 / 32 of |v|, so the lo product is skipped.
+        // P' is carried as f16 hi + lo on heavy steps (kLoThreshold), elsewhere the lo product is skipped
         const bool lo_pass = __any(heavy);
         PREFILL_PHASE_FENCE();
 #pragma unroll
@@ -1173,7 +1169,7 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
             for (int e = 1; e < 8; ++e) {
                 lane_max = fmaxf(lane_max, sc[e]);
             }
-            if (__any(lane_max * mult > run_max[ct]) || window_moved) {
+            if (__any(lane_max * mult > run_max[ct] + kSlack) || window_moved) {
                 const float step_max = wave_max_16x4(lane_max) * mult;
                 const float new_max = fmaxf(run_max[ct], step_max);
                 const float safe_max = new_max == kNegInf ? 0.0f : new_max;
@@ -1198,8 +1194,8 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
             run_sum[ct] += step_sum;
             heavy = heavy || step_sum * kLoThreshold > run_sum[ct];
         }
-        // ---- O^T += V^T . P (Q8g64: P'_g = p * v_scale_g, four output tiles per scale group): f16 hi, and lo while a
-        // lane's probabilities of this step weigh more than 1/8 of its sum ----
+        // ---- O^T += V^T . P (Q8g64: P'_g = p * v_scale_g, four output tiles per scale group): f16 hi, and lo on
+        // heavy steps (kLoThreshold) ----
         const bool lo_pass = __any(heavy);
         PREFILL_PHASE_FENCE();
 #pragma unroll
@@ -1375,11 +1371,14 @@ template <int D, int KV, int SDT, int CT = TileShape<D>::kCT> static hipError_t 
 
 // More tiles of 128 pairs than two rounds of one workgroup a compute unit, f16 rows of head_dim 128: the kernel of which three
 // live on one (gqa_prefill_f16.hip).  Against the better of the tiles of this file (us, 32 / 8 heads where not given): first
-// chunks of 2,300 rows (576 tiles) 133 -> 116, 3,500 231 -> 199, 6,000 422 -> 399, 11,000 1,227 / 1,239; packed segments, 2,600
-// rows in 13 49 -> 39, 4,326 in five 155 -> 133, 16 / 16 heads, 4,100 in nine 66 -> 61, 8,000 in 24 93 -> 77, in one 612 -> 623.
-// Two rounds or less favour the waves of 16 pairs: 1,950 rows (488 tiles) 71 / 86, four segments of 4,096 (512) 98 / 103.
-// Behind a prefix every tile walks about as far, full-size ones read half the keys a pair, and what is gained is their unfilled
-// last round: 2,300 rows at 9,000 (288 full tiles) 670 -> 548, 2,600 at 2,600 (325) 321 -> 281, but 4,096 at 4,000 (512) 489 / 535.
+// chunks of 2,300 rows (576 tiles) 133 -> 123, 3,500 231 -> 205, 6,000 422 -> 410, but 11,000 (1,375 full tiles) 1,227 / 1,255: at
+// more than four rounds of full-size tiles their last one no longer shows; packed segments, 2,600 rows in 13 49 -> 40, 4,326 in
+// five 155 -> 140, 16 / 16 heads, 4,100 in nine 66 -> 62, 8,000 in 24 93 -> 81, 8,000 rows in one 612 / 640 (the host sees only
+// the rows).  Two rounds or less favour the waves of 16 pairs: 1,950 rows (488 tiles) 71 / 86, four segments of 4,096 (512) 98 /
+// 103.  Behind a prefix every tile walks about as far, full-size ones read half the keys a pair, and what is gained is their
+// unfilled last round: 2,300 rows at 9,000 (288 full tiles) 670 -> 556, 2,600 at 2,600 (325) 321 -> 284, but 4,096 at 4,000 (512)
+// 489 / 535.  Far into a document no step is heavy and the results are a hundredth further off (at 26,000 1.21e-4 against 1.20e-4
+// of the 2-norm), so calls behind more than 16,384 keys stay here.
 static bool gqa_prefill_takes_f16(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
                                   unsigned int head_dim, int kv_format)
 {
@@ -1392,7 +1391,7 @@ static bool gqa_prefill_takes_f16(unsigned int rows, unsigned int position, unsi
         return false;
     }
     const unsigned long long full = tiles_of(256u), rounds = (full + kComputeUnitsPrefill - 1) / kComputeUnitsPrefill;
-    return (unsigned long long)position * 4u <= rows || full * 10u <= rounds * kComputeUnitsPrefill * 9u;
+    return rounds <= 4u && position <= 16384u && ((unsigned long long)position * 4u <= rows || full * 10u <= rounds * kComputeUnitsPrefill * 9u);
 }
 
 unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,

@@ -14,6 +14,18 @@ namespace {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kStep = 32;                 // tokens per step
 constexpr float kPBias = 8.0f;            // probabilities are carried as p * 2^8: f16 stays normal down to p = 2^-22
+// The softmax reference of a column follows its maximum only when a score passes it by more than 2^kSlack: a probability is
+// then at most 2^kSlack, and p' = p * v_scale * 2^(kPBias - window) below 2^15 (f16 ends at 2^16).  A running maximum moves in
+// some column of a wave on most of the first hundred steps, and every move reduces across the lanes and rescales the
+// accumulators: 1,000 rows of 32 / 8 heads 45.1 -> 43.0 us, 2,048 of 16 / 4 77 -> 72, 2,048 f16 rows of 256 at 6,144 394 -> 379.
+constexpr float kSlack = 6.0f;
+// P' is carried as f16 hi + lo (22 significant bits) while the probabilities a lane holds of a step weigh more than 1 /
+// kLoThreshold of its running sum.  A lane sums a quarter of the tokens, so below that each is < 1 / 64 of its row's sum, and the
+// hi term's rounding (2^-12 relative, random sign) moves the normalised output by < 2^-12 / 64 of |v|.  8 was enough while the
+// reference was the maximum itself, whose probability is a one and has no rounding error; with 16 the distance from 64 bits
+// (2-norm) is smaller than it was at every size tried: 1,000 rows 4.2e-6 -> 6.1e-7, 4,000 7.3e-5 -> 4.9e-5, 2,048 at 50,000
+// 1.82e-4 -> 1.80e-4 (4,100 f16 rows of 256 in one segment 1.79e-4 -> 1.65e-4; kSlack with 8: 1.87e-4).
+constexpr float kLoThreshold = 16.0f;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 

@@ -10,8 +10,8 @@
 //   The rows go from global memory straight to LDS (no staging registers) two tiles ahead in a ring of three: 48 KB of tiles
 //       and at most 168 registers let three workgroups of four waves live on a compute unit, where eight waves of 16 pairs
 //       around four staged tiles were alone on it.
-// 16 / 4 heads, 4,100 rows in one segment: 285 -> 215 us; in nine segments (16 / 16 heads) 67 -> 62, which are two workgroups a compute unit and last as long as
-// the longest range (36 tiles); 32 / 8 heads, 2,600 rows in 13 50 -> 40, a first chunk of 3,500 rows 231 -> 199.
+// 16 / 4 heads, 4,100 rows in one segment: 285 -> 223 us; in nine segments (16 / 16 heads) 67 -> 62, which are two workgroups a compute unit and last as long as
+// the longest range (36 tiles); 32 / 8 heads, 2,600 rows in 13 50 -> 40, a first chunk of 3,500 rows 231 -> 205.
 #include <type_traits>
 
 #include "gqa_prefill.hpp"
@@ -42,15 +42,11 @@ __device__ __forceinline__ unsigned int swizzle(unsigned int row)
     return ((row & 1u) << 3) | ((row & 2u) << 1) | ((row >> 2) & 3u);
 }
 
-// The softmax reference of a column follows its maximum only when a score passes it by more than 2^kSlack: a probability is
-// then at most 2^kSlack, p * 2^kPBias at most 2^14 (f16 ends at 2^16), and the rescaling of the accumulators, which a running
-// maximum of 32 columns asks for on most of the first steps, is rare (one segment of 4,100 rows 232 -> 215 us).
-constexpr float kSlack = 6.0f;
-// P is carried as f16 hi, and lo while some probability of the step weighs more than 1 / kLoShare of its row: against 64 bits
-// the results are then no further off than those of 16-pair waves, whose reference is always the maximum itself (its
-// probability, a one, has no rounding error) and whose test is per eight tokens: 1.08e-5 / 3.11e-5 (2-norm, this kernel / that
-// one) over nine segments of 4,100 rows, 1.76e-4 / 1.81e-4 over one.
-constexpr float kLoShare = 64.0f;
+// P is carried as f16 hi, and lo while some probability of the step weighs more than 1 / kLoShare of its row: a test of the
+// largest one, which a lane of sixteen tokens has at hand, instead of a sum of eight.  Distance from 64 bits (2-norm), tiles
+// of 16-pair waves / this kernel: nine segments of 4,100 rows 3.1e-5 / 3.7e-6, one 1.81e-4 / 1.58e-4, a first chunk of 3,000 rows
+// 2.9e-5 / 2.0e-5 (with 64 3.0e-5), 2,300 rows at 9,000 4.8e-5 / 4.2e-5 (with 80 5.2e-5).
+constexpr float kLoShare = 96.0f;
 
 // Reduction over a wave inside the vector ALU: rows of sixteen lanes by rotation, then across the rows
 template <class Op> __device__ __forceinline__ unsigned int wave_reduce(unsigned int v, Op op)
