@@ -484,13 +484,22 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
             const bool edge = t0 + kStep > wave_min_hi || t0 < wave_max_lo;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                float x = s[e >> 2][ct][e & 3];
-                if constexpr (SOFTCAP) {
-                    // caps that models use take the five-instruction form (see gqa_prefill_f16), larger ones the precise one
-                    x = small_cap ? cap_log2 * fmaf(-2.0f, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * tanh_arg) + 1.0f), 1.0f)
-                                  : cap_log2 * soft_tanh(x * q_fac * inv_cap);
+                sc[e] = s[e >> 2][ct][e & 3];
+            }
+            if constexpr (SOFTCAP) {
+                // caps that models use take the five-instruction form (see gqa_prefill_tiles), larger ones the precise one; one
+                // branch around the eight scores (a choice per score is a branch per score, and their chains run one by one)
+                if (small_cap) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        sc[e] = cap_log2 * fmaf(-2.0f, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(sc[e] * tanh_arg) + 1.0f), 1.0f);
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        sc[e] = cap_log2 * soft_tanh(sc[e] * q_fac * inv_cap);
+                    }
                 }
-                sc[e] = x;
             }
             if (edge) {
 #pragma unroll
@@ -1142,19 +1151,26 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
             const bool edge = t0 + kStep > wave_min_hi || t0 < wave_max_lo;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                float x = s[e >> 2][ct][e & 3];
-                if constexpr (SOFTCAP) {
-                    // tanh(y) = 1 - 2 / (e^(2y) + 1) for the caps models use: the form cancels for tiny y, and its absolute error,
-                    // a few units of 2^-24, is multiplied by the cap (3e-6 of a score under a cap of 50); larger caps take the
-                    // polynomial-or-exponential form, which keeps the limit of an ever larger cap.  The cap rides in `mult`.
-                    if (small_cap) {
-                        const float e2y = __builtin_amdgcn_exp2f(x * tanh_arg);
-                        x = fmaf(-2.0f, __builtin_amdgcn_rcpf(e2y + 1.0f), 1.0f);
-                    } else {
-                        x = soft_tanh(x * score_mult * inv_cap);
+                sc[e] = s[e >> 2][ct][e & 3];
+            }
+            if constexpr (SOFTCAP) {
+                // tanh(y) = 1 - 2 / (e^(2y) + 1) for the caps models use: the form cancels for tiny y, and its absolute error,
+                // a few units of 2^-24, is multiplied by the cap (3e-6 of a score under a cap of 50); larger caps take the
+                // polynomial-or-exponential form, which keeps the limit of an ever larger cap.  The cap rides in `mult`.  One branch
+                // around the eight scores: a choice per score is a branch per score, and their chains run one by one (2,048
+                // rows at 6,144, 16 / 8 heads of 256, a full and a sliding layer 460 -> 431 us a pass).
+                if (small_cap) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float e2y = __builtin_amdgcn_exp2f(sc[e] * tanh_arg);
+                        sc[e] = fmaf(-2.0f, __builtin_amdgcn_rcpf(e2y + 1.0f), 1.0f);
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        sc[e] = soft_tanh(sc[e] * score_mult * inv_cap);
                     }
                 }
-                sc[e] = x;
             }
             if (edge) {
 #pragma unroll
