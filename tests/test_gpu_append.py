@@ -199,3 +199,24 @@ def test_mla_append_positions_from_device_memory(layout, rotary_dim, rows):
     assert np.array_equal(codes.cpu().numpy(), ref_codes), "codes differ"
     assert np.array_equal(scales.cpu().numpy().view(np.uint16), ref_scales), "scale bits differ"
     assert np.array_equal(rope_cache.cpu().numpy().view(np.uint16), ref_rope), "rope bits differ"
+
+
+@pytest.mark.parametrize("rows", [910, 1025, 2730, 4096, 4097])  # nine, seven, three, two and one waves a row
+@pytest.mark.parametrize("latent", [512, 192])
+def test_mla_append_in_one_call_and_in_pieces(rows, latent):
+    """A long chunk's rows are shared by fewer waves each: the same bytes as in pieces of a hundred rows."""
+    from zllm_amd import ops
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows)
+    x, rope = torch.randn(rows, latent, generator=gen, device="cuda"), torch.randn(rows, 64, generator=gen, device="cuda")
+    cos, sin = torch.randn(rows, 32, generator=gen, device="cuda"), torch.randn(rows, 32, generator=gen, device="cuda")
+    pages = (rows + 15) // 16
+    table = torch.randperm(pages, generator=gen, device="cuda").to(torch.int32)
+    planes = [(torch.zeros(pages * 16, latent, dtype=torch.int8, device="cuda"), torch.zeros(pages * 16, latent // 64, dtype=torch.int16, device="cuda"),
+               torch.zeros(pages * 16, 64, dtype=torch.int16, device="cuda")) for _ in range(2)]
+    ops.mla_append(x, rope, *planes[0], table, 0, 16, cos=cos, sin=sin, rotary_dim=64)
+    for at in range(0, rows, 100):
+        end = min(at + 100, rows)
+        ops.mla_append(x[at:end], rope[at:end], *planes[1], table, at, 16, cos=cos, sin=sin, rotary_dim=64, rope_position=at)
+    for whole, pieces in zip(*planes):
+        assert torch.equal(whole, pieces)

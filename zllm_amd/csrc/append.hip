@@ -90,13 +90,14 @@ __global__ __launch_bounds__(256) void half_append_kernel(HalfAppendParams p)
     p.cache[physical * p.cols + column] = p.dst_dtype == 1 ? f32_to_bf16_bits(value) : f32_to_f16_bits(value);
 }
 
-// Fused MLA append (what paged_cache_append_mla_body computes, paged_mla/source.hip:672-758): one wave per unit of a token
-// row, a unit being one latent group (one value per lane) or the row's rope columns.  The rope columns are written as bf16:
+// Fused MLA append (what paged_cache_append_mla_body computes, paged_mla/source.hip:672-758).  A token row is a list of units, its
+// latent groups (one value per lane) and behind them its rope columns; gridDim.y waves share a row, each taking every
+// gridDim.y-th unit.  The rope columns are written as bf16:
 // those in front of the rotary part are copied, and each lane of the rotary part owns whole rotation pairs -- it loads the
 // pair and its cos / sin once and stores both rotated values.  Products are rounded on their own (no fused multiply-add), so
 // the bits do not depend on the compiler's contraction choices.
 // Nothing but latency bounds it: a row is 2 KiB.  One wave for the whole row quantized its groups one after the other, each a
-// load, a reduction through the lanes and two divisions: one row 7.0 us, now 2.9; 512 rows 8.6 us, now 4.7.
+// load, a reduction through the lanes and two divisions: one row 7.0 us, now 2.9; 512 rows 8.6 us, now 4.7 (in the trace).
 __global__ __launch_bounds__(256) void mla_append_kernel(MlaAppendParams p)
 {
     const unsigned int lane = threadIdx.x & 63u;
@@ -641,8 +642,11 @@ hipError_t launch_mla_append(const MlaAppendParams& p, hipStream_t stream)
     if (p.rows == 0) {
         return hipSuccess;
     }
-    const unsigned int units = p.latent_cols / 64u + 1u;
-    mla_append_kernel<<<dim3((p.rows + 3u) / 4u, units < 65535u ? units : 65535u), dim3(256), 0, stream>>>(p);
+    // As many waves a row as fill the device (8,192 in all), one for long chunks, whose loads then have the rows side by side and
+    // whose per-wave work would only multiply.  Waves a row 1 / 2 / 5 / 9, us: one row 5.7 / 4.1 / 3.0 / 2.7, 1,024 rows 6.6 / 4.8 /
+    // 3.9 / 4.1, 4,096 7.8 / 6.8 / 7.4 / 8.9, 8,192 10.3 / 10.7 / 12.1 / 15.1, 65,536 64.8 / 68.9 / 85.6 / 108.6
+    const unsigned int units = p.latent_cols / 64u + 1u, wanted = p.rows < 8192u ? 8192u / p.rows : 1u;
+    mla_append_kernel<<<dim3((p.rows + 3u) / 4u, units < wanted ? units : wanted), dim3(256), 0, stream>>>(p);
     return hipGetLastError();
 }
 
