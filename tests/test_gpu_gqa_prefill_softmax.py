@@ -1,0 +1,84 @@
+"""The online softmax of the chunk kernels where its reference point moves, behind a prefix of 2,000 keys of two kinds, so that
+the scores of a row are two exact levels.  Against 64-bit attention on three heads."""
+import numpy as np
+import pytest
+import torch
+
+from zllm_amd import capi, ops
+
+pytestmark = pytest.mark.gpu
+
+POSITION = 2000
+PAGE = 16
+# every chunk kernel and tile size: rows, query heads, KV heads, head_dim, cache, scales, query
+KERNELS = {
+    "q8 tiles of 64": (16, 16, 4, 128, "q8", "f16", torch.bfloat16),
+    "q8 tiles of 128": (32, 16, 4, 128, "q8", "f16", torch.bfloat16),
+    "q8 tiles of 128, f32 query": (100, 16, 4, 128, "q8", "f16", torch.float32),
+    "q8 tiles of 256": (100, 16, 4, 128, "q8", "f16", torch.bfloat16),
+    "q8 tiles of 256, f32 scales": (100, 16, 4, 128, "q8", "f32", torch.bfloat16),
+    "q8 64 wide": (100, 16, 4, 64, "q8", "f16", torch.bfloat16),
+    "q8 256 wide": (100, 8, 4, 256, "q8", "f16", torch.bfloat16),
+    "f16 tiles of 128": (32, 16, 4, 128, "f16", None, torch.bfloat16),
+    "f16 tiles of 256": (100, 16, 4, 128, "f16", None, torch.bfloat16),
+    "f16 256 wide": (100, 8, 4, 256, "f16", None, torch.bfloat16),
+    "f16 waves of 32 pairs": (1030, 64, 64, 128, "f16", None, torch.bfloat16),
+}
+
+
+def attend(kernel, q, low, high, rise, k_scale, score_scale):
+    """Distance (2-norm) from 64 bits of a chunk behind POSITION keys.  K of a key is `low` [KV heads, head_dim], from key `rise` on
+    `high`, times k_scale; V is random."""
+    rows, heads, kv_heads, dim, cache, scales, q_dtype = KERNELS[kernel]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + dim)
+    n = POSITION + rows
+    pages = (n + PAGE - 1) // PAGE
+    order = torch.randperm(pages, generator=gen, device="cuda").to(torch.int32)
+    at = (order.long()[:, None] * PAGE + torch.arange(PAGE, device="cuda")).view(-1)[:n]
+    groups = kv_heads * dim // 64
+    k_codes = torch.where(torch.arange(n, device="cuda")[:, None] < rise, low.reshape(1, -1), high.reshape(1, -1))
+    v_codes = torch.randint(-100, 101, (n, kv_heads * dim), generator=gen, device="cuda")
+    planes = []
+    for codes, scale in ((k_codes, k_scale), (v_codes, 2.0**-6)):
+        value = codes.double() * scale
+        if cache == "f16":
+            plane, scale_plane = torch.zeros(pages * PAGE, kv_heads * dim, dtype=torch.float16, device="cuda"), None
+            plane[at] = value.to(torch.float16)
+            assert torch.equal(plane[at].double(), value)
+        else:
+            plane = torch.zeros(pages * PAGE, kv_heads * dim, dtype=torch.int8, device="cuda")
+            scale_plane = torch.full((pages * PAGE, groups), scale, dtype=torch.float16 if scales == "f16" else torch.float32, device="cuda")
+            plane[at] = codes.to(torch.int8)
+        planes.append((plane, scale_plane, value.view(n, kv_heads, dim)))
+    (k_plane, k_scales, k), (v_plane, v_scales, v) = planes
+    q = q.to(q_dtype).view(rows, heads * dim).contiguous()
+    out = ops.gqa_prefill_chunk(q, k_plane, k_scales, v_plane, v_scales, order, POSITION, heads, kv_heads, dim, PAGE, score_scale, workspace=False,
+                                kv_format=capi.KV_F16 if cache == "f16" else capi.KV_Q8G64,
+                                scale_dtype=capi.SCALE_F32 if scales == "f32" else capi.SCALE_F16).view(rows, heads, dim)
+    off = []
+    hidden = torch.arange(n, device="cuda")[None] > POSITION + torch.arange(rows, device="cuda")[:, None]
+    for head in (0, heads // 2, heads - 1):
+        kvh = head // (heads // kv_heads)
+        s = (q.view(rows, heads, dim)[:, head].double() @ k[:, kvh].T.contiguous()) * score_scale
+        want = torch.softmax(s.masked_fill(hidden, float("-inf")), dim=-1) @ v[:, kvh]
+        off.append(((out[:, head].double() - want).norm() / want.norm()).item())
+    assert np.isfinite(off).all(), off
+    return max(off)
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_scores_too_large_to_add_a_few_units_to(kernel):
+    """Scores around 2^25 (base 2), where f32 has multiples of four: a rise by eight units is a rise, not a probability of 2^8, which
+    the f16 of the second product has no room for.  Products and sums are exact: 2^13 times 2^12, and 2^-3 times 0 or 2^6."""
+    rows, heads, kv_heads, dim, _, _, _ = KERNELS[kernel]
+    log2e = np.float32(1.4426950408889634)
+    near = np.float32(np.log(2.0)) + np.arange(-4, 5, dtype=np.float32) * np.float32(2.0**-24)
+    score_scale = next(s for s in near if s * log2e == 1)
+    low, high = torch.zeros(kv_heads, dim, device="cuda"), torch.zeros(kv_heads, dim, device="cuda")
+    low[:, 0] = high[:, 0] = 64.0
+    high[:, -1] = 1.0
+    q = torch.zeros(rows, heads, dim, device="cuda")
+    q[:, :, 0], q[:, :, -1] = 2.0**13, 2.0**-3
+    # numerator and denominator are f32 sums of 2,000 products: 2^-24 sqrt(2000) = 3e-6 each
+    assert attend(kernel, q, low, high, 40, 2.0**6, float(score_scale)) < 1e-5

@@ -517,7 +517,7 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
             }
             // The reference point of the column (a running maximum within 2^kSlack, V window) moves on few steps, so the
             // reduction across the wave's rows and the rescaling sit behind a test of the lane's own maximum.
-            if (__any(lane_max * mult > run_max[ct] + kSlack) || window_moved) {
+            if (__any(lane_max * mult - run_max[ct] > kSlack) || window_moved) {
                 const float step_max = wave_max_16x4(lane_max) * mult;
                 const float new_max = fmaxf(run_max[ct], step_max);
                 const float safe_max = new_max == kNegInf ? 0.0f : new_max;
@@ -1185,7 +1185,7 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
             for (int e = 1; e < 8; ++e) {
                 lane_max = fmaxf(lane_max, sc[e]);
             }
-            if (__any(lane_max * mult > run_max[ct] + kSlack) || window_moved) {
+            if (__any(lane_max * mult - run_max[ct] > kSlack) || window_moved) {
                 const float step_max = wave_max_16x4(lane_max) * mult;
                 const float new_max = fmaxf(run_max[ct], step_max);
                 const float safe_max = new_max == kNegInf ? 0.0f : new_max;

@@ -18,6 +18,7 @@ constexpr float kPBias = 8.0f;            // probabilities are carried as p * 2^
 // then at most 2^kSlack, and p' = p * v_scale * 2^(kPBias - window) below 2^15 (f16 ends at 2^16).  A running maximum moves in
 // some column of a wave on most of the first hundred steps, and every move reduces across the lanes and rescales the
 // accumulators: 1,000 rows of 32 / 8 heads 45.1 -> 43.0 us, 2,048 of 16 / 4 77 -> 72, 2,048 f16 rows of 256 at 6,144 394 -> 379.
+// The difference is compared, which is exact: from 2^25 on f32 rounds a maximum plus six to eight more.
 constexpr float kSlack = 6.0f;
 // P' is carried as f16 hi + lo (22 significant bits) while the probabilities a lane holds of a step weigh more than 1 /
 // kLoThreshold of its running sum.  A lane sums a quarter of the tokens, so below that each is < 1 / 64 of its row's sum, and the

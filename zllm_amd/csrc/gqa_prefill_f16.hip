@@ -366,7 +366,7 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
             upper = fmaxf(fmaxf(upper, s[i + 1]), s[i + 9]);
         }
         lane_max = fmaxf(lane_max, upper);
-        if (__any(lane_max * mult > run_max + kSlack)) {
+        if (__any(lane_max * mult - run_max > kSlack)) {
             const float new_max = fmaxf(run_max, halves_max(lane_max) * mult);
             const float safe_max = new_max == kNegInf ? 0.0f : new_max;
             const float alpha = __builtin_amdgcn_exp2f(run_max - safe_max);
