@@ -82,3 +82,19 @@ def test_scores_too_large_to_add_a_few_units_to(kernel):
     q[:, :, 0], q[:, :, -1] = 2.0**13, 2.0**-3
     # numerator and denominator are f32 sums of 2,000 products: 2^-24 sqrt(2000) = 3e-6 each
     assert attend(kernel, q, low, high, 40, 2.0**6, float(score_scale)) < 1e-5
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_tied_scores_behind_a_rise_lose_no_bits(kernel):
+    """A score that rises by 0.8 to 5.6 units (base 2) after two steps and stays: the probabilities of the 2,000 keys that share the
+    maximum are ones, exact in the f16 of a step that carries no low-order term.  Against a reference left at the first level
+    they are rounded, all by the same 2^-12."""
+    rows, heads, kv_heads, dim, _, _, _ = KERNELS[kernel]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(dim)
+    low = torch.randint(10, 51, (kv_heads, dim), generator=gen, device="cuda") * (torch.randint(0, 2, (kv_heads, dim), generator=gen, device="cuda") * 2 - 1)
+    # scores of the two levels: beta dim^0.5 x (mean magnitude 30) / 64, times one and two
+    beta = torch.linspace(0.55, 3.7, rows * heads, device="cuda")[torch.randperm(rows * heads, generator=gen, device="cuda")].view(rows, heads, 1)
+    q = low.sign().float().repeat_interleave(heads // kv_heads, dim=0)[None] * (beta * dim**-0.5 * 64 / 30)
+    # numerator and denominator are f32 sums of 2,000 products: 2^-24 sqrt(2000) = 3e-6 each
+    assert attend(kernel, q, low, 2 * low, 40, 2.0**-6, dim**-0.5) < 1e-5

@@ -24,7 +24,7 @@
 // The kernel is bound by the vector-ALU instructions it issues, not by the matrix cores, so whatever does not depend on
 // every (token, column) pair stays out of the common path of a step: the tile buffer is a literal (LDS addresses in
 // immediates), edge masks and the low-order P' pass sit behind wave-uniform branches, and a column's reference
-// (a running maximum, V window) is only touched when some lane's score passes it by more than 2^kSlack.
+// (running maximum, V window) is only touched when some lane's score passes it.
 #include <type_traits>
 
 #include "gqa_prefill.hpp"
@@ -351,12 +351,16 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
             acc[ct][t] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
+    constexpr bool kLag = kColTiles == 1; // see kSlack
     float run_max[kColTiles], run_sum[kColTiles];
+    float lane_top[kColTiles]; // the largest score the lane has met (kLag), or that of the step
+    bool two_terms = true;     // the step before carried both terms of its probabilities
     float ref_shift[kColTiles]; // what is added to a scaled score before exp2: bias - V window - running maximum
     unsigned int vis_lo[kColTiles], vis_hi[kColTiles]; // visible tokens [lo, hi) of each column's row
 #pragma unroll
     for (int ct = 0; ct < kColTiles; ++ct) {
         run_max[ct] = kNegInf;
+        lane_top[ct] = kNegInf;
         run_sum[ct] = 0.0f;
         ref_shift[ct] = kPBias;
         const unsigned int pos = p.position + col_row[ct];
@@ -476,7 +480,8 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
         PREFILL_PHASE_FENCE();
         // ---- online softmax per column --------------------------------------------------------------
         float pr[kColTiles][8];
-        bool heavy = false; // some probability of this step is not small against the sum so far
+        bool heavy = false;  // some probability of this step is not small against the sum so far
+        bool behind = false; // some score passed its column's reference, which stayed
 #pragma unroll
         for (int ct = 0; ct < kColTiles; ++ct) {
             float sc[8];
@@ -515,10 +520,12 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
             for (int e = 1; e < 8; ++e) {
                 lane_max = fmaxf(lane_max, sc[e]);
             }
-            // The reference point of the column (a running maximum within 2^kSlack, V window) moves on few steps, so the
-            // reduction across the wave's rows and the rescaling sit behind a test of the lane's own maximum.
-            if (__any(lane_max * mult - run_max[ct] > kSlack) || window_moved) {
-                const float step_max = wave_max_16x4(lane_max) * mult;
+            // The reference point of the column (running maximum, V window) moves on few steps, so the reduction across the
+            // wave's rows and the rescaling sit behind a test of what the lane itself has met.
+            lane_top[ct] = kLag ? fmaxf(lane_top[ct], lane_max * mult) : lane_max * mult;
+            const bool above = __any(lane_top[ct] > run_max[ct]);
+            if ((kLag && two_terms ? __any(lane_top[ct] - run_max[ct] > kSlack) : above) || window_moved) {
+                const float step_max = wave_max_16x4(lane_top[ct]);
                 const float new_max = fmaxf(run_max[ct], step_max);
                 const float safe_max = new_max == kNegInf ? 0.0f : new_max;
                 const float alpha = __builtin_amdgcn_exp2f(run_max[ct] - safe_max) * acc_fix;
@@ -531,6 +538,8 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
                         acc[ct][t] *= alpha;
                     }
                 }
+            } else if (kLag) {
+                behind = behind || above;
             }
             const float shift = ref_shift[ct];
             float step_sum = 0.0f;
@@ -544,8 +553,9 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
             heavy = heavy || step_sum * kLoThreshold > run_sum[ct];
         }
         // ---- O^T += Vcodes^T . P'_g ----------------------------------------------------------------------
-        // P' is carried as f16 hi + lo on heavy steps (kLoThreshold), elsewhere the lo product is skipped
-        const bool lo_pass = __any(heavy);
+        // P' is carried as f16 hi + lo on heavy steps (kLoThreshold) and wherever the reference lags, elsewhere the lo product is skipped
+        two_terms = __any(heavy);
+        const bool lo_pass = two_terms || behind;
         PREFILL_PHASE_FENCE();
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -1028,13 +1038,17 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
             acc[ct][t] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
+    constexpr bool kLag = D == 128 && CT == 1; // see kSlack
     float run_max[CT], run_sum[CT], ref_shift[CT];
+    float lane_top[CT]; // the largest score the lane has met (kLag), or that of the step
+    bool two_terms = true; // the step before carried both terms of its probabilities
     unsigned int vis_lo[CT], vis_hi[CT];
     unsigned int wave_min_hi = 0xffffffffu, wave_max_lo = 0u;
     unsigned int wave_max_hi = 0u, wave_min_lo = 0xffffffffu; // tokens outside [min_lo, max_hi) are nobody's in the wave
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
         run_max[ct] = kNegInf;
+        lane_top[ct] = kNegInf;
         run_sum[ct] = 0.0f;
         ref_shift[ct] = kPBias;
         const unsigned int pos = p.position + col_row[ct];
@@ -1144,7 +1158,7 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
         PREFILL_PHASE_FENCE();
         // ---- online softmax per column ----------------------------------------------------------------
         float pr[CT][8];
-        bool heavy = false;
+        bool heavy = false, behind = false;
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
             float sc[8];
@@ -1185,8 +1199,10 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
             for (int e = 1; e < 8; ++e) {
                 lane_max = fmaxf(lane_max, sc[e]);
             }
-            if (__any(lane_max * mult - run_max[ct] > kSlack) || window_moved) {
-                const float step_max = wave_max_16x4(lane_max) * mult;
+            lane_top[ct] = kLag ? fmaxf(lane_top[ct], lane_max * mult) : lane_max * mult;
+            const bool above = __any(lane_top[ct] > run_max[ct]);
+            if ((kLag && two_terms ? __any(lane_top[ct] - run_max[ct] > kSlack) : above) || window_moved) {
+                const float step_max = wave_max_16x4(lane_top[ct]);
                 const float new_max = fmaxf(run_max[ct], step_max);
                 const float safe_max = new_max == kNegInf ? 0.0f : new_max;
                 const float alpha = __builtin_amdgcn_exp2f(run_max[ct] - safe_max) * acc_fix;
@@ -1199,6 +1215,8 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
                         acc[ct][t] *= alpha;
                     }
                 }
+            } else if (kLag) {
+                behind = behind || above;
             }
             const float shift = ref_shift[ct];
             float step_sum = 0.0f;
@@ -1211,8 +1229,9 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
             heavy = heavy || step_sum * kLoThreshold > run_sum[ct];
         }
         // ---- O^T += V^T . P (Q8g64: P'_g = p * v_scale_g, four output tiles per scale group): f16 hi, and lo on
-        // heavy steps (kLoThreshold) ----
-        const bool lo_pass = __any(heavy);
+        // heavy steps (kLoThreshold) and wherever the reference lags ----
+        two_terms = __any(heavy);
+        const bool lo_pass = two_terms || behind;
         PREFILL_PHASE_FENCE();
 #pragma unroll
         for (int q = 0; q < C::kDT / 4; ++q) {

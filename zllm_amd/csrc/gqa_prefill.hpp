@@ -14,19 +14,22 @@ namespace {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kStep = 32;                 // tokens per step
 constexpr float kPBias = 8.0f;            // probabilities are carried as p * 2^8: f16 stays normal down to p = 2^-22
-// The softmax reference of a column follows its maximum only when a score passes it by more than 2^kSlack: a probability is
-// then at most 2^kSlack, and p' = p * v_scale * 2^(kPBias - window) below 2^15 (f16 ends at 2^16).  A running maximum moves in
-// some column of a wave on most of the first hundred steps, and every move reduces across the lanes and rescales the
-// accumulators: 1,000 rows of 32 / 8 heads 45.1 -> 43.0 us, 2,048 of 16 / 4 77 -> 72, 2,048 f16 rows of 256 at 6,144 394 -> 379.
+// P' is carried as f16 hi + lo (22 significant bits) while the probabilities a lane holds of a step weigh more than 1 /
+// kLoThreshold of its running sum.  A lane sums a quarter of the tokens; where they weigh about the same each is < 1 / 32 of its
+// row's sum below that, and the hi term's rounding (2^-12 relative, random sign) moves the normalised output by < 2^-12 / 32 of |v|
+// (where a lane holds most of its row's sum, by < 2^-12 / 8).
+constexpr float kLoThreshold = 8.0f;
+// The softmax reference of a column is its running maximum: the probability of the maximum, and of every key that ties with it,
+// is a one, which f16 holds.  It moves in some column of a wave on most of the first hundred steps, and every move reduces across
+// the lanes and rescales the accumulators.  Where the registers are there (one column tile of head_dim 128, kLag) it stays while
+// no score passes it by more than 2^kSlack and the steps carry both terms: a probability is then at most 2^kSlack, and p' = p *
+// v_scale * 2^(kPBias - window) below 2^15 (f16 ends at 2^16).  The step after one that needed only the hi term moves every
+// reference up to its maximum, and a step that meets one behind carries both terms, so no rounded probability is measured
+// against anything else.  1,000 rows of 32 / 8 heads 42.4 -> 40.5 us, 2,048 of 16 / 4 71.8 -> 68.7, 1,000 f16 rows of 32 / 8 34.9 -> 33.3.
+// With two column tiles it spills (2,048 rows at 50,000 4.52 -> 5.27 ms), at head_dim 64 the two votes a step cost long chunks more than
+// short ones gain (1,000 rows 39.4 -> 37.2, 2,048 at 30,000 1,056 -> 1,098), at 256 it is level.
 // The difference is compared, which is exact: from 2^25 on f32 rounds a maximum plus six to eight more.
 constexpr float kSlack = 6.0f;
-// P' is carried as f16 hi + lo (22 significant bits) while the probabilities a lane holds of a step weigh more than 1 /
-// kLoThreshold of its running sum.  A lane sums a quarter of the tokens, so below that each is < 1 / 64 of its row's sum, and the
-// hi term's rounding (2^-12 relative, random sign) moves the normalised output by < 2^-12 / 64 of |v|.  8 was enough while the
-// reference was the maximum itself, whose probability is a one and has no rounding error; with 16 the distance from 64 bits
-// (2-norm) is smaller than it was at every size tried: 1,000 rows 4.2e-6 -> 6.1e-7, 4,000 7.3e-5 -> 4.9e-5, 2,048 at 50,000
-// 1.82e-4 -> 1.80e-4 (4,100 f16 rows of 256 in one segment 1.79e-4 -> 1.65e-4; kSlack with 8: 1.87e-4).
-constexpr float kLoThreshold = 16.0f;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 

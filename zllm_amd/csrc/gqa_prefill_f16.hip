@@ -285,6 +285,8 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
         }
     }
     float run_max = kNegInf, run_sum = 0.0f, ref_shift = kPBias;
+    float lane_top = kNegInf; // the largest score the lane has met
+    bool two_terms = true;    // the step before carried both terms of its probabilities (see kSlack)
     unsigned int vis_lo, vis_hi; // visible tokens [lo, hi) of the column's row
     {
         const unsigned int pos = p.position + col_row;
@@ -366,8 +368,11 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
             upper = fmaxf(fmaxf(upper, s[i + 1]), s[i + 9]);
         }
         lane_max = fmaxf(lane_max, upper);
-        if (__any(lane_max * mult - run_max > kSlack)) {
-            const float new_max = fmaxf(run_max, halves_max(lane_max) * mult);
+        lane_top = fmaxf(lane_top, lane_max * mult);
+        bool behind = __any(lane_top > run_max); // some score passed its column's reference, which stays
+        if (two_terms ? __any(lane_top - run_max > kSlack) : behind) {
+            behind = false;
+            const float new_max = fmaxf(run_max, halves_max(lane_top));
             const float safe_max = new_max == kNegInf ? 0.0f : new_max;
             const float alpha = __builtin_amdgcn_exp2f(run_max - safe_max);
             ref_shift = kPBias - safe_max;
@@ -393,7 +398,8 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
         // ---- O^T += V^T . P: f16 hi, on heavy steps lo first, one turn of a loop each (as branches around the products the
         // two forms cost sixty registers of copies) ----
         const float top = __builtin_amdgcn_exp2f(fmaf(lane_max, mult, ref_shift)); // the lane's largest probability
-        const bool lo_pass = __any(top * kLoShare > halves_sum(run_sum));
+        two_terms = __any(top * kLoShare > halves_sum(run_sum));
+        const bool lo_pass = two_terms || behind;
         PREFILL_PHASE_FENCE();
         union VFrag {
             s16x4 s[2];
