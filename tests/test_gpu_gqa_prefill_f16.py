@@ -108,3 +108,25 @@ def test_soft_caps(softcap):
                                                            (torch.float32, True, torch.bfloat16, 4.0)])
 def test_outputs_and_queries(out_dtype, gate, q_dtype, spread):
     run(1030, 0, 64, 64, 16, out_dtype=out_dtype, gate=gate, q_dtype=q_dtype, spread=spread)
+
+
+@pytest.mark.parametrize("spread", [0.02, 0.2, 1.0])
+def test_short_ranges_carry_both_terms(spread):
+    """Segments of up to 400 keys, scores from near-even to ordinary: every step weighs more than a sixteenth of its row, so all
+    probabilities have 22 bits."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(7)
+    rows, heads = 3000, 32
+    lens = torch.tensor([400, 390, 310, 400, 200, 400, 100, 400, 400], device="cuda")
+    ends = torch.cumsum(lens, 0)
+    start, end = torch.repeat_interleave(ends - lens, lens), torch.repeat_interleave(ends, lens)
+    q = (torch.randn(rows, heads * D, generator=gen, device="cuda") * spread).to(torch.bfloat16)
+    k, v = (torch.randn((rows + 63) // 64 * 64, heads * D, generator=gen, device="cuda").to(torch.float16) for _ in range(2))
+    table = torch.arange(len(k) // 64, dtype=torch.int32, device="cuda")
+    out = ops.gqa_prefill_chunk(q, k, None, v, None, table, 0, heads, heads, D, 64, D**-0.5, kv_format=capi.KV_F16, visible_starts=start.to(torch.int32),
+                                visible_ends=end.to(torch.int32)).view(rows, heads, D)
+    for head in (0, heads - 1):
+        want = reference(q.view(rows, heads, D)[:, head], k.view(-1, heads, D)[:rows, head], v.view(-1, heads, D)[:rows, head], start, end, D**-0.5, 0.0)
+        # f32 sums of 400 products in numerator and denominator, 2^-24 sqrt(400) each, and scores of 128 products, 2^-24 sqrt(128) of |s| < 8
+        err = ((out[:, head].double() - want).norm() / want.norm()).item()
+        assert err <= 5e-6, f"head {head}: {err:.2e}"

@@ -42,11 +42,13 @@ __device__ __forceinline__ unsigned int swizzle(unsigned int row)
     return ((row & 1u) << 3) | ((row & 2u) << 1) | ((row >> 2) & 3u);
 }
 
-// P is carried as f16 hi, and lo while some probability of the step weighs more than 1 / kLoShare of its row: a test of the
-// largest one, which a lane of sixteen tokens has at hand, instead of a sum of eight.  Distance from 64 bits (2-norm), tiles
-// of 16-pair waves / this kernel: nine segments of 4,100 rows 3.1e-5 / 3.7e-6, one 1.81e-4 / 1.58e-4, a first chunk of 3,000 rows
-// 2.9e-5 / 2.0e-5 (with 64 3.0e-5), 2,300 rows at 9,000 4.8e-5 / 4.2e-5 (with 80 5.2e-5).
-constexpr float kLoShare = 96.0f;
+// P is carried as f16 hi, and lo while eight probabilities of a lane weigh more than 1 / lo_share of the lane's sum of those (the
+// test of the other chunk kernels, twice a lane).  The share is 16 and behind a prefix longer than the chunk 24, where those kernels
+// use 8: they cut such calls into other parts, and every part begins with both terms.  Distance from 64 bits (2-norm), tiles of 16-pair
+// waves / this kernel, where the standard deviation of the scores is 0.05 and 1: nine segments of 4,100 rows 1.1e-4 / 2.4e-5 and 3.1e-5 /
+// 2.9e-7, a first chunk of 2,300 rows (32 / 8 heads) 3.9e-5 / 2.2e-5 and 1.6e-6 / 2.9e-7, 2,300 rows at 9,000 1.80e-4 / 1.74e-4 and 5.6e-5 / 2.6e-5
+// (with 16 1.83e-4).  A test of the single largest probability against its row passes near-even rows over: 1.5e-4 on the nine segments.
+constexpr float kLoShare = 16.0f, kLoShareBehind = 24.0f;
 
 // Reduction over a wave inside the vector ALU: rows of sixteen lanes by rotation, then across the rows
 template <class Op> __device__ __forceinline__ unsigned int wave_reduce(unsigned int v, Op op)
@@ -284,7 +286,9 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
             acc[t][i] = 0.0f;
         }
     }
-    float run_max = kNegInf, run_sum = 0.0f, ref_shift = kPBias;
+    float run_max = kNegInf, ref_shift = kPBias;
+    float run_sum[2] = {0.0f, 0.0f}; // of the lane's first and second eight tokens of each step
+    const float lo_share = p.position > p.rows ? kLoShareBehind : kLoShare;
     float lane_top = kNegInf; // the largest score the lane has met
     bool two_terms = true;    // the step before carried both terms of its probabilities (see kSlack)
     unsigned int vis_lo, vis_hi; // visible tokens [lo, hi) of the column's row
@@ -376,7 +380,8 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
             const float safe_max = new_max == kNegInf ? 0.0f : new_max;
             const float alpha = __builtin_amdgcn_exp2f(run_max - safe_max);
             ref_shift = kPBias - safe_max;
-            run_sum *= alpha;
+            run_sum[0] *= alpha;
+            run_sum[1] *= alpha;
             run_max = new_max;
             if (__any(alpha != 1.0f)) {
 #pragma unroll
@@ -388,17 +393,22 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
                 }
             }
         }
-        float part_sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        float part_sum[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], mult, ref_shift));
-            part_sum[i & 3] += s[i];
+            part_sum[i >> 3][i & 1] += s[i];
         }
-        run_sum += (part_sum[0] + part_sum[1]) + (part_sum[2] + part_sum[3]);
+        bool heavy = false;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float eight = part_sum[e][0] + part_sum[e][1];
+            run_sum[e] += eight;
+            heavy = heavy || eight * lo_share > run_sum[e];
+        }
         // ---- O^T += V^T . P: f16 hi, on heavy steps lo first, one turn of a loop each (as branches around the products the
         // two forms cost sixty registers of copies) ----
-        const float top = __builtin_amdgcn_exp2f(fmaf(lane_max, mult, ref_shift)); // the lane's largest probability
-        two_terms = __any(top * kLoShare > halves_sum(run_sum));
+        two_terms = __any(heavy);
         const bool lo_pass = two_terms || behind;
         PREFILL_PHASE_FENCE();
         union VFrag {
@@ -470,7 +480,7 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // what was requested past the range lands before the LDS is given back
 
     // ---- normalise and store ----
-    const float total = halves_sum(run_sum);
+    const float total = halves_sum(run_sum[0] + run_sum[1]);
     if (!col_valid) {
         return;
     }
