@@ -415,3 +415,25 @@ def test_planning_entry_points_survive_arbitrary_argument_blocks(lib):
         need = lib.zllm_attn_mla_decode_workspace_bytes(C.byref(m))
         rc = lib.zllm_attn_mla_decode_record_layout(C.byref(m), C.byref(layout))
         assert (need > 0) == (rc == 0)
+
+
+def test_calls_without_k_or_v_are_refused_with_the_librarys_message(lib, monkeypatch):
+    import inspect
+
+    import torch
+
+    from zllm_amd import ops
+
+    monkeypatch.setattr(ops, "_stream", lambda: None)
+    q, kv = torch.zeros(1, 256), torch.zeros(1, 128)
+    codes, scales = torch.zeros(64, 128, dtype=torch.int8), torch.zeros(64, 2, dtype=torch.float16)
+    for k, v in ((None, kv), (kv, None)):
+        with pytest.raises(capi.ZllmAttnError, match="null pointer"):
+            ops.gqa_prologue(q, k, v, None, None, None, None, codes, scales, codes, scales, None, 0, 2, 1, 128, 0, 64)
+    lens = torch.ones(1, dtype=torch.int32)
+    with pytest.raises(capi.ZllmAttnError, match="null pointer"):
+        ops.gqa_decode(q, None, scales, codes, scales, None, lens, 2, 1, 128, 64, 0.1, 64)
+    with pytest.raises(capi.ZllmAttnError, match="null pointer"):
+        ops.gqa_prefill_chunk(q, codes, scales, None, scales, None, 0, 2, 1, 128, 64, 0.1)
+    # what a call does to its argument block is its own affair, not a parameter of the block's builder
+    assert list(inspect.signature(ops.gqa_decode_args).parameters)[-2:] == ["total_kv_tokens", "gate"]

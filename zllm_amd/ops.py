@@ -51,7 +51,7 @@ def gqa_prologue(q, k, v, q_norm, k_norm, cos, sin, k_codes, k_scales, v_codes, 
     rows = q.shape[0]
     q_out = q.new_empty((rows, num_heads * head_dim), dtype=q_out_dtype)
     args = capi.GqaPrologueArgs(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(q_norm), _ptr(k_norm), _ptr(cos), _ptr(sin), q_out.data_ptr(), _ptr(k_codes),
+        q.data_ptr(), _ptr(k), _ptr(v), _ptr(q_norm), _ptr(k_norm), _ptr(cos), _ptr(sin), q_out.data_ptr(), _ptr(k_codes),
         _ptr(k_scales), _ptr(v_codes), _ptr(v_scales), _ptr(table), _ptr(positions), rows, num_heads, num_kv_heads, head_dim, rotary_dim,
         0 if cos is None else cos.shape[0], position, block_tokens, ring_capacity, eps, weight_offset, _DTYPE[q.dtype],
         _DTYPE[q_out_dtype], rule, int(split_half))
@@ -92,10 +92,9 @@ def scatter_rows(plane, rows, table, first, block_tokens, ring_capacity=0):
     capi.check(capi.load().zllm_attn_scatter_rows(C.byref(args), _stream()))
 
 
-def gqa_decode_args(q, k_plane, k_scales, v_plane, v_scales, tables, kv_lens, num_heads, num_kv_heads, head_dim,
-                    block_tokens, score_scale, max_kv_len, first_visible=None, softcap=0.0, ring_capacity=0,
-                    kv_format=capi.KV_Q8G64, scale_dtype=capi.SCALE_F16, out=None, workspace=None, total_kv_tokens=0, gate=None,
-                    launched=False):
+def _gqa_decode_args(launched, q, k_plane, k_scales, v_plane, v_scales, tables, kv_lens, num_heads, num_kv_heads, head_dim,
+                     block_tokens, score_scale, max_kv_len, first_visible=None, softcap=0.0, ring_capacity=0,
+                     kv_format=capi.KV_Q8G64, scale_dtype=capi.SCALE_F16, out=None, workspace=None, total_kv_tokens=0, gate=None):
     batch = q.shape[0]
     if out is None:
         out = q.new_empty((batch, num_heads * head_dim), dtype=torch.float32)
@@ -117,9 +116,17 @@ def gqa_decode_args(q, k_plane, k_scales, v_plane, v_scales, tables, kv_lens, nu
     return args, out, workspace
 
 
+def gqa_decode_args(q, k_plane, k_scales, v_plane, v_scales, tables, kv_lens, num_heads, num_kv_heads, head_dim,
+                    block_tokens, score_scale, max_kv_len, first_visible=None, softcap=0.0, ring_capacity=0,
+                    kv_format=capi.KV_Q8G64, scale_dtype=capi.SCALE_F16, out=None, workspace=None, total_kv_tokens=0, gate=None):
+    return _gqa_decode_args(False, q, k_plane, k_scales, v_plane, v_scales, tables, kv_lens, num_heads, num_kv_heads, head_dim,
+                            block_tokens, score_scale, max_kv_len, first_visible, softcap, ring_capacity, kv_format, scale_dtype, out,
+                            workspace, total_kv_tokens, gate)
+
+
 def gqa_decode(*a, **kw):
     """Batched GQA decode over the paged cache (zllm_attn_gqa_decode).  Returns f32 [batch, Hq*d]."""
-    args, out, workspace = gqa_decode_args(*a, launched=True, **kw)
+    args, out, workspace = _gqa_decode_args(True, *a, **kw)
     capi.check(capi.load().zllm_attn_gqa_decode(C.byref(args), _stream()))
     return out
 
