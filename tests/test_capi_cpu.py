@@ -267,6 +267,24 @@ def test_given_ranges_are_cut_into_kv_splits_behind_a_long_prefix_only(lib):
         assert _ranges_prefill_bytes(lib, rows, position, heads, kv_heads, capi.KV_Q8G64) == 0
 
 
+def _causal_f16_bytes(lib, rows, position, heads=32, kv_heads=8, page=16, table=0x20000):
+    """Workspace of a causal chunk over f16 rows of head_dim 128 (256 compute units where no device says otherwise)."""
+    pre = capi.GqaPrefillArgs(rows=rows, position=position, num_heads=heads, num_kv_heads=kv_heads, head_dim=128, block_tokens=page, score_scale=0.1,
+                              kv_format=capi.KV_F16, q_dtype=capi.DTYPE_BF16, out_dtype=capi.DTYPE_F32, table=table,
+                              table_stride=0 if table is None else (position + rows + page - 1) // page)
+    return lib.zllm_attn_gqa_prefill_workspace_bytes(C.byref(pre))
+
+
+def test_pages_without_scalar_addresses_keep_the_row_tiles_of_256(lib):
+    """2,300 rows behind 9,000 keys are 288 tiles of 256 pairs, a round and an eighth, and cut into seven; the kernel of 32-pair waves
+    would run them as 576 tiles."""
+    seven = 7 * 2300 * 32 * 128 * 4
+    for page, table in ((24, 0x20000), (4, 0x20000), (1, 0x20000), (16, None), (96, None)):
+        assert seven < _causal_f16_bytes(lib, 2300, 9000, page=page, table=table) < 1.1 * seven
+    for page in (8, 16, 1024):
+        assert _causal_f16_bytes(lib, 2300, 9000, page=page) < 0.6 * seven
+
+
 def test_prefill_and_mla_argument_checks_without_a_gpu(lib):
     pre = capi.GqaPrefillArgs()
     pre.rows, pre.num_heads, pre.num_kv_heads, pre.head_dim, pre.block_tokens = 8, 8, 2, 128, 16

@@ -1106,7 +1106,7 @@ void plan_prefill_splits(const zllm_gqa_prefill_args* a, uint32_t* chunk_tokens,
 {
     const uint32_t group = a->num_heads / a->num_kv_heads;
     const uint32_t columns = zllm::gqa_prefill_tile_pairs(a->rows, a->position, a->window, a->num_heads, a->num_kv_heads, a->head_dim, a->kv_format,
-                                                          a->scale_dtype, a->q_dtype, a->visible_starts != nullptr);
+                                                          a->scale_dtype, a->q_dtype, a->visible_starts != nullptr, zllm::prefill_scalar_pages(a->table, a->block_tokens));
     const uint32_t tile_rows = columns / group > 0 ? columns / group : 1u;
     const uint64_t tiles = ((uint64_t)a->rows + tile_rows - 1) / tile_rows;
     uint64_t longest = (uint64_t)a->position + a->rows; // keys the last row tile may see
@@ -1243,7 +1243,7 @@ static bool few_rows_as_decode_items(const zllm_gqa_prefill_args* a)
     const bool half_tiles = a->kv_format == ZLLM_KV_Q8G64 &&
                             a->head_dim == 128 &&
                             zllm::gqa_prefill_tile_pairs(a->rows, a->position, a->window, a->num_heads, a->num_kv_heads, a->head_dim, a->kv_format, a->scale_dtype,
-                                                         a->q_dtype, a->visible_starts != nullptr) <= 128u;
+                                                         a->q_dtype, a->visible_starts != nullptr, zllm::prefill_scalar_pages(a->table, a->block_tokens)) <= 128u;
     return (uint64_t)a->rows * tokens * 34u < tokens * (half_tiles ? 80u : 150u) + 1300000u;
 }
 

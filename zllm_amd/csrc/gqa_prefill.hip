@@ -1412,13 +1412,14 @@ template <int D, int KV, int SDT, int CT = TileShape<D>::kCT> static hipError_t 
 // the rows).  Two rounds or less favour the waves of 16 pairs: 1,950 rows (488 tiles) 71 / 86, four segments of 4,096 (512) 98 /
 // 103.  Behind a prefix every tile walks about as far, full-size ones read half the keys a pair, and what is gained is their
 // unfilled last round: 2,300 rows at 9,000 (288 full tiles) 670 -> 556, 2,600 at 2,600 (325) 321 -> 284, but 4,096 at 4,000 (512)
-// 489 / 535.  Far into a document no step is heavy and the results are a hundredth further off (at 26,000 1.21e-4 against 1.20e-4
+// 489 / 535.  Pages it cannot address by scalars stay here: with an address a lane it spilled 28 registers, some inside its loop, and took
+// 132 us instead of 75 on the nine segments, 250 instead of 163 on the five (24-token pages).  Far into a document no step is heavy and the results are a hundredth further off (at 26,000 1.21e-4 against 1.20e-4
 // of the 2-norm), so calls behind more than 16,384 keys stay here.
 static bool gqa_prefill_takes_f16(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
-                                  unsigned int head_dim, int kv_format)
+                                  unsigned int head_dim, int kv_format, bool scalar_pages)
 {
     const unsigned int group = num_heads / num_kv_heads;
-    if (kv_format != 1 || head_dim != 128u || window != 0u || group == 0u || group > 128u) {
+    if (kv_format != 1 || !scalar_pages || head_dim != 128u || window != 0u || group == 0u || group > 128u) {
         return false;
     }
     auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
@@ -1430,7 +1431,7 @@ static bool gqa_prefill_takes_f16(unsigned int rows, unsigned int position, unsi
 }
 
 unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
-                                    unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges)
+                                    unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges, bool scalar_pages)
 {
     if (head_dim != (unsigned int)kD || (kv_format == 0 && scale_dtype == 2) || num_kv_heads == 0) {
         return head_dim == 256u ? 128u : 256u; // neither gqa_prefill_q8's geometry nor f16 rows of head_dim 128
@@ -1440,7 +1441,7 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
         return 256u;
     }
     auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
-    if (gqa_prefill_takes_f16(rows, position, window, num_heads, num_kv_heads, head_dim, kv_format)) {
+    if (gqa_prefill_takes_f16(rows, position, window, num_heads, num_kv_heads, head_dim, kv_format, scalar_pages)) {
         return 128u;
     }
     if (kv_format == 1 && ranges && (position <= rows || tiles_of(256u) * 5u <= kComputeUnitsPrefill)) {
@@ -1478,10 +1479,11 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
 
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scale_dtype, hipStream_t stream)
 {
+    const bool scalar_pages = prefill_scalar_pages(p.table, p.block_tokens);
     const unsigned int tile_pairs = gqa_prefill_tile_pairs(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scale_dtype,
-                                                           p.q_dtype, p.visible_starts != nullptr);
+                                                           p.q_dtype, p.visible_starts != nullptr, scalar_pages);
     if (kv_format == 1) { // f16 rows
-        if (gqa_prefill_takes_f16(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format)) {
+        if (gqa_prefill_takes_f16(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scalar_pages)) {
             return launch_gqa_prefill_f16(p, stream);
         }
         if (p.head_dim == 128u && tile_pairs == 128u) {

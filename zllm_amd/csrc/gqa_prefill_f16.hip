@@ -12,8 +12,6 @@
 //       around four staged tiles were alone on it.
 // 16 / 4 heads, 4,100 rows in one segment: 285 -> 223 us; in nine segments (16 / 16 heads) 67 -> 62, which are two workgroups a compute unit and last as long as
 // the longest range (36 tiles); 32 / 8 heads, 2,600 rows in 13 50 -> 40, a first chunk of 3,500 rows 231 -> 205.
-#include <type_traits>
-
 #include "gqa_prefill.hpp"
 
 namespace zllm {
@@ -28,6 +26,7 @@ constexpr int kPairs = 32 * kWaves;
 constexpr int kBufs = 3;              // tile buffers: one attended, two on their way
 constexpr int kRun = kStep / kWaves;  // rows of a tile that a wave requests, 4 a load
 constexpr int kLoads = kRun / 4;      // loads of 64 x 16 bytes a wave issues per plane and tile
+static_assert(kRun <= 8, "prefill_scalar_pages: pages of eight tokens hold a wave's rows");
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -94,9 +93,9 @@ __device__ __forceinline__ void load_to_lds(const unsigned char* from, unsigned 
     __builtin_amdgcn_global_load_lds((global_ptr_t)from, (lds_ptr_t)to, 16, 0, 0);
 }
 
-// SOFTCAP: 0 none, 1 caps below 256 (see below), 2 larger ones.  PAGED: pages of a power of two, kRun tokens at least, behind a
-// block table: the rows a wave requests of a tile lie in one page, and their address is scalar but for the lane's constant part.
-template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) void gqa_prefill_f16(GqaPrefillParams p)
+// SOFTCAP: 0 none, 1 caps below 256 (see below), 2 larger ones.  The rows a wave requests of a tile lie in one page
+// (prefill_scalar_pages), and their address is scalar but for the lane's constant part.
+template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 3) void gqa_prefill_f16(GqaPrefillParams p)
 {
     struct Lds {
         unsigned char k[kBufs][kTile];
@@ -188,60 +187,36 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
         lane_col[u] = (m ^ swizzle(wave * kRun + u * 4u + lane_row)) * 16u + kvh * kRow;
         lane_at[u] = lane_col[u] + (u * 4u + lane_row) * k_row;
     }
-    struct Entries {
-        unsigned int e[PAGED ? 1 : kLoads];
-    };
     auto first_of = [&](unsigned int t0) __attribute__((always_inline)) -> unsigned int { // of the wave's rows, inside the range
         const unsigned int t = t0 + wave * kRun;
         return t > last_token ? last_token & ~(unsigned int)(kRun - 1) : t;
     };
-    auto token_of = [&](unsigned int t0, int u) __attribute__((always_inline)) -> unsigned int {
-        return min(t0 + wave * kRun + u * 4u + lane_row, last_token);
+    auto load_entry = [&](unsigned int t0) __attribute__((always_inline)) -> unsigned int {
+        return ((scalar_words_t)(uintptr_t)p.table)[first_of(t0) >> p.block_shift];
     };
-    auto load_entries = [&](Entries& en, unsigned int t0) __attribute__((always_inline)) {
-        if constexpr (PAGED) {
-            en.e[0] = ((scalar_words_t)(uintptr_t)p.table)[first_of(t0) >> p.block_shift];
-        } else {
-#pragma unroll
-            for (int u = 0; u < kLoads; ++u) {
-                const unsigned int page = token_of(t0, u) / p.block_tokens;
-                en.e[u] = p.table != nullptr ? p.table[page] : page;
-            }
-        }
-    };
-    auto load_tile = [&](int buf, unsigned int t0, const Entries& en) __attribute__((always_inline)) {
+    auto load_tile = [&](int buf, unsigned int t0, unsigned int page) __attribute__((always_inline)) {
         unsigned char* const k_to = lds.k[buf] + wave * (kLoads * 1024u);
         unsigned char* const v_to = lds.v[buf] + wave * (kLoads * 1024u);
-        if constexpr (PAGED) {
-            const unsigned int t = first_of(t0), left = last_token - t;
-            const unsigned long long at = (((unsigned long long)en.e[0] << p.block_shift) + (t & (p.block_tokens - 1u))) * k_row;
-            const unsigned char* const kp = p.k_plane + at;
-            const unsigned char* const vp = p.v_plane + at;
+        const unsigned int t = first_of(t0), left = last_token - t;
+        const unsigned long long at = (((unsigned long long)page << p.block_shift) + (t & (p.block_tokens - 1u))) * k_row;
+        const unsigned char* const kp = p.k_plane + at;
+        const unsigned char* const vp = p.v_plane + at;
 #pragma unroll
-            for (int u = 0; u < kLoads; ++u) {
-                unsigned int from = lane_at[u];
-                if (left < kRun - 1u) {
-                    from = lane_col[u] + min(u * 4u + lane_row, left) * k_row;
-                }
-                load_to_lds(kp + from, k_to + u * 1024u);
-                load_to_lds(vp + from, v_to + u * 1024u);
+        for (int u = 0; u < kLoads; ++u) {
+            unsigned int from = lane_at[u];
+            if (left < kRun - 1u) {
+                from = lane_col[u] + min(u * 4u + lane_row, left) * k_row;
             }
-        } else {
-#pragma unroll
-            for (int u = 0; u < kLoads; ++u) {
-                const unsigned long long at = ((unsigned long long)en.e[u] * p.block_tokens + token_of(t0, u) % p.block_tokens) * k_row + lane_col[u];
-                load_to_lds(p.k_plane + at, k_to + u * 1024u);
-                load_to_lds(p.v_plane + at, v_to + u * 1024u);
-            }
+            load_to_lds(kp + from, k_to + u * 1024u);
+            load_to_lds(vp + from, v_to + u * 1024u);
         }
     };
     // the first tiles travel while the query is made ready
-    Entries en;
-    load_entries(en, part.begin);
+    unsigned int page = load_entry(part.begin);
 #pragma unroll
     for (int n = 0; n < kBufs - 1; ++n) {
-        load_tile(n, part.begin + n * kStep, en);
-        load_entries(en, part.begin + (n + 1) * kStep);
+        load_tile(n, part.begin + n * kStep, page);
+        page = load_entry(part.begin + (n + 1) * kStep);
     }
 
     // The wave's queries as f16 after a multiplication by one power of two that puts their largest magnitude into [2^8, 2^9)
@@ -461,8 +436,8 @@ template <int SOFTCAP, bool PAGED> __global__ __launch_bounds__(64 * kWaves, 3) 
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kBufs - 2) * kLoads * 2) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        load_tile((buf + kBufs - 1) % kBufs, t0 + (kBufs - 1) * kStep, en);
-        load_entries(en, t0 + kBufs * kStep);
+        load_tile((buf + kBufs - 1) % kBufs, t0 + (kBufs - 1) * kStep, page);
+        page = load_entry(t0 + kBufs * kStep);
         // a tile of packed segments walks the union of its rows' ranges, a wave only what some row of its own sees
         if (t0 < wave_max_hi && t0 + kStep > wave_min_lo) {
             attend(buf, t0);
@@ -545,18 +520,13 @@ hipError_t launch_gqa_prefill_f16(const GqaPrefillParams& p, hipStream_t stream)
     }
     const unsigned int rows_per_wg = p.group >= (unsigned int)kPairs ? 1u : (unsigned int)kPairs / p.group;
     const dim3 grid((p.rows + rows_per_wg - 1) / rows_per_wg * p.num_kv_heads, 1, p.max_chunks > 1u ? p.max_chunks : 1u);
-    const bool paged = p.table != nullptr && (p.block_tokens & (p.block_tokens - 1u)) == 0 && p.block_tokens >= (unsigned int)kRun;
-    auto launch = [&](auto cap) {
-        constexpr int CAP = decltype(cap)::value;
-        paged ? gqa_prefill_f16<CAP, true><<<grid, dim3(64 * kWaves), 0, stream>>>(p)
-              : gqa_prefill_f16<CAP, false><<<grid, dim3(64 * kWaves), 0, stream>>>(p);
-    };
+    const dim3 block(64 * kWaves);
     if (!(p.softcap > 0.0f)) {
-        launch(std::integral_constant<int, 0>{});
+        gqa_prefill_f16<0><<<grid, block, 0, stream>>>(p);
     } else if (p.softcap < 256.0f) {
-        launch(std::integral_constant<int, 1>{});
+        gqa_prefill_f16<1><<<grid, block, 0, stream>>>(p);
     } else {
-        launch(std::integral_constant<int, 2>{});
+        gqa_prefill_f16<2><<<grid, block, 0, stream>>>(p);
     }
     return hipGetLastError();
 }

@@ -188,7 +188,13 @@ struct MlaDecodeParams {
 // Q8g64 rows, or all pairs fit: half of a workgroup's waves then take every other 32 tokens of the range.  The split
 // planner and the launcher both ask.
 unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
-                                    unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges);
+                                    unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges, bool scalar_pages);
+
+// Pages that gqa_prefill_f16.hip addresses by scalars: a power of two of at least its eight tokens a wave, behind a block table
+inline bool prefill_scalar_pages(const unsigned int* table, unsigned int block_tokens)
+{
+    return table != nullptr && block_tokens >= 8u && (block_tokens & (block_tokens - 1u)) == 0;
+}
 
 // KV heads (= waves) per GQA decode workgroup for a head dimension.
 unsigned int gqa_decode_max_waves(unsigned int head_dim);
