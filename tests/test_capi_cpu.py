@@ -285,6 +285,17 @@ def test_pages_without_scalar_addresses_keep_the_row_tiles_of_256(lib):
         assert _causal_f16_bytes(lib, 2300, 9000, page=page) < 0.6 * seven
 
 
+def test_rows_behind_a_prefix_leave_the_tiles_of_256_for_an_unfilled_last_round_only(lib):
+    """f16 rows of 32 / 8 heads: 64 rows are eight tiles of 256 pairs, 2,048 rows one of each of 256 compute units.  Those tiles are cut
+    where they leave a round unfilled; the 32-pair waves of the other kernel are asked for fewer parts, or none."""
+    record = 32 * 128 * 4
+    # the last round half full, and one tile a KV head more
+    assert _causal_f16_bytes(lib, 3072, 9000) == 0 and _causal_f16_bytes(lib, 3073, 9000) > 2 * 3073 * record
+    assert _causal_f16_bytes(lib, 3300, 9000) > 3 * 3300 * record
+    # no further than 16,384 keys
+    assert _causal_f16_bytes(lib, 3000, 16384) == 0 and _causal_f16_bytes(lib, 3000, 16385) > 2 * 3000 * record
+
+
 def test_prefill_and_mla_argument_checks_without_a_gpu(lib):
     pre = capi.GqaPrefillArgs()
     pre.rows, pre.num_heads, pre.num_kv_heads, pre.head_dim, pre.block_tokens = 8, 8, 2, 128, 16

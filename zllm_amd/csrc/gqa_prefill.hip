@@ -1405,29 +1405,40 @@ template <int D, int KV, int SDT, int CT = TileShape<D>::kCT> static hipError_t 
 } // namespace
 
 // More tiles of 128 pairs than two rounds of one workgroup a compute unit, f16 rows of head_dim 128: the kernel of which three
-// live on one (gqa_prefill_f16.hip).  Against the better of the tiles of this file (us, 32 / 8 heads where not given): first
-// chunks of 2,300 rows (576 tiles) 133 -> 123, 3,500 231 -> 205, 6,000 422 -> 410, but 11,000 (1,375 full tiles) 1,227 / 1,255: at
-// more than four rounds of full-size tiles their last one no longer shows; packed segments, 2,600 rows in 13 49 -> 40, 4,326 in
-// five 155 -> 140, 16 / 16 heads, 4,100 in nine 66 -> 62, 8,000 in 24 93 -> 81, 8,000 rows in one 612 / 640 (the host sees only
-// the rows).  Two rounds or less favour the waves of 16 pairs: 1,950 rows (488 tiles) 71 / 86, four segments of 4,096 (512) 98 /
-// 103.  Behind a prefix every tile walks about as far, full-size ones read half the keys a pair, and what is gained is their
-// unfilled last round: 2,300 rows at 9,000 (288 full tiles) 670 -> 556, 2,600 at 2,600 (325) 321 -> 284, but 4,096 at 4,000 (512)
-// 489 / 535.  Pages it cannot address by scalars stay here: with an address a lane it spilled 28 registers, some inside its loop, and took
-// 132 us instead of 75 on the nine segments, 250 instead of 163 on the five (24-token pages).  Far into a document no step is heavy and the results are a hundredth further off (at 26,000 1.21e-4 against 1.20e-4
-// of the 2-norm), so calls behind more than 16,384 keys stay here.
+// live on one (gqa_prefill_f16.hip).  Against the tiles of this file (us a call, 32 / 8 heads where not given):
+// Nothing before the rows.  First chunks of 2,300 rows (576 tiles) 168 -> 116, 3,500 263 -> 204, 4,096 197 / 196, 6,144 427 -> 421,
+//   8,192 674 / 687; more than four rounds of full-size tiles no longer show their last one, 11,000 rows 1,227 / 1,255.  Two rounds
+//   or less favour the waves of 16 pairs: 1,950 rows (488 tiles) 71 / 86, four segments of 4,096 (512) 98 / 103.
+// Packed segments, also behind a prefix of up to a quarter of the rows: 16 / 16 heads, 4,100 in nine 73 -> 69; 8,000 (512 full-size
+//   tiles, two whole rounds) in 24 104 -> 74, in eight 183 -> 170, in three 339 -> 328, in two 463 -> 410, but in one 616 / 690, which
+//   the host cannot tell from the others: it sees only the rows.
+// Behind a prefix every tile walks about as far, full-size ones read half the keys a pair, and what is gained is their
+//   unfilled last round.  It has to be at most half full: 2,300 rows at 9,000 (288 full-size tiles) 667 -> 592, 5,000 (632) 1,212
+//   -> 1,166, but 3,300 at 13,000 (416) 1,048 / 1,112, 5,500 (688) 1,722 / 1,777, one given range of 3,500 rows at 3,000 (440) 503 /
+//   564.  Causal rows behind fewer keys than rows start at ranges that differ, and only whole rounds lose: 2,600 at 2,600 313 ->
+//   284, 3,500 at 1,000 335 -> 279, but 4,096 at 500 (512) 233 / 257, at 1,000 270 / 314, 8,192 at 500 (1,024) 745 / 758.  From 16,384
+//   keys on the full-size tiles in parts are as fast: 3,000 rows at 16,000 1,054 / 1,061, 3,500 1,345 / 1,350.
+// Pages it cannot address by scalars: with an address a lane it spilled 28 registers, some inside its loop, and took 132 us instead of
+//   75 on the nine segments, 250 instead of 163 on 4,326 rows in five (24-token pages).
 static bool gqa_prefill_takes_f16(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
-                                  unsigned int head_dim, int kv_format, bool scalar_pages)
+                                  unsigned int head_dim, int kv_format, bool ranges, bool scalar_pages)
 {
     const unsigned int group = num_heads / num_kv_heads;
     if (kv_format != 1 || !scalar_pages || head_dim != 128u || window != 0u || group == 0u || group > 128u) {
         return false;
     }
     auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
-    if (tiles_of(128u) <= kComputeUnitsPrefill * 2u) {
+    const unsigned long long full = tiles_of(256u), rounds = (full + kComputeUnitsPrefill - 1) / kComputeUnitsPrefill;
+    if (tiles_of(128u) <= kComputeUnitsPrefill * 2u || rounds > 4u || position > 16384u) {
         return false;
     }
-    const unsigned long long full = tiles_of(256u), rounds = (full + kComputeUnitsPrefill - 1) / kComputeUnitsPrefill;
-    return rounds <= 4u && position <= 16384u && ((unsigned long long)position * 4u <= rows || full * 10u <= rounds * kComputeUnitsPrefill * 9u);
+    if (position == 0u || (ranges && (unsigned long long)position * 4u <= rows)) {
+        return true;
+    }
+    if (!ranges && position <= rows) {
+        return full * 10u <= rounds * kComputeUnitsPrefill * 9u;
+    }
+    return full - (rounds - 1u) * kComputeUnitsPrefill <= kComputeUnitsPrefill / 2u;
 }
 
 unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
@@ -1441,7 +1452,7 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
         return 256u;
     }
     auto tiles_of = [&](unsigned int columns) { return ((unsigned long long)rows + columns / group - 1) / (columns / group) * num_kv_heads; };
-    if (gqa_prefill_takes_f16(rows, position, window, num_heads, num_kv_heads, head_dim, kv_format, scalar_pages)) {
+    if (gqa_prefill_takes_f16(rows, position, window, num_heads, num_kv_heads, head_dim, kv_format, ranges, scalar_pages)) {
         return 128u;
     }
     if (kv_format == 1 && ranges && (position <= rows || tiles_of(256u) * 5u <= kComputeUnitsPrefill)) {
@@ -1483,7 +1494,7 @@ hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scal
     const unsigned int tile_pairs = gqa_prefill_tile_pairs(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scale_dtype,
                                                            p.q_dtype, p.visible_starts != nullptr, scalar_pages);
     if (kv_format == 1) { // f16 rows
-        if (gqa_prefill_takes_f16(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, scalar_pages)) {
+        if (gqa_prefill_takes_f16(p.rows, p.position, p.window, p.num_heads, p.num_kv_heads, p.head_dim, kv_format, p.visible_starts != nullptr, scalar_pages)) {
             return launch_gqa_prefill_f16(p, stream);
         }
         if (p.head_dim == 128u && tile_pairs == 128u) {
