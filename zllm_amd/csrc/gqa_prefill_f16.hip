@@ -162,10 +162,6 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 3) void gqa_pre
             t_end = max(t_end, wave_max_u(union_end));
         }
     }
-    if (p.window != 0 && p.visible_starts == nullptr) {
-        const unsigned int first_pos = p.position + row0 + 1u;
-        t_begin = first_pos > p.window ? first_pos - p.window : 0u;
-    }
     t_begin &= ~31u;
     const SplitRange part = split_range(p, t_begin, t_end);
     if (!part.live) {
@@ -270,7 +266,7 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 3) void gqa_pre
     {
         const unsigned int pos = p.position + col_row;
         unsigned int hi = pos + 1u;
-        unsigned int lo = (p.window != 0 && pos + 1u > p.window) ? pos + 1u - p.window : 0u;
+        unsigned int lo = 0;
         if (p.visible_starts != nullptr) { // the row's range as given
             hi = own_end;
             lo = min(own_start, hi);
@@ -515,9 +511,6 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 3) void gqa_pre
 
 hipError_t launch_gqa_prefill_f16(const GqaPrefillParams& p, hipStream_t stream)
 {
-    if (p.q_dtype == 0) {
-        return hipErrorInvalidValue; // the tiles hold a 16-bit query; f32 ones run as decode items
-    }
     const unsigned int rows_per_wg = p.group >= (unsigned int)kPairs ? 1u : (unsigned int)kPairs / p.group;
     const dim3 grid((p.rows + rows_per_wg - 1) / rows_per_wg * p.num_kv_heads, 1, p.max_chunks > 1u ? p.max_chunks : 1u);
     const dim3 block(64 * kWaves);

@@ -210,7 +210,8 @@ hipError_t launch_gather_rows(const GatherParams& p, hipStream_t stream);
 // kv_format: 0 = Q8g64, 1 = f16; scale_dtype: 0 = bf16, 1 = f16 (Q8 only).
 hipError_t launch_gqa_decode(const GqaDecodeParams& p, int kv_format, int scale_dtype, unsigned int stages, hipStream_t stream);
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scale_dtype, hipStream_t stream);
-// f16 rows at head_dim 128, 16-bit queries, tiles of 128 pairs (gqa_prefill_f16.hip)
+// f16 rows at head_dim 128 in tiles of 128 pairs (gqa_prefill_f16.hip): 16-bit queries, no sliding window, prefill_scalar_pages; the
+// caller has looked at all three
 hipError_t launch_gqa_prefill_f16(const GqaPrefillParams& p, hipStream_t stream);
 hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, hipStream_t stream);
 // The vector-ALU kernels for latent / rope widths other than 512 / 64 and for kv_b in other forms than bf16 (mla_generic.hip).
