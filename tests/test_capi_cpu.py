@@ -292,6 +292,9 @@ def test_rows_behind_a_prefix_leave_the_tiles_of_256_for_an_unfilled_last_round_
     # the last round half full, and one tile a KV head more
     assert _causal_f16_bytes(lib, 3072, 9000) == 0 and _causal_f16_bytes(lib, 3073, 9000) > 2 * 3073 * record
     assert _causal_f16_bytes(lib, 3300, 9000) > 3 * 3300 * record
+    # more than two rounds of tiles of 128 pairs: three parts, five of tiles of 256
+    assert _causal_f16_bytes(lib, 2048, 0) == 0 and 3 * 2049 * record < _causal_f16_bytes(lib, 2049, 0) < 4 * 2049 * record
+    assert _causal_f16_bytes(lib, 2049, 0, page=24) > 5 * 2049 * record
     # no further than 16,384 keys
     assert _causal_f16_bytes(lib, 3000, 16384) == 0 and _causal_f16_bytes(lib, 3000, 16385) > 2 * 3000 * record
 

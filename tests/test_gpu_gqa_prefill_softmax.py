@@ -98,3 +98,50 @@ def test_tied_scores_behind_a_rise_lose_no_bits(kernel):
     q = low.sign().float().repeat_interleave(heads // kv_heads, dim=0)[None] * (beta * dim**-0.5 * 64 / 30)
     # numerator and denominator are f32 sums of 2,000 products: 2^-24 sqrt(2000) = 3e-6 each
     assert attend(kernel, q, low, 2 * low, 40, 2.0**-6, dim**-0.5) < 1e-5
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_a_reference_that_lags_as_far_as_it_may(kernel):
+    """Twelve steps of 32 keys whose scores rise by 5.9 units (base 2) each, under V scales that fill their power of two or pass into
+    the next with every other step, and then the maximum for the rest: the largest values the second product's f16 may meet."""
+    rows, heads, kv_heads, dim, cache, scales, q_dtype = KERNELS[kernel]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + dim)
+    n = POSITION + rows
+    pages = (n + PAGE - 1) // PAGE
+    order = torch.randperm(pages, generator=gen, device="cuda").to(torch.int32)
+    at = (order.long()[:, None] * PAGE + torch.arange(PAGE, device="cuda")).view(-1)[:n]
+    level = torch.clamp(torch.arange(n, device="cuda") // 32, max=12)
+    k_codes = torch.zeros(n, kv_heads, dim, device="cuda")
+    k_codes[:, :, 0] = level[:, None]  # one product a score: exact
+    v_codes = torch.randint(-100, 101, (n, kv_heads * dim), generator=gen, device="cuda")
+    v_scale = 2.0**-6 * 1.9990234375 * 2.0 ** torch.clamp(level // 2, max=4)  # exact in f16
+    planes = []
+    for codes, scale in ((k_codes.view(n, -1), torch.ones(n, device="cuda")), (v_codes, v_scale)):
+        value = codes.double() * scale[:, None].double()
+        if cache == "f16":
+            plane, scale_plane = torch.zeros(pages * PAGE, kv_heads * dim, dtype=torch.float16, device="cuda"), None
+            plane[at] = value.to(torch.float16)
+            value = plane[at].double()
+        else:
+            plane = torch.zeros(pages * PAGE, kv_heads * dim, dtype=torch.int8, device="cuda")
+            scale_plane = torch.zeros((pages * PAGE, kv_heads * dim // 64), dtype=torch.float16 if scales == "f16" else torch.float32, device="cuda")
+            plane[at] = codes.to(torch.int8)
+            scale_plane[at] = scale[:, None].expand(n, kv_heads * dim // 64).to(scale_plane.dtype)
+        planes.append((plane, scale_plane, value.view(n, kv_heads, dim)))
+    (k_plane, k_scales, k), (v_plane, v_scales, v) = planes
+    q = torch.zeros(rows, heads, dim, device="cuda")
+    q[:, :, 0] = 1.0
+    score_scale = 5.9 * float(np.log(2.0))
+    out = ops.gqa_prefill_chunk(q.to(q_dtype).view(rows, heads * dim), k_plane, k_scales, v_plane, v_scales, order, POSITION, heads, kv_heads, dim, PAGE,
+                                score_scale, workspace=False, kv_format=capi.KV_F16 if cache == "f16" else capi.KV_Q8G64,
+                                scale_dtype=capi.SCALE_F32 if scales == "f32" else capi.SCALE_F16).view(rows, heads, dim)
+    hidden = torch.arange(n, device="cuda")[None] > POSITION + torch.arange(rows, device="cuda")[:, None]
+    for head in (0, heads // 2, heads - 1):
+        kvh = head // (heads // kv_heads)
+        s = (q[:, head].double() @ k[:, kvh].T.contiguous()) * score_scale
+        want = torch.softmax(s.masked_fill(hidden, float("-inf")), dim=-1) @ v[:, kvh]
+        # sums of 1,600 tied keys, numerator and denominator, 2^-24 sqrt(1600) = 2.4e-6 each; against a reference left 5.9 units below
+        # the maximum, without the low-order term, the keys would be rounded alike by up to 2^-12
+        off = ((out[:, head].double() - want).norm() / want.norm()).item()
+        assert off < 1e-5, off
