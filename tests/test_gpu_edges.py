@@ -55,3 +55,15 @@ def test_pages_of_one_token_and_of_65536(page, lens):
     case = make_gqa_q8_case(8, lens, 8, 2, 128, block_tokens=page, pool_blocks=len(lens) + 2 if page > 4096 else None)
     got = run_decode(case, 0.09)
     assert_attention_close(got, oracle_gqa_decode(case, 0.09), f"pages of {page}")
+
+
+@pytest.mark.parametrize("raw", [True, False])
+def test_calls_go_to_the_current_stream_with_and_without_torchs_raw_handle(raw, monkeypatch):
+    from zllm_amd import ops
+
+    if not raw:
+        monkeypatch.setattr(ops, "_raw_stream", None)
+    assert ops._stream() == torch.cuda.current_stream().cuda_stream
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert ops._stream() == side.cuda_stream != torch.cuda.default_stream().cuda_stream

@@ -20,8 +20,12 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+# torch.cuda.current_stream() without the Stream object: 0.3 us a call instead of 2.7.  Not a public name: a torch without it takes the public way
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())  # torch.cuda.current_stream() without the Stream object
+    return torch.cuda.current_stream().cuda_stream if _raw_stream is None else _raw_stream(torch.cuda.current_device())
 
 
 def _dev(t, name):
