@@ -145,3 +145,36 @@ def test_a_reference_that_lags_as_far_as_it_may(kernel):
         # the maximum, without the low-order term, the keys would be rounded alike by up to 2^-12
         off = ((out[:, head].double() - want).norm() / want.norm()).item()
         assert off < 1e-5, off
+
+
+@pytest.mark.parametrize("cache,rows,heads,kv_heads,q_dtype", [("q8", 1000, 32, 8, torch.bfloat16), ("q8", 500, 32, 8, torch.float32), ("f16", 500, 64, 8, torch.bfloat16)])
+@pytest.mark.parametrize("spread", [0.05, 0.3])
+def test_the_first_512_keys_of_a_walk_carry_both_terms(cache, rows, heads, kv_heads, q_dtype, spread):
+    """Near-even rows of first chunks in the kernels whose reference lags: a wave walks 512 keys at most (in tiles of 64 pairs each half of
+    the waves takes every other 32 of 1,000), and eight of them weigh more than a sixteenth of their lane's sum."""
+    dim = 128
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + heads)
+    pages = (rows + PAGE - 1) // PAGE
+    table = torch.arange(pages, dtype=torch.int32, device="cuda")
+    planes = []
+    for _ in range(2):
+        if cache == "f16":
+            plane = torch.randn(pages * PAGE, kv_heads * dim, generator=gen, device="cuda").to(torch.float16)
+            planes.append((plane, None, plane.double().view(-1, kv_heads, dim)))
+        else:
+            plane = torch.clamp(torch.randn(pages * PAGE, kv_heads * dim, generator=gen, device="cuda") * 40, -127, 127).to(torch.int8)
+            scales = (0.02 + 0.01 * torch.rand(pages * PAGE, kv_heads * 2, generator=gen, device="cuda")).to(torch.float16)
+            planes.append((plane, scales, (plane.view(-1, kv_heads * 2, 64).double() * scales.double()[:, :, None]).view(-1, kv_heads, dim)))
+    (k_plane, k_scales, k), (v_plane, v_scales, v) = planes
+    q = (torch.randn(rows, heads * dim, generator=gen, device="cuda") * spread).to(q_dtype)
+    out = ops.gqa_prefill_chunk(q, k_plane, k_scales, v_plane, v_scales, table, 0, heads, kv_heads, dim, PAGE, dim**-0.5, workspace=False,
+                                kv_format=capi.KV_F16 if cache == "f16" else capi.KV_Q8G64).view(rows, heads, dim)
+    hidden = torch.ones(rows, rows, dtype=torch.bool, device="cuda").triu(1)
+    for head in (0, heads - 1):
+        kvh = head // (heads // kv_heads)
+        s = (q.view(rows, heads, dim)[:, head].double() @ k[:rows, kvh].T.contiguous()) * dim**-0.5
+        want = torch.softmax(s.masked_fill(hidden, float("-inf")), dim=-1) @ v[:rows, kvh]
+        # f32 sums of 1,000 products in numerator and denominator, 2^-24 sqrt(1000) each, and of 128 products a score, 2^-24 sqrt(128)
+        off = ((out[:, head].double() - want).norm() / want.norm()).item()
+        assert off < 5e-6, off

@@ -550,7 +550,7 @@ __global__ __launch_bounds__(kThreads) void gqa_prefill_q8(GqaPrefillParams p)
             }
             run_sum[ct] += step_sum;
             // the lane's eight probabilities together bound its largest one
-            heavy = heavy || step_sum * kLoThreshold > run_sum[ct];
+            heavy = heavy || step_sum * (kLag ? kLoThresholdLag : kLoThreshold) > run_sum[ct];
         }
         // ---- O^T += Vcodes^T . P'_g ----------------------------------------------------------------------
         // P' is carried as f16 hi + lo on heavy steps (kLoThreshold) and wherever the reference lags, elsewhere the lo product is skipped
@@ -1226,7 +1226,7 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
                 step_sum += pr[ct][e];
             }
             run_sum[ct] += step_sum;
-            heavy = heavy || step_sum * kLoThreshold > run_sum[ct];
+            heavy = heavy || step_sum * (kLag ? kLoThresholdLag : kLoThreshold) > run_sum[ct];
         }
         // ---- O^T += V^T . P (Q8g64: P'_g = p * v_scale_g, four output tiles per scale group): f16 hi, and lo on
         // heavy steps (kLoThreshold) and wherever the reference lags ----

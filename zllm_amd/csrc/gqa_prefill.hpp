@@ -17,8 +17,11 @@ constexpr float kPBias = 8.0f;            // probabilities are carried as p * 2^
 // P' is carried as f16 hi + lo (22 significant bits) while the probabilities a lane holds of a step weigh more than 1 /
 // kLoThreshold of its running sum.  A lane sums a quarter of the tokens; where they weigh about the same each is < 1 / 32 of its
 // row's sum below that, and the hi term's rounding (2^-12 relative, random sign) moves the normalised output by < 2^-12 / 32 of |v|
-// (where a lane holds most of its row's sum, by < 2^-12 / 8).
-constexpr float kLoThreshold = 8.0f;
+// (where a lane holds most of its row's sum, by < 2^-12 / 8).  Kernels whose reference lags (kSlack) take twice the share: their
+// ranges are short, and both terms for the first 512 keys of a walk are what the lag pays with.  Distance from 64 bits (2-norm) with 8
+// / 16, scores of deviation 1: 1,000 rows of 32 / 8 heads 6.9e-7 / 2.4e-7, of deviation 0.05 2.6e-5 / 2.1e-7; 2,000 rows 4.8e-5 / 2.0e-5, 4,000
+// of 16 / 4 7.1e-5 / 4.7e-5.  41.4 / 41.2 us, 90.1 / 91.5, 155 / 162.
+constexpr float kLoThreshold = 8.0f, kLoThresholdLag = 16.0f;
 // The softmax reference of a column is its running maximum: the probability of the maximum, and of every key that ties with it,
 // is a one, which f16 holds.  It moves in some column of a wave on most of the first hundred steps, and every move reduces across
 // the lanes and rescales the accumulators.  Where the registers are there (one column tile of head_dim 128, kLag) it stays while
