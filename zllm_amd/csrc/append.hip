@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void half_append_kernel(HalfAppendParams p)
 // pair and its cos / sin once and stores both rotated values.  Products are rounded on their own (no fused multiply-add), so
 // the bits do not depend on the compiler's contraction choices.
 // Nothing but latency bounds it: a row is 2 KiB.  One wave for the whole row quantized its groups one after the other, each a
-// load, a reduction through the lanes and two divisions: one row 7.0 us, now 2.9; 512 rows 8.6 us, now 4.7 (in the trace).
+// load, a reduction through the lanes and two divisions: one row 6.0 us, now 2.8; 512 rows 5.9 us, now 3.2 (in the trace).
 __global__ __launch_bounds__(256) void mla_append_kernel(MlaAppendParams p)
 {
     const unsigned int lane = threadIdx.x & 63u;

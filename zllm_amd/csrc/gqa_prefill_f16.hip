@@ -1,17 +1,20 @@
-// Chunked-prefill GQA attention over f16 rows at head_dim 128 in tiles of 128 (row, head-in-group) pairs: packed segments and
-// chunks of few row tiles.  What it computes is gqa_prefill_tiles (gqa_prefill.hip); how differs.
+// Chunked-prefill GQA attention over f16 rows at head_dim 128 in tiles of 128 (row, head-in-group) pairs: calls of more than two
+// rounds of such tiles that full-size ones would leave a last round of unfilled, and packed segments (gqa_prefill_takes_f16).  What it
+// computes is gqa_prefill_tiles (gqa_prefill.hip); how differs.
 //
-// Such a launch has a few waves a SIMD and short ranges, and what bounds it is the chain of instructions a wave runs for a
-// 32-token tile, not the matrix cores, memory or LDS: a wave alone on its SIMD takes as long per tile (1,740 cycles, 512 of them
-// matrix work) as one of three.  So the chain is kept short and the waves many:
+// What bounds such a launch is the chain of instructions a wave runs for a 32-token tile, not the matrix cores, memory or LDS: a
+// wave alone on its SIMD takes as long per tile (1,740 cycles, 512 of them matrix work) as one of three.  So the chain is kept short and
+// the waves many:
 //   32x32x16 matrix tiles: a wave owns 32 pairs, a lane sixteen scores of one pair, so the maximum, the sum and the tests of a
 //       step are made once for 32 pairs (twice with 16x16x32 tiles), and every K and V^T fragment read from LDS feeds twice the
 //       work of a 16-pair wave (LDS busy cycles 6.5 M -> 3.5 M on 4,100 rows of 16 heads in nine segments).
 //   The rows go from global memory straight to LDS (no staging registers) two tiles ahead in a ring of three: 48 KB of tiles
 //       and at most 168 registers let three workgroups of four waves live on a compute unit, where eight waves of 16 pairs
 //       around four staged tiles were alone on it.
-// 16 / 4 heads, 4,100 rows in one segment: 285 -> 223 us; in nine segments (16 / 16 heads) 67 -> 62, which are two workgroups a compute unit and last as long as
-// the longest range (36 tiles); 32 / 8 heads, 2,600 rows in 13 50 -> 40, a first chunk of 3,500 rows 231 -> 205.
+//       Six registers are spilled, all outside the loop.
+// 16 / 4 heads, 4,100 rows in one segment: 285 -> 232 us; in nine segments (16 / 16 heads) 69 -> 66, which are two workgroups a compute
+// unit and last as long as the longest walk, 36 tiles of 32 tokens: the longest segment has 21, but a row tile across a boundary walks both its
+// neighbours; 32 / 8 heads, 2,300 rows in eleven 48 -> 42, a first chunk of 3,500 rows 263 -> 204.
 #include "gqa_prefill.hpp"
 
 namespace zllm {
