@@ -393,6 +393,10 @@ typedef struct zllm_gqa_prefill_args {
     const uint32_t* visible_starts; /* [dev] [rows] or NULL */
 } zllm_gqa_prefill_args;
 ZLLM_API uint64_t zllm_attn_gqa_prefill_workspace_bytes(const zllm_gqa_prefill_args* args);
+/* The workspace with which the call is fastest: zllm_attn_gqa_prefill_workspace_bytes, and for chunks of many rows over
+ * Q8g64 rows of head_dim 128 room to convert every K and V row of the call once instead of once a row tile (at most
+ * 1 GiB more).  A call given less runs as described above. */
+ZLLM_API uint64_t zllm_attn_gqa_prefill_preferred_bytes(const zllm_gqa_prefill_args* args);
 ZLLM_API int zllm_attn_gqa_prefill_chunk(const zllm_gqa_prefill_args* args, zllm_stream_t stream);
 
 /* ------------------------------------------------------------------------- *

@@ -1262,6 +1262,23 @@ uint64_t zllm_attn_gqa_prefill_workspace_bytes(const zllm_gqa_prefill_args* a)
     return splits > items ? splits : items;
 }
 
+static uint32_t prefill_staged_tiles(const zllm_gqa_prefill_args* a, uint32_t* first)
+{
+    return zllm::gqa_prefill_staged_tiles(a->rows, a->position, a->window, a->num_heads, a->num_kv_heads, a->head_dim, a->kv_format, a->scale_dtype, a->q_dtype,
+                                          a->visible_ends != nullptr, first);
+}
+
+uint64_t zllm_attn_gqa_prefill_preferred_bytes(const zllm_gqa_prefill_args* a)
+{
+    const uint64_t least = zllm_attn_gqa_prefill_workspace_bytes(a);
+    if (validate_gqa_prefill(a) != 0 || prefill_rows_as_decode_items(a)) {
+        return least;
+    }
+    uint32_t first = 0;
+    const uint32_t tiles = prefill_staged_tiles(a, &first);
+    return tiles == 0 ? least : align_up(least, 256) + zllm::gqa_prefill_staged_bytes(tiles, a->num_kv_heads);
+}
+
 int zllm_attn_gqa_prefill_chunk(const zllm_gqa_prefill_args* a, zllm_stream_t stream)
 {
     const int rc = validate_gqa_prefill(a);
@@ -1354,7 +1371,19 @@ int zllm_attn_gqa_prefill_chunk(const zllm_gqa_prefill_args* a, zllm_stream_t st
             p.max_chunks = max_chunks;
         }
     }
-    const int launched = hip_status(zllm::launch_gqa_prefill(p, a->kv_format, a->scale_dtype, (hipStream_t)stream), "GQA prefill launch");
+    uint32_t staged_first = 0;
+    const uint32_t staged_tiles = prefill_staged_tiles(a, &staged_first);
+    if (staged_tiles != 0 && a->workspace != nullptr && ((uintptr_t)a->workspace & 15u) == 0) { // behind the records
+        const uint64_t least = align_up(max_chunks > 1 ? prefill_split_records(a, max_chunks).total : 0, 256);
+        if (a->workspace_bytes >= least + zllm::gqa_prefill_staged_bytes(staged_tiles, a->num_kv_heads)) {
+            p.staged = (unsigned char*)a->workspace + least;
+            p.staged_first = staged_first;
+            p.staged_tiles = staged_tiles;
+        }
+    }
+    const int launched = p.staged != nullptr
+                             ? hip_status(zllm::launch_gqa_prefill_staged(p, a->scale_dtype, (hipStream_t)stream), "GQA prefill staged launch")
+                             : hip_status(zllm::launch_gqa_prefill(p, a->kv_format, a->scale_dtype, (hipStream_t)stream), "GQA prefill launch");
     if (launched != 0 || p.max_chunks <= 1) {
         return launched;
     }

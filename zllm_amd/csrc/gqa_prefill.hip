@@ -1488,6 +1488,30 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
     return tiles_of(256u) <= kComputeUnitsPrefill ? 128u : 256u;
 }
 
+// Full-size row tiles over Q8g64 rows with the conversion taken out (gqa_prefill_staged.hip), us a call without / with (causal, bf16 queries):
+//   32 / 8 heads behind 2,000 keys: 200 rows (four tiles a KV head) 48 -> 45, 500 82 -> 66, 1,000 130 -> 110, 2,100 374 -> 290, 4,096 513 -> 431;
+//   behind 32,000: 200 rows 253 -> 244, 1,000 851 -> 741, 4,096 3,020 -> 2,532; 64 / 8, 1,000 rows behind 8,000 477 -> 389; 8 / 1, 2,100 behind
+//   8,000 271 -> 207; a window of 1,024 over 2,048 rows 112 -> 99.
+// The staging is a launch and a pass over the keys that few row tiles do not earn back: 80 rows of 32 / 8 (two tiles) 35.8 / 37.9 us behind 2,000,
+// 54 / 58 behind 8,000, of 64 / 8 (three) 225 / 235 behind 32,000; behind 600 keys they do, 48 -> 32.
+// The tiles are bounded by 1 GiB, 253,000 tokens of eight KV heads.
+unsigned int gqa_prefill_staged_tiles(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
+                                      unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ends, unsigned int* first)
+{
+    if (kv_format != 0 || head_dim != 128u || q_dtype == 0 || ends || num_kv_heads == 0u || num_kv_heads > 65535u || num_heads / num_kv_heads > 256u ||
+        gqa_prefill_tile_pairs(rows, position, window, num_heads, num_kv_heads, head_dim, kv_format, scale_dtype, q_dtype, false, false) != 256u) {
+        return 0;
+    }
+    const unsigned int group = num_heads / num_kv_heads, rows_per_tile = 256u / group, end = position + rows;
+    const unsigned int begin = window != 0u && position + 1u > window ? position + 1u - window : 0u;
+    if ((rows + rows_per_tile - 1u) / rows_per_tile < 4u && end - begin > 1024u) {
+        return 0;
+    }
+    *first = begin / (unsigned int)kStep;
+    const unsigned int tiles = (end + (unsigned int)kStep - 1u) / (unsigned int)kStep - *first;
+    return gqa_prefill_staged_bytes(tiles, num_kv_heads) <= (1ull << 30) ? tiles : 0u;
+}
+
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scale_dtype, hipStream_t stream)
 {
     const bool scalar_pages = prefill_scalar_pages(p.table, p.block_tokens);

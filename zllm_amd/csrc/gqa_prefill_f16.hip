@@ -15,7 +15,7 @@
 // 16 / 4 heads, 4,100 rows in one segment: 285 -> 232 us; in nine segments (16 / 16 heads) 69 -> 66, which are two workgroups a compute
 // unit and last as long as the longest walk, 36 tiles of 32 tokens: the longest segment has 21, but a row tile across a boundary walks both its
 // neighbours; 32 / 8 heads, 2,300 rows in eleven 48 -> 42, a first chunk of 3,500 rows 263 -> 204.
-#include "gqa_prefill.hpp"
+#include "gqa_prefill_x32.hpp"
 
 namespace zllm {
 
@@ -31,18 +31,8 @@ constexpr int kRun = kStep / kWaves;  // rows of a tile that a wave requests, 4 
 constexpr int kLoads = kRun / 4;      // loads of 64 x 16 bytes a wave issues per plane and tile
 static_assert(kRun <= 8, "prefill_scalar_pages: pages of eight tokens hold a wave's rows");
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* global_ptr_t;
-typedef const __attribute__((address_space(4))) unsigned int* scalar_words_t;
-
-// Chunk swizzle.  A 16-byte read takes sixteen rows of one chunk at a time, a transposed 8-byte read four rows of four chunks:
-// row bits 0 and 1 go into chunk bits 3 and 2, row bits 2 and 3 into chunk bits 0 and 1, and both meet every bank once
-// (the conflict counter reads 0).
-__device__ __forceinline__ unsigned int swizzle(unsigned int row)
-{
-    return ((row & 1u) << 3) | ((row & 2u) << 1) | ((row >> 2) & 3u);
-}
 
 // P is carried as f16 hi, and lo while eight probabilities of a lane weigh more than 1 / lo_share of the lane's sum of those (the
 // test of the other chunk kernels, twice a lane).  The share is 16 and behind a prefix longer than the chunk 24, where those kernels
@@ -51,41 +41,6 @@ __device__ __forceinline__ unsigned int swizzle(unsigned int row)
 // 2.9e-7, a first chunk of 2,300 rows (32 / 8 heads) 3.9e-5 / 2.2e-5 and 1.6e-6 / 2.9e-7, 2,300 rows at 9,000 1.80e-4 / 1.74e-4 and 5.6e-5 / 2.6e-5
 // (with 16 1.83e-4).  A test of the single largest probability against its row passes near-even rows over: 1.5e-4 on the nine segments.
 constexpr float kLoShare = 16.0f, kLoShareBehind = 24.0f;
-
-// Reduction over a wave inside the vector ALU: rows of sixteen lanes by rotation, then across the rows
-template <class Op> __device__ __forceinline__ unsigned int wave_reduce(unsigned int v, Op op)
-{
-    v = op(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false)); // row_ror:8
-    v = op(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false)); // row_ror:4
-    v = op(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false)); // row_ror:2
-    v = op(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false)); // row_ror:1
-    const u32x2_swap a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    v = op(a.x, a.y);
-    const u32x2_swap b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return __builtin_amdgcn_readfirstlane(op(b.x, b.y));
-}
-
-__device__ __forceinline__ unsigned int wave_min_u(unsigned int v)
-{
-    return wave_reduce(v, [](unsigned int x, unsigned int y) { return min(x, y); });
-}
-
-__device__ __forceinline__ unsigned int wave_max_u(unsigned int v)
-{
-    return wave_reduce(v, [](unsigned int x, unsigned int y) { return max(x, y); });
-}
-
-__device__ __forceinline__ float halves_sum(float v) // lanes l and l ^ 32, the two halves of a column
-{
-    const u32x2_swap b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(b.x) + __uint_as_float(b.y);
-}
-
-__device__ __forceinline__ float halves_max(float v)
-{
-    const u32x2_swap b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b.x), __uint_as_float(b.y));
-}
 
 // 64 x 16 bytes from global memory to 1 KiB of LDS: lane l's bytes land at `to` + 16 l.  The compiler counts these loads and
 // waits for all of them before the first transposed LDS read that follows, which it cannot tell from a read of the tile being
@@ -458,56 +413,7 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 3) void gqa_pre
     if (!col_valid) {
         return;
     }
-    const bool live = total > 0.0f && total < __builtin_inff();
-    if (p.max_chunks > 1u) { // records are in true units: without the bias of the probabilities
-        const size_t rec = ((size_t)col_row * p.max_chunks + blockIdx.z) * p.num_heads + col_head;
-        const float unbias = __builtin_amdgcn_exp2f(-kPBias);
-        if (h == 0u) {
-            p.stats[rec * 2] = live ? run_max : kNegInf;
-            p.stats[rec * 2 + 1] = live ? total * unbias : 0.0f;
-        }
-        float* out = p.partial + rec * (size_t)kD + 4u * h;
-#pragma unroll
-        for (int t = 0; t < kD / 32; ++t) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                *(f32x4*)(out + t * 32 + q * 8) = f32x4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]} * unbias;
-            }
-        }
-        return;
-    }
-    const float inv = live ? 1.0f / total : 0.0f; // accumulators and sum carry the same power of two
-    const size_t base = ((size_t)col_row * p.num_heads + col_head) * kD + 4u * h;
-#pragma unroll
-    for (int t = 0; t < kD / 32; ++t) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            f32x4 v = f32x4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]} * inv;
-            if (inv == 0.0f) {
-                v = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-            const size_t at = base + t * 32 + q * 8;
-            if (p.gate != nullptr) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    v[e] = gated(v[e], p.gate, p.gate_cols, p.gate_dtype, col_row, col_head * kD + 4u * h + t * 32 + q * 8 + e);
-                }
-            }
-            if (p.out_dtype == 0) {
-                *(f32x4*)((float*)p.out + at) = v;
-            } else {
-                unsigned short* o = (unsigned short*)p.out + at;
-                u32x2 packed;
-                if (p.out_dtype == 1) {
-                    packed = u32x2{pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3])};
-                } else {
-                    packed = u32x2{(unsigned int)f32_to_f16_bits(v[0]) | ((unsigned int)f32_to_f16_bits(v[1]) << 16),
-                                   (unsigned int)f32_to_f16_bits(v[2]) | ((unsigned int)f32_to_f16_bits(v[3]) << 16)};
-                }
-                *(u32x2*)o = packed;
-            }
-        }
-    }
+    store_column<kD>(p, col_row, col_head, h, run_max, total, acc, kPBias);
 }
 
 } // namespace

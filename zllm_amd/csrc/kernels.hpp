@@ -139,6 +139,9 @@ struct GqaPrefillParams {
     float* partial;
     float* stats;
     unsigned int chunk_tokens, max_chunks;
+    // K and V as f16 tiles of 32 tokens (gqa_prefill_staged.hip): `staged_tiles` a KV head, the first of them `staged_first`
+    unsigned char* staged;
+    unsigned int staged_first, staged_tiles;
 };
 
 struct MlaDecodeParams {
@@ -190,6 +193,12 @@ struct MlaDecodeParams {
 unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
                                     unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ranges, bool scalar_pages);
 
+// Tiles of 32 tokens, and the first of them, that a call reads of every KV head, where converting them once (gqa_prefill_staged.hip) is faster
+// than once a row tile: 0 for other calls.  What they take in the workspace.
+unsigned int gqa_prefill_staged_tiles(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
+                                      unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ends, unsigned int* first);
+uint64_t gqa_prefill_staged_bytes(unsigned int tiles, unsigned int num_kv_heads);
+
 // Pages that gqa_prefill_f16.hip addresses by scalars: a power of two of at least its eight tokens a wave, behind a block table
 inline bool prefill_scalar_pages(const unsigned int* table, unsigned int block_tokens)
 {
@@ -213,6 +222,9 @@ hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scal
 // f16 rows at head_dim 128 in tiles of 128 pairs (gqa_prefill_f16.hip): 16-bit queries, no sliding window, prefill_scalar_pages; the
 // caller has looked at all three
 hipError_t launch_gqa_prefill_f16(const GqaPrefillParams& p, hipStream_t stream);
+// Q8g64 rows of head_dim 128 converted once a call (gqa_prefill_staged.hip): 16-bit queries, causal or sliding rows; the caller has looked
+// at both, and at the workspace for the tiles
+hipError_t launch_gqa_prefill_staged(const GqaPrefillParams& p, int scale_dtype, hipStream_t stream);
 hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, hipStream_t stream);
 // The vector-ALU kernels for latent / rope widths other than 512 / 64 and for kv_b in other forms than bf16 (mla_generic.hip).
 hipError_t launch_mla_absorb_any(const MlaDecodeParams& p, hipStream_t stream);

@@ -984,7 +984,7 @@ Result<RocmTensor> RocmContext::gqa_attend(const RocmKvCache& cache, size_t laye
     a.q_dtype = abi_dtype(query.dtype);
     a.out_dtype = ZLLM_DTYPE_F32;
     a.visible_ends = visible_ends_dev;
-    const uint64_t need = zllm_attn_gqa_prefill_workspace_bytes(&a);
+    const uint64_t need = zllm_attn_gqa_prefill_preferred_bytes(&a);
     if (need != 0) {
         auto ws = workspace(need);
         if (ws.is_err()) {

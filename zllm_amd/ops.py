@@ -161,7 +161,7 @@ def gqa_prefill_chunk_args(q, k_plane, k_scales, v_plane, v_scales, table, posit
     args.table_stride = 0 if table is None else table.numel()
     scratch = None
     if workspace:
-        need = capi.load().zllm_attn_gqa_prefill_workspace_bytes(C.byref(args))
+        need = capi.load().zllm_attn_gqa_prefill_preferred_bytes(C.byref(args))
         scratch = torch.empty(max(int(need), 256), dtype=torch.uint8, device=q.device)
         args.workspace, args.workspace_bytes = _ptr(scratch), scratch.numel()
     return args, out, scratch
