@@ -1,0 +1,123 @@
+"""Chunked MLA prefill over latents that are converted once a call (mla_staged.hip), taken with the workspace that
+zllm_attn_mla_decode_preferred_bytes names: against the CPU oracle, and against the same call with no room for it."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tests.cases import assert_attention_close, to_torch_bf16, upload
+from tests.test_gpu_mla_decode import make_mla_chunk_case, oracle_mla_chunk, weight_args
+
+torch = pytest.importorskip("torch")
+
+
+def chunk_args(heads, rows, longest, batch=1, **fields):
+    from zllm_amd import capi
+
+    args = capi.MlaDecodeArgs(batch=batch, heads=heads, q_head_dim=192, kv_head_dim=256, latent_dim=512, rope_dim=64, block_tokens=64,
+                              max_ctx_len=longest, table_stride=0, q_dtype=capi.DTYPE_BF16, out_dtype=capi.DTYPE_F32, query_rows=rows)
+    for name, value in fields.items():
+        setattr(args, name, value)
+    return args
+
+
+def staged_bytes(*a, **kw):
+    """What the call asks for beyond the workspace it needs (256 compute units where no device says otherwise)."""
+    from zllm_amd import capi
+
+    args = chunk_args(*a, **kw)
+    return capi.load().zllm_attn_mla_decode_preferred_bytes(C.byref(args)) - capi.load().zllm_attn_mla_decode_workspace_bytes(C.byref(args))
+
+
+def test_which_calls_ask_for_staged_latents():
+    from zllm_amd import capi
+
+    tile = 39 * 1024 + 128
+    assert staged_bytes(128, 512, 16896) >= (16896 // 32) * tile
+    assert staged_bytes(128, 512, 16896, stage_mask=15) > 0
+    assert staged_bytes(128, 20, 10020) == 0 == staged_bytes(64, 16, 30016) == staged_bytes(16, 32, 8032) == staged_bytes(128, 1, 60000)
+    for stages in (1, 2, 14, capi.MLA_WIDE_TILES):
+        assert staged_bytes(128, 512, 16896, stage_mask=stages) == 0  # records for the caller, or another kernel asked for
+    ids = (C.c_uint32 * 1)()
+    assert staged_bytes(128, 512, 16896, selection=C.addressof(ids), top_k=2048) == 0
+    assert staged_bytes(16, 1000, 850000) > 0 and staged_bytes(16, 1000, 870000) == 0  # at most 1 GiB
+
+
+def run_chunk(case, room, out_dtype=None):
+    """The call with the preferred workspace, or with the least; max_ctx_len is the longest context."""
+    from zllm_amd import capi, ops
+
+    weights, form = weight_args(case)
+    rows, heads, batch = case["rows"], case["heads"], len(case["lens"])
+    args = chunk_args(heads, rows, int(case["lens"].max()), batch, block_tokens=case["block_tokens"])
+    lib = capi.load()
+    need = (lib.zllm_attn_mla_decode_preferred_bytes if room else lib.zllm_attn_mla_decode_workspace_bytes)(C.byref(args))
+    assert not room or need > lib.zllm_attn_mla_decode_workspace_bytes(C.byref(args)), "this shape is meant to be staged"
+    workspace = torch.full((need + 4096,), 0x7F, dtype=torch.uint8, device="cuda")
+    out = ops.mla_decode(to_torch_bf16(case["q_bits"], "cuda"), weights, upload(case["codes"]), upload(case["scales"]), upload(case["rope"]),
+                         upload(case["tables"]), upload(case["lens"]), heads, 192, 256, 512, 64, case["block_tokens"], int(case["lens"].max()),
+                         out_dtype=out_dtype or torch.float32, query_rows=rows, workspace=workspace[:need], **form)
+    torch.cuda.synchronize()
+    assert int(workspace[need:].min()) == int(workspace[need:].max()) == 0x7F, "written past the workspace"
+    return out.float().cpu().numpy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,lens,rows,kw", [
+    (1, [1500], 1000, {}),                                             # 128 rows a tile, a last tile of 104
+    (4, [3001], 101, dict(block_tokens=24)),                           # four row tiles, the last with five rows; pages of no power of two
+    (5, [1031, 700], 257, dict(block_tokens=1)),                       # two sequences; 25 rows a tile leave three pairs free
+    (16, [1400], 300, dict(w_std=0.2)),                                # a last tile of four rows; scores of a large spread
+    (8, [900], 900, {}),                                               # a first chunk: the first row sees one token
+    (40, [2200], 180, dict(poison=True)),                              # three rows a tile, the last wave part empty; rows past the end hold NaN
+    (250, [1999], 102, {}),                                            # one row a tile, two blocks of heads, the second three short
+    (8, [1800], 200, dict(latent_gain=2.0 ** np.repeat(np.arange(-9, 9), 100)))])  # the value window moves on, references too
+def test_staged_latents_against_the_oracle(heads, lens, rows, kw):
+    case = make_mla_chunk_case(heads + rows, lens, rows, heads, **kw)
+    want, _ = oracle_mla_chunk(case)
+    outs = [run_chunk(case, room) for room in (True, False)]
+    for got in outs:
+        scale = max(1.0, float(np.abs(want).max()))
+        assert_attention_close(got / scale, want / scale, f"heads={heads} lens={lens} rows={rows}")
+    # the two kernels round the same probabilities and products to f16 (2^-12 a term, independent over the tokens)
+    assert np.linalg.norm(outs[0] - outs[1]) <= 2.0 ** -11 * np.linalg.norm(outs[1])
+
+
+@pytest.mark.gpu
+def test_staged_latents_in_a_graph():
+    """Staging and attention recorded together, replayed over caches that change in between."""
+    from zllm_amd import capi, ops
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    heads, rows, total, page = 8, 240, 2000, 64
+    table = torch.randperm(40, generator=gen, device="cuda")[:32].to(torch.int32)[None].contiguous()
+    codes, scales, rope = (torch.zeros(40 * page, n, dtype=t, device="cuda") for n, t in ((512, torch.int8), (8, torch.int16), (64, torch.int16)))
+    lens = torch.tensor([total], dtype=torch.int32, device="cuda")
+    q = torch.randn(rows, heads * 192, generator=gen, device="cuda", dtype=torch.bfloat16)
+    weights = (torch.randn(heads * 256, 512, generator=gen, device="cuda") / 512 ** 0.5).to(torch.bfloat16)
+    args, out, workspace = ops.mla_decode_args(q, weights, codes, scales, rope, table, lens, heads, 192, 256, 512, 64, page, total, query_rows=rows)
+    lib = capi.load()
+    assert workspace.numel() > lib.zllm_attn_mla_decode_workspace_bytes(C.byref(args)), "this shape is meant to be staged"
+
+    def fill():
+        ops.mla_append(torch.randn(total, 512, generator=gen, device="cuda"), torch.randn(total, 64, generator=gen, device="cuda"), codes, scales, rope,
+                       table[0], 0, page)
+
+    def call():
+        capi.check(lib.zllm_attn_mla_decode(C.byref(args), ops._stream()))
+
+    fill()
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for _ in range(3):
+        fill()
+        call()
+        eager = out.clone()
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager) and float(out.abs().max()) > 0

@@ -9,7 +9,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libzllm_attn.so")
-SOURCES = ["api.hip", "append.hip", "gqa_decode.hip", "mla_decode.hip", "mla_partial_x32.hip", "mla_generic.hip", "gqa_prefill.hip", "gqa_prefill_f16.hip", "gqa_prefill_staged.hip"]
+SOURCES = ["api.hip", "append.hip", "gqa_decode.hip", "mla_decode.hip", "mla_partial_x32.hip", "mla_generic.hip", "mla_staged.hip", "gqa_prefill.hip", "gqa_prefill_f16.hip", "gqa_prefill_staged.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950",
@@ -23,10 +23,14 @@ FLAGS = [
     "-Wno-unknown-warning-option",
 ]
 
+# mla_staged.hip holds more than 256 accumulators and operands a lane: matrix instructions that may write either half of the register file
+# (without it the compiler puts every result into the accumulation half and copies: 284 spills)
+SOURCE_FLAGS = {"mla_staged.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+
 
 def _compile(src: str) -> str:
     obj = os.path.join(CSRC, src.replace(".hip", ".o"))
-    cmd = [HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj]
     result = subprocess.run(cmd, capture_output=True, text=True)
     if result.returncode != 0:
         sys.stderr.write(result.stdout + result.stderr)

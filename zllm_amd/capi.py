@@ -128,6 +128,7 @@ SYMBOLS = {
     "zllm_attn_gqa_prefill_preferred_bytes": (_u64, [C.POINTER(GqaPrefillArgs)]),
     "zllm_attn_gqa_prefill_chunk": (_int, [C.POINTER(GqaPrefillArgs), _ptr]),
     "zllm_attn_mla_decode_workspace_bytes": (_u64, [C.POINTER(MlaDecodeArgs)]),
+    "zllm_attn_mla_decode_preferred_bytes": (_u64, [C.POINTER(MlaDecodeArgs)]),
     "zllm_attn_mla_decode_record_layout": (_int, [C.POINTER(MlaDecodeArgs), C.POINTER(SplitRecordLayout)]),
     "zllm_attn_mla_decode": (_int, [C.POINTER(MlaDecodeArgs), _ptr]),
 }

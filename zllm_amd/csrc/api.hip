@@ -410,6 +410,34 @@ MlaWorkspace mla_workspace(const zllm_mla_decode_args* a, const MlaSplitPlan& pl
     return w;
 }
 
+// A whole call over latents that are converted once (mla_staged.hip): its splits, and the 32-token tiles a sequence.  0 tiles for other calls.
+// A compute unit takes a tile for 128 (row, head) pairs in 2.15 us there; mla_partial_ws takes it for 64 heads of one row in 1.42 us and for
+// up to 32 in 1.05.  The staging is a launch, and as many workgroups leave twice the records: the difference has to come to some 31 us over 256
+// compute units.  Us a call without / with: 128 heads, 20 rows behind 10,000 keys 109 / 116, 500 behind none 171 / 163, 512 behind
+// 16,384 2,824 / 2,330; 64 heads, 16 behind 30,000 116 / 133, 100 behind 3,000 115 / 107, 1,000 behind 8,000 1,504 / 1,239; 32 heads, 64
+// behind 4,000 69 / 75, behind 30,000 287 / 194, 1,000 behind none 157 / 137; 16 heads, 32 behind 8,000 58 / 66, 300 behind none 60 / 62,
+// behind 3,000 193 / 99, 1,000 behind 2,000 378 / 167.  The tiles are bounded by 1 GiB, 856,000 tokens.
+uint32_t plan_mla_staged(const zllm_mla_decode_args* a, MlaSplitPlan* plan)
+{
+    const uint32_t stages = a->stage_mask & 31u;
+    const uint64_t rows = mla_query_rows(a);
+    if ((stages != 0u && stages != 15u) || a->latent_dim != 512u || a->rope_dim != 64u || a->selection != nullptr || rows < 2u) {
+        return 0;
+    }
+    const uint32_t heads_here = a->heads < 128u ? a->heads : 128u;
+    const uint64_t units = (rows + 128u / heads_here - 1u) / (128u / heads_here) * a->batch * ((a->heads + heads_here - 1u) / heads_here);
+    const uint64_t tiles = ((uint64_t)a->max_ctx_len + 31u) / 32u;
+    const uint64_t steps = (a->max_ctx_len - (a->max_ctx_len < rows ? a->max_ctx_len : rows) / 2u) / 32u; // of a middle row
+    const uint64_t there = 215u * units, here = (a->heads <= 32u ? 105u : 142u) * rows * a->batch * ((a->heads + 63u) / 64u);
+    if (here <= there || steps * (here - there) < 800000u || units > 65535u || zllm::mla_staged_bytes((uint32_t)tiles, a->batch) > (1ull << 30)) {
+        return 0;
+    }
+    plan->dense = false;
+    plan_splits(a->max_ctx_len, units, 1, 64, &plan->chunk_tokens, &plan->max_chunks);
+    plan->record_rows = (uint64_t)a->batch * rows * plan->max_chunks;
+    return (uint32_t)tiles;
+}
+
 } // namespace
 
 extern "C" {
@@ -960,6 +988,18 @@ uint64_t zllm_attn_mla_decode_workspace_bytes(const zllm_mla_decode_args* a)
     return mla_workspace(a, plan_mla_decode(a)).total;
 }
 
+uint64_t zllm_attn_mla_decode_preferred_bytes(const zllm_mla_decode_args* a)
+{
+    const uint64_t least = zllm_attn_mla_decode_workspace_bytes(a);
+    MlaSplitPlan plan;
+    const uint32_t tiles = least == 0 ? 0 : plan_mla_staged(a, &plan);
+    if (tiles == 0) {
+        return least;
+    }
+    const uint64_t staged = align_up(mla_workspace(a, plan).total, 256) + zllm::mla_staged_bytes(tiles, a->batch);
+    return staged > least ? staged : least;
+}
+
 int zllm_attn_mla_decode_record_layout(const zllm_mla_decode_args* a, zllm_split_record_layout* out)
 {
     const int rc = validate_mla_decode(a);
@@ -998,10 +1038,23 @@ int zllm_attn_mla_decode(const zllm_mla_decode_args* a, zllm_stream_t stream)
     }
     zllm::MlaDecodeParams p;
     memset(&p, 0, sizeof(p));
-    const MlaSplitPlan plan = plan_mla_decode(a);
+    MlaSplitPlan plan;
+    MlaWorkspace w;
+    const uint32_t staged_tiles = plan_mla_staged(a, &plan);
+    if (staged_tiles != 0) {
+        w = mla_workspace(a, plan);
+        const uint64_t records = align_up(w.total, 256);
+        if (a->workspace_bytes >= records + zllm::mla_staged_bytes(staged_tiles, a->batch)) {
+            p.staged = (unsigned char*)a->workspace + records;
+            p.staged_tiles = staged_tiles;
+        }
+    }
+    if (p.staged == nullptr) {
+        plan = plan_mla_decode(a);
+        w = mla_workspace(a, plan);
+    }
     p.chunk_tokens = plan.chunk_tokens;
     p.max_chunks = plan.max_chunks;
-    const MlaWorkspace w = mla_workspace(a, plan);
     if (a->workspace_bytes < w.total) {
         return fail(-1, "MLA decode: workspace %llu bytes, need %llu", (unsigned long long)a->workspace_bytes, (unsigned long long)w.total);
     }

@@ -123,17 +123,6 @@ template <int SDT> __global__ __launch_bounds__(256) void gqa_stage_q8(GqaPrefil
     }
 }
 
-// 64 x 16 bytes (WIDE) or 64 x 4 from `from` + the lane's offset to LDS at `to` + AT + 16 or 4 times the lane.  In assembly, because the
-// compiler would wait for all of these loads before every LDS read that follows.
-template <bool WIDE, unsigned int AT> __device__ __forceinline__ void load_to_lds(const unsigned char* from, unsigned int lane_at, unsigned int to)
-{
-    if constexpr (WIDE) {
-        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" ::"s"(to), "n"(AT), "v"(lane_at), "s"(from) : "memory", "scc");
-    } else {
-        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %3" ::"s"(to), "n"(AT), "v"(lane_at), "s"(from) : "memory", "scc");
-    }
-}
-
 // SOFTCAP: 0 none, 1 caps below 256, 2 larger ones (see gqa_prefill_f16)
 template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_prefill_staged(GqaPrefillParams p)
 {

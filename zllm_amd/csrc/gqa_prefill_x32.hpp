@@ -92,6 +92,17 @@ __device__ __forceinline__ void row_lane_fmac4(float& t0, float& t1, float& t2, 
 #undef ROW_FMAC
 }
 
+// 64 x 16 bytes (WIDE) or 64 x 4 from `from` + the lane's offset to LDS at `to` + AT + 16 or 4 times the lane.  In assembly, because the
+// compiler would wait for all of these loads before every LDS read that follows.
+template <bool WIDE, unsigned int AT> __device__ __forceinline__ void load_to_lds(const unsigned char* from, unsigned int lane_at, unsigned int to)
+{
+    if constexpr (WIDE) {
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" ::"s"(to), "n"(AT), "v"(lane_at), "s"(from) : "memory", "scc");
+    } else {
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %3" ::"s"(to), "n"(AT), "v"(lane_at), "s"(from) : "memory", "scc");
+    }
+}
+
 // A finished column: `acc` and `total` carry 2^v_shift.  Split calls leave records in true units, others the normalised row.
 template <int D>
 __device__ __forceinline__ void store_column(const GqaPrefillParams& p, unsigned int row, unsigned int head, unsigned int h, float run_max, float total,

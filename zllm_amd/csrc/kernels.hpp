@@ -180,6 +180,9 @@ struct MlaDecodeParams {
     // (a prefill chunk, causal inside the chunk): `batch` counts query rows over all sequences, row v belongs to
     // sequence v / query_rows and sees ctx_lens[sequence] - (query_rows - 1 - v % query_rows) tokens.
     unsigned int query_rows;
+    // Tiles of 32 converted tokens (mla_staged.hip), `staged_tiles` a sequence
+    unsigned char* staged;
+    unsigned int staged_tiles;
 };
 
 // (row, query head) pairs of a row tile of the chunked-prefill kernels: 256, 128 at head_dim 256, and at head_dim 128 over
@@ -226,6 +229,10 @@ hipError_t launch_gqa_prefill_f16(const GqaPrefillParams& p, hipStream_t stream)
 // at both, and at the workspace for the tiles
 hipError_t launch_gqa_prefill_staged(const GqaPrefillParams& p, int scale_dtype, hipStream_t stream);
 hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, hipStream_t stream);
+// The partial stage of a chunk over latents converted once a call (mla_staged.hip): 512 + 64 columns, no selection, records by query row and
+// split; the caller has looked at the workspace for the tiles.  What `tiles` of each of `batch` sequences take there.
+hipError_t launch_mla_partial_staged(const MlaDecodeParams& p, hipStream_t stream);
+uint64_t mla_staged_bytes(unsigned int tiles, unsigned int batch);
 // The vector-ALU kernels for latent / rope widths other than 512 / 64 and for kv_b in other forms than bf16 (mla_generic.hip).
 hipError_t launch_mla_absorb_any(const MlaDecodeParams& p, hipStream_t stream);
 hipError_t launch_mla_partial_any(const MlaDecodeParams& p, hipStream_t stream);

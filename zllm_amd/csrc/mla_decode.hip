@@ -2360,7 +2360,12 @@ hipError_t launch_mla_decode(const MlaDecodeParams& p, unsigned int stage_mask, 
         const bool narrow = p.heads <= 32u; // two head tiles at most: the score waves split a step's tokens, the value waves the columns four ways
         const bool aligned = p.block_tokens % kStepTokens == 0 && p.chunk_tokens % kStepTokens == 0;
         const bool pow2_tables = (p.block_tokens & (p.block_tokens - 1u)) == 0 && p.tables != nullptr;
-        if ((stage_mask & 16u) != 0 && mla_partial_x32_takes(p)) { // ZLLM_MLA_WIDE_TILES: the caller asks for the 32x32x16-tile kernel
+        if (p.staged != nullptr) {
+            err = launch_mla_partial_staged(p, stream);
+            if (err != hipSuccess) {
+                return err;
+            }
+        } else if ((stage_mask & 16u) != 0 && mla_partial_x32_takes(p)) { // ZLLM_MLA_WIDE_TILES: the caller asks for the 32x32x16-tile kernel
             err = launch_mla_partial_x32(p, stream);
             if (err != hipSuccess) {
                 return err;

@@ -1603,9 +1603,9 @@ Result<RocmTensor> RocmContext::mla_decode_impl(const RocmTensor& query, const R
         a.kv_b_group = (uint32_t)kv_b.group_size;
         a.kv_b_scale_dtype = kv_b.scale_dtype == DType::F32 ? ZLLM_SCALE_F32 : (kv_b.scale_dtype == DType::F16 ? ZLLM_SCALE_F16 : ZLLM_SCALE_BF16);
     }
-    const uint64_t need = zllm_attn_mla_decode_workspace_bytes(&a);
+    const uint64_t need = zllm_attn_mla_decode_preferred_bytes(&a);
     if (need == 0) {
-        return abi_error("zllm_attn_mla_decode_workspace_bytes", -1);
+        return abi_error("zllm_attn_mla_decode_preferred_bytes", -1);
     }
     auto ws = workspace(need);
     if (ws.is_err()) {
