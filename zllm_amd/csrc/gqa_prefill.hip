@@ -1512,6 +1512,17 @@ unsigned int gqa_prefill_staged_tiles(unsigned int rows, unsigned int position, 
     return gqa_prefill_staged_bytes(tiles, num_kv_heads) <= (1ull << 30) ? tiles : 0u;
 }
 
+// f16 rows of head_dim 256: the kernel of two halves (gqa_prefill_f16_256.hip) where a row tile is full and its walk pays for their
+// meeting.  Us a call, tiles / halves (16 / 8 heads; with a window of 1,024 and a soft cap, a layer of each): 2,048 rows behind 6,144 keys
+// 437 / 391, 4,096 behind none 367 / 341, 1,000 104 / 97, 700 behind 5,000 208 / 198, 300 behind 30,000 319 / 303; one full layer, 200
+// behind 3,000 (parts of 400 keys) 43.8 / 44.0, behind 5,500 58.6 / 54.8, 400 behind none 36.2 / 35.9; but 100 behind none 34.0 / 37.4,
+// and 30 rows, half a tile, behind 10,000 56.6 / 65.4.  Runs of sixteen rows lie in one page; other pages keep the tiles, an address a lane.
+static bool gqa_prefill_takes_f16_256(const GqaPrefillParams& p, bool scalar_pages)
+{
+    const unsigned long long keys = p.window != 0u ? min((unsigned long long)p.window, (unsigned long long)p.position + p.rows) : (unsigned long long)p.position + p.rows;
+    return scalar_pages && p.block_tokens >= 16u && p.q_dtype != 0 && p.group <= 128u && (unsigned long long)p.rows * p.group >= 128u && keys >= 256u;
+}
+
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scale_dtype, hipStream_t stream)
 {
     const bool scalar_pages = prefill_scalar_pages(p.table, p.block_tokens);
@@ -1526,6 +1537,9 @@ hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scal
         }
         if (p.head_dim == 128u) {
             return launch_prefill_tiles<128, 1, 0>(p, stream);
+        }
+        if (p.head_dim == 256u && gqa_prefill_takes_f16_256(p, scalar_pages)) {
+            return launch_gqa_prefill_f16_256(p, stream);
         }
         if (p.head_dim == 256u) {
             return launch_prefill_tiles<256, 1, 0>(p, stream);
