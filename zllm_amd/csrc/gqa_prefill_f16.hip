@@ -11,7 +11,9 @@
 //   The rows go from global memory straight to LDS (no staging registers) two tiles ahead in a ring of three: 48 KB of tiles
 //       and at most 168 registers let three workgroups of four waves live on a compute unit, where eight waves of 16 pairs
 //       around four staged tiles were alone on it.
-//       Six registers are spilled, all outside the loop.
+//       Five registers are spilled, all outside the loop.
+//   The exponentials of a tile's second sixteen tokens stand between the matrix instructions of the first sixteen: what a wave places between its
+//       own hides, the other waves' hardly does.  Nine segments (appends included) 75.1 -> 73.0 us, a first chunk of 2,300 rows 122 -> 119.
 // 16 / 4 heads, 4,100 rows in one segment: 285 -> 232 us; in nine segments (16 / 16 heads) 69 -> 66, which are two workgroups a compute
 // unit and last as long as the longest walk, 36 tiles of 32 tokens: the longest segment has 21, but a row tile across a boundary walks both its
 // neighbours; 32 / 8 heads, 2,300 rows in eleven 48 -> 42, a first chunk of 3,500 rows 263 -> 204.
@@ -322,23 +324,13 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 3) void gqa_pre
                 }
             }
         }
+        // ---- O^T += V^T . P: f16 hi, with the second half's exponentials under the products of the first, then on heavy steps lo, one turn of a
+        // loop each (as branches around the products the two forms cost sixty registers of copies) ----
         float part_sum[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
+        auto weigh = [&](int i) __attribute__((always_inline)) {
             s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], mult, ref_shift));
             part_sum[i >> 3][i & 1] += s[i];
-        }
-        bool heavy = false;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const float eight = part_sum[e][0] + part_sum[e][1];
-            run_sum[e] += eight;
-            heavy = heavy || eight * lo_share > run_sum[e];
-        }
-        // ---- O^T += V^T . P: f16 hi, on heavy steps lo first, one turn of a loop each (as branches around the products the
-        // two forms cost sixty registers of copies) ----
-        two_terms = __any(heavy);
-        const bool lo_pass = two_terms || behind;
+        };
         PREFILL_PHASE_FENCE();
         union VFrag {
             s16x4 s[2];
@@ -352,32 +344,54 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 3) void gqa_pre
                 vf.s[r8] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(at));
             }
         };
-        for (int term = lo_pass ? 1 : 0; term >= 0; --term) {
-            VFrag vf[2][2]; // [parity][output tile of a pair]
-            load_v(vf[0][0], 0, 0);
-            load_v(vf[0][1], 1, 0);
-            Frag ph[2];
-            if (term == 0) {
+        for (bool hi = true;; hi = false) {
+            constexpr int kRing = 2; // a third fragment spills in the loop
+            VFrag vf[kRing];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    ph[e >> 2].u[e & 3] = pack_f16_hw(s[2 * e], s[2 * e + 1]);
+            for (int n = 0; n < kRing; ++n) {
+                load_v(vf[n], n % 4, n / 4);
+            }
+            Frag ph[2];
+            if (hi) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    weigh(2 * e);
+                    weigh(2 * e + 1);
+                    ph[0].u[e] = pack_f16_hw(s[2 * e], s[2 * e + 1]);
                 }
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const f16x2 hi = __builtin_bit_cast(f16x2, pack_f16_hw(s[2 * e], s[2 * e + 1]));
-                    ph[e >> 2].u[e & 3] = pack_f16_hw(s[2 * e] - (float)hi[0], s[2 * e + 1] - (float)hi[1]);
+                    const f16x2 dropped = __builtin_bit_cast(f16x2, pack_f16_hw(s[2 * e], s[2 * e + 1]));
+                    ph[e >> 2].u[e & 3] = pack_f16_hw(s[2 * e] - (float)dropped[0], s[2 * e + 1] - (float)dropped[1]);
                 }
             }
 #pragma unroll
-            for (int n = 0; n < 4; ++n) { // output tiles 2 (n / 2) .. + 2, tokens 16 (n % 2) .. + 16
-                if (n < 3) { // the fragments after these travel while these multiply
-                    load_v(vf[(n + 1) & 1][0], (n + 1) / 2 * 2, (n + 1) & 1);
-                    load_v(vf[(n + 1) & 1][1], (n + 1) / 2 * 2 + 1, (n + 1) & 1);
+            for (int n = 0; n < 8; ++n) { // output tile n % 4, tokens 16 (n / 4) .. + 16
+                acc[n % 4] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[n % kRing].h, ph[n / 4].h, acc[n % 4], 0, 0, 0);
+                if (n + kRing < 8) { // the fragments after these travel while these multiply
+                    load_v(vf[n % kRing], (n + kRing) % 4, (n + kRing) / 4);
                 }
-                acc[n / 2 * 2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[n & 1][0].h, ph[n & 1].h, acc[n / 2 * 2], 0, 0, 0);
-                acc[n / 2 * 2 + 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[n & 1][1].h, ph[n & 1].h, acc[n / 2 * 2 + 1], 0, 0, 0);
+                if (hi && n < 4) {
+                    weigh(8 + 2 * n);
+                    weigh(8 + 2 * n + 1);
+                    ph[1].u[n] = pack_f16_hw(s[8 + 2 * n], s[8 + 2 * n + 1]);
+                }
                 PREFILL_PHASE_FENCE(); // or every fragment is requested at once, into registers that are not there
+            }
+            if (!hi) {
+                break;
+            }
+            bool heavy = false;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float eight = part_sum[e][0] + part_sum[e][1];
+                run_sum[e] += eight;
+                heavy = heavy || eight * lo_share > run_sum[e];
+            }
+            two_terms = __any(heavy);
+            if (!two_terms && !behind) {
+                break;
             }
         }
     };
