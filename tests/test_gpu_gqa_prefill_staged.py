@@ -36,7 +36,9 @@ def test_which_calls_ask_for_staged_rows():
         assert staged_bytes(2048, 50000, 32, 8, **other) == 0
     ends = (C.c_uint32 * 1)()
     assert staged_bytes(2048, 50000, 32, 8, visible_ends=C.addressof(ends)) == 0
-    assert staged_bytes(2048, 0, 32, 8) == 0  # a first chunk: half-size row tiles
+    # a first chunk: half-size row tiles, more than one a compute unit
+    assert staged_bytes(1024, 0, 32, 8) == 0 < staged_bytes(1025, 0, 32, 8)
+    assert staged_bytes(16, 500, 32, 8) == 0
 
 
 @pytest.mark.gpu
@@ -50,7 +52,12 @@ def test_which_calls_ask_for_staged_rows():
     (1200, 260, 8, 2, dict(softcap=30.0, rule=O.RULE_ROCM_MLA)),
     (800, 140, 8, 2, dict(softcap=400.0, rule=O.RULE_CUDA_GQA)),     # the precise form of the soft cap; f32 scales
     (2500, 200, 8, 2, dict(rule=O.RULE_ROCM_MLA, block_tokens=64, v_gain=2.0 ** np.repeat(np.arange(-10, 10), 135))),  # the V window moves on
-    (400, 40, 130, 1, {})])                                          # one row a tile
+    (400, 40, 130, 1, {}),                                           # one row a tile
+    # half-size tiles, the keys in two halves: first chunks
+    (0, 1031, 32, 8, dict(block_tokens=24)),                         # 33 tiles of keys: the odd half ends a pass earlier; a last tile of seven rows
+    (0, 1000, 33, 11, {}),                                           # the fewest keys; row tiles that see one tile, or the even half's only
+    (7, 1100, 56, 8, dict(softcap=30.0, rule=O.RULE_ROCM_MLA, gate_cols=1)),
+    (0, 1200, 32, 8, dict(rule=O.RULE_ROCM_MLA, block_tokens=64, v_gain=2.0 ** np.repeat(np.arange(-10, 10), 60)))])  # the halves' windows differ
 def test_staged_rows_against_the_oracle(prefix, chunk, hq, hkv, kw):
     named = {"rule": "scale_dtype", "block_tokens": "block_tokens", "window": "window"}
     fields = {named[n]: v for n, v in kw.items() if n in named}

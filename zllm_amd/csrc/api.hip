@@ -1155,11 +1155,15 @@ static int validate_gqa_prefill(const zllm_gqa_prefill_args* a)
 // as a decode call's is -- whole rounds of the CUs, splits of at least 256 tokens (a workgroup first loads and
 // normalises a tile of queries) -- and the parts meet in the split merge.  The records are
 // rows x splits x heads x head_dim floats: a plan whose records would pass 256 MiB keeps fewer splits.
-void plan_prefill_splits(const zllm_gqa_prefill_args* a, uint32_t* chunk_tokens, uint32_t* max_chunks)
+uint32_t prefill_tile_pairs(const zllm_gqa_prefill_args* a)
+{
+    return zllm::gqa_prefill_tile_pairs(a->rows, a->position, a->window, a->num_heads, a->num_kv_heads, a->head_dim, a->kv_format, a->scale_dtype, a->q_dtype,
+                                        a->visible_starts != nullptr, zllm::prefill_scalar_pages(a->table, a->block_tokens));
+}
+
+void plan_prefill_splits(const zllm_gqa_prefill_args* a, uint32_t columns, uint32_t* chunk_tokens, uint32_t* max_chunks)
 {
     const uint32_t group = a->num_heads / a->num_kv_heads;
-    const uint32_t columns = zllm::gqa_prefill_tile_pairs(a->rows, a->position, a->window, a->num_heads, a->num_kv_heads, a->head_dim, a->kv_format,
-                                                          a->scale_dtype, a->q_dtype, a->visible_starts != nullptr, zllm::prefill_scalar_pages(a->table, a->block_tokens));
     const uint32_t tile_rows = columns / group > 0 ? columns / group : 1u;
     const uint64_t tiles = ((uint64_t)a->rows + tile_rows - 1) / tile_rows;
     uint64_t longest = (uint64_t)a->position + a->rows; // keys the last row tile may see
@@ -1309,16 +1313,31 @@ uint64_t zllm_attn_gqa_prefill_workspace_bytes(const zllm_gqa_prefill_args* a)
         return prefill_decode_route_bytes(a);
     }
     uint32_t chunk_tokens, max_chunks;
-    plan_prefill_splits(a, &chunk_tokens, &max_chunks);
+    plan_prefill_splits(a, prefill_tile_pairs(a), &chunk_tokens, &max_chunks);
     const uint64_t splits = max_chunks > 1 ? prefill_split_records(a, max_chunks).total : 0; /* unsplit, the chunk kernel keeps all of its state on chip */
     const uint64_t items = few_rows_as_decode_items(a) ? prefill_decode_route_bytes(a) : 0;
     return splits > items ? splits : items;
 }
 
-static uint32_t prefill_staged_tiles(const zllm_gqa_prefill_args* a, uint32_t* first)
+// A call over rows that are converted once: its tiles, its splits, and where the tiles lie in the workspace, behind the split records.  tiles == 0
+// for other calls.
+struct PrefillStaged {
+    uint32_t tiles, first, chunk_tokens, max_chunks;
+    bool halves;
+    uint64_t at, total;
+};
+
+static PrefillStaged plan_prefill_staged(const zllm_gqa_prefill_args* a)
 {
-    return zllm::gqa_prefill_staged_tiles(a->rows, a->position, a->window, a->num_heads, a->num_kv_heads, a->head_dim, a->kv_format, a->scale_dtype, a->q_dtype,
-                                          a->visible_ends != nullptr, first);
+    PrefillStaged s = {};
+    s.tiles = zllm::gqa_prefill_staged_tiles(a->rows, a->position, a->window, a->num_heads, a->num_kv_heads, a->head_dim, a->kv_format, a->scale_dtype,
+                                             a->q_dtype, a->visible_ends != nullptr, &s.first, &s.halves);
+    if (s.tiles != 0) {
+        plan_prefill_splits(a, s.halves ? 128u : 256u, &s.chunk_tokens, &s.max_chunks);
+        s.at = align_up(s.max_chunks > 1 ? prefill_split_records(a, s.max_chunks).total : 0, 256);
+        s.total = s.at + zllm::gqa_prefill_staged_bytes(s.tiles, a->num_kv_heads);
+    }
+    return s;
 }
 
 uint64_t zllm_attn_gqa_prefill_preferred_bytes(const zllm_gqa_prefill_args* a)
@@ -1327,9 +1346,8 @@ uint64_t zllm_attn_gqa_prefill_preferred_bytes(const zllm_gqa_prefill_args* a)
     if (validate_gqa_prefill(a) != 0 || prefill_rows_as_decode_items(a)) {
         return least;
     }
-    uint32_t first = 0;
-    const uint32_t tiles = prefill_staged_tiles(a, &first);
-    return tiles == 0 ? least : align_up(least, 256) + zllm::gqa_prefill_staged_bytes(tiles, a->num_kv_heads);
+    const PrefillStaged staged = plan_prefill_staged(a);
+    return staged.total > least ? staged.total : least;
 }
 
 int zllm_attn_gqa_prefill_chunk(const zllm_gqa_prefill_args* a, zllm_stream_t stream)
@@ -1414,7 +1432,17 @@ int zllm_attn_gqa_prefill_chunk(const zllm_gqa_prefill_args* a, zllm_stream_t st
     }
     // KV splits when the chunk has too few row tiles for the device and the caller brought the room for their records
     uint32_t chunk_tokens = 0, max_chunks = 1;
-    plan_prefill_splits(a, &chunk_tokens, &max_chunks);
+    const PrefillStaged staged = plan_prefill_staged(a);
+    if (staged.tiles != 0 && a->workspace != nullptr && ((uintptr_t)a->workspace & 15u) == 0 && a->workspace_bytes >= staged.total) {
+        chunk_tokens = staged.chunk_tokens;
+        max_chunks = staged.max_chunks;
+        p.staged = (unsigned char*)a->workspace + staged.at;
+        p.staged_first = staged.first;
+        p.staged_tiles = staged.tiles;
+        p.staged_halves = staged.halves;
+    } else {
+        plan_prefill_splits(a, prefill_tile_pairs(a), &chunk_tokens, &max_chunks);
+    }
     if (max_chunks > 1) {
         const PrefillSplitRecords w = prefill_split_records(a, max_chunks);
         if (a->workspace != nullptr && a->workspace_bytes >= w.total && ((uintptr_t)a->workspace & 15u) == 0) {
@@ -1422,16 +1450,6 @@ int zllm_attn_gqa_prefill_chunk(const zllm_gqa_prefill_args* a, zllm_stream_t st
             p.stats = (float*)((char*)a->workspace + w.stats);
             p.chunk_tokens = chunk_tokens;
             p.max_chunks = max_chunks;
-        }
-    }
-    uint32_t staged_first = 0;
-    const uint32_t staged_tiles = prefill_staged_tiles(a, &staged_first);
-    if (staged_tiles != 0 && a->workspace != nullptr && ((uintptr_t)a->workspace & 15u) == 0) { // behind the records
-        const uint64_t least = align_up(max_chunks > 1 ? prefill_split_records(a, max_chunks).total : 0, 256);
-        if (a->workspace_bytes >= least + zllm::gqa_prefill_staged_bytes(staged_tiles, a->num_kv_heads)) {
-            p.staged = (unsigned char*)a->workspace + least;
-            p.staged_first = staged_first;
-            p.staged_tiles = staged_tiles;
         }
     }
     const int launched = p.staged != nullptr

@@ -1495,16 +1495,25 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
 // The staging is a launch and a pass over the keys that few row tiles do not earn back: 80 rows of 32 / 8 (two tiles) 35.8 / 37.9 us behind 2,000,
 // 54 / 58 behind 8,000, of 64 / 8 (three) 225 / 235 behind 32,000; behind 600 keys they do, 48 -> 32.
 // The tiles are bounded by 1 GiB, 253,000 tokens of eight KV heads.
+// First chunks whose full-size tiles are at most a workgroup a compute unit have tiles of 128 pairs above and halves of the keys here: 32 / 8 heads,
+// 1,500 rows 92 -> 88, behind 300 keys 113 -> 104, 2,048 110 -> 99; 64 / 8, 1,000 rows 71 -> 67; 16 / 4, 4,000 rows 178 -> 150.  Below 1,000 keys the
+// staging shows (560 rows of 64 / 8 52 / 53).  One round of such tiles or less keeps the tiles of 64 and both terms of
+// every probability, which the halves would have to carry as well to be as close to 64 bits (1,000 rows of 32 / 8 54 / 53 without).
 unsigned int gqa_prefill_staged_tiles(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
-                                      unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ends, unsigned int* first)
+                                      unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ends, unsigned int* first, bool* halves)
 {
-    if (kv_format != 0 || head_dim != 128u || q_dtype == 0 || ends || num_kv_heads == 0u || num_kv_heads > 65535u || num_heads / num_kv_heads > 256u ||
-        gqa_prefill_tile_pairs(rows, position, window, num_heads, num_kv_heads, head_dim, kv_format, scale_dtype, q_dtype, false, false) != 256u) {
+    if (kv_format != 0 || head_dim != 128u || q_dtype == 0 || ends || num_kv_heads == 0u || num_kv_heads > 65535u) {
         return 0;
     }
-    const unsigned int group = num_heads / num_kv_heads, rows_per_tile = 256u / group, end = position + rows;
+    const unsigned int group = num_heads / num_kv_heads, end = position + rows;
+    const unsigned int pairs = gqa_prefill_tile_pairs(rows, position, window, num_heads, num_kv_heads, head_dim, kv_format, scale_dtype, q_dtype, false, false);
+    *halves = pairs != 256u;
+    if (group > pairs || pairs < 128u) {
+        return 0;
+    }
+    const unsigned int rows_per_tile = pairs / group, row_tiles = (rows + rows_per_tile - 1u) / rows_per_tile;
     const unsigned int begin = window != 0u && position + 1u > window ? position + 1u - window : 0u;
-    if ((rows + rows_per_tile - 1u) / rows_per_tile < 4u && end - begin > 1024u) {
+    if (*halves ? (unsigned long long)row_tiles * num_kv_heads <= kComputeUnitsPrefill || end < 1000u : row_tiles < 4u && end - begin > 1024u) {
         return 0;
     }
     *first = begin / (unsigned int)kStep;

@@ -28,13 +28,13 @@ constexpr int kTile = kStep * kD * 2; // bytes of one 32-token tile as f16
 constexpr int kGroups = kD / 64;
 constexpr int kScales = kGroups * kStep * 4; // bytes of a tile's f32 scales, [token][group]
 constexpr int kWaves = 8; // of 32 pairs each
-constexpr int kPairs = 32 * kWaves;
 constexpr int kBufs = 6; // three passes of two tiles: one attended, one complete or on its way, one requested
 // A staged tile: K | V | K scales | V scales | the (biased) exponent of the largest V scale.  K and V lie as the matrix instructions take
 // them, 1 KiB a fragment, 16 bytes a lane: K fragment ks holds columns 16 ks + 8 h .. + 8 of token c (lane 32 h + c), V fragment 2 t + kk
 // column 32 t + c of tokens 16 kk + 4 h .. + 4 and eight further.
 constexpr int kKsAt = 2 * kTile, kVsAt = 2 * kTile + kScales, kTopAt = 2 * kTile + 2 * kScales;
 constexpr int kBlock = kTopAt + 128;
+constexpr float kLoThresholdHalves = 24.0f; // see kLoThreshold: a half's walk is short, as those of the kernels whose reference lags are (16)
 constexpr int kBlocksBehind = 8; // a part's requests run up to seven tiles past its last
 
 // One tile of one KV head a workgroup; bound by the memory it reads and writes.
@@ -124,14 +124,27 @@ template <int SDT> __global__ __launch_bounds__(256) void gqa_stage_q8(GqaPrefil
 }
 
 // SOFTCAP: 0 none, 1 caps below 256, 2 larger ones (see gqa_prefill_f16)
-template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_prefill_staged(GqaPrefillParams p)
+// HALVES 1: eight waves of 32 pairs, a wave attends both tiles of a pass.  HALVES 2: four waves of 32 pairs for even tiles and four for odd ones,
+// which meet once, at the end: first chunks, whose last row tiles walk longest.  Their reference lags (kSlack): with the maximum itself 2,048 rows of
+// 32 / 8 heads 101 -> 97 us (the kernel it stands in for: 111).  Distance from 64 bits there (2-norm) 2.4e-5 in that kernel, 2.8e-6 here.
+template <int SOFTCAP, int HALVES> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_prefill_staged(GqaPrefillParams p)
 {
     struct Lds {
         unsigned char k[kBufs][kTile];
         unsigned char v[kBufs][kTile];
         float scales[kBufs][2][kStep][kGroups]; // of K and V
     };
-    __shared__ __align__(1024) Lds lds;
+    constexpr int kSide = kWaves / HALVES; // waves of a half
+    constexpr unsigned int kPairs = 32 * kSide;
+    struct Meeting { // of the halves, over the tiles
+        float acc[kD / 8][kSide][64][4];
+        float stats[3][kSide][64];
+    };
+    __shared__ __align__(1024) union {
+        Lds lds;
+        Meeting meeting;
+    } shared;
+    Lds& lds = shared.lds;
 
     const unsigned int tid = threadIdx.x;
     const unsigned int lane = tid & 63u;
@@ -141,10 +154,11 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
     const unsigned int h = lane >> 5;
     // row tiles with the longest range first, the KV head as the fast index (see gqa_prefill_q8)
     const unsigned int kvh = blockIdx.x % p.num_kv_heads;
-    const unsigned int rows_per_wg = max(1u, (unsigned int)kPairs / p.group);
+    const unsigned int half = HALVES == 1 ? 0u : wave / kSide, side = HALVES == 1 ? wave : wave % kSide;
+    const unsigned int rows_per_wg = max(1u, kPairs / p.group);
     const unsigned int row0 = (gridDim.x / p.num_kv_heads - 1u - blockIdx.x / p.num_kv_heads) * rows_per_wg;
     const unsigned int cols_used = rows_per_wg * p.group;
-    const unsigned int col = wave * 32u + c;
+    const unsigned int col = side * 32u + c;
     const unsigned int col_row = row0 + col / p.group;
     const unsigned int col_head = kvh * p.group + col % p.group;
     const bool col_valid = col < cols_used && col_row < p.rows;
@@ -170,37 +184,40 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
     t_begin &= ~31u;
     const SplitRange part = split_range(p, t_begin, t_end);
     if (!part.live) {
-        if (col_valid && h == 0u) {
+        if (col_valid && h == 0u && half == 0u) {
             store_empty_record(p, col_row, col_head);
         }
         return;
     }
     const unsigned int steps = (part.end - part.begin + kStep - 1) / kStep;
 
-    // ---- staging.  Pass n of the loop attends tiles 2 n and 2 n + 1 and multiplies the keys of 2 n + 1 and 2 n + 2: their K are loaded beside
-    // the V of the first two, a fragment of each a wave, and a piece of the scales (the waves' pieces repeat).  Requests run past the range
+    // ---- staging.  Pass n of the loop attends tiles 2 n and 2 n + 1 and multiplies the keys of the HALVES tiles ahead of them: their K are loaded
+    // beside the V of the first two, a fragment of each a wave, and a piece of the scales (the waves' pieces repeat).  Requests run past the range
     // into what follows in the workspace (kBlocksBehind); nothing of that is attended.
     const unsigned char* const staged = p.staged + ((size_t)kvh * p.staged_tiles + (part.begin / kStep - p.staged_first)) * kBlock;
     const unsigned int lds_base = (unsigned int)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&lds;
     const unsigned int lane16 = lane * 16u, lane4 = lane * 4u;
     const unsigned int wave_lds = lds_base + wave * 1024u;
     const bool scales_of_v = (wave & 2u) != 0u;
-    const unsigned int scales_tile = (wave & 1u) + (scales_of_v ? 0u : 1u); // of the pass: 0, 1, or 2 for K
+    const unsigned int scales_tile = (wave & 1u) + (scales_of_v ? 0u : (unsigned int)HALVES); // of the pass: HALVES more for K
     const unsigned int scales_from = scales_tile * kBlock + kKsAt + (scales_of_v ? kScales : 0u);
     const unsigned int scales_lds = lds_base + offsetof(Lds, scales) + (scales_of_v ? kScales : 0u);
     auto load_pass = [&](auto which, const unsigned char* at) __attribute__((always_inline)) { // tiles from `at` on
         constexpr int set = decltype(which)::value;
         constexpr unsigned int k_at = offsetof(Lds, k), v_at = offsetof(Lds, v);
         const unsigned char* const from = at + wave * 1024u;
-        load_to_lds<true, k_at + (2 * set + 1) * kTile>(from + kBlock, lane16, wave_lds);
+        load_to_lds<true, k_at + (2 * set + HALVES) % kBufs * kTile>(from + HALVES * kBlock, lane16, wave_lds);
         load_to_lds<true, v_at + 2 * set * kTile>(from + kTile, lane16, wave_lds);
-        load_to_lds<true, k_at + (2 * set + 2) % kBufs * kTile>(from + 2 * kBlock, lane16, wave_lds);
+        load_to_lds<true, k_at + (2 * set + 1 + HALVES) % kBufs * kTile>(from + (1 + HALVES) * kBlock, lane16, wave_lds);
         load_to_lds<true, v_at + (2 * set + 1) * kTile>(from + kBlock + kTile, lane16, wave_lds);
-        const unsigned int buf = set == 2 && scales_tile == 2u ? 0u : 2u * set + scales_tile;
+        const unsigned int buf = set == 2 && scales_tile >= 2u ? scales_tile - 2u : 2u * set + scales_tile;
         load_to_lds<false, 0>(at + scales_from, lane4, scales_lds + buf * (2 * kScales));
     };
-    load_to_lds<true, offsetof(Lds, k)>(staged + wave * 1024u, lane16, wave_lds);
-    load_to_lds<false, offsetof(Lds, scales)>(staged + kKsAt, lane4, lds_base);
+#pragma unroll
+    for (int n = 0; n < HALVES; ++n) { // the first keys
+        load_to_lds<true, offsetof(Lds, k)>(staged + n * kBlock + wave * 1024u, lane16, wave_lds + n * kTile);
+        load_to_lds<false, offsetof(Lds, scales)>(staged + n * kBlock + kKsAt, lane4, lds_base + n * (2 * kScales));
+    }
     load_pass(std::integral_constant<int, 0>{}, staged);
     load_pass(std::integral_constant<int, 1>{}, staged + 2 * kBlock);
 
@@ -245,6 +262,8 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
         }
     }
     float run_max = kNegInf, ref_shift = kPBias;
+    [[maybe_unused]] float lane_top = kNegInf; // halves: the largest score the lane has met
+    bool two_terms = true; // the tile before carried both terms of its probabilities
     float run_sum[2] = {0.0f, 0.0f}; // of the lane's first and second eight tokens of each step
     unsigned int vis_lo, vis_hi;     // visible tokens [lo, hi) of the column's row
     {
@@ -255,7 +274,9 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
     // the tokens that every column of the wave sees are [max_lo, min_hi)
     const unsigned int wave_min_hi = wave_min_u(vis_hi), wave_max_lo = wave_max_u(vis_lo);
 
-    const unsigned int scale_token = 8u * (m >> 2) + 4u * h + (m & 3u); // lane m of a row of sixteen holds the scales of element m's token
+    // a half's tiles lie in the buffer of its number behind the pass's first
+    const unsigned int frag_at = lane16 + half * kTile;
+    const unsigned int scale_at = (8u * (m >> 2) + 4u * h + (m & 3u)) * kGroups + half * (2u * kStep * kGroups); // lane m of a row of sixteen: element m's token
 
     f32x16 s; // the tile's scores, up to the query's power of two; multiplied a step ahead
     f32x16 d[kGroups];
@@ -272,12 +293,12 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
 #pragma unroll
             for (int g = 0; g < kGroups; ++g) {
                 Frag kf;
-                kf.u = *(const u32x4*)(lds.k[buf] + lane16 + (g * 4 + ks) * 1024);
+                kf.u = *(const u32x4*)(lds.k[buf] + frag_at + (g * 4 + ks) * 1024);
                 d[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf.h, qf[g * 4 + ks].h, d[g], 0, 0, 0);
             }
         }
     };
-    auto scales_of = [&](int buf, int plane) __attribute__((always_inline)) { return *(const f32x2*)(&lds.scales[buf][plane][scale_token][0]); };
+    auto scales_of = [&](int buf, int plane) __attribute__((always_inline)) { return *(const f32x2*)(&lds.scales[buf][plane][0][0] + scale_at); };
     // s = sum_g scale_g d_g, four elements; `settled`: an element of d[1] times something, which the compiler has waited for
     auto scale_scores = [&](const f32x2& scale, int q, float settled) __attribute__((always_inline)) {
         float t[4];
@@ -293,15 +314,15 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
     };
 
     auto attend = [&](int buf, unsigned int t0, float v_shift, float acc_fix, bool window_moved) __attribute__((always_inline)) {
-        const int next = (buf + 1) % kBufs;
-                constexpr int kAhead = 3, kRing = kAhead + 1;
+        const int next = (buf + HALVES) % kBufs;
+        constexpr int kAhead = 3, kRing = kAhead + 1;
         Frag frag[kRing];
         auto request = [&](int n) __attribute__((always_inline)) { // of slot n
             if (n < 8) {
-                frag[n % kRing].u = *(const u32x4*)(lds.k[next] + lane16 + ((n & 1) * 4 + n / 2) * 1024);
+                frag[n % kRing].u = *(const u32x4*)(lds.k[next] + frag_at + ((n & 1) * 4 + n / 2) * 1024);
             } else if (n < 16) {
                 const int j = n - 8, t = (j >> 2) * 2 + (j & 1), kk = (j >> 1) & 1;
-                frag[n % kRing].u = *(const u32x4*)(lds.v[buf] + lane16 + (2 * t + kk) * 1024);
+                frag[n % kRing].u = *(const u32x4*)(lds.v[buf] + frag_at + (2 * t + kk) * 1024);
             }
         };
 #pragma unroll
@@ -337,7 +358,16 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
             upper = fmaxf(fmaxf(upper, s[i + 1]), s[i + 9]);
         }
         lane_max = fmaxf(lane_max, upper) * mult;
-        if (__any(lane_max > run_max) || window_moved) {
+        bool behind = false, move;
+        if constexpr (HALVES == 1) {
+            move = __any(lane_max > run_max);
+        } else { // first chunks: the reference lags while the tiles carry both terms (see kSlack)
+            lane_max = lane_top = fmaxf(lane_top, lane_max);
+            behind = __any(lane_top > run_max);
+            move = two_terms ? __any(lane_top - run_max > kSlack) : behind;
+        }
+        if (move || window_moved) {
+            behind = false;
             const float new_max = fmaxf(run_max, halves_max(lane_max));
             const float safe_max = new_max == kNegInf ? 0.0f : new_max;
             const float alpha = __builtin_amdgcn_exp2f(run_max - safe_max) * acc_fix;
@@ -416,9 +446,14 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
         for (int e = 0; e < 2; ++e) {
             const float eight = part_sum[e][0] + part_sum[e][1];
             run_sum[e] += eight;
-            heavy = heavy || eight * kLoThreshold > run_sum[e];
+            heavy = heavy || (HALVES == 1 && eight * kLoThreshold > run_sum[e]);
         }
-        const bool lo_pass = __any(heavy);
+        if constexpr (HALVES == 2) { // the two sums of a half are those of a quarter of the row's tokens, as in the kernels whose reference lags
+            const float most = fmaxf(part_sum[0][0] + part_sum[0][1], part_sum[1][0] + part_sum[1][1]);
+            heavy = most * kLoThresholdHalves > run_sum[0] + run_sum[1];
+        }
+        two_terms = __any(heavy);
+        const bool lo_pass = two_terms || behind;
         if (lo_pass) { // what f16 has dropped of the probabilities
 #pragma unroll
             for (int g = 0; g < kGroups; ++g) {
@@ -436,7 +471,7 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
 #pragma unroll
                     for (int t = 2 * g; t < 2 * g + 2; ++t) {
                         Frag vf;
-                        vf.u = *(const u32x4*)(lds.v[buf] + lane16 + (2 * t + kk) * 1024);
+                        vf.u = *(const u32x4*)(lds.v[buf] + frag_at + (2 * t + kk) * 1024);
                         acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf.h, pl[kk].h, acc[t], 0, 0, 0);
                     }
                 }
@@ -452,11 +487,11 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
     auto load_top = [&](unsigned int tile) __attribute__((always_inline)) -> unsigned int { // `tile` tiles past the pass's first
         return *(scalar_words_t)(uintptr_t)(pass_at + tile * kBlock + kTopAt);
     };
-    unsigned int top_now = load_top(0), top_next = load_top(1);
+    unsigned int top_now = load_top(half), top_next = load_top(half + 1u * HALVES);
     auto attend_tile = [&](unsigned int step, int buf) __attribute__((always_inline)) {
         const unsigned int wv_now = max(wv, top_now);
         top_now = top_next;
-        top_next = load_top(2u + (buf & 1));
+        top_next = load_top(HALVES == 1 ? 2u + (buf & 1) : half + 4u);
         const bool window_moved = wv_now != wv; // rare: a V scale above everything met so far
         float acc_fix = 1.0f;
         if (window_moved) {
@@ -477,13 +512,23 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
         constexpr int set = decltype(which)::value;
         wait_pass();
         load_pass(std::integral_constant<int, (set + 2) % 3>{}, pass_at + 4 * kBlock);
-        attend_tile(step, 2 * set);
-        if (step + 1u < steps) {
-            attend_tile(step + 1u, 2 * set + 1);
+        if constexpr (HALVES == 1) {
+            attend_tile(step, 2 * set);
+            if (step + 1u < steps) {
+                attend_tile(step + 1u, 2 * set + 1);
+            }
+        } else if (step + half < steps) {
+            attend_tile(step + half, 2 * set);
         }
         pass_at += 2 * kBlock;
     };
-    wait_pass();
+    if constexpr (HALVES == 1) {
+        wait_pass();
+    } else { // the first keys of both halves are behind the loads of two passes
+        asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    }
     multiply_keys(0);
     {
         float settled = d[1][0] * mult;
@@ -509,7 +554,40 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves, 2) void gqa_pre
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // what was requested past the range lands before the LDS is given back
 
-    const float total = halves_sum(run_sum[0] + run_sum[1]);
+    float total = halves_sum(run_sum[0] + run_sum[1]);
+    if constexpr (HALVES == 2) {
+        Meeting& meeting = shared.meeting;
+        __syncthreads(); // the tiles are read no more
+        if (half == 1u) {
+            meeting.stats[0][side][lane] = run_max;
+            meeting.stats[1][side][lane] = total;
+            meeting.stats[2][side][lane] = v_shift;
+#pragma unroll
+            for (int n = 0; n < kD / 8; ++n) {
+                *(f32x4*)meeting.acc[n][side][lane] = f32x4{acc[n / 4][n % 4 * 4], acc[n / 4][n % 4 * 4 + 1], acc[n / 4][n % 4 * 4 + 2], acc[n / 4][n % 4 * 4 + 3]};
+            }
+        }
+        __syncthreads();
+        if (half == 1u) {
+            return;
+        }
+        // to the larger reference and the larger window (a half whose sum is zero may have seen nothing)
+        const float other_max = meeting.stats[0][side][lane], other_total = meeting.stats[1][side][lane], other_shift = meeting.stats[2][side][lane];
+        const float common = fmaxf(run_max, other_max), shift = fminf(v_shift, other_shift);
+        const float own_fac = run_max == kNegInf ? 0.0f : __builtin_amdgcn_exp2f((run_max - common) + (shift - v_shift));
+        const float other_fac = other_max == kNegInf ? 0.0f : __builtin_amdgcn_exp2f((other_max - common) + (shift - other_shift));
+        total = total * own_fac + other_total * other_fac;
+#pragma unroll
+        for (int n = 0; n < kD / 8; ++n) {
+            const f32x4 other = *(const f32x4*)meeting.acc[n][side][lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc[n / 4][n % 4 * 4 + e] = acc[n / 4][n % 4 * 4 + e] * own_fac + other[e] * other_fac;
+            }
+        }
+        run_max = common;
+        v_shift = shift;
+    }
     if (!col_valid) {
         return;
     }
@@ -533,16 +611,22 @@ hipError_t launch_gqa_prefill_staged(const GqaPrefillParams& p, int scale_dtype,
     } else {
         gqa_stage_q8<2><<<tiles, dim3(256), 0, stream>>>(p);
     }
-    const unsigned int rows_per_wg = p.group >= (unsigned int)kPairs ? 1u : (unsigned int)kPairs / p.group;
-    const dim3 grid((p.rows + rows_per_wg - 1) / rows_per_wg * p.num_kv_heads, 1, p.max_chunks > 1u ? p.max_chunks : 1u);
-    const dim3 block(64 * kWaves);
-    if (!(p.softcap > 0.0f)) {
-        gqa_prefill_staged<0><<<grid, block, 0, stream>>>(p);
-    } else if (p.softcap < 256.0f) {
-        gqa_prefill_staged<1><<<grid, block, 0, stream>>>(p);
-    } else {
-        gqa_prefill_staged<2><<<grid, block, 0, stream>>>(p);
-    }
+    auto launch = [&](auto softcap, auto halves) {
+        constexpr unsigned int kPairs = 32 * kWaves / decltype(halves)::value;
+        const unsigned int rows_per_wg = p.group >= kPairs ? 1u : kPairs / p.group;
+        const dim3 grid((p.rows + rows_per_wg - 1) / rows_per_wg * p.num_kv_heads, 1, p.max_chunks > 1u ? p.max_chunks : 1u);
+        gqa_prefill_staged<decltype(softcap)::value, decltype(halves)::value><<<grid, dim3(64 * kWaves), 0, stream>>>(p);
+    };
+    auto launch_halves = [&](auto halves) {
+        if (!(p.softcap > 0.0f)) {
+            launch(std::integral_constant<int, 0>{}, halves);
+        } else if (p.softcap < 256.0f) {
+            launch(std::integral_constant<int, 1>{}, halves);
+        } else {
+            launch(std::integral_constant<int, 2>{}, halves);
+        }
+    };
+    p.staged_halves ? launch_halves(std::integral_constant<int, 2>{}) : launch_halves(std::integral_constant<int, 1>{});
     return hipGetLastError();
 }
 

@@ -142,6 +142,7 @@ struct GqaPrefillParams {
     // K and V as f16 tiles of 32 tokens (gqa_prefill_staged.hip): `staged_tiles` a KV head, the first of them `staged_first`
     unsigned char* staged;
     unsigned int staged_first, staged_tiles;
+    bool staged_halves; // row tiles of 128 pairs, the keys in two halves
 };
 
 struct MlaDecodeParams {
@@ -199,7 +200,7 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
 // Tiles of 32 tokens, and the first of them, that a call reads of every KV head, where converting them once (gqa_prefill_staged.hip) is faster
 // than once a row tile: 0 for other calls.  What they take in the workspace.
 unsigned int gqa_prefill_staged_tiles(unsigned int rows, unsigned int position, unsigned int window, unsigned int num_heads, unsigned int num_kv_heads,
-                                      unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ends, unsigned int* first);
+                                      unsigned int head_dim, int kv_format, int scale_dtype, int q_dtype, bool ends, unsigned int* first, bool* halves);
 uint64_t gqa_prefill_staged_bytes(unsigned int tiles, unsigned int num_kv_heads);
 
 // Pages that gqa_prefill_f16.hip addresses by scalars: a power of two of at least its eight tokens a wave, behind a block table
