@@ -203,7 +203,8 @@ def mla_decode_args(q, kv_b, latent_codes, latent_scales, rope_cache, tables, ct
     if selection is not None:  # [batch, top_k] token positions (uint32 / int32)
         args.selection, args.top_k = _ptr(selection), selection.shape[1]
         args.selection_counts = _ptr(selection_counts)
-    need = capi.load().zllm_attn_mla_decode_preferred_bytes(C.byref(args))
+    lib = capi.load()  # a caller's own workspace is taken as it is
+    need = (lib.zllm_attn_mla_decode_preferred_bytes if workspace is None else lib.zllm_attn_mla_decode_workspace_bytes)(C.byref(args))
     if need == 0:
         raise capi.ZllmAttnError(-1, capi.last_error())
     if workspace is None:
