@@ -524,10 +524,13 @@ typedef struct zllm_mla_decode_args {
     int kv_b_scale_dtype;
 } zllm_mla_decode_args;
 ZLLM_API uint64_t zllm_attn_mla_decode_workspace_bytes(const zllm_mla_decode_args* args);
-/* The workspace with which the call is fastest: zllm_attn_mla_decode_workspace_bytes, and for chunks (query_rows > 1) room to convert every
- * latent row of the call once instead of once a query row (at most 1 GiB more).  A call given less runs without. */
+/* The workspace with which a whole call is fastest: zllm_attn_mla_decode_workspace_bytes, and for chunks (query_rows > 1) room to convert every
+ * latent row of the call once instead of once a query row (at most 1 GiB more).  A call asks for that by this very number in
+ * workspace_bytes; with another one, smaller or larger, it runs without. */
 ZLLM_API uint64_t zllm_attn_mla_decode_preferred_bytes(const zllm_mla_decode_args* args);
-/* The record layout of a call, as zllm_attn_gqa_decode_record_layout gives it for GQA; record groups are query rows. */
+/* The record layout of a call, as zllm_attn_gqa_decode_record_layout gives it for GQA; record groups are query rows.  Like every stage
+ * of the call it follows workspace_bytes where that is zllm_attn_mla_decode_preferred_bytes: calls that take up the records of another
+ * one state the same number. */
 ZLLM_API int zllm_attn_mla_decode_record_layout(const zllm_mla_decode_args* args, zllm_split_record_layout* layout);
 ZLLM_API int zllm_attn_mla_decode(const zllm_mla_decode_args* args, zllm_stream_t stream);
 

@@ -43,6 +43,32 @@ def test_which_calls_ask_for_staged_latents():
     assert staged_bytes(16, 1000, 850000) > 0 and staged_bytes(16, 1000, 870000) == 0  # at most 1 GiB
 
 
+def record_layout(args):
+    from zllm_amd import capi
+
+    layout = capi.SplitRecordLayout()
+    capi.check(capi.load().zllm_attn_mla_decode_record_layout(C.byref(args), C.byref(layout)))
+    return [getattr(layout, name) for name, _ in layout._fields_]
+
+
+def test_the_workspace_size_names_the_plan_of_every_stage():
+    """Records lie under one plan for all stage masks and for the layout; only the preferred size itself asks for that of the converted latents."""
+    from zllm_amd import capi
+
+    args = chunk_args(16, 1000, 3000)
+    lib = capi.load()
+    least, preferred = lib.zllm_attn_mla_decode_workspace_bytes(C.byref(args)), lib.zllm_attn_mla_decode_preferred_bytes(C.byref(args))
+    plain = record_layout(args)
+    args.workspace_bytes = preferred
+    staged = record_layout(args)
+    assert staged != plain
+    for stages in (0, 1, 2, 3, 8, 12, 15, 2 | capi.MLA_WIDE_TILES):
+        args.stage_mask = stages
+        for size, want in ((preferred, staged), (0, plain), (least, plain), (preferred - 1, plain), (preferred + 1, plain), (1 << 40, plain)):
+            args.workspace_bytes = size
+            assert record_layout(args) == want, (stages, size)
+
+
 def run_chunk(case, room, out_dtype=None):
     """The call with the preferred workspace, or with the least; max_ctx_len is the longest context."""
     from zllm_amd import capi, ops
@@ -81,6 +107,46 @@ def test_staged_latents_against_the_oracle(heads, lens, rows, kw):
         assert_attention_close(got / scale, want / scale, f"heads={heads} lens={lens} rows={rows}")
     # the two kernels round the same probabilities and products to f16 (2^-12 a term, independent over the tokens)
     assert np.linalg.norm(outs[0] - outs[1]) <= 2.0 ** -11 * np.linalg.norm(outs[1])
+
+
+@pytest.mark.gpu
+def test_later_stages_take_up_the_records_of_a_whole_call():
+    """With the preferred workspace, more, and the least: merge and projection again over the records that a whole call has left, and the
+    call stage by stage, give the bits of the whole call; the layout's statistics are those of every live split."""
+    from zllm_amd import capi, ops
+
+    heads, rows, lens = 16, 300, [2400, 1700]
+    case = make_mla_chunk_case(3, lens, rows, heads, block_tokens=64)
+    keep = [upload(case[n]) for n in ("codes", "scales", "rope", "tables", "lens")]
+    weights, form = weight_args(case)
+    args, out, workspace = ops.mla_decode_args(to_torch_bf16(case["q_bits"], "cuda"), weights, *keep, heads, 192, 256, 512, 64, 64, max(lens),
+                                               query_rows=rows, **form)
+    lib = capi.load()
+    preferred, least = args.workspace_bytes, lib.zllm_attn_mla_decode_workspace_bytes(C.byref(args))
+    assert preferred > least, "this shape is meant to be staged"
+    workspace = torch.empty(preferred + 4096, dtype=torch.uint8, device="cuda")
+    args.workspace = workspace.data_ptr()
+    for size in (preferred, preferred + 4096, least):
+        args.workspace_bytes = size
+        workspace.fill_(0xFF)
+        outs = []
+        for masks in ((0,), (12,), (3, 12), (1, 2, 4, 8)):
+            out.zero_()
+            for mask in masks:
+                args.stage_mask = mask
+                capi.check(lib.zllm_attn_mla_decode(C.byref(args), ops._stream()))
+            outs.append(out.clone())
+            layout = capi.SplitRecordLayout()
+            capi.check(lib.zllm_attn_mla_decode_record_layout(C.byref(args), C.byref(layout)))
+            stats = workspace[layout.stats_offset:layout.stats_offset + layout.record_rows * heads * 8].view(torch.float32).view(-1, heads, 2)
+            for row in (0, rows - 1, rows, 2 * rows - 1):
+                length = lens[row // rows] - (rows - 1 - row % rows)
+                live = stats[row * layout.max_chunks:row * layout.max_chunks + -(-length // layout.chunk_tokens)]
+                assert bool(torch.isfinite(live).all()) and float(live[..., 1].min()) > 0
+        assert float(outs[0].abs().max()) > 0
+        # merge and projection are one kernel in a whole call and two stage by stage: f32 sums in another order
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+        assert float((outs[3] - outs[0]).norm() / outs[0].norm()) <= 1e-5
 
 
 @pytest.mark.gpu

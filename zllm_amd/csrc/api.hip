@@ -410,7 +410,7 @@ MlaWorkspace mla_workspace(const zllm_mla_decode_args* a, const MlaSplitPlan& pl
     return w;
 }
 
-// A whole call over latents that are converted once (mla_staged.hip): its splits, and the 32-token tiles a sequence.  0 tiles for other calls.
+// A chunk over latents that are converted once (mla_staged.hip): its splits, and the 32-token tiles a sequence.  0 tiles for other calls.
 // A compute unit takes a tile for 128 (row, head) pairs in 2.15 us there; mla_partial_ws takes it for 64 heads of one row in 1.42 us and for
 // up to 32 in 1.05.  The staging is a launch, and as many workgroups leave twice the records: the difference has to come to some 31 us over 256
 // compute units.  Us a call without / with: 128 heads, 20 rows behind 10,000 keys 109 / 116, 500 behind none 171 / 163, 512 behind
@@ -419,9 +419,8 @@ MlaWorkspace mla_workspace(const zllm_mla_decode_args* a, const MlaSplitPlan& pl
 // behind 3,000 193 / 99, 1,000 behind 2,000 378 / 167.  The tiles are bounded by 1 GiB, 856,000 tokens.
 uint32_t plan_mla_staged(const zllm_mla_decode_args* a, MlaSplitPlan* plan)
 {
-    const uint32_t stages = a->stage_mask & 31u;
     const uint64_t rows = mla_query_rows(a);
-    if ((stages != 0u && stages != 15u) || a->latent_dim != 512u || a->rope_dim != 64u || a->selection != nullptr || rows < 2u) {
+    if (a->latent_dim != 512u || a->rope_dim != 64u || a->selection != nullptr || rows < 2u) {
         return 0;
     }
     const uint32_t heads_here = a->heads < 128u ? a->heads : 128u;
@@ -436,6 +435,43 @@ uint32_t plan_mla_staged(const zllm_mla_decode_args* a, MlaSplitPlan* plan)
     plan_splits(a->max_ctx_len, units, 1, 64, &plan->chunk_tokens, &plan->max_chunks);
     plan->record_rows = (uint64_t)a->batch * rows * plan->max_chunks;
     return (uint32_t)tiles;
+}
+
+// What a call runs with: its splits, where its arrays lie, and for chunks over converted latents their tiles, behind the arrays.
+struct MlaCallPlan {
+    MlaSplitPlan splits;
+    MlaWorkspace workspace;
+    uint32_t staged_tiles; // a sequence; 0: none
+    uint64_t staged_at;
+};
+
+// Workspace of a chunk over converted latents, 0 for other calls; `plan` is what it runs with.  At least what the call needs without them.
+uint64_t plan_mla_preferred(const zllm_mla_decode_args* a, MlaCallPlan* plan)
+{
+    plan->staged_tiles = plan_mla_staged(a, &plan->splits);
+    if (plan->staged_tiles == 0) {
+        return 0;
+    }
+    plan->workspace = mla_workspace(a, plan->splits);
+    plan->staged_at = align_up(plan->workspace.total, 256);
+    const uint64_t bytes = plan->staged_at + zllm::mla_staged_bytes(plan->staged_tiles, a->batch), least = mla_workspace(a, plan_mla_decode(a)).total;
+    return bytes > least ? bytes : least + 1u; // never the number that asks for the other plan
+}
+
+// One plan for every stage of a call, for the record layout and for later calls that take up its records: it follows from the host arguments
+// alone.  workspace_bytes asks for the converted latents by being that very number -- a larger workspace does not, or a caller who keeps one
+// for all of its calls and asks for the layout before would find the records of another plan.
+MlaCallPlan plan_mla_call(const zllm_mla_decode_args* a)
+{
+    MlaCallPlan plan;
+    const uint64_t preferred = plan_mla_preferred(a, &plan);
+    if (preferred == 0 || a->workspace_bytes != preferred) {
+        plan.splits = plan_mla_decode(a);
+        plan.workspace = mla_workspace(a, plan.splits);
+        plan.staged_tiles = 0;
+        plan.staged_at = 0;
+    }
+    return plan;
 }
 
 } // namespace
@@ -991,13 +1027,13 @@ uint64_t zllm_attn_mla_decode_workspace_bytes(const zllm_mla_decode_args* a)
 uint64_t zllm_attn_mla_decode_preferred_bytes(const zllm_mla_decode_args* a)
 {
     const uint64_t least = zllm_attn_mla_decode_workspace_bytes(a);
-    MlaSplitPlan plan;
-    const uint32_t tiles = least == 0 ? 0 : plan_mla_staged(a, &plan);
-    if (tiles == 0) {
+    const uint32_t whole = ZLLM_MLA_ABSORB | ZLLM_MLA_PARTIAL | ZLLM_MLA_MERGE | ZLLM_MLA_PROJECT;
+    if (least == 0 || (a->stage_mask != 0u && a->stage_mask != whole)) {
         return least;
     }
-    const uint64_t staged = align_up(mla_workspace(a, plan).total, 256) + zllm::mla_staged_bytes(tiles, a->batch);
-    return staged > least ? staged : least;
+    MlaCallPlan plan;
+    const uint64_t preferred = plan_mla_preferred(a, &plan);
+    return preferred != 0 ? preferred : least;
 }
 
 int zllm_attn_mla_decode_record_layout(const zllm_mla_decode_args* a, zllm_split_record_layout* out)
@@ -1009,8 +1045,9 @@ int zllm_attn_mla_decode_record_layout(const zllm_mla_decode_args* a, zllm_split
     if (out == nullptr) {
         return fail(-1, "MLA decode record layout: null output");
     }
-    const MlaSplitPlan plan = plan_mla_decode(a);
-    const MlaWorkspace w = mla_workspace(a, plan);
+    const MlaCallPlan call = plan_mla_call(a);
+    const MlaSplitPlan& plan = call.splits;
+    const MlaWorkspace& w = call.workspace;
     out->record_rows = plan.record_rows;
     out->partial_offset = w.partial;
     out->stats_offset = w.stats;
@@ -1038,20 +1075,12 @@ int zllm_attn_mla_decode(const zllm_mla_decode_args* a, zllm_stream_t stream)
     }
     zllm::MlaDecodeParams p;
     memset(&p, 0, sizeof(p));
-    MlaSplitPlan plan;
-    MlaWorkspace w;
-    const uint32_t staged_tiles = plan_mla_staged(a, &plan);
-    if (staged_tiles != 0) {
-        w = mla_workspace(a, plan);
-        const uint64_t records = align_up(w.total, 256);
-        if (a->workspace_bytes >= records + zllm::mla_staged_bytes(staged_tiles, a->batch)) {
-            p.staged = (unsigned char*)a->workspace + records;
-            p.staged_tiles = staged_tiles;
-        }
-    }
-    if (p.staged == nullptr) {
-        plan = plan_mla_decode(a);
-        w = mla_workspace(a, plan);
+    const MlaCallPlan call = plan_mla_call(a);
+    const MlaSplitPlan& plan = call.splits;
+    const MlaWorkspace& w = call.workspace;
+    if (call.staged_tiles != 0 && (a->stage_mask & ZLLM_MLA_WIDE_TILES) == 0) {
+        p.staged = (unsigned char*)a->workspace + call.staged_at;
+        p.staged_tiles = call.staged_tiles;
     }
     p.chunk_tokens = plan.chunk_tokens;
     p.max_chunks = plan.max_chunks;

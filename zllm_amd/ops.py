@@ -203,13 +203,17 @@ def mla_decode_args(q, kv_b, latent_codes, latent_scales, rope_cache, tables, ct
     if selection is not None:  # [batch, top_k] token positions (uint32 / int32)
         args.selection, args.top_k = _ptr(selection), selection.shape[1]
         args.selection_counts = _ptr(selection_counts)
-    lib = capi.load()  # a caller's own workspace is taken as it is
-    need = (lib.zllm_attn_mla_decode_preferred_bytes if workspace is None else lib.zllm_attn_mla_decode_workspace_bytes)(C.byref(args))
-    if need == 0:
+    lib = capi.load()
+    need = least = lib.zllm_attn_mla_decode_workspace_bytes(C.byref(args))
+    if least == 0:
         raise capi.ZllmAttnError(-1, capi.last_error())
+    if query_rows > 1:
+        need = lib.zllm_attn_mla_decode_preferred_bytes(C.byref(args))
     if workspace is None:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     args.workspace, args.workspace_bytes = _ptr(workspace), workspace.numel()
+    if workspace.numel() >= need > least:  # the number asks for the larger workspace's plan
+        args.workspace_bytes = need
     return args, out, workspace
 
 
