@@ -5,6 +5,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import oracle as O
 from tests.cases import assert_attention_close, to_torch_bf16, upload
 from tests.test_gpu_mla_decode import make_mla_chunk_case, oracle_mla_chunk, weight_args
 
@@ -107,6 +108,42 @@ def test_staged_latents_against_the_oracle(heads, lens, rows, kw):
         assert_attention_close(got / scale, want / scale, f"heads={heads} lens={lens} rows={rows}")
     # the two kernels round the same probabilities and products to f16 (2^-12 a term, independent over the tokens)
     assert np.linalg.norm(outs[0] - outs[1]) <= 2.0 ** -11 * np.linalg.norm(outs[1])
+
+
+def rope_score_chunk(heads, rows, length, first_gain, spread):
+    """A chunk whose scores come from the rope columns alone, its first 64 latents `first_gain` above the others and seen with a weight of some
+    e^-40; and its attention in 64 bits, before the projection by the value rows, which pick columns 4 v of the latents.  The case's context is `length`."""
+    case = make_mla_chunk_case(11, [length], rows, heads, block_tokens=64, latent_gain=np.where(np.arange(length) < 64, first_gain, 1.0))
+    rng = np.random.default_rng(5)
+    direction = rng.standard_normal(64)
+    q = rng.standard_normal((rows, heads, 192)) * 0.5
+    q[..., 128:] = (q[..., 128:] + direction) * spread * np.sqrt(192.0) / np.sqrt(64 * 1.25)  # scores of deviation `spread`
+    kv_b = np.zeros((heads, 256, 512), dtype=np.float32)
+    kv_b[:, 128 + np.arange(128), 4 * np.arange(128)] = 1.0
+    k_rope = rng.standard_normal((length, 64)) - np.where(np.arange(length) < 64, 6.0 / spread, 0.0)[:, None] * direction
+    case["q_bits"], case["kv_b_bits"] = O.f32_to_bf16(q.reshape(rows, -1).astype(np.float32)), O.f32_to_bf16(kv_b.reshape(-1, 512))
+    pages = case["tables"][0].astype(np.int64)
+    at = (pages[:, None] * 64 + np.arange(64)).reshape(-1)[:length]
+    case["rope"][at] = O.f32_to_bf16(k_rope.astype(np.float32))
+    latents = case["codes"][at].astype(np.float64) * np.repeat(O.bf16_to_f32(case["scales"][at]).astype(np.float64), 64, axis=1)
+    q64 = O.bf16_to_f32(case["q_bits"]).astype(np.float64).reshape(rows, heads, 192)[..., 128:]
+    scores = q64 @ O.bf16_to_f32(case["rope"][at]).astype(np.float64).T / np.sqrt(192.0)
+    scores = np.where(np.arange(length) < length - rows + 1 + np.arange(rows)[:, None, None], scores, -np.inf)
+    p = np.exp(scores - scores.max(axis=2, keepdims=True))
+    return case, (p / p.sum(axis=2, keepdims=True)) @ latents[:, ::4]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spread", [0.5, 2.0])
+@pytest.mark.parametrize("gain", [8, 14, 17, 20, 24])
+def test_scales_that_fall_keep_their_bits(gain, spread):
+    """Latents 2^gain below those before them, which hold the exponent window of the values: the staged call is as far from 64 bits as the
+    call that converts them for every row (f16 weights and products whose factors are rounded alike, in another order)."""
+    case, want = rope_score_chunk(8, 300, 2000, 2.0 ** gain, spread)
+    staged, plain = (run_chunk(case, room).reshape(want.shape) for room in (True, False))
+    err = [float(np.linalg.norm(got - want) / np.linalg.norm(want)) for got in (staged, plain)]
+    print("mla falling scales", gain, spread, err)
+    assert err[0] <= 1.05 * err[1]
 
 
 @pytest.mark.gpu

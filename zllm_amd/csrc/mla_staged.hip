@@ -415,7 +415,13 @@ __global__ __launch_bounds__(64 * kWaves, 1) void mla_partial_staged(MlaDecodePa
             }
         }
     };
-    // behind the softmax: the probabilities as f16, brought to the accumulators' window
+    // Behind the softmax: the probabilities as f16, the accumulators and the scales of the values in one window.  A tile 2^k below the accumulators'
+    // window brings its probabilities down by it, up to k = 8 (what they lose then counts for nothing beside the rounding of the products).
+    // Further below, its scales are written anew from f32, 2^min(k, 16) lower, which leaves the largest normal (every wave writes the same table and
+    // reads it behind its own writes), and the probabilities take what is left.  k = 20 (3,000 keys, scores of deviation 1), 2-norm from 64
+    // bits: 7.0e-4; all of it on the probabilities 2.5e-3, all on the scales, as mla_partial_ws has it, 2.8e-3; up to k = 12 2.7e-4
+    // whichever way.  Written for every tile below the window (by 2, among latents of one size) the table costs 512 rows of 128 heads
+    // behind 16,384 keys 3 %.
     auto take_probabilities = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -424,8 +430,21 @@ __global__ __launch_bounds__(64 * kWaves, 1) void mla_partial_staged(MlaDecodePa
         if (tile_window > window) {
             acc_fix *= __uint_as_float((unsigned int)(127 - min(tile_window - window, 126)) << 23);
             window = tile_window;
-        } else if (tile_window < window) { // not past the end of f16: what is below counts for nothing beside the window's scales
-            const float down = __uint_as_float((unsigned int)(127 - min(window - tile_window, 30)) << 23);
+        } else if (tile_window < window) {
+            int rest = window - tile_window;
+            if (rest > 8) {
+                rest = min(max(rest - 16, 0), 14);
+                const float into_window = __uint_as_float((unsigned int)(127 - kPShift - window + rest) << 23);
+                unsigned int to = lane, from;
+                asm volatile("" : "+v"(to)); // or the addresses take registers of the loop
+                from = keys_at + kScaleAt + (to >> 4) * 128u + (to & 15u) * 4u;
+                to = keys_at + kScale16At + to * 2u;
+#pragma unroll 1
+                for (unsigned int i = 0; i < kGroups / 2; ++i) { // two groups of 32 tokens
+                    *(_Float16*)(lds + to + i * 128) = (_Float16)(*(const float*)(lds + from + i * 512) * into_window);
+                }
+            }
+            const float down = __uint_as_float((unsigned int)(127 - rest) << 23);
             const unsigned int down2 = pack_f16_hw(down, down);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
