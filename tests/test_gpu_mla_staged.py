@@ -147,6 +147,31 @@ def test_scales_that_fall_keep_their_bits(gain, spread):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,rows,length", [(16, 300, 2403), (128, 110, 4005), (40, 185, 2231), (1, 1001, 1500)])  # 8, 1, 3 and 128 rows a workgroup
+def test_rows_are_independent_of_later_tokens(heads, rows, length):
+    """The last five tokens hold infinite scales, NaN and NaN rope columns: rows that do not see them come out as with ordinary ones there."""
+    case = make_mla_chunk_case(heads + 1, [length], rows, heads, block_tokens=64)
+    clean = run_chunk(case, True)[:rows - 5]
+    assert (length - 5) % 64 <= 59
+    at = int(case["tables"][0][(length - 5) // 64]) * 64 + (length - 5) % 64  # five tokens of one page
+    case["scales"][at:at + 2], case["scales"][at + 2:at + 4], case["rope"][at + 4] = 0x7F80, 0x7FC0, 0x7FC0
+    for room in (True, False):
+        got = run_chunk(case, room)[:rows - 5]
+        assert np.linalg.norm(got - clean) <= 2.0 ** -11 * np.linalg.norm(clean)
+
+
+@pytest.mark.gpu
+def test_a_row_keeps_its_bits_before_a_far_larger_token():
+    """One row a workgroup: a last token 2^24 above the others is no part of the rows before it, though it lies in their last tile."""
+    case, want = rope_score_chunk(128, 110, 4007, 1.0, 2.0)
+    at = int(case["tables"][0][4006 // 64]) * 64 + 4006 % 64
+    case["scales"][at] = O.f32_to_bf16(O.bf16_to_f32(case["scales"][at]) * np.float32(2.0 ** 24))
+    err = [float(np.linalg.norm((run_chunk(case, room).reshape(want.shape) - want)[:109]) / np.linalg.norm(want[:109])) for room in (True, False)]
+    print("mla row before a large token", err)
+    assert err[0] <= 1.05 * err[1]
+
+
+@pytest.mark.gpu
 def test_later_stages_take_up_the_records_of_a_whole_call():
     """With the preferred workspace, more, and the least: merge and projection again over the records that a whole call has left, and the
     call stage by stage, give the bits of the whole call; the layout's statistics are those of every live split."""

@@ -39,7 +39,7 @@ constexpr int kScale16At = kScaleAt + 64 * kGroups * 4;
 constexpr int kTile = kScale16At + kStep * kGroups * 2;
 static_assert(kTile % 1024 == 0, "tiles are moved in whole wave loads");
 constexpr int kLoads = kTile / 1024;
-constexpr int kWindowAt = kTile; // the tile's exponent window, read by scalar loads
+constexpr int kWindowAt = kTile; // exponent windows of the tile's first 1, 2 ... 32 tokens, read by scalar loads
 constexpr int kBlock = kTile + 128;
 constexpr int kBufs = 3;
 constexpr int kBlocksBehind = 4; // a part's requests run up to three tiles past its last
@@ -78,6 +78,9 @@ __global__ __launch_bounds__(256) void mla_stage(MlaDecodeParams p)
     }
     const u32x4 rope = *(const u32x4*)((const unsigned char*)p.rope_cache + row * (kRope * 2) + part * 16u);
     const float scale = t0 + token < end ? bf16_bits_to_f32(p.latent_scales[row * kGroups + part]) : 0.0f;
+    // An infinite scale or a NaN makes the scores of its token NaN, and with them whatever sees the token.  Nothing else: it counts as zero for the
+    // values and the windows, where rows of the workgroup that do not see it would meet it with a probability of zero.
+    const float value_scale = fabsf(scale) < __builtin_inff() ? scale : 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
@@ -94,22 +97,32 @@ __global__ __launch_bounds__(256) void mla_stage(MlaDecodeParams p)
         }
     }
     *(u32x4*)(block + kRopeAt + (part >> 1) * 1024u + (part & 1u) * 512u + token * 16u) = rope;
-    __shared__ unsigned int tops[4];
-    const unsigned int wave_top = wave_max_u(__float_as_uint(fmaxf(scale, 0.0f)));
-    if ((tid & 63u) == 0u) {
-        tops[tid >> 6] = wave_top;
+    __shared__ unsigned int tops[kStep];
+    unsigned int token_top = __float_as_uint(fmaxf(value_scale, 0.0f));
+#pragma unroll
+    for (int d = 1; d < kGroups; d <<= 1) {
+        token_top = max(token_top, (unsigned int)__shfl_xor((int)token_top, d));
+    }
+    if (part == 0u) {
+        tops[token] = token_top;
     }
     __syncthreads();
-    const unsigned int top = max(max(tops[0], tops[1]), max(tops[2], tops[3]));
-    const int window = min(max((int)((top >> 23) & 0xffu) - 133, -96), 112); // as in mla_partial_ws
+    unsigned int top = tops[tid & 31u]; // of the tokens up to this one
+#pragma unroll
+    for (int d = 1; d < kStep; d <<= 1) {
+        const unsigned int before = (unsigned int)__shfl_up((int)top, d, kStep);
+        top = max(top, (tid & 31u) >= (unsigned int)d ? before : 0u);
+    }
+    const int up_to = min(max((int)((top >> 23) & 0xffu) - 133, -96), 112); // as in mla_partial_ws
+    const int window = __builtin_amdgcn_readlane(up_to, 31);
     const unsigned int element = 4u * (token >> 3) + (token & 3u), half = (token >> 2) & 1u;
 #pragma unroll
     for (unsigned int row = 0; row < 2; ++row) { // both rows of sixteen lanes of the half
-        ((float*)(block + kScaleAt))[part * 64u + 32u * half + 16u * row + element] = scale;
+        ((float*)(block + kScaleAt))[part * 64u + 32u * half + 16u * row + element] = value_scale == scale ? scale : __builtin_nanf("");
     }
-    ((_Float16*)(block + kScale16At))[part * 32u + half * 16u + element] = (_Float16)(scale * __uint_as_float((unsigned int)(127 - kPShift - window) << 23));
-    if (tid == 0u) {
-        *(int*)(block + kWindowAt) = window;
+    ((_Float16*)(block + kScale16At))[part * 32u + half * 16u + element] = (_Float16)(value_scale * __uint_as_float((unsigned int)(127 - kPShift - window) << 23));
+    if (tid < (unsigned int)kStep) {
+        ((int*)(block + kWindowAt))[tid] = up_to;
     }
 }
 
@@ -415,6 +428,19 @@ __global__ __launch_bounds__(64 * kWaves, 1) void mla_partial_staged(MlaDecodePa
             }
         }
     };
+    // the f16 scales of the tile at `at` from its f32 ones, for the window given; none for tokens from `seen` on
+    auto write_scales = [&](unsigned int at, int to_window, unsigned int seen) __attribute__((always_inline)) {
+        const float into_window = __uint_as_float((unsigned int)(127 - kPShift - to_window) << 23);
+        unsigned int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); // the lane again: no registers of the loop
+        asm volatile("" : "+v"(l));
+        const bool live = 8u * ((l >> 2) & 3u) + 4u * ((l >> 4) & 1u) + (l & 3u) < seen;
+        const unsigned int from = at + kScaleAt + (l >> 4) * 128u + (l & 15u) * 4u, to = at + kScale16At + l * 2u;
+#pragma unroll 1
+        for (unsigned int i = 0; i < kGroups / 2; ++i) { // two groups of 32 tokens
+            const float scale = *(const float*)(lds + from + i * 512);
+            *(_Float16*)(lds + to + i * 128) = (_Float16)(live && scale == scale ? scale * into_window : 0.0f);
+        }
+    };
     // Behind the softmax: the probabilities as f16, the accumulators and the scales of the values in one window.  A tile 2^k below the accumulators'
     // window brings its probabilities down by it, up to k = 8 (what they lose then counts for nothing beside the rounding of the products).
     // Further below, its scales are written anew from f32, 2^min(k, 16) lower, which leaves the largest normal (every wave writes the same table and
@@ -434,15 +460,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void mla_partial_staged(MlaDecodePa
             int rest = window - tile_window;
             if (rest > 8) {
                 rest = min(max(rest - 16, 0), 14);
-                const float into_window = __uint_as_float((unsigned int)(127 - kPShift - window + rest) << 23);
-                unsigned int to = lane, from;
-                asm volatile("" : "+v"(to)); // or the addresses take registers of the loop
-                from = keys_at + kScaleAt + (to >> 4) * 128u + (to & 15u) * 4u;
-                to = keys_at + kScale16At + to * 2u;
-#pragma unroll 1
-                for (unsigned int i = 0; i < kGroups / 2; ++i) { // two groups of 32 tokens
-                    *(_Float16*)(lds + to + i * 128) = (_Float16)(*(const float*)(lds + from + i * 512) * into_window);
-                }
+                write_scales(keys_at, window - rest, kStep);
             }
             const float down = __uint_as_float((unsigned int)(127 - rest) << 23);
             const unsigned int down2 = pack_f16_hw(down, down);
@@ -453,8 +471,13 @@ __global__ __launch_bounds__(64 * kWaves, 1) void mla_partial_staged(MlaDecodePa
         }
     };
 
-    const unsigned char* window_of = staged + kBlock; // of tile n + 1
-    auto load_window = [&](const unsigned char* block) __attribute__((always_inline)) { return *(const __attribute__((address_space(4))) int*)(uintptr_t)(block + kWindowAt); };
+    // A tile's window is that of its whole, in the last tile that of the tokens which some row of the workgroup sees: neither windows nor values hang
+    // on what only later rows see.  (Rows of one workgroup share their windows, as the row tiles of the GQA chunk kernels do.)
+    const unsigned int last_tile_at = (steps - 1u) * kBlock, last_seen = min(end_of_rows - (begin + (steps - 1u) * kStep), (unsigned int)kStep);
+    const unsigned int last_window_at = last_tile_at + kWindowAt + (last_seen - 1u) * 4u;
+    unsigned int window_at = min((unsigned int)kWindowAt + (kStep - 1) * 4u, last_window_at); // of tile n + 1
+    auto load_window = [&](unsigned int at) __attribute__((always_inline)) { return *(const __attribute__((address_space(4))) int*)(uintptr_t)(staged + at); };
+    const int seen_window = load_window(last_window_at), whole_window = load_window(last_tile_at + kWindowAt + (kStep - 1) * 4);
     auto next_buf = [](unsigned int at) __attribute__((always_inline)) { return at == (kBufs - 1u) * kTile ? 0u : at + kTile; };
     auto wait_tile = [&](auto left) __attribute__((always_inline)) { // a wave for its own loads and reads, the barrier for the others'
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(left)::value) : "memory");
@@ -545,7 +568,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void mla_partial_staged(MlaDecodePa
     }
 
     // tile 0: keys and softmax alone
-    window = tile_window = load_window(staged);
+    window = tile_window = load_window(window_at);
+    window_at = min(window_at + kBlock, last_window_at);
     keys_at = 0;
     values_at = 0;
     wait_tile(std::integral_constant<int, 2 * kOwn>{});
@@ -559,7 +583,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void mla_partial_staged(MlaDecodePa
         softmax_slot(n, begin);
     }
     take_probabilities(); // acc_fix of the first tile multiplies zeros
-    tile_window = load_window(window_of);
+    tile_window = load_window(window_at);
     wait_tile(std::integral_constant<int, kOwn>{});
     keys_at = kTile;
     open_keys();
@@ -568,8 +592,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void mla_partial_staged(MlaDecodePa
         multiply_keys(true);
         accumulate(std::integral_constant<bool, true>{}, begin + step * kStep, upcoming_at);
         take_probabilities();
-        window_of += kBlock;
-        tile_window = load_window(window_of);
+        window_at = min(window_at + kBlock, last_window_at);
+        tile_window = load_window(window_at);
         fix_accumulators();
         values_at = keys_at;
         keys_at = upcoming_at;
@@ -577,6 +601,10 @@ __global__ __launch_bounds__(64 * kWaves, 1) void mla_partial_staged(MlaDecodePa
 #pragma unroll
     for (int n = 0; n < kRing; ++n) {
         request_value(n);
+    }
+    if (whole_window != seen_window) { // the last tile's scales are in the window of its whole: as take_probabilities has left the others
+        const int rest = window - seen_window;
+        write_scales(values_at, rest > 8 ? window - min(max(rest - 16, 0), 14) : seen_window, last_seen);
     }
     accumulate(std::integral_constant<bool, false>{}, 0u, 0u);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // what was requested past the range lands before the LDS is given back
