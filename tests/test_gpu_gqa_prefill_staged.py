@@ -77,6 +77,38 @@ def test_staged_rows_against_the_oracle(prefix, chunk, hq, hkv, kw):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,prefix,tile_rows", [(290, 300, 64), (1100, 7, 32)])  # a row tile of 256 pairs; of 128, the keys in two halves
+@pytest.mark.parametrize("k_bits,v_bits", [(0x7E00, 0x7C00), (0x0001, 0x7BFF)])  # a NaN and an infinity; the smallest and the largest scale
+def test_row_tiles_are_independent_of_later_tokens(rows, prefix, tile_rows, k_bits, v_bits):
+    """A token in the 32-token tile in which a row tile ends, but behind its rows: they come out bit for bit as with an ordinary one there."""
+    from zllm_amd import capi, ops
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(9)
+    total, page = prefix + rows, 16
+    table = torch.randperm((total + page - 1) // page, generator=gen, device="cuda").to(torch.int32)
+    planes = [torch.zeros(table.numel() * page, n, dtype=t, device="cuda") for n, t in ((1024, torch.int8), (16, torch.int16)) * 2]
+    for n in (0, 2):
+        ops.q8g64_append(torch.randn(total, 1024, generator=gen, device="cuda", dtype=torch.bfloat16), planes[n], planes[n + 1], table, 0, page,
+                         capi.QUANT_METAL_GQA)
+    q = torch.randn(rows, 32 * 128, generator=gen, device="cuda", dtype=torch.bfloat16)
+    assert staged_bytes(rows, prefix, 32, 8) > 0
+
+    def call():
+        return ops.gqa_prefill_chunk(q, *planes, table, prefix, 32, 8, 128, page, 128 ** -0.5)
+
+    clean = call()
+    seen = 3 * tile_rows  # rows of the first three tiles
+    token = (prefix + seen) | 31  # the last of the 32 tokens in which they end
+    assert (prefix + seen) % 32 and token < total
+    at = int(table[token // page]) * page + token % page
+    planes[1][at], planes[3][at] = k_bits, v_bits
+    got = call()
+    assert torch.equal(got[:seen], clean[:seen])
+    assert not torch.equal(got[seen:], clean[seen:])
+
+
+@pytest.mark.gpu
 def test_staged_rows_in_a_graph():
     """Staging and attention recorded together, replayed over caches that change in between."""
     from zllm_amd import capi, ops

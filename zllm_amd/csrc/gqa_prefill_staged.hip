@@ -29,7 +29,7 @@ constexpr int kGroups = kD / 64;
 constexpr int kScales = kGroups * kStep * 4; // bytes of a tile's f32 scales, [token][group]
 constexpr int kWaves = 8; // of 32 pairs each
 constexpr int kBufs = 6; // three passes of two tiles: one attended, one complete or on its way, one requested
-// A staged tile: K | V | K scales | V scales | the (biased) exponent of the largest V scale.  K and V lie as the matrix instructions take
+// A staged tile: K | V | K scales | V scales | the (biased) exponents of the largest V scale of its first 1, 2 ... 32 tokens.  K and V lie as the matrix instructions take
 // them, 1 KiB a fragment, 16 bytes a lane: K fragment ks holds columns 16 ks + 8 h .. + 8 of token c (lane 32 h + c), V fragment 2 t + kk
 // column 32 t + c of tokens 16 kk + 4 h .. + 4 and eight further.
 constexpr int kKsAt = 2 * kTile, kVsAt = 2 * kTile + kScales, kTopAt = 2 * kTile + 2 * kScales;
@@ -115,9 +115,15 @@ template <int SDT> __global__ __launch_bounds__(256) void gqa_stage_q8(GqaPrefil
         const float fold = of_v ? 1.0f : p.softcap > 0.0f ? p.score_scale : p.score_scale * kLog2e;
         ((float*)(block + kKsAt))[tid] = scale * fold;
         if (of_v) { // the second wave
-            const float top = __uint_as_float(wave_max_u(__float_as_uint(fmaxf(scale, 0.0f))));
-            if (tid == kGroups * kStep) { // clamped away from the ends of the f32 range
-                *(unsigned int*)(block + kTopAt) = min(max((__float_as_uint(top) >> 23) & 0xffu, 2u), 252u);
+            unsigned int top = __float_as_uint(fmaxf(scale, 0.0f));
+            top = max(top, (unsigned int)__shfl_xor((int)top, 1));
+#pragma unroll
+            for (int d = kGroups; d < 64; d <<= 1) {
+                const unsigned int before = (unsigned int)__shfl_up((int)top, d);
+                top = max(top, (tid & 63u) >= (unsigned int)d ? before : 0u);
+            }
+            if (group == 0u) { // clamped away from the ends of the f32 range
+                ((unsigned int*)(block + kTopAt))[token] = min(max((top >> 23) & 0xffu, 2u), 252u);
             }
         }
     }
@@ -345,6 +351,11 @@ template <int SOFTCAP, int HALVES> __global__ __launch_bounds__(64 * kWaves, 2) 
         if (t0 + kStep > wave_min_hi || t0 < wave_max_lo) { // only steps at an edge of some column need the per-token masks
             unsigned int first = t0 + 4u * h;
             asm volatile("" : "+v"(first)); // or sixteen additions leave the branch
+            // What the tile's last rows do not see counts as zero, or an infinite V scale there would meet their probabilities of zero: every wave
+            // clears the same scales and reads them behind its own writes.
+            if (t0 + kStep > part.end && first + 8u * (m >> 2) + (m & 3u) >= part.end) {
+                *(f32x2*)(&lds.scales[buf][1][0][0] + scale_at) = f32x2{0.0f, 0.0f};
+            }
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const unsigned int token = first + 8u * (i >> 2) + (i & 3);
@@ -485,11 +496,12 @@ template <int SOFTCAP, int HALVES> __global__ __launch_bounds__(64 * kWaves, 2) 
     // the exponents come by scalar loads, two tiles ahead
     const unsigned char* pass_at = staged;
     auto load_top = [&](unsigned int tile) __attribute__((always_inline)) -> unsigned int { // `tile` tiles past the pass's first
-        return *(scalar_words_t)(uintptr_t)(pass_at + tile * kBlock + kTopAt);
+        return *(scalar_words_t)(uintptr_t)(pass_at + tile * kBlock + kTopAt + (kStep - 1) * 4);
     };
+    const unsigned int last_top = *(scalar_words_t)(uintptr_t)(staged + (steps - 1u) * kBlock + kTopAt + (part.end - part.begin - (steps - 1u) * kStep - 1u) * 4u); // of what its rows see
     unsigned int top_now = load_top(half), top_next = load_top(half + 1u * HALVES);
     auto attend_tile = [&](unsigned int step, int buf) __attribute__((always_inline)) {
-        const unsigned int wv_now = max(wv, top_now);
+        const unsigned int wv_now = max(wv, step + 1u == steps ? last_top : top_now);
         top_now = top_next;
         top_next = load_top(HALVES == 1 ? 2u + (buf & 1) : half + 4u);
         const bool window_moved = wv_now != wv; // rare: a V scale above everything met so far
