@@ -1,5 +1,6 @@
-"""The chunk kernel over f16 rows of head_dim 256 (gqa_prefill_f16_256.hip): pages it addresses by scalars and others, ranges that end in
-either half's tile and inside a run of sixteen rows, windows, given and empty ranges, groups, KV splits, against 64-bit attention."""
+"""Chunks over f16 rows of head_dim 256, the walks of 576 keys and more in two halves (gqa_prefill_f16_256.hpp): pages they address by scalars and
+others, ranges that end in either half's tile and inside a run of sixteen rows, windows, given and empty ranges, groups, KV splits, row
+tiles on both sides of the line in one call, against 64-bit attention."""
 import numpy as np
 import pytest
 import torch
@@ -33,7 +34,7 @@ def run(rows, position, heads, kv_heads, page=16, window=0, softcap=0.0, given=N
         hi = torch.minimum((r // 50 + 1) * 50, torch.tensor(rows, device="cuda")) + position
         kw = dict(visible_ends=hi.to(torch.int32))
     elif given == "segments":  # the rows of the third see nothing
-        cuts = torch.tensor([0, 3, 64, 131], device="cuda")
+        cuts = torch.tensor([0, 3, 64, 131] if rows < 300 else [0, 300, 360, 610, 1250, 1256], device="cuda")
         which = torch.searchsorted(cuts, r, right=True) - 1
         lo, hi = cuts[which], torch.cat([cuts[1:], torch.tensor([rows], device="cuda")])[which]
         hi = torch.where(which == 2, lo, hi)
@@ -53,9 +54,15 @@ def run(rows, position, heads, kv_heads, page=16, window=0, softcap=0.0, given=N
 @pytest.mark.parametrize("page", [16, 64, 256, 8, 24])  # the last two keep the tile kernel
 def test_pages(page):
     run(150, 300, 16, 8, page)
+    run(150, 700, 16, 8, page, workspace=False)
 
 
-# ranges that end at every edge: a run of sixteen rows, a tile of 32, a pass of two tiles; 128 pairs over 256 keys are the least it takes
+# ranges that end at every edge: a run of sixteen rows, a tile of 32, a pass of two tiles; walks of 576 keys are the shortest in halves
+@pytest.mark.parametrize("rows,position", [(64, 511), (64, 512), (64, 513), (65, 527), (65, 528), (79, 529), (64, 544), (97, 543), (575, 0), (576, 0), (700, 3)])
+def test_edges_of_halves(rows, position):
+    run(rows, position, 4, 2, workspace=False)
+
+
 @pytest.mark.parametrize("rows,position", [(64, 192), (64, 193), (65, 207), (65, 208), (79, 209), (64, 224), (97, 223), (255, 0), (256, 0), (257, 0), (289, 2),
                                            (63, 300), (64, 191)])
 def test_edges(rows, position):
@@ -65,9 +72,10 @@ def test_edges(rows, position):
 @pytest.mark.parametrize("heads,kv_heads,rows", [(3, 3, 140), (12, 4, 90), (16, 1, 40), (128, 1, 60), (100, 1, 60)])
 def test_groups(heads, kv_heads, rows):
     run(rows, 200, heads, kv_heads)
+    run(rows, 600, heads, kv_heads, workspace=False)
 
 
-@pytest.mark.parametrize("window", [200, 256, 300, 1024])  # from 256 on
+@pytest.mark.parametrize("window", [200, 256, 511, 512, 1024])  # a row tile of 64 and a window of 512: 575 keys from a tile's first on, in halves
 def test_windows(window):
     run(170, 900, 4, 2, window=window)
     run(300, 0, 4, 2, window=window)
@@ -78,6 +86,13 @@ def test_given_ranges(given, position):
     run(260, position, 8, 2, given=given)
 
 
+# walks on both sides of the line in one launch: segments of 300, 60, none, 640, 6 and 150 rows, their row tiles across them, and ends inside a prefix
+@pytest.mark.parametrize("heads,kv_heads", [(8, 2), (16, 16), (6, 3)])
+@pytest.mark.parametrize("given,position,workspace", [("segments", 0, True), ("segments", 0, False), ("ends", 0, False), ("ends", 530, False), ("ends", 530, True)])
+def test_given_ranges_of_both_lengths(heads, kv_heads, given, position, workspace):
+    run(1406, position, heads, kv_heads, given=given, workspace=workspace)
+
+
 @pytest.mark.parametrize("workspace", [True, False])
 def test_splits(workspace):  # parts of a length that is no multiple of a pass
     run(70, 5003, 4, 1, workspace=workspace)
@@ -86,4 +101,5 @@ def test_splits(workspace):  # parts of a length that is no multiple of a pass
 @pytest.mark.parametrize("softcap,spread,gain,q_dtype", [(50.0, 1.0, 1.0, torch.float16), (5.0, 4.0, 1.0, torch.bfloat16), (300.0, 1.0, 1.0, torch.bfloat16),
                                                          (0.0, 4.0, 8.0, torch.float16), (0.0, 0.05, 1.0, torch.bfloat16)])
 def test_scores(softcap, spread, gain, q_dtype):
+    run(200, 400, 8, 4, softcap=softcap, spread=spread, gain=gain, q_dtype=q_dtype, workspace=False)
     run(200, 1500, 8, 4, softcap=softcap, spread=spread, gain=gain, q_dtype=q_dtype)

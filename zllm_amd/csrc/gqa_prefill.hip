@@ -27,7 +27,7 @@
 // (running maximum, V window) is only touched when some lane's score passes it.
 #include <type_traits>
 
-#include "gqa_prefill.hpp"
+#include "gqa_prefill_f16_256.hpp"
 
 namespace zllm {
 
@@ -798,9 +798,19 @@ template <int D> struct TileShape {
     __device__ static __forceinline__ unsigned int swizzle(unsigned int row) { return swz(row) & (unsigned int)(kChunks - 1); }
 };
 
+// Keys of a workgroup's walk from which the halves of gqa_prefill_f16_256.hpp pay for their prologue and their meeting, some 3.5 us a workgroup: 8 %
+// less a tile.  Us a call, tiles / halves / by this line (16 / 4 heads of 256): segments of 50, 8,000 rows 89 / 104 / 89; of 200, 4,100 rows
+// 79 / 81 / 79; of 400, 2,000 rows 65 / 66 / 64; of 800, 4,100 rows 156 / 140 / 140; of 2,000, 8,000 rows 454 / 395 / 396; 1,097 causal rows
+// (16 / 8, three parts of up to 384 keys a row tile) 62 / 67 / 62.  A line of 512 costs segments of 200, whose row tiles meet two or three
+// of them, 12 %; 640 segments of 800 4 %.
+constexpr unsigned int kHalvesKeys = 576;
+
 // KV: 0 = Q8g64 (SDT names the scale type: bf16, f16 or f32), 1 = f16 rows
 // CT: 16-column MFMA tiles per wave, TileShape<D>::kCT or, for f16 rows at head_dim 128, one (gqa_prefill_tile_pairs)
-template <int D, int KV, int SDT, bool SOFTCAP, bool POW2, int CT = TileShape<D>::kCT>
+// HALVES: f16 rows of head_dim 256 in pages that can be addressed by scalars; a walk of kHalvesKeys and more runs in two halves
+// (0 no soft cap, 1 and 2 the forms of it in gqa_prefill_f16_256.hpp).  The walk is known here and not on the host: given ranges may be as long
+// as the rows or a few keys.  -1 for all other calls
+template <int D, int KV, int SDT, bool SOFTCAP, bool POW2, int CT = TileShape<D>::kCT, int HALVES = -1>
 __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
 {
     using C = TileShape<D>;
@@ -817,7 +827,12 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
         unsigned char k[4][C::kTile];
         unsigned char v[4][C::kTile];
     };
-    __shared__ __align__(16) Lds lds;
+    union WithHalves {
+        Lds tiles;
+        halves256::Shared halves;
+    };
+    __shared__ __align__(16) std::conditional_t<(HALVES >= 0), WithHalves, Lds> shared;
+    Lds& lds = (Lds&)shared;
     auto& lds_k = lds.k;
     auto& lds_v = lds.v;
     auto& lds_ks = lds.ks;
@@ -860,6 +875,12 @@ __global__ __launch_bounds__(512) void gqa_prefill_tiles(GqaPrefillParams p)
             }
         }
         return;
+    }
+    if constexpr (HALVES >= 0) {
+        if (part.end - part.begin >= kHalvesKeys) {
+            halves256::attend_part<HALVES>(p, shared.halves, part, t_end);
+            return;
+        }
     }
     const unsigned int steps = (part.end - part.begin + kStep - 1) / kStep;
 
@@ -1402,6 +1423,20 @@ template <int D, int KV, int SDT, int CT = TileShape<D>::kCT> static hipError_t 
     return hipGetLastError();
 }
 
+static hipError_t launch_prefill_halves(const GqaPrefillParams& p, hipStream_t stream)
+{
+    const unsigned int rows_per_wg = p.group >= 128u ? 1u : 128u / p.group;
+    const dim3 grid((p.rows + rows_per_wg - 1) / rows_per_wg * p.num_kv_heads, 1, p.max_chunks > 1u ? p.max_chunks : 1u);
+    if (!(p.softcap > 0.0f)) {
+        gqa_prefill_tiles<256, 1, 0, false, true, 1, 0><<<grid, dim3(512), 0, stream>>>(p);
+    } else if (p.softcap < 256.0f) {
+        gqa_prefill_tiles<256, 1, 0, true, true, 1, 1><<<grid, dim3(512), 0, stream>>>(p);
+    } else {
+        gqa_prefill_tiles<256, 1, 0, true, true, 1, 2><<<grid, dim3(512), 0, stream>>>(p);
+    }
+    return hipGetLastError();
+}
+
 } // namespace
 
 // More tiles of 128 pairs than two rounds of one workgroup a compute unit, f16 rows of head_dim 128: the kernel of which three
@@ -1521,15 +1556,14 @@ unsigned int gqa_prefill_staged_tiles(unsigned int rows, unsigned int position, 
     return gqa_prefill_staged_bytes(tiles, num_kv_heads) <= (1ull << 30) ? tiles : 0u;
 }
 
-// f16 rows of head_dim 256: the kernel of two halves (gqa_prefill_f16_256.hip) where a row tile is full and its walk pays for their
-// meeting.  Us a call, tiles / halves (16 / 8 heads; with a window of 1,024 and a soft cap, a layer of each): 2,048 rows behind 6,144 keys
-// 437 / 391, 4,096 behind none 367 / 341, 1,000 104 / 97, 700 behind 5,000 208 / 198, 300 behind 30,000 319 / 303; one full layer, 200
-// behind 3,000 (parts of 400 keys) 43.8 / 44.0, behind 5,500 58.6 / 54.8, 400 behind none 36.2 / 35.9; but 100 behind none 34.0 / 37.4,
-// and 30 rows, half a tile, behind 10,000 56.6 / 65.4.  Runs of sixteen rows lie in one page; other pages keep the tiles, an address a lane.
-static bool gqa_prefill_takes_f16_256(const GqaPrefillParams& p, bool scalar_pages)
+// f16 rows of head_dim 256: the kernel that may walk in two halves (gqa_prefill_f16_256.hpp), where a row tile is full and some walk can be long
+// enough.  Us a call, tiles / halves (16 / 8 heads; with a window of 1,024 and a soft cap, a layer of each): 2,048 rows behind 6,144 keys
+// 436 / 387, 4,096 behind none 369 / 340, 700 behind 5,000 208 / 198, 300 behind 30,000 322 / 302; but 30 rows, half a tile, behind
+// 10,000 56.6 / 65.4.  Runs of sixteen rows lie in one page; other pages keep the tiles, an address a lane.
+static bool gqa_prefill_takes_halves(const GqaPrefillParams& p, bool scalar_pages)
 {
     const unsigned long long keys = p.window != 0u ? min((unsigned long long)p.window, (unsigned long long)p.position + p.rows) : (unsigned long long)p.position + p.rows;
-    return scalar_pages && p.block_tokens >= 16u && p.q_dtype != 0 && p.group <= 128u && (unsigned long long)p.rows * p.group >= 128u && keys >= 256u;
+    return scalar_pages && p.block_tokens >= 16u && p.q_dtype != 0 && p.group <= 128u && (unsigned long long)p.rows * p.group >= 128u && keys >= kHalvesKeys;
 }
 
 hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scale_dtype, hipStream_t stream)
@@ -1547,8 +1581,8 @@ hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scal
         if (p.head_dim == 128u) {
             return launch_prefill_tiles<128, 1, 0>(p, stream);
         }
-        if (p.head_dim == 256u && gqa_prefill_takes_f16_256(p, scalar_pages)) {
-            return launch_gqa_prefill_f16_256(p, stream);
+        if (p.head_dim == 256u && gqa_prefill_takes_halves(p, scalar_pages)) {
+            return launch_prefill_halves(p, stream);
         }
         if (p.head_dim == 256u) {
             return launch_prefill_tiles<256, 1, 0>(p, stream);

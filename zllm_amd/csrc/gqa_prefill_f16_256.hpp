@@ -1,4 +1,4 @@
-// Chunked-prefill GQA attention over f16 rows at head_dim 256: what it computes is gqa_prefill_tiles (gqa_prefill.hip), for pages that it can
+// Chunked-prefill GQA attention over f16 rows at head_dim 256: the long walks of gqa_prefill_tiles (gqa_prefill.hip, kHalvesKeys), over pages that it can
 // address by scalars (sixteen tokens at least, see prefill_scalar_pages).
 //
 // A workgroup is 128 (row, head-in-group) pairs, as there: the models of this head dimension have few query heads a KV head, and tiles of 256
@@ -12,11 +12,15 @@
 // other's (46 % and 47 % of the cycles); what hides is what stands between a wave's own matrix instructions: with the exponentials
 // of a tile's second sixteen tokens under the first sixteen's products 407 -> 391.  Tried: the odd half half a pass behind
 // (spills in the loop, 457), raised priority for either phase (level), 64 pairs a wave and one wave a SIMD (70 spills).
+#pragma once
+
 #include "gqa_prefill_x32.hpp"
 
 namespace zllm {
 
 namespace {
+
+namespace halves256 {
 
 constexpr int kD = 256;
 constexpr int kRow = kD * 2;         // bytes of one token of one KV head
@@ -36,20 +40,22 @@ constexpr int kLoads = 4;            // loads a wave issues per plane and pass
 // row's tokens, sixteen of each second tile, as in gqa_prefill_tiles.  With a sixteenth 403 -> 413 us.
 constexpr float kLoShare = 8.0f;
 
+struct Lds {
+    unsigned char tile[2][kHalves][2][kTile]; // [buffer][half][K, V]
+};
+struct Meeting { // of the halves, over the tiles
+    float acc[kD / 32 * 4][kWaves][64][4];
+    float stats[2][kWaves][64];
+};
+union Shared {
+    Lds lds;
+    Meeting meeting;
+};
+
+// One workgroup of 512 threads: keys [part.begin, part.end) of a row tile whose visible range ends at t_end.
 // SOFTCAP: 0 none, 1 caps below 256, 2 larger ones (see gqa_prefill_f16)
-template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves * kHalves, 2) void gqa_prefill_f16_256(GqaPrefillParams p)
+template <int SOFTCAP> __device__ __forceinline__ void attend_part(const GqaPrefillParams& p, Shared& shared, const SplitRange& part, unsigned int t_end)
 {
-    struct Lds {
-        unsigned char tile[2][kHalves][2][kTile]; // [buffer][half][K, V]
-    };
-    struct Meeting { // of the halves, over the tiles
-        float acc[kD / 32 * 4][kWaves][64][4];
-        float stats[2][kWaves][64];
-    };
-    __shared__ __align__(1024) union {
-        Lds lds;
-        Meeting meeting;
-    } shared;
     Lds& lds = shared.lds;
 
     const unsigned int tid = threadIdx.x;
@@ -71,18 +77,13 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves * kHalves, 2) vo
     const unsigned int last_row = min(row0 + rows_per_wg, p.rows) - 1u;
 
     // ---- given ranges, then the query's rows, are requested before anything waits ----
-    unsigned int own_end = 0, own_start = 0, union_end = 0, union_start = 0xffffffffu;
+    unsigned int own_end = 0, own_start = 0;
     if (p.visible_ends != nullptr) {
-        const unsigned int lane_row = min(row0 + lane, last_row), own_row = min(col_row, last_row);
-        const unsigned int lane_end = p.visible_ends[lane_row], end = p.visible_ends[own_row];
-        unsigned int lane_start = 0;
+        const unsigned int own_row = min(col_row, last_row);
+        own_end = min(p.visible_ends[own_row], p.position + p.rows);
         if (p.visible_starts != nullptr) {
-            lane_start = p.visible_starts[lane_row];
             own_start = p.visible_starts[own_row];
         }
-        own_end = min(end, p.position + p.rows);
-        union_end = min(lane_end, p.position + p.rows);
-        union_start = min(lane_start, union_end);
     }
     Frag qf[kD / 16];
     {
@@ -95,35 +96,6 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves * kHalves, 2) vo
             }
         }
     }
-    unsigned int t_end = p.position + last_row + 1u;
-    unsigned int t_begin = 0;
-    if (p.window != 0) {
-        const unsigned int first_pos = p.position + row0 + 1u;
-        t_begin = first_pos > p.window ? first_pos - p.window : 0u;
-    }
-    if (p.visible_ends != nullptr) { // the union over the rows; a lane has taken one of the first 64
-        for (unsigned int r = row0 + 64u + lane; r <= last_row; r += 64u) {
-            const unsigned int end = min(p.visible_ends[r], p.position + p.rows);
-            union_end = max(union_end, end);
-            if (p.visible_starts != nullptr) {
-                union_start = min(union_start, min(p.visible_starts[r], end));
-            }
-        }
-        if (p.visible_starts != nullptr) {
-            t_end = wave_max_u(union_end);
-            t_begin = wave_min_u(union_start);
-        } else {
-            t_end = max(t_end, wave_max_u(union_end));
-        }
-    }
-    t_begin &= ~31u;
-    const SplitRange part = split_range(p, t_begin, t_end);
-    if (!part.live) {
-        if (col_valid && h == 0u && half == 0u) {
-            store_empty_record(p, col_row, col_head);
-        }
-        return;
-    }
     const unsigned int passes = (part.end - part.begin + kPass - 1) / kPass;
 
     // ---- staging.  Wave (half, quarter) requests pairs 4 quarter .. + 4 of its half's tile: tokens 8 e + 4 (lane / 32) + q of a run of
@@ -131,8 +103,7 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves * kHalves, 2) vo
     const unsigned int k_row = p.num_kv_heads * kRow;
     const unsigned int last_token = max(t_end, 1u) - 1u;
     const unsigned int q0 = 2u * (quarter & 1u);
-    const unsigned int lane_col = (c ^ h) * 16u + kvh * kRow;
-    const unsigned int lane_at = lane_col + 4u * h * k_row;
+    const unsigned int lane_at = (c ^ h) * 16u + kvh * kRow + 4u * h * k_row;
     const unsigned int lds_base = (unsigned int)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&lds;
     const unsigned int lds_to = lds_base + half * (2 * kTile) + 4u * quarter * kPairStride;
     auto first_of = [&](unsigned int t0) __attribute__((always_inline)) -> unsigned int { // of the wave's run, inside the range
@@ -154,7 +125,8 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves * kHalves, 2) vo
             const unsigned int token = 8u * (u & 1) + q0 + (u >> 1);
             unsigned int from = lane_at + token * k_row;
             if (!whole) {
-                from = lane_col + min(token + 4u * h, left) * k_row;
+                const unsigned int l = fresh_lane(), lh = l >> 5;
+                from = ((l & 31u) ^ lh) * 16u + kvh * kRow + min(token + 4u * lh, left) * k_row;
             }
             load_to_lds<true, 0>(kp, from, to + u * kPairStride);
             load_to_lds<true, kTile>(vp, from, to + u * kPairStride);
@@ -292,9 +264,10 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves * kHalves, 2) vo
             }
         }
         if (t0 + kStep > wave_min_hi || t0 < wave_max_lo) { // only steps at an edge of some column need the per-token masks
+            const unsigned int first = t0 + (fresh_lane() >> 5) * 4u;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const unsigned int token = t0 + 8u * (i >> 2) + 4u * h + (i & 3);
+                const unsigned int token = first + 8u * (i >> 2) + (i & 3);
                 s[i] = (token >= vis_lo && token < vis_hi) ? s[i] : kNegInf;
             }
         }
@@ -444,21 +417,8 @@ template <int SOFTCAP> __global__ __launch_bounds__(64 * kWaves * kHalves, 2) vo
     store_column<kD>(p, col_row, col_head, h, common, total, acc, kPBias);
 }
 
-} // namespace
+} // namespace halves256
 
-hipError_t launch_gqa_prefill_f16_256(const GqaPrefillParams& p, hipStream_t stream)
-{
-    const unsigned int rows_per_wg = p.group >= (unsigned int)kPairs ? 1u : (unsigned int)kPairs / p.group;
-    const dim3 grid((p.rows + rows_per_wg - 1) / rows_per_wg * p.num_kv_heads, 1, p.max_chunks > 1u ? p.max_chunks : 1u);
-    const dim3 block(64 * kWaves * kHalves);
-    if (!(p.softcap > 0.0f)) {
-        gqa_prefill_f16_256<0><<<grid, block, 0, stream>>>(p);
-    } else if (p.softcap < 256.0f) {
-        gqa_prefill_f16_256<1><<<grid, block, 0, stream>>>(p);
-    } else {
-        gqa_prefill_f16_256<2><<<grid, block, 0, stream>>>(p);
-    }
-    return hipGetLastError();
-}
+} // namespace
 
 } // namespace zllm

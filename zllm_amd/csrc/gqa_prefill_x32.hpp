@@ -19,6 +19,14 @@ __device__ __forceinline__ unsigned int swizzle(unsigned int row)
     return ((row & 1u) << 3) | ((row & 2u) << 1) | ((row >> 2) & 3u);
 }
 
+// The lane number again, for places off the main path: what is formed from it there takes no register of the loop around them
+__device__ __forceinline__ unsigned int fresh_lane()
+{
+    unsigned int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
 // Reduction over a wave inside the vector ALU: rows of sixteen lanes by rotation, then across the rows
 template <class Op> __device__ __forceinline__ unsigned int wave_reduce(unsigned int v, Op op)
 {

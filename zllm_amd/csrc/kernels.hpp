@@ -226,9 +226,6 @@ hipError_t launch_gqa_prefill(const GqaPrefillParams& p, int kv_format, int scal
 // f16 rows at head_dim 128 in tiles of 128 pairs (gqa_prefill_f16.hip): 16-bit queries, no sliding window, prefill_scalar_pages; the
 // caller has looked at all three
 hipError_t launch_gqa_prefill_f16(const GqaPrefillParams& p, hipStream_t stream);
-// f16 rows at head_dim 256 (gqa_prefill_f16_256.hip): 16-bit queries, prefill_scalar_pages of at least sixteen tokens, at most 128 query
-// heads a KV head; the caller has looked at all three
-hipError_t launch_gqa_prefill_f16_256(const GqaPrefillParams& p, hipStream_t stream);
 // Q8g64 rows of head_dim 128 converted once a call (gqa_prefill_staged.hip): 16-bit queries, causal or sliding rows; the caller has looked
 // at both, and at the workspace for the tiles
 hipError_t launch_gqa_prefill_staged(const GqaPrefillParams& p, int scale_dtype, hipStream_t stream);
