@@ -44,6 +44,28 @@ def test_which_calls_ask_for_staged_latents():
     assert staged_bytes(16, 1000, 850000) > 0 and staged_bytes(16, 1000, 870000) == 0  # at most 1 GiB
 
 
+def test_few_rows_over_many_tokens_are_not_staged():
+    """Converting a token costs about as much as attending to it with four rows of 16 heads: speculated tokens and short chunks stay out, alone
+    and in batches, and so do ragged batches whose records follow the tokens there are."""
+    assert staged_bytes(16, 4, 64000, 8) == staged_bytes(16, 3, 48000, 16) == staged_bytes(16, 4, 300000) == staged_bytes(32, 8, 64000, 8) == 0
+    assert staged_bytes(16, 16, 64000, 8) > 0 < staged_bytes(16, 16, 300000)
+    ragged = dict(total_ctx_tokens=101500)
+    assert staged_bytes(16, 8, 100000, 4, **ragged) == staged_bytes(64, 4, 100000, 4, **ragged) == 0 < staged_bytes(16, 32, 100000, 4, **ragged)
+
+
+@pytest.mark.parametrize("heads,rows,length", [(128, 300, 1400), (128, 850, 1150), (32, 700, 1500)])
+def test_splits_have_to_save_more_than_their_records_cost(heads, rows, length):
+    """Some more than one round of workgroups with two splits' worth of keys: unsplit."""
+    args = chunk_args(heads, rows, length)
+    assert staged_bytes(heads, rows, length) > 0
+    from zllm_amd import capi
+
+    args.workspace_bytes = capi.load().zllm_attn_mla_decode_preferred_bytes(C.byref(args))
+    layout = capi.SplitRecordLayout()
+    capi.check(capi.load().zllm_attn_mla_decode_record_layout(C.byref(args), C.byref(layout)))
+    assert layout.max_chunks == 1 and layout.record_rows == rows
+
+
 def record_layout(args):
     from zllm_amd import capi
 

@@ -411,28 +411,64 @@ MlaWorkspace mla_workspace(const zllm_mla_decode_args* a, const MlaSplitPlan& pl
 }
 
 // A chunk over latents that are converted once (mla_staged.hip): its splits, and the 32-token tiles a sequence.  0 tiles for other calls.
-// A compute unit takes a tile for 128 (row, head) pairs in 2.15 us there; mla_partial_ws takes it for 64 heads of one row in 1.42 us and for
-// up to 32 in 1.05.  The staging is a launch, and as many workgroups leave twice the records: the difference has to come to some 31 us over 256
-// compute units.  Us a call without / with: 128 heads, 20 rows behind 10,000 keys 109 / 116, 500 behind none 171 / 163, 512 behind
-// 16,384 2,824 / 2,330; 64 heads, 16 behind 30,000 116 / 133, 100 behind 3,000 115 / 107, 1,000 behind 8,000 1,504 / 1,239; 32 heads, 64
-// behind 4,000 69 / 75, behind 30,000 287 / 194, 1,000 behind none 157 / 137; 16 heads, 32 behind 8,000 58 / 66, 300 behind none 60 / 62,
-// behind 3,000 193 / 99, 1,000 behind 2,000 378 / 167.  The tiles are bounded by 1 GiB, 856,000 tokens.
+// Us a call without / with, 16 heads: 8 sequences of 64,000 tokens, 4 rows 282 / 481 (the conversion costs more than the rows save), 16 rows 1,053 /
+// 630; 300 rows behind 3,000 193 / 99; 32 heads: 64 rows behind 30,000 287 / 194, behind 4,000 69 / 75; 64 heads: 16 rows behind 64,000 199 / 214,
+// 1,000 behind 8,000 1,504 / 1,239; 128 heads: 512 behind 16,384 2,824 / 2,330, 20 behind 10,000 109 / 116.  Splits that only fill the
+// last round cost more in records than they save: 300 rows of 128 heads behind 1,100 keys 273 without, 342 in three splits, 244 in
+// one; 850 behind 300 431, 612, 403.  Over 590 shapes of 2 to 1,024 rows the estimate below is wrong by up to 4 % where it takes a call
+// (64 heads, 700 rows behind 2,500 444 / 464) and by 9 % where it does not (128 rows of 32 behind 4,000 99 / 90).
 uint32_t plan_mla_staged(const zllm_mla_decode_args* a, MlaSplitPlan* plan)
 {
     const uint64_t rows = mla_query_rows(a);
     if (a->latent_dim != 512u || a->rope_dim != 64u || a->selection != nullptr || rows < 2u) {
         return 0;
     }
+    const MlaSplitPlan plain = plan_mla_decode(a);
     const uint32_t heads_here = a->heads < 128u ? a->heads : 128u;
     const uint64_t units = (rows + 128u / heads_here - 1u) / (128u / heads_here) * a->batch * ((a->heads + heads_here - 1u) / heads_here);
+    const uint64_t plain_units = rows * a->batch * ((a->heads + 63u) / 64u);
     const uint64_t tiles = ((uint64_t)a->max_ctx_len + 31u) / 32u;
-    const uint64_t steps = (a->max_ctx_len - (a->max_ctx_len < rows ? a->max_ctx_len : rows) / 2u) / 32u; // of a middle row
-    const uint64_t there = 215u * units, here = (a->heads <= 32u ? 105u : 142u) * rows * a->batch * ((a->heads + 63u) / 64u);
-    if (here <= there || steps * (here - there) < 800000u || units > 65535u || zllm::mla_staged_bytes((uint32_t)tiles, a->batch) > (1ull << 30)) {
+    if (plain.dense || units > 65535u) { // dense: a ragged batch of few rows, whose records and workgroups follow the tokens there are
+        return 0;
+    }
+    // What both take, in us.  A compute unit walks a token for 128 (row, head) pairs in 67 ns here, for 64 heads of one row in 44 and for up to
+    // 32 in 36 (mla_partial_ws); a workgroup's ends are worth 64 tokens of its walk; a record is written and read at 4 TB/s; converting a token
+    // takes 0.65 ns, and 10 us whatever is converted.
+    const double cus = compute_units(), batch = a->batch, longest = a->max_ctx_len;
+    const bool ragged = a->total_ctx_tokens != 0 && a->total_ctx_tokens < batch * longest;
+    const double context = ragged ? a->total_ctx_tokens / batch : longest; // of the mean sequence
+    const double mean = context - (rows < context ? rows : context) / 2;   // of its middle row
+    const double record_us = batch * rows * a->heads * 4112.0 / 4e6;       // a split
+    auto attention_us = [&](uint64_t groups, uint32_t chunk, uint32_t splits, double ns) {
+        const double walk = (double)(chunk < a->max_ctx_len ? chunk : a->max_ctx_len) + 64;
+        if (ragged) { // the work there is, and half of a longest walk that starts late
+            return (groups * mean / cus + walk / 2) * ns / 1e3 + splits * record_us;
+        }
+        const double rounds = (double)((groups * splits + (uint64_t)cus - 1) / (uint64_t)cus);
+        return rounds * walk * (mean / longest) * ns / 1e3 + splits * record_us;
+    };
+    double here_us = 0;
+    for (uint32_t rounds = 0; rounds <= 8; ++rounds) { // one split, or those that fill 1, 2, ... rounds (see plan_splits)
+        const uint64_t per_unit = rounds == 0 ? 1 : rounds * (uint64_t)cus / units;
+        if (per_unit == 0) {
+            continue;
+        }
+        uint64_t chunk = (a->max_ctx_len + per_unit - 1) / per_unit;
+        chunk = align_up(chunk < 64 ? 64 : chunk, 32);
+        const uint32_t splits = (uint32_t)((a->max_ctx_len + chunk - 1) / chunk);
+        const double us = attention_us(units, (uint32_t)chunk, splits, 67);
+        if (rounds == 0 || us < here_us) {
+            here_us = us;
+            plan->chunk_tokens = (uint32_t)chunk;
+            plan->max_chunks = splits;
+        }
+    }
+    const double plain_us = attention_us(plain_units, plain.chunk_tokens, plain.max_chunks, a->heads <= 32u ? 36 : 44);
+    const double convert_us = 10 + 0.65e-3 * batch * context;
+    if (here_us + convert_us >= plain_us || zllm::mla_staged_bytes((uint32_t)tiles, a->batch) > (1ull << 30)) {
         return 0;
     }
     plan->dense = false;
-    plan_splits(a->max_ctx_len, units, 1, 64, &plan->chunk_tokens, &plan->max_chunks);
     plan->record_rows = (uint64_t)a->batch * rows * plan->max_chunks;
     return (uint32_t)tiles;
 }
