@@ -44,6 +44,18 @@ def test_which_calls_ask_for_staged_latents():
     assert staged_bytes(16, 1000, 850000) > 0 and staged_bytes(16, 1000, 870000) == 0  # at most 1 GiB
 
 
+def test_the_preferred_workspace_is_at_most_a_gigabyte_more():
+    """Tiles and records together, over shapes drawn up to where the bound bites; the four are some that went beyond it."""
+    rng = np.random.default_rng(7)
+    shapes = [(8, 208, 213548, 4), (4, 2093, 844747, 1), (128, 23, 835389, 1), (16, 1000, 850000, 1)]
+    for _ in range(4000):
+        batch = int(np.exp(rng.uniform(0, np.log(32))))
+        rows = min(int(np.exp(rng.uniform(np.log(2), np.log(8000)))), 65535 // batch)
+        shapes.append((int(rng.choice([1, 4, 8, 16, 32, 64, 128, 200])), rows, int(np.exp(rng.uniform(np.log(500), np.log(1e6)))), batch))
+    more = np.array([staged_bytes(*shape) for shape in shapes])
+    assert more.max() <= 1 << 30 and np.count_nonzero(more > 900 << 20) > 10
+
+
 def test_few_rows_over_many_tokens_are_not_staged():
     """Converting a token costs about as much as attending to it with four rows of 16 heads: speculated tokens and short chunks stay out, alone
     and in batches, and so do ragged batches whose records follow the tokens there are."""

@@ -447,7 +447,10 @@ uint32_t plan_mla_staged(const zllm_mla_decode_args* a, MlaSplitPlan* plan)
         const double rounds = (double)((groups * splits + (uint64_t)cus - 1) / (uint64_t)cus);
         return rounds * walk * (mean / longest) * ns / 1e3 + splits * record_us;
     };
+    // Room beside what the call needs anyway: at most 1 GiB (856,000 tokens), by fewer splits where there is a choice
+    const uint64_t tile_bytes = zllm::mla_staged_bytes((uint32_t)tiles, a->batch), least = mla_workspace(a, plain).total;
     double here_us = 0;
+    plan->max_chunks = 0;
     for (uint32_t rounds = 0; rounds <= 8; ++rounds) { // one split, or those that fill 1, 2, ... rounds (see plan_splits)
         const uint64_t per_unit = rounds == 0 ? 1 : rounds * (uint64_t)cus / units;
         if (per_unit == 0) {
@@ -456,21 +459,19 @@ uint32_t plan_mla_staged(const zllm_mla_decode_args* a, MlaSplitPlan* plan)
         uint64_t chunk = (a->max_ctx_len + per_unit - 1) / per_unit;
         chunk = align_up(chunk < 64 ? 64 : chunk, 32);
         const uint32_t splits = (uint32_t)((a->max_ctx_len + chunk - 1) / chunk);
+        MlaSplitPlan cut = {(uint32_t)chunk, splits, (uint64_t)a->batch * rows * splits, false};
+        if (align_up(mla_workspace(a, cut).total, 256) + tile_bytes > least + (1ull << 30)) {
+            continue;
+        }
         const double us = attention_us(units, (uint32_t)chunk, splits, 67);
-        if (rounds == 0 || us < here_us) {
+        if (plan->max_chunks == 0 || us < here_us) {
             here_us = us;
-            plan->chunk_tokens = (uint32_t)chunk;
-            plan->max_chunks = splits;
+            *plan = cut;
         }
     }
     const double plain_us = attention_us(plain_units, plain.chunk_tokens, plain.max_chunks, a->heads <= 32u ? 36 : 44);
     const double convert_us = 10 + 0.65e-3 * batch * context;
-    if (here_us + convert_us >= plain_us || zllm::mla_staged_bytes((uint32_t)tiles, a->batch) > (1ull << 30)) {
-        return 0;
-    }
-    plan->dense = false;
-    plan->record_rows = (uint64_t)a->batch * rows * plan->max_chunks;
-    return (uint32_t)tiles;
+    return plan->max_chunks == 0 || here_us + convert_us >= plain_us ? 0u : (uint32_t)tiles;
 }
 
 // What a call runs with: its splits, where its arrays lie, and for chunks over converted latents their tiles, behind the arrays.
