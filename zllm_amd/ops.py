@@ -34,6 +34,17 @@ def _dev(t, name):
     return t
 
 
+def _workspace(preferred, least_of, args, device):
+    """Device memory of the size with which a call is fastest, or of the least with which it runs where the device has not that much left."""
+    try:
+        return torch.empty(preferred, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        least = least_of(C.byref(args))
+        if least >= preferred:
+            raise
+    return torch.empty(max(least, 256), dtype=torch.uint8, device=device)
+
+
 def init(device: int = 0) -> int:
     cu = C.c_int(0)
     capi.check(capi.load().zllm_attn_init(device, C.byref(cu)))
@@ -161,8 +172,9 @@ def gqa_prefill_chunk_args(q, k_plane, k_scales, v_plane, v_scales, table, posit
     args.table_stride = 0 if table is None else table.numel()
     scratch = None
     if workspace:
-        need = capi.load().zllm_attn_gqa_prefill_preferred_bytes(C.byref(args))
-        scratch = torch.empty(max(int(need), 256), dtype=torch.uint8, device=q.device)
+        lib = capi.load()
+        need = max(lib.zllm_attn_gqa_prefill_preferred_bytes(C.byref(args)), 256)
+        scratch = _workspace(need, lib.zllm_attn_gqa_prefill_workspace_bytes, args, q.device)
         args.workspace, args.workspace_bytes = _ptr(scratch), scratch.numel()
     return args, out, scratch
 
@@ -210,7 +222,7 @@ def mla_decode_args(q, kv_b, latent_codes, latent_scales, rope_cache, tables, ct
     if query_rows > 1:
         need = lib.zllm_attn_mla_decode_preferred_bytes(C.byref(args))
     if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        workspace = _workspace(need, lib.zllm_attn_mla_decode_workspace_bytes, args, q.device)
     args.workspace, args.workspace_bytes = _ptr(workspace), workspace.numel()
     if workspace.numel() >= need > least:  # the number asks for the larger workspace's plan
         args.workspace_bytes = need
