@@ -847,6 +847,75 @@ static void test_steady_state_counters(const RocmContext& ctx)
     CHECK(ctx.synchronize().is_ok(), "synchronize");
 }
 
+// Chunks take a larger workspace as an option: refused, the call runs with what it needs, and a prompt's chunks neither double it nor grow it
+// one by one.
+static void test_preferred_workspace()
+{
+    GqaSpec spec;
+    spec.num_heads = 16;
+    spec.num_kv_heads = 4;
+    spec.head_dim = 128;
+    spec.score_scale = 1.0f / sqrtf(128.0f);
+    MlaSpec mla;
+    mla.kv_lora_rank = 512;
+    mla.qk_rope_head_dim = 64;
+    mla.num_heads = 16;
+    mla.q_projection_size = mla.num_heads * 192;
+    mla.kv_projection_size = mla.num_heads * 256;
+    mla.q_lora_rank = 1536;
+    const size_t rows = 300, chunks = 6;
+    std::vector<float> outs[3];
+    size_t held[3] = {0, 0, 0};
+    for (int limited = 0; limited < 3; ++limited) { // no limit, none allowed, and 40 MiB, which hold the first chunks
+        std::mt19937 rng(59);
+        auto ctx_r = RocmContext::create(0);
+        CHECK(ctx_r.is_ok(), "context");
+        RocmContext ctx = ctx_r.unwrap();
+        if (limited != 0) {
+            CHECK(ctx.limit_preferred_workspace(limited == 1 ? 0 : 40u << 20).is_ok(), "limit");
+        }
+        RocmKvCache cache = RocmKvCache::new_gqa(1, 4, 128, 16, 2048, TablePolicy::Scrambled).unwrap();
+        RocmKvCache latents = RocmKvCache::new_mla(1, 512, 64, 64, 2048, TablePolicy::Scrambled).unwrap();
+        auto weight = ctx.prepare_mla_kv_b(randn(rng, mla.kv_projection_size * 512, true), mla.kv_projection_size, 512);
+        size_t allocations = 0;
+        for (size_t c = 0; c < chunks; ++c) {
+            auto q = ctx.tensor_from_f32(randn(rng, rows * 2048, true), rows, 2048, DType::BF16);
+            auto kv = ctx.tensor_from_f32(randn(rng, rows * 512, false), rows, 512);
+            auto rope = ctx.tensor_from_f32(randn(rng, rows * 64, false), rows, 64);
+            auto mq = ctx.tensor_from_f32(randn(rng, rows * mla.q_projection_size, true), rows, mla.q_projection_size, DType::BF16);
+            auto out = ctx.gqa_prefill_attention_cached(cache, 0, c * rows, q.unwrap(), kv.unwrap(), kv.unwrap(), spec, true);
+            auto mout = ctx.mla_prefill_attention(mq.unwrap(), kv.unwrap(), rope.unwrap(), weight.unwrap(), &latents, 0, mla);
+            CHECK(out.is_ok() && mout.is_ok(), "chunk %zu, workspace form %d: %s", c, limited,
+                  out.is_err() ? out.unwrap_err().to_string().c_str() : mout.is_err() ? mout.unwrap_err().to_string().c_str() : "");
+            if (out.is_err() || mout.is_err()) {
+                return;
+            }
+            for (const auto& t : {out.unwrap(), mout.unwrap()}) {
+                const auto x = ctx.tensor_to_f32(t).unwrap();
+                outs[limited].insert(outs[limited].end(), x.begin(), x.end());
+            }
+            const size_t now = ctx.counters().preferred_workspace_bytes;
+            allocations += now != held[limited];
+            held[limited] = now;
+        }
+        CHECK(limited != 0 || (held[0] >= 64u << 20 && held[0] % (64u << 20) == 0 && allocations <= 2), "preferred workspace %zu bytes after %zu growths", held[0],
+              allocations);
+        CHECK(ctx.limit_preferred_workspace(0).is_ok() && ctx.counters().preferred_workspace_bytes == 0, "given back");
+    }
+    CHECK(held[1] == 0 && held[2] > 0 && held[2] <= 40u << 20, "limits: %zu and %zu bytes held", held[1], held[2]);
+    double diff[2] = {0, 0}, norm = 0;
+    for (size_t i = 0; i < outs[0].size(); ++i) {
+        norm += (double)outs[0][i] * outs[0][i];
+        for (int n = 0; n < 2; ++n) {
+            const double d = (double)outs[n + 1][i] - outs[0][i];
+            diff[n] += d * d;
+        }
+    }
+    // f16 weights round 2^-12 a term, independently over the tokens; MLA chunks come back as bf16, 2^-9 a value where a rounding falls the other way
+    printf("preferred workspace: with / without %.3e, with / partly %.3e\n", sqrt(diff[0] / norm), sqrt(diff[1] / norm));
+    CHECK(norm > 0 && sqrt(diff[0] / norm) <= 1.0 / 512 && sqrt(diff[1] / norm) <= 1.0 / 512, "the workspace changes results");
+}
+
 // MLA at another latent / rope width with kv_b as W8A16 and W4A16 codes (RocmQuantizedWeight, src/backend/rocm/attention.rs:181-192):
 // the oracle gets the f32 values the codes stand for
 static void test_mla_other_widths_and_quantized_weights(const RocmContext& ctx)
@@ -949,6 +1018,7 @@ int main()
     test_block_attention(ctx.unwrap());
     test_mla_other_widths_and_quantized_weights(ctx.unwrap());
     test_steady_state_counters(ctx.unwrap());
+    test_preferred_workspace();
     printf(failures == 0 ? "ALL PASSED\n" : "%d FAILED\n", failures);
     return failures == 0 ? 0 : 1;
 }

@@ -391,7 +391,10 @@ struct RocmContext::Scratch {
     static constexpr size_t kStageBytes = 1 << 20;       // pinned ring for small arrays
     static constexpr size_t kPoolKeepBytes = 2ull << 30; // idle blocks kept beyond this are released
     hipStream_t stream = nullptr;
+    static constexpr size_t kPreferredStep = 64u << 20;  // a prompt's chunks prefer more and more: grown in steps, each waits for the stream
     DeviceBuffer workspace;
+    DeviceBuffer preferred;               // what chunks are fastest with, beside the workspace that they need otherwise
+    size_t preferred_limit = SIZE_MAX;    // sizes from here on are not asked for: the caller's limit, or refused by the device
     uint32_t* meta_host = nullptr; // pinned, kSlots records of four u32
     DeviceBuffer meta_dev;
     size_t next = 0;
@@ -485,7 +488,10 @@ Result<RocmContext> RocmContext::create(int device_id)
 
 HostCounters RocmContext::counters() const
 {
-    return scratch_->counters;
+    HostCounters now = scratch_->counters;
+    now.workspace_bytes = scratch_->workspace.bytes();
+    now.preferred_workspace_bytes = scratch_->preferred.bytes();
+    return now;
 }
 
 Result<Unit> RocmContext::wait_for_stream() const
@@ -660,6 +666,54 @@ Result<void*> RocmContext::workspace(size_t bytes) const
         s.workspace = grown.unwrap();
     }
     return s.workspace.data();
+}
+
+Result<RocmContext::Workspace> RocmContext::workspace(uint64_t least, uint64_t preferred) const
+{
+    Scratch& s = *scratch_;
+    if (preferred > least && preferred <= s.preferred_limit) {
+        if (preferred > s.preferred.bytes()) {
+            auto waited = wait_for_stream();
+            if (waited.is_err()) {
+                return waited.unwrap_err();
+            }
+            s.preferred = DeviceBuffer(); // given back first: old and new never add up
+            const size_t stepped = (preferred + Scratch::kPreferredStep - 1) / Scratch::kPreferredStep * Scratch::kPreferredStep;
+            auto grown = DeviceBuffer::allocate(std::min(stepped, s.preferred_limit));
+            if (grown.is_err()) {
+                (void)hipGetLastError(); // answered here: the next launch is not to find it
+                s.preferred_limit = (size_t)preferred - 1u;
+            } else {
+                ++s.counters.device_allocations;
+                s.preferred = grown.unwrap();
+            }
+        }
+        if (preferred <= s.preferred.bytes()) {
+            return Workspace{s.preferred.data(), preferred};
+        }
+    }
+    if (least == 0) {
+        return Workspace{nullptr, 0};
+    }
+    auto needed = workspace((size_t)least);
+    if (needed.is_err()) {
+        return needed.unwrap_err();
+    }
+    return Workspace{needed.unwrap(), least};
+}
+
+Result<Unit> RocmContext::limit_preferred_workspace(size_t bytes) const
+{
+    Scratch& s = *scratch_;
+    if (s.preferred.bytes() > bytes) {
+        auto waited = wait_for_stream();
+        if (waited.is_err()) {
+            return waited.unwrap_err();
+        }
+        s.preferred = DeviceBuffer();
+    }
+    s.preferred_limit = bytes;
+    return Unit{};
 }
 
 Result<const uint32_t*> RocmContext::upload_meta(const uint32_t (&values)[4]) const
@@ -984,15 +1038,12 @@ Result<RocmTensor> RocmContext::gqa_attend(const RocmKvCache& cache, size_t laye
     a.q_dtype = abi_dtype(query.dtype);
     a.out_dtype = ZLLM_DTYPE_F32;
     a.visible_ends = visible_ends_dev;
-    const uint64_t need = zllm_attn_gqa_prefill_preferred_bytes(&a);
-    if (need != 0) {
-        auto ws = workspace(need);
-        if (ws.is_err()) {
-            return ws.unwrap_err();
-        }
-        a.workspace = ws.unwrap();
-        a.workspace_bytes = need;
+    auto ws = workspace(zllm_attn_gqa_prefill_workspace_bytes(&a), zllm_attn_gqa_prefill_preferred_bytes(&a));
+    if (ws.is_err()) {
+        return ws.unwrap_err();
     }
+    a.workspace = ws.unwrap().data;
+    a.workspace_bytes = ws.unwrap().bytes;
     const int rc = zllm_attn_gqa_prefill_chunk(&a, stream_);
     if (rc != 0) {
         return abi_error("zllm_attn_gqa_prefill_chunk", rc);
@@ -1603,16 +1654,16 @@ Result<RocmTensor> RocmContext::mla_decode_impl(const RocmTensor& query, const R
         a.kv_b_group = (uint32_t)kv_b.group_size;
         a.kv_b_scale_dtype = kv_b.scale_dtype == DType::F32 ? ZLLM_SCALE_F32 : (kv_b.scale_dtype == DType::F16 ? ZLLM_SCALE_F16 : ZLLM_SCALE_BF16);
     }
-    const uint64_t need = zllm_attn_mla_decode_preferred_bytes(&a);
-    if (need == 0) {
-        return abi_error("zllm_attn_mla_decode_preferred_bytes", -1);
+    const uint64_t least = zllm_attn_mla_decode_workspace_bytes(&a);
+    if (least == 0) {
+        return abi_error("zllm_attn_mla_decode_workspace_bytes", -1);
     }
-    auto ws = workspace(need);
+    auto ws = workspace(least, chunk ? zllm_attn_mla_decode_preferred_bytes(&a) : least);
     if (ws.is_err()) {
         return ws.unwrap_err();
     }
-    a.workspace = ws.unwrap();
-    a.workspace_bytes = need;
+    a.workspace = ws.unwrap().data;
+    a.workspace_bytes = ws.unwrap().bytes;
     const int rc = zllm_attn_mla_decode(&a, stream_);
     if (rc != 0) {
         return abi_error("zllm_attn_mla_decode", rc);

@@ -235,6 +235,7 @@ struct HostCounters {
     size_t rope_table_uploads = 0;  // uploads of a cos/sin prefix
     size_t stream_waits = 0;        // hipStreamSynchronize calls made inside attention and append methods
     size_t staged_uploads = 0;      // small host arrays (visible ends, selections) sent through the pinned ring
+    size_t workspace_bytes = 0, preferred_workspace_bytes = 0; // held now: what calls need, and what chunks are fastest with
 };
 
 // One context drives one HIP stream and keeps that stream's scratch.  A context and its copies (they share the scratch)
@@ -245,6 +246,9 @@ class RocmContext {
   public:
     static Result<RocmContext> create(int device_id);
     HostCounters counters() const;
+    // Device memory that chunks may take to run faster (zllm_attn_*_preferred_bytes, up to 1 GiB more than they need): a call that would
+    // take more, or that the device refuses it, runs with what it needs.  Unlimited unless said otherwise; 0 gives back what is held.
+    Result<Unit> limit_preferred_workspace(size_t bytes) const;
     int device_id() const { return device_id_; }
     hipStream_t stream() const { return stream_; }
     Result<Unit> synchronize() const;
@@ -324,14 +328,20 @@ class RocmContext {
 
   private:
     // Device scratch of the context's stream, kept between calls: the split-KV workspace (grown when a call needs
-    // more), a ring of small metadata records (lengths, window starts) and a ring for small arrays (visible ends,
+    // more), the larger one that chunks prefer (optional), a ring of small metadata records (lengths, window starts) and a ring for small arrays (visible ends,
     // selections) that travel host -> device from pinned memory, a pool that output tensors and scratch planes are
     // taken from and returned to, an identity block table and the cos/sin tables already on the device -- so that a
     // call in steady state neither allocates nor waits for the stream.  Blocks are reused in stream order: everything
     // the context launches runs on its one stream, so a block that went back to the pool is next written by work
     // queued behind its last reader.
     struct Scratch;
+    struct Workspace {
+        void* data;
+        uint64_t bytes;
+    };
     Result<void*> workspace(size_t bytes) const;
+    // of `preferred` bytes where the device has them to spare, else of `least` (which may be 0)
+    Result<Workspace> workspace(uint64_t least, uint64_t preferred) const;
     Result<const uint32_t*> upload_meta(const uint32_t (&values)[4]) const;
     Result<DeviceBuffer> pooled(size_t bytes) const;
     Result<DeviceBuffer> upload_words(const uint32_t* words, size_t count) const;
