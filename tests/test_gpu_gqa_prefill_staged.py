@@ -32,6 +32,9 @@ def test_which_calls_ask_for_staged_rows():
     assert staged_bytes(65, 959, 32, 8) > 0 and staged_bytes(65, 960, 32, 8) == 0          # few tiles: up to 1,024 keys
     assert 0 < staged_bytes(400, 50000, 32, 8, window=600) < 8 * 33 * (tile + 256) + 9 * tile  # only what a window leaves
     assert staged_bytes(512, 240000, 32, 8) > 0 and staged_bytes(512, 260000, 32, 8) == 0  # at most 1 GiB
+    for scales in (capi.SCALE_F32, capi.SCALE_F16):  # few tiles: half of one has to be filled, whatever the scales
+        assert staged_bytes(31, 100, 32, 8, scale_dtype=scales) == 0 == staged_bytes(127, 500, 16, 16, scale_dtype=scales)
+        assert staged_bytes(33, 100, 32, 8, scale_dtype=scales) > 0 == staged_bytes(24, 8, 64, 8, scale_dtype=scales)
     for other in (dict(q_dtype=capi.DTYPE_F32), dict(kv_format=capi.KV_F16), dict(head_dim=64), dict(head_dim=256)):
         assert staged_bytes(2048, 50000, 32, 8, **other) == 0
     ends = (C.c_uint32 * 1)()

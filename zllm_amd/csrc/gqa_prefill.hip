@@ -1528,7 +1528,10 @@ unsigned int gqa_prefill_tile_pairs(unsigned int rows, unsigned int position, un
 //   behind 32,000: 200 rows 253 -> 244, 1,000 851 -> 741, 4,096 3,020 -> 2,532; 64 / 8, 1,000 rows behind 8,000 477 -> 389; 8 / 1, 2,100 behind
 //   8,000 271 -> 207; a window of 1,024 over 2,048 rows 112 -> 99.
 // The staging is a launch and a pass over the keys that few row tiles do not earn back: 80 rows of 32 / 8 (two tiles) 35.8 / 37.9 us behind 2,000,
-// 54 / 58 behind 8,000, of 64 / 8 (three) 225 / 235 behind 32,000; behind 600 keys they do, 48 -> 32.
+// 54 / 58 behind 8,000, of 64 / 8 (three) 225 / 235 behind 32,000; over 1,024 keys and less they do: 33 to 600 rows behind 0 to 900 keys in 175
+// shapes of 16-bit scales 36 -> 27 us a call, 0.60 to 1.05 of the time without.  f32 scales have full-size tiles whatever the rows: those
+// that fill half of one gain as much (33 rows of 32 / 8 behind 400 36 -> 26; 0.58 to 1.10), fewer lose (17 rows behind 100 13.6 / 14.7,
+// 48 of 16 / 16 behind 900 24 / 29), and so does a single tile of keys (24 first rows of 64 / 8 11.0 / 12.6).
 // The tiles are bounded by 1 GiB, 253,000 tokens of eight KV heads.
 // First chunks whose full-size tiles are at most a workgroup a compute unit have tiles of 128 pairs above and halves of the keys here: 32 / 8 heads,
 // 1,500 rows 92 -> 88, behind 300 keys 113 -> 104, 2,048 110 -> 99; 64 / 8, 1,000 rows 71 -> 67; 16 / 4, 4,000 rows 178 -> 150.  Below 1,000 keys the
@@ -1548,6 +1551,9 @@ unsigned int gqa_prefill_staged_tiles(unsigned int rows, unsigned int position, 
     }
     const unsigned int rows_per_tile = pairs / group, row_tiles = (rows + rows_per_tile - 1u) / rows_per_tile;
     const unsigned int begin = window != 0u && position + 1u > window ? position + 1u - window : 0u;
+    if ((unsigned long long)rows * group < 128u || end - begin <= (unsigned int)kStep) {
+        return 0;
+    }
     if (*halves ? (unsigned long long)row_tiles * num_kv_heads <= kComputeUnitsPrefill || end < 1000u : row_tiles < 4u && end - begin > 1024u) {
         return 0;
     }
