@@ -213,9 +213,9 @@ def test_later_stages_take_up_the_records_of_a_whole_call():
 
     heads, rows, lens = 16, 300, [2400, 1700]
     case = make_mla_chunk_case(3, lens, rows, heads, block_tokens=64)
-    keep = [upload(case[n]) for n in ("codes", "scales", "rope", "tables", "lens")]
-    weights, form = weight_args(case)
-    args, out, workspace = ops.mla_decode_args(to_torch_bf16(case["q_bits"], "cuda"), weights, *keep, heads, 192, 256, 512, 64, 64, max(lens),
+    keep = [upload(case[n]) for n in ("codes", "scales", "rope", "tables", "lens")]  # the argument block holds addresses only
+    q, (weights, form) = to_torch_bf16(case["q_bits"], "cuda"), weight_args(case)
+    args, out, workspace = ops.mla_decode_args(q, weights, *keep, heads, 192, 256, 512, 64, 64, max(lens),
                                                query_rows=rows, **form)
     lib = capi.load()
     preferred, least = args.workspace_bytes, lib.zllm_attn_mla_decode_workspace_bytes(C.byref(args))
