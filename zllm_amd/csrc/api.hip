@@ -449,8 +449,13 @@ uint32_t plan_mla_staged(const zllm_mla_decode_args* a, MlaSplitPlan* plan)
     };
     // Room beside what the call needs anyway: at most 1 GiB (856,000 tokens), by fewer splits where there is a choice
     const uint64_t tile_bytes = zllm::mla_staged_bytes((uint32_t)tiles, a->batch), least = mla_workspace(a, plain).total;
+    const double plain_us = attention_us(plain_units, plain.chunk_tokens, plain.max_chunks, a->heads <= 32u ? 36 : 44);
+    const double convert_us = 10 + 0.65e-3 * batch * context;
     double here_us = 0;
     plan->max_chunks = 0;
+    if (convert_us >= plain_us) {
+        return 0;
+    }
     for (uint32_t rounds = 0; rounds <= 8; ++rounds) { // one split, or those that fill 1, 2, ... rounds (see plan_splits)
         const uint64_t per_unit = rounds == 0 ? 1 : rounds * (uint64_t)cus / units;
         if (per_unit == 0) {
@@ -469,8 +474,6 @@ uint32_t plan_mla_staged(const zllm_mla_decode_args* a, MlaSplitPlan* plan)
             *plan = cut;
         }
     }
-    const double plain_us = attention_us(plain_units, plain.chunk_tokens, plain.max_chunks, a->heads <= 32u ? 36 : 44);
-    const double convert_us = 10 + 0.65e-3 * batch * context;
     return plan->max_chunks == 0 || here_us + convert_us >= plain_us ? 0u : (uint32_t)tiles;
 }
 
@@ -501,12 +504,15 @@ uint64_t plan_mla_preferred(const zllm_mla_decode_args* a, MlaCallPlan* plan)
 MlaCallPlan plan_mla_call(const zllm_mla_decode_args* a)
 {
     MlaCallPlan plan;
-    const uint64_t preferred = plan_mla_preferred(a, &plan);
-    if (preferred == 0 || a->workspace_bytes != preferred) {
-        plan.splits = plan_mla_decode(a);
-        plan.workspace = mla_workspace(a, plan.splits);
-        plan.staged_tiles = 0;
-        plan.staged_at = 0;
+    plan.splits = plan_mla_decode(a);
+    plan.workspace = mla_workspace(a, plan.splits);
+    plan.staged_tiles = 0;
+    plan.staged_at = 0;
+    if (a->workspace_bytes > plan.workspace.total) { // the preferred size is always beyond the least
+        MlaCallPlan preferred;
+        if (plan_mla_preferred(a, &preferred) == a->workspace_bytes) {
+            return preferred;
+        }
     }
     return plan;
 }

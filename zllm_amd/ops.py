@@ -219,7 +219,7 @@ def mla_decode_args(q, kv_b, latent_codes, latent_scales, rope_cache, tables, ct
     need = least = lib.zllm_attn_mla_decode_workspace_bytes(C.byref(args))
     if least == 0:
         raise capi.ZllmAttnError(-1, capi.last_error())
-    if query_rows > 1:
+    if query_rows > 1 and (workspace is None or workspace.numel() > least):
         need = lib.zllm_attn_mla_decode_preferred_bytes(C.byref(args))
     if workspace is None:
         workspace = _workspace(need, lib.zllm_attn_mla_decode_workspace_bytes, args, q.device)
