@@ -88,7 +88,7 @@ def test_given_ranges(given, position):
 
 # walks on both sides of the line in one launch: segments of 300, 60, none, 640, 6 and 150 rows, their row tiles across them, and ends inside a prefix
 @pytest.mark.parametrize("heads,kv_heads", [(8, 2), (16, 16), (6, 3)])
-@pytest.mark.parametrize("given,position,workspace", [("segments", 0, True), ("segments", 0, False), ("ends", 0, False), ("ends", 530, False), ("ends", 530, True)])
+@pytest.mark.parametrize("given,position,workspace", [("segments", 0, True), ("segments", 0, False), ("segments", 37, True), ("segments", 1100, False), ("ends", 0, False), ("ends", 530, False), ("ends", 530, True)])
 def test_given_ranges_of_both_lengths(heads, kv_heads, given, position, workspace):
     run(1406, position, heads, kv_heads, given=given, workspace=workspace)
 

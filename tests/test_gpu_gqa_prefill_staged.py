@@ -55,6 +55,7 @@ def test_which_calls_ask_for_staged_rows():
     (1200, 260, 8, 2, dict(softcap=30.0, rule=O.RULE_ROCM_MLA)),
     (800, 140, 8, 2, dict(softcap=400.0, rule=O.RULE_CUDA_GQA)),     # the precise form of the soft cap; f32 scales
     (2500, 200, 8, 2, dict(rule=O.RULE_ROCM_MLA, block_tokens=64, v_gain=2.0 ** np.repeat(np.arange(-10, 10), 135))),  # the V window moves on
+    (2500, 200, 8, 2, dict(rule=O.RULE_ROCM_MLA, block_tokens=64, v_gain=2.0 ** np.repeat(np.arange(20, 0, -1), 135))),  # and scales that fall behind it
     (400, 40, 130, 1, {}),                                           # one row a tile
     # half-size tiles, the keys in two halves: first chunks
     (0, 1031, 32, 8, dict(block_tokens=24)),                         # 33 tiles of keys: the odd half ends a pass earlier; a last tile of seven rows

@@ -104,20 +104,21 @@ def test_the_workspace_size_names_the_plan_of_every_stage():
             assert record_layout(args) == want, (stages, size)
 
 
-def run_chunk(case, room, out_dtype=None):
-    """The call with the preferred workspace, or with the least; max_ctx_len is the longest context."""
+def run_chunk(case, room, out_dtype=None, hint=False):
+    """The call with the preferred workspace, or with the least; max_ctx_len is the longest context, `hint` states the tokens there are."""
     from zllm_amd import capi, ops
 
     weights, form = weight_args(case)
     rows, heads, batch = case["rows"], case["heads"], len(case["lens"])
-    args = chunk_args(heads, rows, int(case["lens"].max()), batch, block_tokens=case["block_tokens"])
+    args = chunk_args(heads, rows, int(case["lens"].max()), batch, block_tokens=case["block_tokens"],
+                      total_ctx_tokens=int(case["lens"].sum()) if hint else 0)
     lib = capi.load()
     need = (lib.zllm_attn_mla_decode_preferred_bytes if room else lib.zllm_attn_mla_decode_workspace_bytes)(C.byref(args))
     assert not room or need > lib.zllm_attn_mla_decode_workspace_bytes(C.byref(args)), "this shape is meant to be staged"
     workspace = torch.full((need + 4096,), 0x7F, dtype=torch.uint8, device="cuda")
     out = ops.mla_decode(to_torch_bf16(case["q_bits"], "cuda"), weights, upload(case["codes"]), upload(case["scales"]), upload(case["rope"]),
                          upload(case["tables"]), upload(case["lens"]), heads, 192, 256, 512, 64, case["block_tokens"], int(case["lens"].max()),
-                         out_dtype=out_dtype or torch.float32, query_rows=rows, workspace=workspace[:need], **form)
+                         out_dtype=out_dtype or torch.float32, query_rows=rows, workspace=workspace[:need], total_ctx_tokens=args.total_ctx_tokens, **form)
     torch.cuda.synchronize()
     assert int(workspace[need:].min()) == int(workspace[need:].max()) == 0x7F, "written past the workspace"
     return out.float().cpu().numpy()
@@ -165,6 +166,18 @@ def rope_score_chunk(heads, rows, length, first_gain, spread):
     scores = np.where(np.arange(length) < length - rows + 1 + np.arange(rows)[:, None, None], scores, -np.inf)
     p = np.exp(scores - scores.max(axis=2, keepdims=True))
     return case, (p / p.sum(axis=2, keepdims=True)) @ latents[:, ::4]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens", [[2600, 901, 700], [1400, 300, 301]])
+def test_ragged_batches_with_the_token_count(lens):
+    """Sequences of unequal lengths whose sum is stated, one of them no longer than its chunk: each split of each sequence where the merges
+    look for it, and the workgroups behind a short one's end write that they have seen nothing."""
+    case = make_mla_chunk_case(21, lens, 300, 16, block_tokens=64)
+    want, _ = oracle_mla_chunk(case)
+    scale = max(1.0, float(np.abs(want).max()))
+    for hint in (True, False):
+        assert_attention_close(run_chunk(case, True, hint=hint) / scale, want / scale, f"lens={lens} hint={hint}")
 
 
 @pytest.mark.gpu
