@@ -233,7 +233,7 @@ def run_mla_prefill(args):
         "pct_of_mfma_peak": round(100.0 * tflops / MFMA_BF16_PEAK_TFLOPS, 2),
         "tokens_per_s": round(rows / (ms_step * 1e-3), 1),
         "stage_ms": {k: round(v, 5) for k, v in stage_ms.items()},
-        "roofline": {"bound": "mfma", "kernel": "mla_partial_ws", "achieved": round(achieved, 1), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
+        "roofline": {"bound": "mfma", "kernel": "mla_partial_staged (mla_stage included)", "achieved": round(achieved, 1), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / MFMA_BF16_PEAK_TFLOPS, 4), "traffic": None, "kernel_ms": round(stage_ms["partial"], 5)},
     }
     if not args.no_cpu_baseline:
