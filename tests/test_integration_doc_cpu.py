@@ -102,3 +102,15 @@ def test_the_parsers_see_the_whole_surface():
     from zllm_amd import capi
 
     assert set(functions) == set(capi.SYMBOLS)
+
+
+def test_the_build_script_names_every_source_and_its_flags():
+    from zllm_amd import build
+
+    text = open(os.path.join(ROOT, "INTEGRATION.md"), encoding="utf-8").read()
+    block = text[text.index("let src = ["):text.index("cc::Build::new()")]
+    assert re.findall(r'"(\w+\.hip)"', block[:block.index("];")]) == build.SOURCES
+    for source, flags in build.SOURCE_FLAGS.items():
+        assert f'if file == "{source}" {{ &[{", ".join(chr(34) + flag + chr(34) for flag in flags)}]' in block
+    readme = open(os.path.join(ROOT, "README.md"), encoding="utf-8").read()
+    assert all(source in readme for source in build.SOURCES)
