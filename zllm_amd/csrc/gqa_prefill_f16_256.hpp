@@ -5,12 +5,12 @@
 // would leave half the device idle.  Its eight waves are four of 32 pairs for even 32-token tiles and four for odd ones, each half with
 // a softmax of its own, and the halves meet once, at the end, in LDS.  So 32x32x16 tiles (a fragment feeds 32 pairs), two waves a SIMD
 // and no exchange in the loop, where gqa_prefill_tiles has eight waves of 16 pairs.
-// 2,048 rows behind 6,144 keys (16 / 8 heads, soft cap 50), a full layer and one of window 1,024 together: 437 -> 391 us a pass, appends
-// included.  Distance from 64 bits (2-norm) there 1.55e-4 -> 1.44e-4 and 6.6e-5 -> 3.4e-5, 64 rows behind 30,000 6.0e-5 -> 2.2e-5.
+// 2,048 rows behind 6,144 keys (16 / 8 heads, soft cap 50), a full layer and one of window 1,024 together: 437 -> 387 us a pass, appends
+// included (382 to 394 by the card).  Distance from 64 bits (2-norm) there 1.55e-4 -> 1.44e-4 and 6.6e-5 -> 3.4e-5, 64 rows behind 30,000 6.0e-5 -> 2.2e-5.
 //
 // What bounds the loop: both waves of a SIMD run the matrix instructions and the vector ALU one after the other and hide little of one behind the
-// other's (46 % and 47 % of the cycles); what hides is what stands between a wave's own matrix instructions: with the exponentials
-// of a tile's second sixteen tokens under the first sixteen's products 407 -> 391.  Tried: the odd half half a pass behind
+// other's (44 % and 50 % of the cycles in the full layer); what hides is what stands between a wave's own matrix instructions: with the exponentials
+// of a tile's second sixteen tokens under the first sixteen's products 407 -> 391, and without spills in the loop (fresh_lane) 391 -> 387.  Tried: the odd half half a pass behind
 // (spills in the loop, 457), raised priority for either phase (level), 64 pairs a wave and one wave a SIMD (70 spills).
 #pragma once
 

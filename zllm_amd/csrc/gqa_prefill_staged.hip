@@ -4,14 +4,15 @@
 // gqa_stage_q8 writes K and V of the call into the workspace as f16 integers (exact), in the order in which the matrix instructions take
 // them, with the f32 scales beside them.  gqa_prefill_staged then moves tiles straight from memory to LDS: no registers, conversions,
 // addresses or LDS stores in its loop, where gqa_prefill_q8 spends a fifth of its vector instructions on them, and every row tile does.
-// 2,048 rows behind 50,000 keys (64 / 8 heads): 4,499 -> 3,666 us a call.  Distance from 64 bits as before (2-norm, scores of deviation 1):
+// 2,048 rows behind 50,000 keys (64 / 8 heads): 4,500 -> 3,840 us a pass, appends included (3,735 on the fastest card met; the kernel 3,710, the
+// staging 69).  Distance from 64 bits as before (2-norm, scores of deviation 1):
 // 1.43e-4 there, 1,000 rows behind 20,000 (32 / 8) 1.51e-4 -> 1.50e-4, 333 behind 3,000 (24 / 8) 1.4e-6 -> 1.2e-6.
 //
-// What bounds the loop: the vector ALU beside the matrix cores, and the power of both: the device holds 2.4 GHz under neither kernel, and
-// falls from 2.25 to 2.0 as the waits go, so that instructions and LDS bytes count even where they are hidden.  Hence
+// What bounds the loop: the vector ALU (68 % of a SIMD's cycles) beside the matrix cores (44 %), and the power of both: of its 2.4 GHz the
+// device holds 2.0 to 2.1, so that instructions and LDS bytes count even where they are hidden.  Hence
 //   32x32x16 tiles: a wave owns 32 pairs and the vector ALU runs beside the matrix cores (with 16x16x32 tiles it hardly does).
 //   Scales come to a lane as two words a tile and are multiplied as lane reads of the row of sixteen (row_lane): read from LDS element by
-//       element they were half of its traffic (16 of 32 reads a tile and wave; 4,105 -> 3,847 us, built without any scales 20 % less).
+//       element they were half of its traffic (16 of 32 reads a tile and wave; 4,105 -> 3,850 us, built without any scales 20 % less).
 //   A tile is sixteen slots of one matrix instruction and the vector instructions that do not wait for it: the keys of the next tile
 //       under the exponentials, the values under the packing and the scaling of the next scores (4,586 -> 4,105 us against scores,
 //       softmax and values one after the other; three workgroups of four such waves on a compute unit, in parts, 4,424).

@@ -1,11 +1,11 @@
 // Split-KV attention of chunked MLA prefill (512 latent + 64 rope columns) over latents that are converted once a call: what it computes is
-// mla_partial_ws (mla_decode.hip), for calls whose workspace has the room (mla_staged_takes).
+// mla_partial_ws (mla_decode.hip), for calls whose workspace asks for it (plan_mla_staged, plan_mla_call in api.hip).
 //
 // mla_stage writes every 32-token tile of the call into the workspace as it is to lie in LDS: the codes as f16 integers (exact), the rope
 // columns as the matrix instructions take them, the group scales in f32 for the scores and in f16 over the tile's exponent window for the
 // values.  mla_partial_staged moves such tiles straight from memory to LDS.
 //
-// 512 rows of 128 heads behind 16,384 keys: 2,855 -> 2,365 us a call (1,060 TFLOP/s in the kernel), 1,000 rows of 16 heads behind 2,000 keys
+// 512 rows of 128 heads behind 16,384 keys: 2,830 to 2,890 -> 2,340 to 2,400 us a call, by the card (1,010 to 1,060 TFLOP/s in the kernel), 1,000 rows of 16 heads behind 2,000 keys
 // 378 -> 167 (a workgroup there is eight rows, where mla_partial_ws is one).  Distance from 64 bits (2-norm), 64 rows of 24 heads behind 30,000
 // keys 1.0e-4 -> 7.5e-5, 200 of 32 (192 / 256) behind 3,000 2.2e-4 -> 1.8e-4.
 //
