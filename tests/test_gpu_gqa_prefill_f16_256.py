@@ -75,7 +75,7 @@ def test_groups(heads, kv_heads, rows):
     run(rows, 600, heads, kv_heads, workspace=False)
 
 
-@pytest.mark.parametrize("window", [200, 256, 511, 512, 1024])  # a row tile of 64 and a window of 512: 575 keys from a tile's first on, in halves
+@pytest.mark.parametrize("window", [200, 256, 300, 511, 512, 1024])  # a row tile of 64 and a window of 512: 575 keys from a tile's first on, in halves
 def test_windows(window):
     run(170, 900, 4, 2, window=window)
     run(300, 0, 4, 2, window=window)
