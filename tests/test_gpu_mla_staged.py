@@ -239,7 +239,7 @@ def test_later_stages_take_up_the_records_of_a_whole_call():
         args.workspace_bytes = size
         workspace.fill_(0xFF)
         outs = []
-        for masks in ((0,), (12,), (3, 12), (1, 2, 4, 8)):
+        for masks in ((0,), (12,), (3, 12), (1, 2, 4, 8), (1, 2 | capi.MLA_WIDE_TILES, 12)):
             out.zero_()
             for mask in masks:
                 args.stage_mask = mask
@@ -256,6 +256,9 @@ def test_later_stages_take_up_the_records_of_a_whole_call():
         # merge and projection are one kernel in a whole call and two stage by stage: f32 sums in another order
         assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
         assert float((outs[3] - outs[0]).norm() / outs[0].norm()) <= 1e-5
+        # the other partial kernels write the same places: an f16 weight is within 2^-11 of its value in
+        # each of the two kernels, so a term of one is within 2^-10 of the other's
+        assert float((outs[4] - outs[0]).norm() / outs[0].norm()) <= 2.0 ** -10
 
 
 @pytest.mark.gpu
